@@ -93,38 +93,53 @@ __device__ __forceinline__ bool teno_cut(double g, double gs) {
     return g - P < E - 0x1p-70 * gs;
 }
 
-// The left reconstruction at a face reads c0..c4 and the mirrored right one
-// c5..c1 (fillScalarWENOStencils<6>, SF_WENO.h:79-98).  Two of the three
-// candidate stencils are the same three nodes on both sides, so their
-// candidate values (the same parabola at the same face) and the
-// second-difference part of their smoothness indicators are formed once;
-// the two final divisions share one reciprocal.  Each side's weights are
-// those of WENO5::weno5_core (SF_WENO5.cpp:42-62) or TENO5::teno5_core
-// (SF_TENO5.cpp:44-92).
+// Reconstruction in differences.  Every candidate value is the upwind node
+// plus a combination of the differences d_k = c_{k+1} - c_k of neighbouring
+// nodes, and every smoothness indicator is a function of them alone, so the
+// functions below take the NS - 1 projected differences of a stencil and
+// return the increments to add to the upwind nodes: the left one to node
+// NS/2 - 1, the right one to node NS/2 (left reads d_0.., the mirrored right
+// side the same differences in reverse).  Against projecting the NS nodes
+// and rebuilding the differences per field this takes a fifth of a WENO5
+// face's FP64 instructions away (721 -> 597 with HLLC) and half of a WENO7
+// face's, and it rounds less: what is rounded is the increment, not the
+// node.  The faces are bound by FP64 issue, so the sweeps follow: a whole
+// 512^3 WENO5/HLLC pass 86.4 -> 79.5 ms, 256^3 WENO7/Rusanov 23.5 -> 14.4,
+// 2048^2 TENO5/HLLC 7.0 -> 6.3 (together with the HLLC flux below).
+//
+// WENO5 / TENO5 indicators, scaled by 4 (exactly) so that the squared first
+// difference needs no factor: b = 13/3 s^2 + f^2 + eps with s the second
+// difference and f the one-sided or central first difference
+// (SF_WENO5.cpp:42-62).  Two of the three second differences of each side
+// belong to the other side too.
 struct PairTerms {
-    double qL0, qR0, Sa, Sb;     // candidates (x6): left S0, right S0, shared
-    double bL[3], bR[3];         // smoothness indicators
+    double fL[3], fR[3];   // first-difference terms of the candidates
+    double bL[3], bR[3];   // 4 (beta + eps)
 };
 
-// The indicators come out as beta + eps: eps enters as the addend of the
-// innermost fused multiply-add of each, so the weights' eps + beta costs no
-// separate addition (eps = 0 gives beta itself).
-__device__ __forceinline__ PairTerms pair_terms(double c0, double c1, double c2, double c3,
-                                                double c4, double c5, double eps) {
+__device__ __forceinline__ PairTerms pair_terms(const double (&d)[5], double eps4) {
     PairTerms t;
-    t.qL0 = 2.0 * c0 - 7.0 * c1 + 11.0 * c2;
-    t.qR0 = 2.0 * c5 - 7.0 * c4 + 11.0 * c3;
-    t.Sa = -c1 + 5.0 * c2 + 2.0 * c3;   // left S1 = right S2
-    t.Sb = 2.0 * c2 + 5.0 * c3 - c4;    // left S2 = right S1
-    constexpr double k = 13.0 / 12.0;
-    const double dB = sq(c1 - 2.0 * c2 + c3);
-    const double dC = sq(c2 - 2.0 * c3 + c4);
-    t.bL[0] = fma(k, sq(c0 - 2.0 * c1 + c2), fma(0.25, sq(c0 - 4.0 * c1 + 3.0 * c2), eps));
-    t.bL[1] = fma(0.25, sq(c1 - c3), fma(k, dB, eps));
-    t.bL[2] = fma(0.25, sq(3.0 * c2 - 4.0 * c3 + c4), fma(k, dC, eps));
-    t.bR[0] = fma(k, sq(c5 - 2.0 * c4 + c3), fma(0.25, sq(c5 - 4.0 * c4 + 3.0 * c3), eps));
-    t.bR[1] = fma(0.25, sq(c4 - c2), fma(k, dC, eps));
-    t.bR[2] = fma(0.25, sq(3.0 * c3 - 4.0 * c2 + c1), fma(k, dB, eps));
+    constexpr double k = 13.0 / 3.0;
+    double s[4], g[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+        s[i] = d[i + 1] - d[i];
+        g[i] = fma(k * s[i], s[i], eps4);
+    }
+    // 3 d1 - d0, d3 - 3 d2, ...: through s, so that the factor is 2, which
+    // the instruction holds (a literal 3 would cost a register move each)
+    t.fL[0] = fma(2.0, d[1], s[0]);
+    t.fL[1] = d[1] + d[2];
+    t.fL[2] = fma(-2.0, d[2], s[2]);
+    t.fR[0] = fma(-2.0, d[3], s[3]);
+    t.fR[1] = d[3] + d[2];
+    t.fR[2] = fma(2.0, d[2], s[1]);
+    t.bL[0] = fma(t.fL[0], t.fL[0], g[0]);
+    t.bL[1] = fma(t.fL[1], t.fL[1], g[1]);
+    t.bL[2] = fma(t.fL[2], t.fL[2], g[2]);
+    t.bR[0] = fma(t.fR[0], t.fR[0], g[3]);
+    t.bR[1] = fma(t.fR[1], t.fR[1], g[2]);
+    t.bR[2] = fma(t.fR[2], t.fR[2], g[1]);
     return t;
 }
 
@@ -138,22 +153,24 @@ __device__ __forceinline__ void div_pair(double a, double b, double c, double d,
     y = c * b * r;
 }
 
+// WENO5::weno5_core (SF_WENO5.cpp:42-62).  With AL = e1 e2, BL = e0 e2,
+// CL = e0 e1 (e = b^2) the weights are (AL, 6 BL, 3 CL) / (AL + 6 BL + 3 CL);
+// the candidates' increments are (5 d1 - 2 d0)/6 = (2 fL0 - d1)/6,
+// (d1 + 2 d2)/6 and (4 d2 - d3)/6, whose factors 6 and 3 cancel those of the
+// weights.
 template <int NR>
-__device__ __forceinline__ void weno5_pair(double c0, double c1, double c2, double c3,
-                                           double c4, double c5, double& left,
-                                           double& right) {
-    const PairTerms t = pair_terms(c0, c1, c2, c3, c4, c5, 1e-6);   // beta + eps
-    const double eL0 = sq(t.bL[0]), eL1 = sq(t.bL[1]), eL2 = sq(t.bL[2]);
-    const double eR0 = sq(t.bR[0]), eR1 = sq(t.bR[1]), eR2 = sq(t.bR[2]);
-    // alpha_k e0 e1 e2 / 10 with d = (0.1, 0.6, 0.3): (1, 6, 3) x the
-    // products of the other two e; the candidates carry a factor 6, so the
-    // denominator is 6 x (A + 6B + 3C)
-    const double AL = eL1 * eL2, BL = eL0 * eL2, CL = eL0 * eL1;
-    const double AR = eR1 * eR2, BR = eR0 * eR2, CR = eR0 * eR1;
-    const double nL = AL * t.qL0 + (6.0 * BL) * t.Sa + (3.0 * CL) * t.Sb;
-    const double nR = AR * t.qR0 + (6.0 * BR) * t.Sb + (3.0 * CR) * t.Sa;
-    div_pair<NR>(nL, 6.0 * AL + 36.0 * BL + 18.0 * CL, nR, 6.0 * AR + 36.0 * BR + 18.0 * CR, left,
-             right);
+__device__ __forceinline__ void weno5_pair(const double (&d)[5], double& left, double& right) {
+    const PairTerms t = pair_terms(d, 4e-6);
+    const double AL = sq(t.bL[1] * t.bL[2]), BL = sq(t.bL[0] * t.bL[2]), CL = sq(t.bL[0] * t.bL[1]);
+    const double AR = sq(t.bR[1] * t.bR[2]), BR = sq(t.bR[0] * t.bR[2]), CR = sq(t.bR[0] * t.bR[1]);
+    constexpr double s6 = 1.0 / 6.0, s3 = 1.0 / 3.0;
+    const double h2 = 0.5 * d[2];
+    const double nL = fma(AL, fma(s3, t.fL[0], -s6 * d[1]),
+                          fma(BL, t.fL[1] + d[2], CL * fma(-0.5, t.fL[2], h2)));
+    const double nR = fma(AR, fma(s3, t.fR[0], s6 * d[3]),
+                          -fma(BR, t.fR[1] + d[2], CR * fma(0.5, t.fR[2], h2)));
+    const double dL = fma(3.0, CL, fma(6.0, BL, AL)), dR = fma(3.0, CR, fma(6.0, BR, AR));
+    div_pair<NR>(nL, dL, nR, dR, left, right);
 }
 
 // TENO5's stencil selection (SF_TENO5.cpp:60-89): gamma_k = (1 + tau5 /
@@ -162,20 +179,20 @@ __device__ __forceinline__ void weno5_pair(double c0, double c1, double c2, doub
 // quotients change a result only where a ratio lies within rounding of the
 // cutoff.  Returns false where the sum of the gammas is not finite, which
 // the reference treats as fatal (requireFiniteGammaSum, SF_TENO5.cpp:33-40).
+// b[k] = 4 (beta_k + 1e-40): the factor cancels in the quotients.
 __device__ __forceinline__ bool teno5_weights(const double b[3], double& c0, double& c1,
                                               double& c2) {
     const double tau5 = fabs(b[0] - b[2]);
-    // tau5 / e_k for the three k from one reciprocal of e0 e1 e2 (each
-    // e_k >= 1e-40, so the product stays far above the subnormal range)
-    const double e0 = b[0] + 1.0e-40, e1 = b[1] + 1.0e-40, e2 = b[2] + 1.0e-40;
-    const double e01 = e0 * e1;
-    const double t = tau5 * frcp(e01 * e2);
+    // tau5 / b_k for the three k from one reciprocal of b0 b1 b2 (each
+    // b_k >= 4e-40, so the product stays far above the subnormal range)
+    const double e01 = b[0] * b[1];
+    const double t = tau5 * frcp(e01 * b[2]);
     auto p6 = [](double x) {   // three products: within a few ulps of x^6
         const double x3 = x * x * x;
         return x3 * x3;
     };
-    const double g0 = p6(1.0 + t * (e1 * e2));
-    const double g1 = p6(1.0 + t * (e0 * e2));
+    const double g0 = p6(1.0 + t * (b[1] * b[2]));
+    const double g1 = p6(1.0 + t * (b[0] * b[2]));
     const double g2 = p6(1.0 + t * e01);
     const double gs = g0 + g1 + g2;
     c0 = teno_cut(g0, gs) ? 0.0 : 1.0;
@@ -184,121 +201,97 @@ __device__ __forceinline__ bool teno5_weights(const double b[3], double& c0, dou
     return gs < INFINITY;
 }
 
-__device__ __forceinline__ void teno5_pair(double c0, double c1, double c2, double c3,
-                                           double c4, double c5, double& left, double& right,
+// The kept candidates' linear weights (0.1, 0.6, 0.3), scaled by 10, times
+// the increments as in weno5_pair.
+__device__ __forceinline__ void teno5_pair(const double (&d)[5], double& left, double& right,
                                            unsigned& flags) {
-    const PairTerms t = pair_terms(c0, c1, c2, c3, c4, c5, 0.0);
+    const PairTerms t = pair_terms(d, 4e-40);
     double l0, l1, l2, r0, r1, r2;
     const bool fin = teno5_weights(t.bL, l0, l1, l2) & teno5_weights(t.bR, r0, r1, r2);
-    const double aL = 0.1 * l0 + 0.6 * l1 + 0.3 * l2;
-    const double aR = 0.1 * r0 + 0.6 * r1 + 0.3 * r2;
+    const double aL = fma(3.0, l2, fma(6.0, l1, l0));
+    const double aR = fma(3.0, r2, fma(6.0, r1, r0));
     if (!fin || !(aL > 0.0) || !(aR > 0.0)) flags |= kFlagTeno;
-    const double nL = 0.1 * l0 * t.qL0 + 0.6 * l1 * t.Sa + 0.3 * l2 * t.Sb;
-    const double nR = 0.1 * r0 * t.qR0 + 0.6 * r1 * t.Sb + 0.3 * r2 * t.Sa;
-    div_pair(nL, 6.0 * aL, nR, 6.0 * aR, left, right);
+    constexpr double s6 = 1.0 / 6.0, s3 = 1.0 / 3.0;
+    const double h2 = 0.5 * d[2];
+    const double nL = fma(l0, fma(s3, t.fL[0], -s6 * d[1]),
+                          fma(l1, t.fL[1] + d[2], l2 * fma(-0.5, t.fL[2], h2)));
+    const double nR = fma(r0, fma(s3, t.fR[0], s6 * d[3]),
+                          -fma(r1, t.fR[1] + d[2], r2 * fma(0.5, t.fR[2], h2)));
+    div_pair(nL, aL, nR, aR, left, right);
 }
 
-// WENO3::weno3_core (SF_WENO3.cpp:42-57) on both sides of a face: the left
-// side reads c0..c3 and the right one c3..c0 (fillScalarWENOStencils<4>,
-// SF_WENO.h:79-98).  The right side's two candidates and smoothness
-// indicators are the left side's, exchanged, so each is formed once; the
-// weights are those of the reference, normalised with one division per
-// side (alpha_k = d_k / e_k multiplied through by e_A e_B) and the two
-// divisions share one reciprocal.
+// WENO3::weno3_core (SF_WENO3.cpp:42-57) on both sides of a face.  The two
+// candidates and the two squared spreads serve both sides; the weights are
+// normalised with one division per side (alpha_k = d_k / e_k multiplied
+// through by 3 e_A e_B) and the two divisions share one reciprocal.
 template <int NR>
-__device__ __forceinline__ void weno3_pair(const double c[4], double& left, double& right) {
-    const double A = -c[0] + 5.0 * c[1] + 2.0 * c[2];   // 6 x left S0 = right S1
-    const double B = 2.0 * c[1] + 5.0 * c[2] - c[3];    // 6 x left S1 = right S0
+__device__ __forceinline__ void weno3_pair(const double (&d)[3], double& left, double& right) {
     const double eps = 1e-6;
-    const double eA = sq(fma(c[2] - c[0], c[2] - c[0], eps));
-    const double eB = sq(fma(c[3] - c[1], c[3] - c[1], eps));
-    const double d0 = 1.0 / 3.0, d1 = 2.0 / 3.0;
-    const double nL = d0 * eB * A + d1 * eA * B, nR = d0 * eA * B + d1 * eB * A;
-    const double sL = d0 * eB + d1 * eA, sR = d0 * eA + d1 * eB;
-    div_pair<NR>(nL, 6.0 * sL, nR, 6.0 * sR, left, right);
+    const double fA = d[0] + d[1], fB = d[1] + d[2];
+    const double eA = sq(fma(fA, fA, eps)), eB = sq(fma(fB, fB, eps));
+    // 6 x increments: candidates A and B from node 1 (left), node 2 (right)
+    const double AL = fma(2.0, d[1], d[0]), BL = fma(4.0, d[1], -d[2]);
+    const double AR = fma(-4.0, d[1], d[0]), BR = fma(-2.0, d[1], -d[2]);
+    const double e2A = 2.0 * eA, e2B = 2.0 * eB;
+    const double nL = fma(eB, AL, e2A * BL), nR = fma(eA, BR, e2B * AR);
+    div_pair<NR>(nL, 6.0 * (eB + e2A), nR, 6.0 * (eA + e2B), left, right);
 }
 
-// Smoothness of one four-node WENO7 candidate over the cell [a, b] of its
-// local coordinate, as beta4 (SF_WENO7.cpp:43-68) forms it: the integral
-// of the squared first, second and third derivatives of the cubic with
-// forward differences d1, 2 d2, 6 d3.  b - a = 1 for every candidate, and
-// the second-derivative coefficients D = 2 d2 - 6 d3, E = 6 d3 of the
-// reference equal B and 2 C.
-struct W7Interval {
-    double i2, i3, i4, i5;   // F(b) - F(a) for x^2, x^3/3, x^4/2, x^5/5
-};
-
-constexpr W7Interval w7_interval(double a, double b) {
-    return {b * b - a * a, b * b * b / 3.0 - a * a * a / 3.0,
-            (b * b) * (b * b) / 2.0 - (a * a) * (a * a) / 2.0,
-            b * b * b * b * b / 5.0 - a * a * a * a * a / 5.0};
-}
-
-// Returns beta + eps, eps added inside the last fused multiply-add.
-__device__ __forceinline__ double w7_beta(double v0, double v1, double v2, double v3,
-                                          const W7Interval& I, double eps) {
-    const double d1 = v1 - v0;
-    const double d2 = (v2 - 2.0 * v1 + v0) * 0.5;
-    const double d3 = (v3 - 3.0 * v2 + 3.0 * v1 - v0) * (1.0 / 6.0);
-    const double A = d1 - d2 + 2.0 * d3;
-    const double B = 2.0 * d2 - 6.0 * d3;
-    const double C = 3.0 * d3;
-    const double E = 2.0 * C;
-    const double beta1 = A * A + A * B * I.i2 + (B * B + 2.0 * A * C) * I.i3 + B * C * I.i4 +
-                         C * C * I.i5;
-    const double beta2 = B * B + B * E * I.i2 + E * E * I.i3;
-    const double beta3 = fma(36.0 * d3, d3, eps);
-    return beta1 + beta2 + beta3;
-}
-
-// WENO7::weno7_core (SF_WENO7.cpp:70-98) on both sides of a face: left
-// reads c0..c6, right c7..c1 (fillScalarWENOStencils<8>).  Three of the
-// four candidates of each side are candidates of the other side too (the
-// same four nodes in reverse, the same polynomial at the same face), so
-// five candidate values are formed; the smoothness intervals differ
-// between the sides (each side's target cell is its own upwind node), so
-// all eight indicators are formed.  Each side's weights are normalised
-// with one division (alpha_k = d_k / e_k multiplied through by the
-// product of the four e_j) and the two divisions share one reciprocal.
-__device__ __forceinline__ void weno7_side_weights(const double b[4], double w[4]) {
-    constexpr double d0 = 1.0 / 35.0, d1 = 12.0 / 35.0, d2 = 18.0 / 35.0, d3 = 4.0 / 35.0;
-    // b[k] = beta_k + eps (w7_beta)
-    const double e0 = sq(b[0]), e1 = sq(b[1]);
-    const double e2 = sq(b[2]), e3 = sq(b[3]);
+// WENO7::weno7_core (SF_WENO7.cpp:43-98) on both sides of a face.  The
+// indicator of a four-node candidate over its target cell (beta4: the
+// integral of the squared first, second and third derivatives of the
+// cubic), written about the cell's centre, is a sum of three squares,
+//   beta = G^2 + 13/12 B^2 + 781/720 t^2,
+// with t the candidate's third difference, B its second derivative at the
+// centre (a second difference, or one extrapolated by t) and G its first
+// derivative there plus t/24: for the target cell between differences d_l
+// and d_r (d_l to its left),
+//   d_l + s/2 + 3/8 t   outermost upwind candidate (s, t its last ones)
+//   (d_l + d_r)/2 - t/8 the two candidates around the cell
+//   d_r - s/2 + 3/8 t   outermost downwind candidate (s, t its first ones).
+// This takes 52 operations for the eight indicators of a field against
+// about 240 for the polynomial form.  The weights (1, 12, 18, 4) / e_k are
+// multiplied through by the product of the four e and normalised with one
+// division per side; the two divisions share one reciprocal.
+__device__ __forceinline__ void weno7_side(const double b[4], double q0, double q1, double q2,
+                                           double q3, double& num, double& den) {
+    const double e0 = sq(b[0]), e1 = sq(b[1]), e2 = sq(b[2]), e3 = sq(b[3]);
     const double e01 = e0 * e1, e23 = e2 * e3;
-    w[0] = d0 * (e1 * e23);
-    w[1] = d1 * (e0 * e23);
-    w[2] = d2 * (e01 * e3);
-    w[3] = d3 * (e01 * e2);
+    const double w1 = 12.0 * e0, w2 = 18.0 * e3, w3 = 4.0 * e2;
+    num = fma(e23, fma(e1, q0, w1 * q1), e01 * fma(w2, q2, w3 * q3));
+    den = fma(e23, e1 + w1, e01 * (w2 + w3));
 }
 
-__device__ __forceinline__ void weno7_pair(const double c[8], double& left, double& right) {
-    constexpr W7Interval I0 = w7_interval(2.5, 3.5), I1 = w7_interval(1.5, 2.5);
-    constexpr W7Interval I2 = w7_interval(0.5, 1.5), I3 = w7_interval(-0.5, 0.5);
-    // 12 x candidates: left S0, the shared ones (left S1 = right S3, left
-    // S2 = right S2, left S3 = right S1), right S0
-    const double L0 = -3.0 * c[0] + 13.0 * c[1] - 23.0 * c[2] + 25.0 * c[3];
-    const double P1 = c[1] - 5.0 * c[2] + 13.0 * c[3] + 3.0 * c[4];
-    const double P2 = -c[2] + 7.0 * c[3] + 7.0 * c[4] - c[5];
-    const double P3 = 3.0 * c[3] + 13.0 * c[4] - 5.0 * c[5] + c[6];
-    const double R0 = -3.0 * c[7] + 13.0 * c[6] - 23.0 * c[5] + 25.0 * c[4];
-    constexpr double eps = 1e-6;
-    double bL[4], bR[4];
-    bL[0] = w7_beta(c[0], c[1], c[2], c[3], I0, eps);
-    bL[1] = w7_beta(c[1], c[2], c[3], c[4], I1, eps);
-    bL[2] = w7_beta(c[2], c[3], c[4], c[5], I2, eps);
-    bL[3] = w7_beta(c[3], c[4], c[5], c[6], I3, eps);
-    bR[0] = w7_beta(c[7], c[6], c[5], c[4], I0, eps);
-    bR[1] = w7_beta(c[6], c[5], c[4], c[3], I1, eps);
-    bR[2] = w7_beta(c[5], c[4], c[3], c[2], I2, eps);
-    bR[3] = w7_beta(c[4], c[3], c[2], c[1], I3, eps);
-    double wL[4], wR[4];
-    weno7_side_weights(bL, wL);
-    weno7_side_weights(bR, wR);
-    const double nL = wL[0] * L0 + wL[1] * P1 + wL[2] * P2 + wL[3] * P3;
-    const double nR = wR[0] * R0 + wR[1] * P3 + wR[2] * P2 + wR[3] * P1;
-    div_pair(nL, 12.0 * (wL[0] + wL[1] + wL[2] + wL[3]), nR,
-             12.0 * (wR[0] + wR[1] + wR[2] + wR[3]), left, right);
+__device__ __forceinline__ void weno7_pair(const double (&d)[7], double& left, double& right) {
+    constexpr double k2 = 13.0 / 12.0, k3 = 781.0 / 720.0, eps = 1e-6;
+    double s[6], t[5], T[5];
+#pragma unroll
+    for (int i = 0; i < 6; ++i) s[i] = d[i + 1] - d[i];
+#pragma unroll
+    for (int i = 0; i < 5; ++i) {
+        t[i] = s[i + 1] - s[i];
+        T[i] = fma(k3 * t[i], t[i], eps);
+    }
+    auto beta = [](double G, double B, double Tt) { return fma(G, G, fma(k2 * B, B, Tt)); };
+    const double DL = 0.5 * (d[2] + d[3]), DR = 0.5 * (d[3] + d[4]);
+    double bL[4], bR[4];   // beta + eps
+    bL[0] = beta(fma(0.5, s[1], fma(0.375, t[0], d[2])), s[1] + t[0], T[0]);
+    bL[1] = beta(fma(-0.125, t[1], DL), s[2], T[1]);
+    bL[2] = beta(fma(-0.125, t[2], DL), s[2], T[2]);
+    bL[3] = beta(fma(-0.5, s[3], fma(0.375, t[3], d[3])), s[3] - t[3], T[3]);
+    bR[0] = beta(fma(-0.5, s[4], fma(0.375, t[4], d[4])), s[4] - t[4], T[4]);
+    bR[1] = beta(fma(-0.125, t[3], DR), s[3], T[3]);
+    bR[2] = beta(fma(-0.125, t[2], DR), s[3], T[2]);
+    bR[3] = beta(fma(0.5, s[2], fma(0.375, t[1], d[3])), s[2] + t[1], T[1]);
+    // 12 x increments of the candidates: the outermost ones, and the three
+    // that both sides use, from node 3 (left) and node 4 (right)
+    const double L0 = fma(13.0, d[2], fma(-10.0, d[1], 3.0 * d[0]));
+    const double R0 = fma(-13.0, d[4], fma(10.0, d[5], -3.0 * d[6]));
+    const double p1 = fma(4.0, d[2], -d[1]), p2 = d[2] - d[4], p3 = fma(-4.0, d[4], d[5]);
+    double nL, nR, dL, dR;
+    weno7_side(bL, L0, fma(3.0, d[3], p1), fma(6.0, d[3], p2), fma(9.0, d[3], p3), nL, dL);
+    weno7_side(bR, R0, fma(-3.0, d[3], p3), fma(-6.0, d[3], p2), fma(-9.0, d[3], p1), nR, dR);
+    div_pair(nL, 12.0 * dL, nR, 12.0 * dR, left, right);
 }
 
 // Scheme ids (SF_SCHEME_*) and their stencils (SF_stencil.h:12-17):
@@ -315,12 +308,12 @@ template <> struct Stencil<2> { static constexpr int ns = 4, newton = 1; };
 template <> struct Stencil<3> { static constexpr int ns = 8, newton = 2; };
 
 template <int SCHEME, int NR>
-__device__ __forceinline__ void recon_pair(const double (&ch)[Stencil<SCHEME>::ns], double& left,
+__device__ __forceinline__ void recon_pair(const double (&d)[Stencil<SCHEME>::ns - 1], double& left,
                                            double& right, unsigned& flags) {
-    if constexpr (SCHEME == 1) teno5_pair(ch[0], ch[1], ch[2], ch[3], ch[4], ch[5], left, right, flags);
-    else if constexpr (SCHEME == 2) weno3_pair<NR>(ch, left, right);
-    else if constexpr (SCHEME == 3) weno7_pair(ch, left, right);
-    else weno5_pair<NR>(ch[0], ch[1], ch[2], ch[3], ch[4], ch[5], left, right);
+    if constexpr (SCHEME == 1) teno5_pair(d, left, right, flags);
+    else if constexpr (SCHEME == 2) weno3_pair<NR>(d, left, right);
+    else if constexpr (SCHEME == 3) weno7_pair(d, left, right);
+    else weno5_pair<NR>(d, left, right);
 }
 
 // Closure of SingleFluidStateModel::close + PerfectGasEOS
@@ -334,14 +327,12 @@ struct Closed {
 template <int NR = 2>
 __device__ __forceinline__ Closed close_state_r(const double q[5], double gamma, double inv_rho) {
     Closed s;
-    const double rho = q[0];
     s.inv_rho = inv_rho;
     s.u[0] = q[1] * s.inv_rho;
     s.u[1] = q[2] * s.inv_rho;
     s.u[2] = q[3] * s.inv_rho;
-    const double kinetic = 0.5 * rho * (s.u[0] * s.u[0] + s.u[1] * s.u[1] + s.u[2] * s.u[2]);
-    const double e = (q[4] - kinetic) * s.inv_rho;
-    s.p = (gamma - 1.0) * rho * e;
+    const double mu = q[1] * s.u[0] + q[2] * s.u[1] + q[3] * s.u[2];
+    s.p = (gamma - 1.0) * fma(-0.5, mu, q[4]);
     s.c = fsqrt<NR>(gamma * s.p * s.inv_rho);
     return s;
 }
@@ -351,6 +342,11 @@ __device__ __forceinline__ Closed close_state(const double q[5], double gamma) {
     return close_state_r<NR>(q, gamma, frcp<NR>(q[0]));
 }
 
+// Whether x is positive and finite: one class test (positive subnormal or
+// normal) instead of two comparisons.
+__device__ __forceinline__ bool positive_finite(double x) {
+    return __builtin_amdgcn_class(x, 0x180);
+}
 
 // The closure's validity test, as PerfectGasEOS::fromDensityEnergy makes
 // it on each face state the Rusanov flux closes (SF_perfectGasEOS.h:26-33
@@ -359,18 +355,7 @@ __device__ __forceinline__ Closed close_state(const double q[5], double gamma) {
 // when p is): the reference stops on a face whose reconstructed state
 // fails it.
 __device__ __forceinline__ bool closed_ok(const double q[5], const Closed& s) {
-    return q[0] > 0.0 && q[0] < INFINITY && s.p > 0.0 && s.p < INFINITY;
-}
-
-// physicalFlux (SF_rusanovEOS.cpp:14-32) for n = e_ND.
-template <int ND>
-__device__ __forceinline__ void physical_flux(const double q[5], const Closed& s,
-                                              double f[5]) {
-    const double un = s.u[ND];
-    f[0] = q[0] * un;
-#pragma unroll
-    for (int d = 0; d < 3; ++d) f[1 + d] = (d == ND) ? q[1 + d] * un + s.p : q[1 + d] * un;
-    f[4] = (q[4] + s.p) * un;
+    return positive_finite(q[0]) && positive_finite(s.p);
 }
 
 // RusanovEOS::faceFlux, SF_rusanovEOS.cpp:47-77.
@@ -379,19 +364,35 @@ __device__ __forceinline__ void rusanov(const double qL[5], const double qR[5],
                                         double gamma, double out[5], unsigned& flags) {
     const Closed l = close_state<NR>(qL, gamma), r = close_state<NR>(qR, gamma);
     if (!closed_ok(qL, l) || !closed_ok(qR, r)) flags |= kFlagFlux;
-    double fL[5], fR[5];
-    physical_flux<ND>(qL, l, fL);
-    physical_flux<ND>(qR, r, fR);
-    const double lambda = fmax(fabs(l.u[ND]) + l.c, fabs(r.u[ND]) + r.c);
+    // (F(qL) + F(qR) - lambda (qR - qL)) / 2 with F the physical flux
+    // (physicalFlux, SF_rusanovEOS.cpp:14-32), whose mass component is the
+    // normal momentum
+    const double unL = l.u[ND], unR = r.u[ND];
+    const double lambda = fmax(fabs(unL) + l.c, fabs(unR) + r.c);
+    out[0] = 0.5 * fma(-lambda, qR[0] - qL[0], qL[1 + ND] + qR[1 + ND]);
 #pragma unroll
-    for (int v = 0; v < 5; ++v)
-        out[v] = 0.5 * (fL[v] + fR[v]) - 0.5 * lambda * (qR[v] - qL[v]);
+    for (int d = 0; d < 3; ++d) {
+        double f = fma(qR[1 + d], unR, qL[1 + d] * unL);
+        if (d == ND) f += l.p + r.p;
+        out[1 + d] = 0.5 * fma(-lambda, qR[1 + d] - qL[1 + d], f);
+    }
+    out[4] = 0.5 * fma(-lambda, qR[4] - qL[4], fma(qR[4] + r.p, unR, (qL[4] + l.p) * unL));
 }
 
 // HLLC (no reference counterpart).  Toro, "Riemann Solvers and Numerical
 // Methods for Fluid Dynamics", 3rd ed.: Einfeldt wave speeds from Roe
 // averages, contact speed eq. (10.37), star states eq. (10.39) with the
 // tangential velocity of each side carried unchanged, flux eq. (10.38).
+//
+// The flux of eq. (10.38) through the star region of side K is the physical
+// flux of its star state moving with the contact: with a = S_K - u_K,
+// g = S - u_K, S the contact speed,
+//   rho* = rho_K a / (S_K - S),  p* = p_K + rho_K a g,
+//   E* = (a E_K - p_K u_K + p* S) / (S_K - S),
+//   F = (rho* S, rho* S u + p* n, (E* + p*) S).
+// The same formulas at S = u_K give side K's own physical flux, which is
+// what the two supersonic regions take, so one choice of S serves all four
+// regions and only side K's values are selected.
 template <int ND, int NR = 2>
 __device__ __forceinline__ void hllc(const double qL[5], const double qR[5],
                                      double gamma, double out[5], unsigned& flags) {
@@ -414,33 +415,27 @@ __device__ __forceinline__ void hllc(const double qL[5], const double qR[5],
     const double SR = fmax(unR + r.c, ut[ND] + ct);
     const double mL = qL[0] * (SL - unL), mR = qR[0] * (SR - unR);
     const double Ss = fdiv<NR>(r.p - l.p + unL * mL - unR * mR, mL - mR);
-    // One side's physical flux serves all three regions: the left state's
-    // where the fan leaves the face to the right (0 <= S_L) or the contact
-    // does (0 <= S*), the right state's otherwise; the star correction
-    // applies between the outer waves only.
+    // The left side where the fan leaves the face to the right (0 <= S_L) or
+    // the contact does (0 <= S*), the right side otherwise.
     const bool supL = 0.0 <= SL, supR = SR <= 0.0;
     const bool left = supL || (!supR && 0.0 <= Ss);
-    double q[5];
-#pragma unroll
-    for (int v = 0; v < 5; ++v) q[v] = left ? qL[v] : qR[v];
-    const Closed& s = left ? l : r;
+    constexpr int t1 = ND == 0 ? 1 : 0, t2 = ND == 2 ? 1 : 2;
+    const double E = left ? qL[4] : qR[4];
+    const double p = left ? l.p : r.p;
     const double un = left ? unL : unR;
+    const double ut1 = left ? l.u[t1] : r.u[t1], ut2 = left ? l.u[t2] : r.u[t2];
     const double SK = left ? SL : SR;
     const double mK = left ? mL : mR;
-    double f[5];
-    physical_flux<ND>(q, s, f);
-    // scale = mK / (SK - Ss); the pressure term p / mK * scale = p / (SK - Ss)
-    const double rs = frcp<NR>(SK - Ss);
-    const double scale = mK * rs;
-    double us[5];
-    us[0] = scale;
-#pragma unroll
-    for (int d = 0; d < 3; ++d)
-        us[1 + d] = scale * ((d == ND) ? s.u[d] + (Ss - un) : s.u[d]);
-    us[4] = scale * (q[4] * s.inv_rho + (Ss - un) * Ss) + (Ss - un) * (s.p * rs);
-    const bool star = !supL && !supR;
-#pragma unroll
-    for (int v = 0; v < 5; ++v) out[v] = star ? f[v] + SK * (us[v] - q[v]) : f[v];
+    const double S = (supL || supR) ? un : Ss;
+    const double rs = frcp<NR>(SK - S);
+    const double ps = fma(mK, S - un, p);
+    const double Es = rs * fma(SK - un, E, fma(ps, S, -p * un));
+    const double m = mK * rs * S;
+    out[0] = m;
+    out[1 + ND] = fma(m, S, ps);
+    out[1 + t1] = m * ut1;
+    out[1 + t2] = m * ut2;
+    out[4] = (Es + ps) * S;
 }
 
 // Pressure as Numerics::pressure forms it (SF_utility.h:24-29), the form
@@ -550,18 +545,19 @@ __device__ __forceinline__ void euler_flux(const double q[5], const Legacy& s, d
 // form used by the projections below.
 template <int AXIS, int NR = 2>
 struct CharBasis {
-    double u[3], hq2, c, H, un, ul, um, b2, x1;
+    double u[3], hq2, c, H, un, ul, um, b2, x1, xn, cn;
 
+    // q may carry any common factor: the basis depends on ratios only.
     __device__ __forceinline__ CharBasis(const double q[5], double gamma, unsigned& flags) {
         using B = Basis<AXIS>;
         const double invR = frcp<NR>(q[0]);
-        const double ke = 0.5 * (q[1] * q[1] + q[2] * q[2] + q[3] * q[3]) * invR;
-        const double p = (gamma - 1.0) * (q[4] - ke);
-        if (!(q[0] > 0.0) || !(p > 0.0)) flags |= kFlagChar;
         u[0] = q[1] * invR;
         u[1] = q[2] * invR;
         u[2] = q[3] * invR;
-        hq2 = 0.5 * (u[0] * u[0] + u[1] * u[1] + u[2] * u[2]);
+        const double ke = 0.5 * (q[1] * u[0] + q[2] * u[1] + q[3] * u[2]);
+        const double p = (gamma - 1.0) * (q[4] - ke);
+        if (!(q[0] > 0.0) || !(p > 0.0)) flags |= kFlagChar;
+        hq2 = ke * invR;
         const double cz = gamma * p * invR;
         const double rc = frsqrt<NR>(cz);
         c = cz * rc;
@@ -571,6 +567,8 @@ struct CharBasis {
         um = B::sm * u[B::mi];
         b2 = 0.5 * ((gamma - 1.0) * (rc * rc));
         x1 = 0.5 * rc;
+        xn = x1 * un;
+        cn = c * un;
     }
 
     // w = L q (gemv5, SF_riemann.h:33-37).  With P = b2 (q2/2 rho - u.m + E)
@@ -580,31 +578,33 @@ struct CharBasis {
     __device__ __forceinline__ void project(const double q[5], double w[5]) const {
         using B = Basis<AXIS>;
         const double r = q[0];
-        const double um_dot = u[0] * q[1] + u[1] * q[2] + u[2] * q[3];
-        const double P = b2 * (hq2 * r - um_dot + q[4]);
-        const double X = x1 * (un * r - q[1 + B::nd]);
-        w[0] = r - 2.0 * P;
-        w[1] = -ul * r + B::sl * q[1 + B::li];
-        w[2] = -um * r + B::sm * q[1 + B::mi];
+        const double e = fma(-u[0], q[1], fma(-u[1], q[2], fma(-u[2], q[3], q[4])));
+        const double P = b2 * fma(hq2, r, e);
+        const double X = fma(xn, r, -x1 * q[1 + B::nd]);
+        w[0] = fma(-2.0, P, r);
+        w[1] = fma(-ul, r, B::sl * q[1 + B::li]);
+        w[2] = fma(-um, r, B::sm * q[1 + B::mi]);
         w[3] = P + X;
         w[4] = P - X;
     }
 
-    // q = R w.  Every column of R carries u in the momentum rows except the
-    // acoustic -+c on the normal and the shear units, so q_m = u q_rho +
-    // (the rest).
-    __device__ __forceinline__ void back(const double w[5], double q[5]) const {
+    // q = base + R w.  Every column of R carries u in the momentum rows
+    // except the acoustic -+c on the normal and the shear units, so
+    // q_m = u q_rho + (the rest).
+    __device__ __forceinline__ void back(const double base[5], const double w[5],
+                                         double q[5]) const {
         using B = Basis<AXIS>;
-        const double r = w[0] + w[3] + w[4];
+        const double sw = w[3] + w[4];
+        const double r = w[0] + sw;
         const double dw = w[4] - w[3];
-        q[0] = r;
+        q[0] = base[0] + r;
 #pragma unroll
         for (int d = 0; d < 3; ++d) {
-            if (d == B::nd) q[1 + d] = u[d] * r + c * dw;
-            else if (d == B::li) q[1 + d] = u[d] * r + B::sl * w[1];
-            else q[1 + d] = u[d] * r + B::sm * w[2];
+            if (d == B::nd) q[1 + d] = fma(u[d], r, fma(c, dw, base[1 + d]));
+            else if (d == B::li) q[1 + d] = fma(u[d], r, fma(B::sl, w[1], base[1 + d]));
+            else q[1 + d] = fma(u[d], r, fma(B::sm, w[2], base[1 + d]));
         }
-        q[4] = hq2 * w[0] + ul * w[1] + um * w[2] + H * (w[3] + w[4]) + (c * un) * dw;
+        q[4] = fma(hq2, w[0], fma(ul, w[1], fma(um, w[2], fma(H, sw, fma(cn, dw, base[4])))));
     }
 };
 
@@ -656,8 +656,9 @@ __device__ __forceinline__ void roe(const double qL[5], const double qR[5], doub
     al[2] *= lam0;
     al[3] *= lam3;
     al[4] *= lam4;
+    const double zero[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
     double dis[5];
-    cb.back(al, dis);
+    cb.back(zero, al, dis);
     double fL[5], fR[5];
     euler_flux<ND>(qL, l, fL);
     euler_flux<ND>(qR, r, fR);
@@ -702,37 +703,60 @@ __device__ __forceinline__ void riemann_flux(const double qL[5], const double qR
 
 // Flux::characteristicWENOFaceFlux<NS> (SF_WENO.h:185-245) on a face of
 // axis AXIS whose cofactor is area * e_AXIS.  st[s][v] holds the stencil
-// nodes at offsets 1-NS/2 .. NS/2 around the face.  Returns the
-// area-weighted flux.
-template <int AXIS, int SCHEME, int FLUX>
-__device__ __forceinline__ void face_flux(const double (&st)[Stencil<SCHEME>::ns][5],
-                                          double gamma, double area, double out[5],
-                                          unsigned& flags, double lw = 0.0) {
+// nodes at offsets 1-NS/2 .. NS/2 around the face; base(side, q) gives the
+// node on the face's left (side 0, st[NS/2-1]) or right (side 1, st[NS/2])
+// once more, after the reconstruction: a caller whose nodes lie in LDS reads
+// them again there, so that no register holds them across the
+// reconstruction.  Returns the area-weighted flux.
+template <int AXIS, int SCHEME, int FLUX, class Base>
+__device__ __forceinline__ void face_flux_from(const double (&st)[Stencil<SCHEME>::ns][5],
+                                               Base base, double gamma, double area,
+                                               double out[5], unsigned& flags, double lw = 0.0) {
     constexpr int NS = Stencil<SCHEME>::ns;
     constexpr int NR = Stencil<SCHEME>::newton;
-    // face average (SF_WENO.h:207-211) and its characteristic basis
+    // the characteristic basis of the face average (SF_WENO.h:207-211), from
+    // twice the average
     double qa[5];
 #pragma unroll
-    for (int v = 0; v < 5; ++v) qa[v] = 0.5 * (st[NS / 2 - 1][v] + st[NS / 2][v]);
+    for (int v = 0; v < 5; ++v) qa[v] = st[NS / 2 - 1][v] + st[NS / 2][v];
     const CharBasis<AXIS, NR> cb(qa, gamma, flags);
-    double ch[5][NS];
+    double ch[5][NS - 1];
 #pragma unroll
-    for (int s = 0; s < NS; ++s) {
-        double w[5];
-        cb.project(st[s], w);
+    for (int s = 0; s < NS - 1; ++s) {
+        double dq[5], w[5];
+#pragma unroll
+        for (int v = 0; v < 5; ++v) dq[v] = st[s + 1][v] - st[s][v];
+        cb.project(dq, w);
 #pragma unroll
         for (int v = 0; v < 5; ++v) ch[v][s] = w[v];
     }
     double wL[5], wR[5];
 #pragma unroll
     for (int v = 0; v < 5; ++v) recon_pair<SCHEME, NR>(ch[v], wL[v], wR[v], flags);
-    double qL[5], qR[5];
-    cb.back(wL, qL);
-    cb.back(wR, qR);
+    double qb[5], qL[5], qR[5];
+    base(0, qb);
+    cb.back(qb, wL, qL);
+    base(1, qb);
+    cb.back(qb, wR, qR);
     double f[5];
     riemann_flux<AXIS, FLUX, NR>(qL, qR, gamma, lw, f, flags);
 #pragma unroll
     for (int v = 0; v < 5; ++v) out[v] = f[v] * area;
+}
+
+// face_flux_from with the two nodes taken from the stencil.
+template <int AXIS, int SCHEME, int FLUX>
+__device__ __forceinline__ void face_flux(const double (&st)[Stencil<SCHEME>::ns][5],
+                                          double gamma, double area, double out[5],
+                                          unsigned& flags, double lw = 0.0) {
+    constexpr int NS = Stencil<SCHEME>::ns;
+    face_flux_from<AXIS, SCHEME, FLUX>(
+        st,
+        [&st](int side, double (&q)[5]) {
+#pragma unroll
+            for (int v = 0; v < 5; ++v) q[v] = st[NS / 2 - 1 + side][v];
+        },
+        gamma, area, out, flags, lw);
 }
 
 }  // namespace sfamd
