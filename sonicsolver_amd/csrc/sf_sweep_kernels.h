@@ -365,9 +365,15 @@ __attribute__((amdgpu_waves_per_eu(3, 8))) void k_sweep_xl(GridDev G, const doub
 constexpr int kMarchBlock = 64;
 
 // The WENO5 ring (10 KB per wave) leaves room for four waves per SIMD; the
-// register count decides how many run: the WENO5 / WENO3 marches with the
-// Rusanov or HLLC flux fit 128 registers and run four, the other fluxes'
-// need a few more and run three (holding them to 128 spills).
+// register count decides how many run: the WENO5, TENO5 and WENO3 marches
+// with the Rusanov or HLLC flux fit 128 registers and run four, the other
+// fluxes' need a few more and run three (holding them to 128 spills).
+// Bound by FP64 issue.  On 512^3 with WENO5/HLLC the z / y march took 4.03 /
+// 4.33 ms; 3.51 / 3.90 with the shorter face arithmetic and the face's two
+// nodes read from the ring again after the reconstruction (120 registers;
+// held across it they cost the fourth wave); 3.41 / 3.71 with the y march's
+// sums requested before the Riemann solver and without the wait for the
+// previous node's stores at the head of the loop.
 template <int AXIS, int SCHEME, int FLUX, int MODE>
 __global__ __launch_bounds__(kMarchBlock)
 void k_sweep_march(GridDev G,
@@ -407,6 +413,11 @@ void k_sweep_march(GridDev G,
         id += (H - 1) * step;  // node a0 - 1
         int head = 0;          // slot of the oldest node
         double fprev[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+        // Pinned, so that the wait for the carried node stands here and not at
+        // the head of the loop, where it would also wait for the stores of
+        // the previous node.
+#pragma unroll
+        for (int v = 0; v < 5; ++v) asm volatile("" : "+v"(carried[v]));
 #pragma clang loop unroll(disable)
         for (int a = a0 - 1; a < a1; ++a, id += step) {
             double st[NS][5];
@@ -426,8 +437,26 @@ void k_sweep_march(GridDev G,
                 carried[v] = st[NS - 1][v];
             }
             head = (head == W - 1) ? 0 : head + 1;
+            // the face's two nodes a and a+1: ring slots H-1 and H of the
+            // window as it was (slots H-2 and H-1 from the new head); for
+            // WENO3, whose ring holds two nodes, the right one is the node
+            // that just entered.  The sum this face's difference is added to
+            // is requested here too, so that the Riemann solver hides its
+            // latency (the node a0 - 1, whose sum goes unused, lies in the
+            // padded grid).
+            double sold[5];
+            const auto base = [&](int side, double (&b)[5]) {
+                if (MODE == kAccumS && side == 0) {
+#pragma unroll
+                    for (int v = 0; v < 5; ++v) sold[v] = S[v * G.P + id];
+                }
+                const int s = H - 2 + side;
+                const int slot = (head + s >= W) ? head + s - W : head + s;
+#pragma unroll
+                for (int v = 0; v < 5; ++v) b[v] = win[slot][v][lane];
+            };
             double f[5];
-            face_flux<AXIS, SCHEME, FLUX>(st, G.gamma, G.area[AXIS], f, flags, lw);
+            face_flux_from<AXIS, SCHEME, FLUX>(st, base, G.gamma, G.area[AXIS], f, flags, lw);
             double s5[5];
 #pragma unroll
             for (int v = 0; v < 5; ++v) {
@@ -435,10 +464,15 @@ void k_sweep_march(GridDev G,
                 s5[v] = f[v] - fprev[v];
                 fprev[v] = f[v];
             }
-            if (a < a0) continue;
+            if (MODE == kAccumS) {
+                // pinned, so that the loads of sold stay where they are
 #pragma unroll
-            for (int v = 0; v < 5; ++v)
-                if (MODE != kCopyS) s5[v] = S[v * G.P + id] + s5[v];
+                for (int v = 0; v < 5; ++v) {
+                    s5[v] = sold[v] + s5[v];
+                    asm volatile("" : "+v"(s5[v]));
+                }
+            }
+            if (a < a0) continue;
 #pragma unroll
             for (int v = 0; v < 5; ++v) S[v * G.P + id] = s5[v];
         }
