@@ -66,6 +66,7 @@ int launch_sweep_fm(const SweepCall& c, int axis) {
             // the tiles.
             // The line walk addresses a lane's stage operands by a 32-bit
             // byte offset of up to one variable (8 P bytes) past the tile.
+            const SweepArgs W{G, c.q, c.S, c.A};
             const long long lines = (long long)G.n[1] * G.n[2];
             const bool fits = (long long)G.P * 8 + 1024 < (1LL << 32);
             const bool by_lines =
@@ -76,7 +77,7 @@ int launch_sweep_fm(const SweepCall& c, int axis) {
                 const long long groups = (lines + kLineGroup - 1) / kLineGroup;
                 const unsigned nb = (unsigned)std::min<long long>(groups, 16384);
 #define SF_LAUNCH_XL(T) \
-    k_sweep_xl<SCHEME, FLUX, T><<<nb, kXBlock, 0, c.stream>>>(G, c.q, c.S, c.A)
+    k_sweep_xl<SCHEME, FLUX, T><<<nb, kXBlock, 0, c.stream>>>(W)
                 switch (c.A.time) {
                 case 0: SF_LAUNCH_XL(0); break;
                 case 1: SF_LAUNCH_XL(1); break;
@@ -92,7 +93,7 @@ int launch_sweep_fm(const SweepCall& c, int axis) {
             const long long tiles = (faces - 1 + kXBlock - 2) / (kXBlock - 1);
 #define SF_LAUNCH_X(T)                                                            \
     k_sweep_x<SCHEME, FLUX, T><<<x_blocks<SCHEME, FLUX, T>(c.cus, tiles), kXBlock, 0, \
-                                c.stream>>>(G, c.q, c.S, c.A)
+                                c.stream>>>(W)
             switch (c.A.time) {
             case 0: SF_LAUNCH_X(0); break;
             case 1: SF_LAUNCH_X(1); break;

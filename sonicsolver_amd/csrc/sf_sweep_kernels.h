@@ -20,6 +20,31 @@ namespace sfamd {
 // ---------------------------------------------------------------------------
 constexpr int kXBlock = 64;
 
+// The x sweeps' arguments, and the wave's own view of them in the kernel
+// argument segment.  A sweep has about 90 uniform values (variable pointers,
+// grid constants, ranges of ghost copies); held across the tile loop they
+// exceed the scalar registers, and each restored one costs a v_readlane in
+// the loop that the FP64 pipe is waiting for (90 of an x line tile's 880
+// vector instructions).  sweep_args() hides where its pointer comes from, so
+// that what is read through it is loaded where it is used, by scalar loads
+// from the constant cache: 880 -> 800 vector instructions per x line tile
+// with WENO5/HLLC.  The 256^3 WENO7/Rusanov x sweep took 919 and takes 779
+// us; the 512^3 WENO5/HLLC one keeps its 4.77 ms, in which it moves 21.7 GB,
+// 95% of the rate of a large copy.
+struct SweepArgs {
+    GridDev G;
+    const double* q;
+    const double* S;
+    StageArgs A;
+};
+
+__device__ __forceinline__ const SweepArgs& sweep_args() {
+    auto p = (const __attribute__((address_space(4))) SweepArgs*)
+        __builtin_amdgcn_kernarg_segment_ptr();
+    asm volatile("" : "+s"(p));
+    return *(const SweepArgs*)p;
+}
+
 // The value of lane t-1 (lane 0 receives 0): one DPP wave shift per 32-bit
 // half, a VALU move with no LDS round trip.
 __device__ __forceinline__ double lane_shift_up1(double x) {
@@ -37,26 +62,29 @@ __device__ __forceinline__ double lane63(double x) {
     return __longlong_as_double(((long long)hi << 32) | (unsigned)lo);
 }
 
-// The final sweep's operands for node id: its current value, the flux
-// difference the y and z sweeps accumulated and its step-start value.  All
-// three are loaded for every lane, without a test: every lane's node index
-// lies in the padded grid (a lane without a node of its own takes node
-// (-1 or 0, j, k)); on a grid without a y axis no sweep writes S, which
-// keeps the zeros it was created with, so its sum is the x difference
-// alone; where the recipe does not read q0 (Euler, the first SSPRK3
-// stage) the values go unused, and there q0 is the stage input itself, so
-// the loads hit the lines the stencil loads bring in.
-template <int TIME>
-__device__ __forceinline__ void stage_operands(const GridDev& G, const StageArgs& A,
-                                               const double* __restrict__ q,
-                                               const double* __restrict__ S, long long id,
-                                               double (&pq)[5], double (&ps)[5],
-                                               double (&pq0)[5]) {
+// The double `nodes` past base + off bytes: a uniform base, a lane's 32-bit
+// byte offset and a constant, which one load instruction takes as they are.
+__device__ __forceinline__ double at(const double* base, unsigned off, int nodes = 0) {
+    return *(const double*)((const char*)base + off + 8 * nodes);
+}
+
+// The final sweep's operands for the node `off` bytes past node id0: its
+// current value, the flux difference the y and z sweeps accumulated and its
+// step-start value.  All three are loaded for every lane, without a test:
+// every lane's node index lies in the padded grid (a lane without a node of
+// its own takes the tile's first); on a grid without a y axis no sweep
+// writes S, which keeps the zeros it was created with, so its sum is the x
+// difference alone; where the recipe does not read q0 (Euler, the first
+// SSPRK3 stage) the values go unused, and there q0 is the stage input
+// itself, so the loads hit the lines the stencil loads bring in.
+__device__ __forceinline__ void stage_operands(long long id0, unsigned off, double (&pq)[5],
+                                               double (&ps)[5], double (&pq0)[5]) {
+    const SweepArgs& W = sweep_args();
 #pragma unroll
     for (int v = 0; v < 5; ++v) {
-        pq[v] = q[v * G.P + id];
-        ps[v] = S[v * G.P + id];
-        pq0[v] = A.q0[v * G.P + id];
+        pq[v] = at(W.q + v * W.G.P + id0, off);
+        ps[v] = at(W.S + v * W.G.P + id0, off);
+        pq0[v] = at(W.A.q0 + v * W.G.P + id0, off);
     }
 }
 
@@ -69,19 +97,18 @@ __device__ __forceinline__ void stage_operands(const GridDev& G, const StageArgs
 // code for the other recipes).
 template <int SCHEME, int FLUX, int TIME>
 __global__ __launch_bounds__(kXBlock)
-__attribute__((amdgpu_waves_per_eu(3, 8))) void k_sweep_x(GridDev G, const double* __restrict__ q,
-                                                     const double* __restrict__ S, StageArgs A) {
-    if (*A.flags) return;   // a fault was raised: keep the step-start state
+__attribute__((amdgpu_waves_per_eu(3, 8))) void k_sweep_x(SweepArgs W) {
+    if (*W.A.flags) return;   // a fault was raised: keep the step-start state
     // face numbers fit 32 bits: the host rejects grids with 2^32 - 2^8
     // faces or more along x
     const int t = threadIdx.x;
-    const unsigned per_line = G.n[0] + 1;
-    const unsigned faces = per_line * G.n[1] * G.n[2];
+    const unsigned per_line = W.G.n[0] + 1;
+    const unsigned faces = per_line * W.G.n[1] * W.G.n[2];
     const unsigned tiles = (faces - 1 + kXBlock - 2) / (kXBlock - 1);
     unsigned flags = 0;
     double dt_local = INFINITY;
-    const double dt_step = TIME == 3 ? 0.0 : *A.dt;   // the step's dt, read once
-    const double lw = (FLUX == 5) ? *A.dt / G.d[0] : 0.0;   // Lax-Wendroff dt / spacing
+    const double dt_step = TIME == 3 ? 0.0 : *W.A.dt;   // the step's dt, read once
+    const double lw = (FLUX == 5) ? *W.A.dt / W.G.d[0] : 0.0;   // Lax-Wendroff dt / spacing
     // Blocks are dealt to the 8 XCDs round-robin (block b runs on XCD b % 8),
     // each with its own L2; tiles are numbered so that the blocks of one XCD
     // take consecutive tiles and share the stencil halo between them in that
@@ -89,6 +116,8 @@ __attribute__((amdgpu_waves_per_eu(3, 8))) void k_sweep_x(GridDev G, const doubl
     const unsigned per_xcd = gridDim.x >> 3;
     const unsigned first = (blockIdx.x & 7u) * per_xcd + (blockIdx.x >> 3);
     for (unsigned T = first; T < tiles; T += gridDim.x) {
+        const SweepArgs& F = sweep_args();
+        const GridDev& G = F.G;
         const unsigned f = T * (kXBlock - 1) + t;
         const bool face = f < faces;
         const unsigned line = face ? fast_div(f, G.div_line) : 0;
@@ -96,23 +125,29 @@ __attribute__((amdgpu_waves_per_eu(3, 8))) void k_sweep_x(GridDev G, const doubl
         const unsigned kz = fast_div(line, G.div_n1);
         const int j = (int)(line - kz * (unsigned)G.n[1]), k = (int)kz;
         double f5[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+        // A tile's nodes lie within a few lines, in ascending order, so a
+        // lane addresses its node by a 32-bit offset from the first lane's.
         // The final sweep's stage operands for the node this lane updates
-        // (the lower node of its face): loaded before the face arithmetic,
-        // so that their latency hides behind it -- except for WENO7, whose
-        // eight-node stencil leaves no registers to hold them at three waves
-        // per SIMD; it loads them after the face.
+        // (the lower node of its face) are loaded before the face
+        // arithmetic, so that their latency hides behind it -- except for
+        // WENO7, whose eight-node stencil leaves no registers to hold them at
+        // three waves per SIMD; it loads them after the face.
         const bool upd = t >= 1 && face && a >= 0;
-        const long long id = node_index(G, a, j, k);
+        const unsigned uid = (unsigned)node_index(G, a, j, k);
+        const unsigned id0 = __builtin_amdgcn_readfirstlane(uid);
+        const unsigned off = face ? (uid - id0) * 8u : 0u;
         double pq[5], ps[5], pq0[5];
         constexpr bool kEarly = SCHEME != 3;
-        if (kEarly) stage_operands<TIME>(G, A, q, S, id, pq, ps, pq0);
+        if (kEarly) stage_operands(id0, off, pq, ps, pq0);
         if (face) {
             constexpr int NS = Stencil<SCHEME>::ns;
             double st[NS][5];
 #pragma unroll
-            for (int s = 0; s < NS; ++s)
+            for (int v = 0; v < 5; ++v) {
+                const double* row = F.q + v * G.P + id0;
 #pragma unroll
-                for (int v = 0; v < 5; ++v) st[s][v] = q[v * G.P + id + (s + 1 - NS / 2)];
+                for (int s = 0; s < NS; ++s) st[s][v] = at(row, off, s + 1 - NS / 2);
+            }
             face_flux<0, SCHEME, FLUX>(st, G.gamma, G.area[0], f5, flags, lw);
             if (!finite_sum5(f5)) flags |= kFlagFlux;
         }
@@ -120,7 +155,9 @@ __attribute__((amdgpu_waves_per_eu(3, 8))) void k_sweep_x(GridDev G, const doubl
 #pragma unroll
         for (int v = 0; v < 5; ++v) lower[v] = lane_shift_up1(f5[v]);
         if (upd) {
-            if (!kEarly) stage_operands<TIME>(G, A, q, S, id, pq, ps, pq0);
+            const SweepArgs& U = F;
+            if (!kEarly) stage_operands(id0, off, pq, ps, pq0);
+            const long long id = uid;
             double s5[5];
 #pragma unroll
             for (int v = 0; v < 5; ++v) {
@@ -129,21 +166,24 @@ __attribute__((amdgpu_waves_per_eu(3, 8))) void k_sweep_x(GridDev G, const doubl
             }
             double dl = INFINITY;
             double qn[5];
-            if (solved_node(G, a, j, k)) {
-                stage_update_dt<TIME>(G, A, id, pq, pq0, s5, dt_step, flags, dl, qn);
+            if (solved_node(U.G, a, j, k)) {
+                stage_update_dt<TIME>(U.G, U.A, id, pq, pq0, s5, dt_step, flags, dl, qn);
             } else if (TIME != 3) {
 #pragma unroll
                 for (int v = 0; v < 5; ++v) {
                     qn[v] = pq[v];   // carry_node
-                    A.qout[v * G.P + id] = qn[v];
+                    U.A.qout[v * U.G.P + id] = qn[v];
                 }
             }
-            if (TIME != 3 && G.images) write_images(G, A.qout, a, j, k, id, qn);
+            if (TIME != 3) {
+                const SweepArgs& V = sweep_args();
+                if (V.G.images) write_images(V.G, V.A.qout, a, j, k, id, qn);
+            }
             dt_local = fmin(dt_local, dl);
         }
     }
-    raise_fault(flags, A.flags, A.fault_tag, A.tag);
-    if (A.reduce_dt) wave_min_atomic(dt_local, A.dtmin);
+    raise_fault(flags, W.A.flags, W.A.fault_tag, W.A.tag);
+    if (W.A.reduce_dt) wave_min_atomic(dt_local, W.A.dtmin);
 }
 
 // ---------------------------------------------------------------------------
@@ -177,17 +217,16 @@ constexpr int kRowLanes = kRow / 2;           // lanes of 16 bytes per row
 
 template <int SCHEME, int FLUX, int TIME>
 __global__ __launch_bounds__(kXBlock)
-__attribute__((amdgpu_waves_per_eu(3, 8))) void k_sweep_xl(GridDev G, const double* __restrict__ q,
-                                                      const double* __restrict__ S, StageArgs A) {
-    if (*A.flags) return;   // a fault was raised: keep the step-start state
+__attribute__((amdgpu_waves_per_eu(3, 8))) void k_sweep_xl(SweepArgs W) {
+    if (*W.A.flags) return;   // a fault was raised: keep the step-start state
     constexpr int NS = Stencil<SCHEME>::ns;
     static_assert(NS / 2 <= kHalo, "the halo covers the stencil");
     __shared__ double first[5][kLineGroup];   // each line's face -1/2
     __shared__ __attribute__((aligned(16))) double qb[2][5][kRow];
     __shared__ __attribute__((aligned(16))) double pk[10][kXBlock];   // S 0-4, q0 5-9
     const int t = threadIdx.x;
-    const int n0 = G.n[0];
-    const unsigned lines = (unsigned)G.n[1] * (unsigned)G.n[2];
+    const int n0 = W.G.n[0];
+    const unsigned lines = (unsigned)W.G.n[1] * (unsigned)W.G.n[2];
     const unsigned groups = (lines + kLineGroup - 1) / kLineGroup;
     const int tiles = (n0 + kXBlock - 1) / kXBlock;
     const int last_needed = n0 - 1 + NS / 2;   // the highest node a stencil reads
@@ -195,11 +234,11 @@ __attribute__((amdgpu_waves_per_eu(3, 8))) void k_sweep_xl(GridDev G, const doub
     // variable of a copy, and of the upper variable (P doubles further;
     // the host keeps 8 P + 1024 below 2^32)
     const int pair = t & 31;
-    const unsigned up = (t >> 5) ? (unsigned)G.P * 8u : 0u;
+    const unsigned up = (t >> 5) ? (unsigned)W.G.P * 8u : 0u;
     unsigned flags = 0;
     double dt_local = INFINITY;
-    const double dt_step = TIME == 3 ? 0.0 : *A.dt;   // the step's dt, read once
-    const double lw = (FLUX == 5) ? *A.dt / G.d[0] : 0.0;   // Lax-Wendroff dt / spacing
+    const double dt_step = TIME == 3 ? 0.0 : *W.A.dt;   // the step's dt, read once
+    const double lw = (FLUX == 5) ? *W.A.dt / W.G.d[0] : 0.0;   // Lax-Wendroff dt / spacing
 
     // the 72 nodes 64m-4 .. 64m+67 of line (j, k), all five variables, into
     // buffer b; lanes 0-35 take two nodes each, a lane whose first node no
@@ -207,12 +246,13 @@ __attribute__((amdgpu_waves_per_eu(3, 8))) void k_sweep_xl(GridDev G, const doub
     // pair is at most one past the last ghost, which every row holds)
     auto fetch_q = [&](int b, int m, int j, int k) {
         if (t < kRowLanes) {
+            const SweepArgs& T = sweep_args();
             const int node0 = m * kXBlock - kHalo;
-            const long long id = node_index(G, node0, j, k);
+            const long long id = node_index(T.G, node0, j, k);
             const unsigned off = (node0 + 2 * t <= last_needed ? (unsigned)t : 0u) * 16u;
 #pragma unroll
             for (int v = 0; v < 5; ++v) {
-                const char* base = (const char*)(q + v * G.P + id);
+                const char* base = (const char*)(T.q + v * T.G.P + id);
                 __builtin_amdgcn_global_load_lds(
                     (__attribute__((address_space(1))) void*)(base + off),
                     (__attribute__((address_space(3))) void*)&qb[b][v][0], 16, 0, 0);
@@ -228,6 +268,9 @@ __attribute__((amdgpu_waves_per_eu(3, 8))) void k_sweep_xl(GridDev G, const doub
     for (unsigned grp = blockIdx.x; grp < groups; grp += gridDim.x) {
         const unsigned line0 = grp * kLineGroup;
         const unsigned nl = min((unsigned)kLineGroup, lines - line0);
+        const SweepArgs& W1 = sweep_args();
+        const GridDev& G = W1.G;
+        const int n1 = G.n[1];
         int j, k;
         {
             const unsigned kz = fast_div(line0, G.div_n1);
@@ -246,7 +289,7 @@ __attribute__((amdgpu_waves_per_eu(3, 8))) void k_sweep_xl(GridDev G, const doub
 #pragma unroll
                 for (int s = 0; s < NS; ++s)
 #pragma unroll
-                    for (int v = 0; v < 5; ++v) st[s][v] = q[v * G.P + id + (s + 1 - NS / 2)];
+                    for (int v = 0; v < 5; ++v) st[s][v] = W1.q[v * G.P + id + (s + 1 - NS / 2)];
                 double f5[5];
                 face_flux<0, SCHEME, FLUX>(st, G.gamma, G.area[0], f5, flags, lw);
                 if (!finite_sum5(f5)) flags |= kFlagFlux;
@@ -265,7 +308,8 @@ __attribute__((amdgpu_waves_per_eu(3, 8))) void k_sweep_xl(GridDev G, const doub
                 const int a = m * kXBlock + t;   // this lane's node
                 const int rem = n0 - m * kXBlock;
                 const bool node = t < rem;
-                const long long id0 = node_index(G, m * kXBlock, j, k);
+                const SweepArgs& T = sweep_args();
+                const long long id0 = node_index(T.G, m * kXBlock, j, k);
                 // the next tile's variables (next line's first tile at the
                 // end of a line, none after the group's last)
                 {
@@ -274,7 +318,7 @@ __attribute__((amdgpu_waves_per_eu(3, 8))) void k_sweep_xl(GridDev G, const doub
                     if (mn == tiles) {
                         mn = 0;
                         more = l + 1 < nl;
-                        if (++jn == G.n[1]) { jn = 0; ++kn; }
+                        if (++jn == n1) { jn = 0; ++kn; }
                     }
                     if (more) fetch_q(b ^ 1, mn, jn, kn);
                 }
@@ -282,12 +326,12 @@ __attribute__((amdgpu_waves_per_eu(3, 8))) void k_sweep_xl(GridDev G, const doub
                 // line's end copies the tile's first two again
                 {
                     const unsigned lo = (unsigned)(2 * pair < rem ? pair : 0) * 16u;
-                    const double* const src[2] = {S, A.q0};
+                    const double* const src[2] = {T.S, T.A.q0};
 #pragma unroll
                     for (int c = 0; c < 6; ++c) {
                         const int arr = c / 3, v = 2 * (c % 3);
                         if (v < 4 || t < 32) {
-                            const char* base = (const char*)(src[arr] + v * G.P + id0);
+                            const char* base = (const char*)(src[arr] + v * T.G.P + id0);
                             const unsigned off = lo + (v < 4 ? up : 0u);
                             __builtin_amdgcn_global_load_lds(
                                 (__attribute__((address_space(1))) void*)(base + off),
@@ -305,7 +349,7 @@ __attribute__((amdgpu_waves_per_eu(3, 8))) void k_sweep_xl(GridDev G, const doub
 #pragma unroll
                     for (int v = 0; v < 5; ++v) st[s][v] = qb[b][v][ti + kHalo + s + 1 - NS / 2];
                 double f5[5];
-                face_flux<0, SCHEME, FLUX>(st, G.gamma, G.area[0], f5, flags, lw);
+                face_flux<0, SCHEME, FLUX>(st, T.G.gamma, T.G.area[0], f5, flags, lw);
                 if (!finite_sum5(f5)) flags |= kFlagFlux;
                 double lower[5];
 #pragma unroll
@@ -316,6 +360,7 @@ __attribute__((amdgpu_waves_per_eu(3, 8))) void k_sweep_xl(GridDev G, const doub
                 }
                 wait_copies();
                 if (node) {
+                    const SweepArgs& U = sweep_args();
                     const long long id = id0 + t;
                     double pq[5], ps[5], pq0[5];
 #pragma unroll
@@ -332,26 +377,29 @@ __attribute__((amdgpu_waves_per_eu(3, 8))) void k_sweep_xl(GridDev G, const doub
                     }
                     double dl = INFINITY;
                     double qn[5];
-                    if (solved_node(G, a, j, k)) {
-                        stage_update_dt<TIME>(G, A, id, pq, pq0, s5, dt_step, flags, dl, qn);
+                    if (solved_node(U.G, a, j, k)) {
+                        stage_update_dt<TIME>(U.G, U.A, id, pq, pq0, s5, dt_step, flags, dl, qn);
                     } else if (TIME != 3) {
 #pragma unroll
                         for (int v = 0; v < 5; ++v) {
                             qn[v] = pq[v];   // carry_node
-                            A.qout[v * G.P + id] = qn[v];
+                            U.A.qout[v * U.G.P + id] = qn[v];
                         }
                     }
-                    if (TIME != 3 && G.images) write_images(G, A.qout, a, j, k, id, qn);
+                    if (TIME != 3) {
+                        const SweepArgs& V = sweep_args();
+                        if (V.G.images) write_images(V.G, V.A.qout, a, j, k, id, qn);
+                    }
                     dt_local = fmin(dt_local, dl);
                 }
                 b ^= 1;
             }
-            if (++j == G.n[1]) { j = 0; ++k; }
+            if (++j == n1) { j = 0; ++k; }
         }
         __syncthreads();
     }
-    raise_fault(flags, A.flags, A.fault_tag, A.tag);
-    if (A.reduce_dt) wave_min_atomic(dt_local, A.dtmin);
+    raise_fault(flags, W.A.flags, W.A.fault_tag, W.A.tag);
+    if (W.A.reduce_dt) wave_min_atomic(dt_local, W.A.dtmin);
 }
 
 // ---------------------------------------------------------------------------
