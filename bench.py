@@ -570,9 +570,13 @@ def main():
     final = axis == 0  # the x sweep applies the stage update
     fl = flops.sweep_flops((n, n, n), axis, scheme, flux, final=final, dim=3, time=tscheme,
                            fold_dt=1.0 / 3.0 if final else 0.0)
+    fused = prof["sweep_y"][1] == 0   # the y faces run in the x sweep's launch
+    if final and fused:
+        fl += flops.sweep_flops((n, n, n), 1, scheme, flux, final=False, dim=3, time=tscheme)
     achieved_tf = fl / (avg_ms * 1e-3) / 1e12
-    kernel_names = {"sweep_x": "the x sweep: k_sweep_xl on grids with many x lines (512^3), "
-                               "else k_sweep_x (x faces + stage update + CFL fold)",
+    kernel_names = {"sweep_x": "k_stage_yx (y and x faces + stage update + CFL fold)" if fused
+                    else "the x sweep: k_sweep_xl on grids with many x lines, else k_sweep_x "
+                         "(x faces + stage update + CFL fold)",
                     "sweep_y": "k_sweep_march<1> (y faces, accumulates S)",
                     "sweep_z": "k_sweep_march<2> (z faces, writes S)"}
     traffic, traffic_src = traffic_measurement(name)

@@ -200,18 +200,21 @@ int sf_error_flags(sf_grid *grid, uint32_t *flags, int clear);
  * the start or commit of the step, 7 = the CFL scan before it).  Any
  * output may be NULL. */
 int sf_fault_check(sf_grid *grid, uint32_t *flags, long long *step, int *phase);
-/* Nodes per segment of the y / z marching sweeps (1..4096), or 0 for the
- * automatic choice (64 where that leaves at least 8192 one-wave blocks,
- * else 32 halved down to 8 until there are 4096).  No reference
- * counterpart; results do not depend on it. */
+/* Nodes per segment of the y / z marching sweeps (1..4096; the launch that
+ * takes the y and x faces together caps it at 32), or 0 for the automatic
+ * choice (the length that weighs the extra work at a segment's start against
+ * filling the device).  No reference counterpart; results do not depend on
+ * it. */
 int sf_grid_set_march_segment(sf_grid *grid, int nodes);
 /* How the x sweep walks the grid: 1 by whole x lines in 64-node tiles,
- * 0 by tiles of 63 faces over all lines numbered as one sequence, -1 (the
- * default) by lines where nx >= 64 and the grid has at least 256 x lines
- * per compute unit (65536 lines on a 256-CU device: 256^3 and up), else by
- * flattened tiles.  Grids whose
- * variables exceed 2^32 - 1024 bytes always take the flattened tiles.  No
- * reference counterpart; results do not depend on it. */
+ * 0 by tiles of 63 faces over all lines numbered as one sequence, both as a
+ * launch of their own after the y march; -1 (the default) in one launch with
+ * the y faces on 2D and 3D grids, except on grids narrower than 32 nodes
+ * that fill the device anyway.  1D grids, those narrow ones and sf_residual
+ * choose between the two walks by the number of lines (lines where nx >= 64
+ * and there are at least 256 per compute unit).  Grids whose variables exceed
+ * 2^32 - 1024 bytes never walk by lines.  No reference counterpart; results
+ * do not depend on it. */
 int sf_grid_set_x_walk(sf_grid *grid, int mode);
 /* Wait for the grid's queued work. */
 int sf_synchronize(sf_grid *grid);
@@ -244,8 +247,9 @@ int sf_face_flux(int device, int scheme, int flux, int axis, double gamma, doubl
  * the grid's stream; sf_profile_read waits for them and returns the summed
  * duration and the launch count.  Enabling resets the counters. */
 enum {
-    SF_KERNEL_SWEEP_X = 0,   /* x-face flux sweep                               */
-    SF_KERNEL_SWEEP_Y = 1,   /* y-face flux sweep                               */
+    SF_KERNEL_SWEEP_X = 0,   /* x-face flux sweep and stage update, with the y
+                                faces where one launch takes both               */
+    SF_KERNEL_SWEEP_Y = 1,   /* y-face flux sweep of its own                    */
     SF_KERNEL_SWEEP_Z = 2,   /* z-face flux sweep                               */
     SF_KERNEL_GHOST = 3,     /* one ghost fill (all its boundary kernels)       */
     SF_KERNEL_CFL = 4,       /* standalone CFL scan                             */

@@ -252,7 +252,7 @@ class Grid:
 
     def set_x_walk(self, mode: int):
         """x sweep by whole lines (1), by flattened face tiles (0) or the
-        automatic choice (-1)."""
+        automatic choice (-1: with the y faces in one launch where it can)."""
         _check(load().sf_grid_set_x_walk(self._h, int(mode)))
 
     def profile(self, enable: bool = True):

@@ -21,6 +21,8 @@ ARCH = os.environ.get("SONIC_AMD_ARCH", "gfx950")
 SOURCES = [PKG / "csrc" / "sf_capi.hip", PKG / "csrc" / "sf_batch.hip", PKG / "csrc" / "sf_diag.hip",
            PKG / "csrc" / "sf_sweep_weno5.hip", PKG / "csrc" / "sf_sweep_teno5.hip",
            PKG / "csrc" / "sf_sweep_weno3.hip", PKG / "csrc" / "sf_sweep_weno7.hip",
+           PKG / "csrc" / "sf_yx_weno5.hip", PKG / "csrc" / "sf_yx_teno5.hip",
+           PKG / "csrc" / "sf_yx_weno3.hip", PKG / "csrc" / "sf_yx_weno7.hip",
            PKG / "host" / "sf_provider.cpp", PKG / "host" / "sf_server.cpp",
            PKG / "host" / "sf_yaml.cpp", PKG / "host" / "sf_case.cpp", PKG / "host" / "sf_vts.cpp"]
 HEADERS = list((PKG / "csrc").glob("*.h")) + list((PKG / "host").glob("*.h")) + \

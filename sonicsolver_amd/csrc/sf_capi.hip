@@ -208,19 +208,31 @@ int fill_ghosts(sf_grid* g, double* q, int all, long long tag) {
 // the last bit at most.
 int run_sweeps(sf_grid* g, const double* q, const StageArgs& A) {
     SweepCall c{g->G, q, g->S, A, g->stream, g->march_seg, g->cus, g->x_walk};
+    auto sweep = [&](int axis, int mode) {
+        switch (g->desc.scheme) {
+        case SF_SCHEME_TENO5: return launch_sweep<1>(c, g->desc.flux, axis, mode);
+        case SF_SCHEME_WENO3: return launch_sweep<2>(c, g->desc.flux, axis, mode);
+        case SF_SCHEME_WENO7: return launch_sweep<3>(c, g->desc.flux, axis, mode);
+        default: return launch_sweep<0>(c, g->desc.flux, axis, mode);
+        }
+    };
+    auto fused = [&](const YxShape& sh) {
+        switch (g->desc.scheme) {
+        case SF_SCHEME_TENO5: return launch_yx<1>(c, g->desc.flux, sh);
+        case SF_SCHEME_WENO3: return launch_yx<2>(c, g->desc.flux, sh);
+        case SF_SCHEME_WENO7: return launch_yx<3>(c, g->desc.flux, sh);
+        default: return launch_yx<0>(c, g->desc.flux, sh);
+        }
+    };
+    const YxShape yx = yx_shape(c);
     int axes[3], na = 0;
     for (int a = 2; a >= 0; --a)
-        if (g->G.active[a]) axes[na++] = a;
+        if (g->G.active[a] && !(a == 1 && yx.blocks)) axes[na++] = a;
     for (int t = 0; t < na; ++t) {
-        const int mode = (t == na - 1) ? kFinal : (t == 0) ? kCopyS : kAccumS;
+        const bool last = t == na - 1;
+        const int mode = last ? kFinal : (t == 0) ? kCopyS : kAccumS;
         const int ev = prof_start(g, SF_KERNEL_SWEEP_X + axes[t]);
-        int rc;
-        switch (g->desc.scheme) {
-        case SF_SCHEME_TENO5: rc = launch_sweep<1>(c, g->desc.flux, axes[t], mode); break;
-        case SF_SCHEME_WENO3: rc = launch_sweep<2>(c, g->desc.flux, axes[t], mode); break;
-        case SF_SCHEME_WENO7: rc = launch_sweep<3>(c, g->desc.flux, axes[t], mode); break;
-        default: rc = launch_sweep<0>(c, g->desc.flux, axes[t], mode); break;
-        }
+        const int rc = last && yx.blocks ? fused(yx) : sweep(axes[t], mode);
         prof_stop(g, ev);
         if (rc) return fail(SF_E_STATE, "run_sweeps: no kernel for this sweep axis and mode");
     }

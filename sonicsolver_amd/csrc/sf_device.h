@@ -135,10 +135,11 @@ template <class GT>
 __device__ __forceinline__ double local_dt(const GT& G, const double q[5], double cfl,
                                            unsigned& flags) {
     const Closed s = close_state(q, G.gamma);
+    const double c = s.c();
     double spectral = 0.0;
 #pragma unroll
     for (int d = 0; d < 3; ++d)
-        if (cfl_axis(G, d)) spectral += fabs(s.u[d] * G.metric[d]) + s.c * G.metric[d];
+        if (cfl_axis(G, d)) spectral += fma(c, G.metric[d], fabs(s.u[d] * G.metric[d]));
     if (!(spectral > 0.0) || !isfinite(spectral)) flags |= kFlagDt;
     return cfl / spectral;
 }
@@ -258,17 +259,17 @@ __device__ __forceinline__ void stage_update_dt(const GT& G, const StageArgs& A,
     for (int v = 0; v < 5; ++v) {
         const double R = G.jac * S[v];
         if (time == 1) {
-            const double euler = qc[v] - dt * R;
-            qn[v] = A.base * q0v[v] + A.incr * euler;   // base = 0 in stage 1
+            const double euler = fma(-dt, R, qc[v]);
+            qn[v] = fma(A.incr, euler, A.base * q0v[v]);   // base = 0 in stage 1
         } else if (time == 0) {
-            qn[v] = qc[v] - dt * R;
+            qn[v] = fma(-dt, R, qc[v]);
         } else if (A.stage < 3) {
             A.k[A.stage][v * G.P + id] = R;
-            qn[v] = q0v[v] - A.incr * dt * R;
+            qn[v] = fma(-(A.incr * dt), R, q0v[v]);
         } else {
-            qn[v] = q0v[v]
-                  - dt / 6.0 * (A.k[0][v * G.P + id] + 2.0 * A.k[1][v * G.P + id]
-                                + 2.0 * A.k[2][v * G.P + id] + R);
+            const double sum = fma(2.0, A.k[2][v * G.P + id],
+                                   fma(2.0, A.k[1][v * G.P + id], A.k[0][v * G.P + id])) + R;
+            qn[v] = fma(-(dt / 6.0), sum, q0v[v]);
         }
         A.qout[v * G.P + id] = qn[v];
     }
@@ -276,8 +277,8 @@ __device__ __forceinline__ void stage_update_dt(const GT& G, const StageArgs& A,
     // (p has the sign of the internal energy; with the refined reciprocal
     // of the density instead of a division, that sign can differ only where
     // the internal energy is within an ulp of the kinetic energy)
-    const double ke = 0.5 * (qn[1] * qn[1] + qn[2] * qn[2] + qn[3] * qn[3]) * frcp(qn[0]);
-    const double eint = qn[4] - ke;
+    const double ke = 0.5 * dot3(qn + 1, qn + 1);
+    const double eint = fma(-ke, frcp(qn[0]), qn[4]);
     if (!(qn[0] > 0.0) || !(eint > 0.0) || !isfinite(eint)) flags |= kFlagState;
     if (A.reduce_dt) dt_local = local_dt(G, qn, A.cfl, flags);
 }
@@ -353,9 +354,9 @@ __device__ __forceinline__ double pressure_of(const double* q, long long P, long
 __device__ __forceinline__ double energy_from_pressure(const double* q, long long P, long long id,
                                                        double gamma, double p) {
     const double r = q[id], m1 = q[P + id], m2 = q[2 * P + id], m3 = q[3 * P + id];
-    const double e = 0.0 + p / ((gamma - 1.0) * r);
-    const double kinetic = 0.5 * (1.0 / r) * (m1 * m1 + m2 * m2 + m3 * m3);
-    return r * e + kinetic;
+    const double e = p / ((gamma - 1.0) * r);
+    const double kinetic = 0.5 * (1.0 / r) * fma(m3, m3, fma(m2, m2, m1 * m1));
+    return fma(r, e, kinetic);
 }
 
 }  // namespace sfamd

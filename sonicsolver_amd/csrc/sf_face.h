@@ -12,11 +12,18 @@
 // instruction sequence on CDNA, so where the reference divides several
 // times by one quantity the code takes one reciprocal, and the WENO
 // weights are normalised with a single division (each definition says
-// where).  With hipcc's FMA contraction, results differ from the
+// where).  With its fused multiply-adds, results differ from the
 // reference in the last few bits only.
+//
+// Every fused multiply-add below is written out and the compiler fuses none
+// of its own (which of two products a sum would be fused with depends on
+// what else a kernel does with them), so a face has the same bits in every
+// kernel that evaluates it.
 #pragma once
 
 #include <hip/hip_runtime.h>
+
+#pragma clang fp contract(off)
 
 namespace sfamd {
 
@@ -44,6 +51,10 @@ template <> struct Basis<2> {
 };
 
 __device__ __forceinline__ double sq(double x) { return x * x; }
+
+__device__ __forceinline__ double dot3(const double* a, const double* b) {
+    return fma(a[2], b[2], fma(a[1], b[1], a[0] * b[0]));
+}
 
 // Reciprocal, quotient and reciprocal square root from the hardware
 // estimate (good to about 5e-8 relative) refined by NR Newton steps: with
@@ -87,10 +98,9 @@ __device__ __forceinline__ double fsqrt(double z) { return z * frsqrt<NR>(z); }
 // the boundary g - P is exact (Sterbenz), so the comparison below decides
 // exactly as the division does (up to a tie at the midpoint).
 __device__ __forceinline__ bool teno_cut(double g, double gs) {
-#pragma clang fp contract(off)
     const double P = 1.0e-5 * gs;
     const double E = __builtin_fma(1.0e-5, gs, -P);
-    return g - P < E - 0x1p-70 * gs;
+    return g - P < fma(-0x1p-70, gs, E);
 }
 
 // Reconstruction in differences.  Every candidate value is the upwind node
@@ -191,9 +201,9 @@ __device__ __forceinline__ bool teno5_weights(const double b[3], double& c0, dou
         const double x3 = x * x * x;
         return x3 * x3;
     };
-    const double g0 = p6(1.0 + t * (b[1] * b[2]));
-    const double g1 = p6(1.0 + t * (b[0] * b[2]));
-    const double g2 = p6(1.0 + t * e01);
+    const double g0 = p6(fma(t, b[1] * b[2], 1.0));
+    const double g1 = p6(fma(t, b[0] * b[2], 1.0));
+    const double g2 = p6(fma(t, e01, 1.0));
     const double gs = g0 + g1 + g2;
     c0 = teno_cut(g0, gs) ? 0.0 : 1.0;
     c1 = teno_cut(g1, gs) ? 0.0 : 1.0;
@@ -320,7 +330,9 @@ __device__ __forceinline__ void recon_pair(const double (&d)[Stencil<SCHEME>::ns
 // (SF_singleFluidStateModel.cpp:49-71, SF_perfectGasEOS.h:24-32).
 // One reciprocal of the density replaces the five divisions by rho.
 struct Closed {
-    double u[3], p, c, inv_rho;
+    double u[3], p, inv_rho;
+    double c2, rc;   // squared sound speed and its reciprocal root: c = c2 rc
+    __device__ __forceinline__ double c() const { return c2 * rc; }
 };
 
 // close_state with the reciprocal of the density given.
@@ -331,9 +343,10 @@ __device__ __forceinline__ Closed close_state_r(const double q[5], double gamma,
     s.u[0] = q[1] * s.inv_rho;
     s.u[1] = q[2] * s.inv_rho;
     s.u[2] = q[3] * s.inv_rho;
-    const double mu = q[1] * s.u[0] + q[2] * s.u[1] + q[3] * s.u[2];
+    const double mu = dot3(q + 1, s.u);
     s.p = (gamma - 1.0) * fma(-0.5, mu, q[4]);
-    s.c = fsqrt<NR>(gamma * s.p * s.inv_rho);
+    s.c2 = gamma * s.p * s.inv_rho;
+    s.rc = frsqrt<NR>(s.c2);
     return s;
 }
 
@@ -368,7 +381,7 @@ __device__ __forceinline__ void rusanov(const double qL[5], const double qR[5],
     // (physicalFlux, SF_rusanovEOS.cpp:14-32), whose mass component is the
     // normal momentum
     const double unL = l.u[ND], unR = r.u[ND];
-    const double lambda = fmax(fabs(unL) + l.c, fabs(unR) + r.c);
+    const double lambda = fmax(fma(l.c2, l.rc, fabs(unL)), fma(r.c2, r.rc, fabs(unR)));
     out[0] = 0.5 * fma(-lambda, qR[0] - qL[0], qL[1 + ND] + qR[1 + ND]);
 #pragma unroll
     for (int d = 0; d < 3; ++d) {
@@ -403,18 +416,19 @@ __device__ __forceinline__ void hllc(const double qL[5], const double qR[5],
     if (!closed_ok(qL, l) || !closed_ok(qR, r)) flags |= kFlagFlux;
     const double unL = l.u[ND], unR = r.u[ND];
     // Roe weights sqrt(rho_K) / (sqrt(rho_L) + sqrt(rho_R))
-    const double inv = frcp<NR>(qL[0] * yL + qR[0] * yR);
-    const double wL = qL[0] * yL * inv, wR = qR[0] * yR * inv;
+    const double sL = qL[0] * yL, sR = qR[0] * yR;
+    const double inv = frcp<NR>(sL + sR);
+    const double wL = sL * inv, wR = sR * inv;
     double ut[3];
 #pragma unroll
-    for (int d = 0; d < 3; ++d) ut[d] = wL * l.u[d] + wR * r.u[d];
+    for (int d = 0; d < 3; ++d) ut[d] = fma(wL, l.u[d], wR * r.u[d]);
     const double HL = (qL[4] + l.p) * l.inv_rho, HR = (qR[4] + r.p) * r.inv_rho;
-    const double Ht = wL * HL + wR * HR;
-    const double ct = fsqrt<NR>((gamma - 1.0) * (Ht - 0.5 * (ut[0] * ut[0] + ut[1] * ut[1] + ut[2] * ut[2])));
-    const double SL = fmin(unL - l.c, ut[ND] - ct);
-    const double SR = fmax(unR + r.c, ut[ND] + ct);
+    const double Ht = fma(wL, HL, wR * HR);
+    const double ct2 = (gamma - 1.0) * fma(-0.5, dot3(ut, ut), Ht), rct = frsqrt<NR>(ct2);
+    const double SL = fmin(fma(-l.c2, l.rc, unL), fma(-ct2, rct, ut[ND]));
+    const double SR = fmax(fma(r.c2, r.rc, unR), fma(ct2, rct, ut[ND]));
     const double mL = qL[0] * (SL - unL), mR = qR[0] * (SR - unR);
-    const double Ss = fdiv<NR>(r.p - l.p + unL * mL - unR * mR, mL - mR);
+    const double Ss = fdiv<NR>(fma(-unR, mR, fma(unL, mL, r.p - l.p)), mL - mR);
     // The left side where the fan leaves the face to the right (0 <= S_L) or
     // the contact does (0 <= S*), the right side otherwise.
     const bool supL = 0.0 <= SL, supR = SR <= 0.0;
@@ -449,7 +463,7 @@ template <int NR = 2>
 __device__ __forceinline__ Legacy legacy_state(const double q[5], double gamma) {
     Legacy s;
     s.inv_rho = frcp<NR>(q[0]);
-    const double ke = 0.5 * (q[1] * q[1] + q[2] * q[2] + q[3] * q[3]) * s.inv_rho;
+    const double ke = 0.5 * dot3(q + 1, q + 1) * s.inv_rho;
     s.p = (gamma - 1.0) * (q[4] - ke);
     s.u[0] = q[1] * s.inv_rho;
     s.u[1] = q[2] * s.inv_rho;
@@ -469,23 +483,23 @@ __device__ __forceinline__ void steger_half(const double q[5], double gamma, dou
     if (!s.ok) flags |= kFlagFlux;
     const double a = fsqrt<NR>(gamma * s.p * s.inv_rho);
     const double un = s.u[ND];
-    const double q2 = s.u[0] * s.u[0] + s.u[1] * s.u[1] + s.u[2] * s.u[2];
+    const double q2 = dot3(s.u, s.u);
     auto split = [](double lam) {
         const double eps_sw = 0.01;
         double lp;
-        if (fabs(lam) < 2.0 * eps_sw) lp = 0.5 * (lam * lam * (1.0 / (4.0 * eps_sw)) + lam + eps_sw);
+        if (fabs(lam) < 2.0 * eps_sw) lp = 0.5 * (fma(lam * (1.0 / (4.0 * eps_sw)), lam, lam) + eps_sw);
         else lp = 0.5 * (lam + fabs(lam));
         return POS ? lp : lam - lp;
     };
     const double l0 = split(un), l3 = split(un + a), l4 = split(un - a);
-    const double W1 = 2.0 * (gamma - 1.0) * l0 + l3 + l4;
+    const double W1 = fma(2.0 * (gamma - 1.0), l0, l3) + l4;
     const double W2 = l3 - l4;
     const double W3 = l3 + l4;
     const double common = q[0] * frcp<NR>(2.0 * gamma);
     f[0] = common * W1;
 #pragma unroll
-    for (int d = 0; d < 3; ++d) f[1 + d] = common * ((d == ND) ? s.u[d] * W1 + a * W2 : s.u[d] * W1);
-    f[4] = common * (0.5 * q2 * W1 + a * un * W2 + (a * a) * frcp<NR>(gamma - 1.0) * W3);
+    for (int d = 0; d < 3; ++d) f[1 + d] = common * ((d == ND) ? fma(a, W2, s.u[d] * W1) : s.u[d] * W1);
+    f[4] = common * fma((a * a) * frcp<NR>(gamma - 1.0), W3, fma(a * un, W2, 0.5 * q2 * W1));
 }
 
 // StegerWarmingFlux::flux (SF_sw.cpp:21-27): F+(qL) + F-(qR).
@@ -513,10 +527,10 @@ __device__ __forceinline__ void laxf_half(const double q[5], double gamma, doubl
     double F[5];
     F[0] = q[0] * un;
 #pragma unroll
-    for (int d = 0; d < 3; ++d) F[1 + d] = (d == ND) ? q[1 + d] * un + s.p : q[1 + d] * un;
+    for (int d = 0; d < 3; ++d) F[1 + d] = (d == ND) ? fma(q[1 + d], un, s.p) : q[1 + d] * un;
     F[4] = (q[4] + s.p) * un;
 #pragma unroll
-    for (int v = 0; v < 5; ++v) f[v] = 0.5 * (F[v] + lam * q[v]);
+    for (int v = 0; v < 5; ++v) f[v] = 0.5 * fma(lam, q[v], F[v]);
 }
 
 // LaxFriedrichsFlux::flux (SF_lxF.cpp:21-27).
@@ -536,7 +550,7 @@ __device__ __forceinline__ void euler_flux(const double q[5], const Legacy& s, d
     const double un = s.u[ND];
     f[0] = q[0] * un;
 #pragma unroll
-    for (int d = 0; d < 3; ++d) f[1 + d] = (d == ND) ? q[0] * s.u[d] * un + s.p : q[0] * s.u[d] * un;
+    for (int d = 0; d < 3; ++d) f[1 + d] = (d == ND) ? fma(q[0] * s.u[d], un, s.p) : q[0] * s.u[d] * un;
     f[4] = (q[4] + s.p) * un;
 }
 
@@ -554,7 +568,7 @@ struct CharBasis {
         u[0] = q[1] * invR;
         u[1] = q[2] * invR;
         u[2] = q[3] * invR;
-        const double ke = 0.5 * (q[1] * u[0] + q[2] * u[1] + q[3] * u[2]);
+        const double ke = 0.5 * dot3(q + 1, u);
         const double p = (gamma - 1.0) * (q[4] - ke);
         if (!(q[0] > 0.0) || !(p > 0.0)) flags |= kFlagChar;
         hq2 = ke * invR;
@@ -627,17 +641,17 @@ __device__ __forceinline__ void roe(const double qL[5], const double qR[5], doub
     const double inv = frcp<NR>(sL + sR);
     double ut[3];
 #pragma unroll
-    for (int d = 0; d < 3; ++d) ut[d] = (sL * l.u[d] + sR * r.u[d]) * inv;
-    const double ht = (sL * hL + sR * hR) * inv;
-    const double q2t = ut[0] * ut[0] + ut[1] * ut[1] + ut[2] * ut[2];
-    const double a2 = gm1 * (ht - 0.5 * q2t);
+    for (int d = 0; d < 3; ++d) ut[d] = fma(sL, l.u[d], sR * r.u[d]) * inv;
+    const double ht = fma(sL, hL, sR * hR) * inv;
+    const double q2t = dot3(ut, ut);
+    const double a2 = gm1 * fma(-0.5, q2t, ht);
     if (!(a2 > 0.0)) flags |= kFlagFlux;
     const double at = fsqrt<NR>(a2);
     const double unt = ut[ND];
     const double delta = 0.1 * at;
     auto fix = [delta](double lam) {
         const double v = fabs(lam);
-        return v < 2.0 * delta ? 0.5 * (v * v * frcp<NR>(2.0 * delta) + delta) : v;
+        return v < 2.0 * delta ? 0.5 * fma(v * v, frcp<NR>(2.0 * delta), delta) : v;
     };
     const double lam0 = fix(unt), lam3 = fix(unt + at), lam4 = fix(unt - at);
     const double rt = sL * sR;
@@ -645,7 +659,7 @@ __device__ __forceinline__ void roe(const double qL[5], const double qR[5], doub
     qt[0] = rt;
 #pragma unroll
     for (int d = 0; d < 3; ++d) qt[1 + d] = rt * ut[d];
-    qt[4] = rt * (0.5 * q2t + a2 * frcp<NR>(gm1));
+    qt[4] = rt * fma(a2, frcp<NR>(gm1), 0.5 * q2t);
     const CharBasis<AXIS, NR> cb(qt, gamma, flags);
     double dq[5], al[5];
 #pragma unroll
@@ -680,7 +694,7 @@ __device__ __forceinline__ void lax_wendroff(const double qL[5], const double qR
     euler_flux<ND>(qR, r, fR);
     double qh[5];
 #pragma unroll
-    for (int v = 0; v < 5; ++v) qh[v] = 0.5 * (qL[v] + qR[v]) - 0.5 * lambda * (fR[v] - fL[v]);
+    for (int v = 0; v < 5; ++v) qh[v] = fma(-0.5 * lambda, fR[v] - fL[v], 0.5 * (qL[v] + qR[v]));
     const Legacy h = legacy_state<NR>(qh, gamma);
     if (!h.ok) flags |= kFlagFlux;
     euler_flux<ND>(qh, h, out);

@@ -7,21 +7,22 @@
 // (m_d = n_d + 2 g) and none on an inactive one.  Work per RK stage:
 //
 //   ghost fill (O(surface))      k_bc_copy4 / k_bc_energy / k_bc_periodic
-//   x sweep                      k_sweep_x:     one lane per x face, the
-//                                               flux difference by a
-//                                               cross-lane shift; on grids
-//                                               with many x lines
-//                                               k_sweep_xl walks whole
-//                                               lines in 64-node tiles
-//   y / z sweeps                 k_sweep_march: one lane per (x, column
+//   z sweep                      k_sweep_march: one lane per (x, column
 //                                               segment), marching along the
 //                                               axis with the stencil window
 //                                               in LDS, so each node is
 //                                               loaded once and each face
 //                                               evaluated once
-//   the last sweep (x) also applies the stage update, validates the new
-//   state and (on the last stage) folds the CFL scan of the next step into
-//   a wave-level minimum (DPP moves) plus one 64-bit atomic per wave.
+//   y and x sweeps               k_stage_yx:    the same march along y with
+//                                               the x faces of each row taken
+//                                               from the window's rows
+//   separately, where yx_shape   k_sweep_march, then k_sweep_x (one lane per
+//   says so                      x face, the flux difference by a cross-lane
+//                                shift) or k_sweep_xl (whole lines in 64-node
+//                                tiles)
+//   the last launch also applies the stage update, validates the new state
+//   and (on the last stage) folds the CFL scan of the next step into a
+//   wave-level minimum (DPP moves) plus one 64-bit atomic per wave.
 //
 // Sweeps accumulate S = sum_d (F_d(i) - F_d(i-1)) and the update multiplies
 // by Jac once, as Math::localSpatialResidual does

@@ -22,6 +22,23 @@ struct SweepCall {
     int x_walk;        // x sweep by lines (1), by flat tiles (0), automatic (-1)
 };
 
+// Cost, in face evaluations of one wave, of a march whose one-wave blocks
+// evaluate `faces` faces each, on a device of `cus` compute units (four SIMDs
+// each).  Blocks are dealt evenly, so the SIMD with the most of them sets the
+// time.  Measured on 2D and 3D grids with the fused y / x march: one wave on
+// a SIMD takes 1.73 times as long per face as each of three or more, two
+// take 1.3 times, and a block's start (its window's loads) costs as much as
+// five faces where nothing hides it and 1.5 where other waves do.
+// 853^2, WENO5/HLLC, per stage: 52 us with 1008 blocks of 12 rows, 73 with
+// 1092 of 11, 47 with 2002 of 6, 45 with 2996 of 4.
+inline double march_cost(long long blocks, double faces, int cus) {
+    const long long simds = 4LL * std::max(cus, 8);
+    const long long w = (blocks + simds - 1) / simds;
+    if (w <= 1) return 1.73 * (faces + 5.0);
+    if (w == 2) return 2.6 * (faces + 4.0);
+    return 1.07 * (double)w * (faces + (w <= 4 ? 3.0 : 1.5));
+}
+
 // Grid of the x sweep (a multiple of 8 for the XCD mapping): one block per
 // 128 tiles, at least as many as the device holds at once (compute units x
 // the kernel's resident blocks per unit) and at most 16384.  Blocks beyond
@@ -110,22 +127,19 @@ int launch_sweep_fm(const SweepCall& c, int axis) {
         const unsigned other = (unsigned)(axis == 1 ? G.n[2] : G.n[1]);
         const unsigned cols = (unsigned)((G.n[0] + kMarchBlock - 1) / kMarchBlock);
         // Each segment re-reads the stencil window and evaluates one extra
-        // face at its start, so segments of 64 nodes are used wherever that
-        // still leaves 8192 one-wave blocks or more to fill the chip
-        // (512^3); where 32-node segments leave fewer than 4096 blocks
-        // (2048^2 in 2D: 2048), the segment is halved down to 8 nodes until
-        // there are 4096, four waves per SIMD.  A face's arithmetic does not
-        // depend on the segment length, so neither does the result.
-        // c.seg > 0 fixes the length instead.
-        auto blocks = [&](int s) {
-            return (long long)cols * other * ((G.n[axis] + s - 1) / s);
-        };
+        // face at its start; march_cost weighs that against filling the
+        // chip.  A face's arithmetic does not depend on the segment length,
+        // so neither does the result.  c.seg > 0 fixes the length instead.
         int seg = c.seg;
         if (seg <= 0) {
-            seg = 32;
-            if (blocks(2 * seg) >= 8192) seg *= 2;
-            else
-                while (seg > 8 && blocks(seg) < 4096) seg /= 2;
+            double least = 0.0;
+            for (int s = 1; s <= 64; ++s) {
+                const long long blocks = (long long)cols * other * ((G.n[axis] + s - 1) / s);
+                const double cost = march_cost(blocks, s + 1.0, c.cus);
+                if (seg > 0 && cost >= least) continue;
+                least = cost;
+                seg = s;
+            }
         }
         const dim3 grid(cols, other, (unsigned)((G.n[axis] + seg - 1) / seg));
         if (axis == 1)
@@ -143,6 +157,41 @@ int launch_sweep_f(const SweepCall& c, int axis, int mode) {
     if (mode == kCopyS) return launch_sweep_fm<SCHEME, FLUX, kCopyS>(c, axis);
     if (mode == kAccumS) return launch_sweep_fm<SCHEME, FLUX, kAccumS>(c, axis);
     return launch_sweep_fm<SCHEME, FLUX, kFinal>(c, axis);
+}
+
+// The y and x faces and the stage update in one launch (k_stage_yx).
+// Returns -1 for a time recipe that is not compiled.
+template <int SCHEME, int FLUX>
+int launch_yx_f(const SweepCall& c, const YxShape& sh) {
+    const SweepArgs W{c.G, c.q, c.S, c.A};
+    const unsigned nb = (sh.blocks + 7) & ~7u;
+#define SF_LAUNCH_YX(T)                                                                       \
+    do {                                                                                      \
+        if (c.G.active[2])                                                                    \
+            k_stage_yx<SCHEME, FLUX, T, true><<<nb, kXBlock, 0, c.stream>>>(W, sh);           \
+        else                                                                                  \
+            k_stage_yx<SCHEME, FLUX, T, false><<<nb, kXBlock, 0, c.stream>>>(W, sh);          \
+    } while (0)
+    switch (c.A.time) {
+    case 0: SF_LAUNCH_YX(0); break;
+    case 1: SF_LAUNCH_YX(1); break;
+    case 2: SF_LAUNCH_YX(2); break;
+    default: return -1;
+    }
+#undef SF_LAUNCH_YX
+    return 0;
+}
+
+template <int SCHEME>
+int launch_yx(const SweepCall& c, int flux, const YxShape& sh) {
+    switch (flux) {
+    case 0: return launch_yx_f<SCHEME, 0>(c, sh);
+    case 1: return launch_yx_f<SCHEME, 1>(c, sh);
+    case 2: return launch_yx_f<SCHEME, 2>(c, sh);
+    case 3: return launch_yx_f<SCHEME, 3>(c, sh);
+    case 4: return launch_yx_f<SCHEME, 4>(c, sh);
+    default: return launch_yx_f<SCHEME, 5>(c, sh);
+    }
 }
 
 // One sweep of scheme SCHEME with face flux `flux` (SF_FLUX_*) along
@@ -163,5 +212,47 @@ extern template int launch_sweep<0>(const SweepCall&, int, int, int);
 extern template int launch_sweep<1>(const SweepCall&, int, int, int);
 extern template int launch_sweep<2>(const SweepCall&, int, int, int);
 extern template int launch_sweep<3>(const SweepCall&, int, int, int);
+extern template int launch_yx<0>(const SweepCall&, int, const YxShape&);
+extern template int launch_yx<1>(const SweepCall&, int, const YxShape&);
+extern template int launch_yx<2>(const SweepCall&, int, const YxShape&);
+extern template int launch_yx<3>(const SweepCall&, int, const YxShape&);
+
+// Shape of the fused y / x launch of a stage, or blocks = 0 where the
+// separate sweeps take it: the residual-only mode, a chosen x walk, and grids
+// narrower than half a wave that fill the device more than twice over, whose
+// x faces the flattened tiles pack into whole waves (24 x 200 x 200,
+// WENO5/HLLC, 3 steps: 2.64 ms separately, 2.73 fused; 32 x 150 x 150: 1.91
+// and 1.93; 40 x 100 x 100: 1.41 and 1.30).  Everywhere else the fused
+// launch was faster, e.g. 512^3 77.3 -> 72.0 ms a pass of two steps, 2048^2
+// TENO5/HLLC 6.39 -> 5.75, 853^2 5.22 -> 4.23, 256^2 TENO5/HLLC 2.40 ->
+// 1.36, 64^3 4.32 -> 2.87, 40^2 1.05 -> 0.76 (the small ones by shorter
+// segments in the z march, too).
+inline YxShape yx_shape(const SweepCall& c) {
+    YxShape best{};
+    const GridDev& G = c.G;
+    if (!G.active[1] || c.x_walk >= 0 || c.A.time == 3) return best;
+    double least = 0.0;
+    // columns a block advances: 64 with its first x faces evaluated
+    // beforehand, or 63 with lane 0 evaluating them
+    for (int cols = kXBlock; cols >= kXBlock - 1; --cols) {
+        YxShape sh{};
+        sh.cols = cols;
+        sh.nx = (G.n[0] + cols - 1) / cols;
+        for (int rows = 1; rows <= kYxRows; ++rows) {
+            if (c.seg > 0 && rows != std::min(c.seg, kYxRows)) continue;
+            sh.rows = rows;
+            sh.ny = (G.n[1] + rows - 1) / rows;
+            const long long blocks = (long long)sh.nx * sh.ny * G.n[2];
+            const double cost =
+                march_cost(blocks, 2.0 * rows + 1.0 + (cols == kXBlock ? 1.0 : 0.0), c.cus);
+            if (best.blocks && cost >= least) continue;
+            least = cost;
+            best = sh;
+            best.blocks = (unsigned)blocks;
+        }
+    }
+    if (2 * G.n[0] < kXBlock && best.blocks > 8u * (unsigned)std::max(c.cus, 8)) best.blocks = 0;
+    return best;
+}
 
 }  // namespace sfamd

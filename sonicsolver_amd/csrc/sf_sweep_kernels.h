@@ -528,4 +528,231 @@ void k_sweep_march(GridDev G,
     raise_fault(flags, A.flags, A.fault_tag, A.tag);
 }
 
+// ---------------------------------------------------------------------------
+// y and x faces and the stage update in one march along y: a block (one
+// wave) takes 64 columns of one z plane and up to kYxRows rows.  At row a
+// every lane evaluates its upper y face from its own column, as
+// k_sweep_march does, and its upper x face from the same row of the LDS
+// ring, whose rows carry the NS - 1 halo columns the x stencils reach; the
+// lower x face comes from lane t-1 by the cross-lane shift.  Lane 0 takes it
+// from the block's first faces, which the lanes evaluate beforehand, one row
+// each (cols = 64), or is itself only there to evaluate it (cols = 63, the
+// blocks overlapping by a column).  Faces, sums and updates are formed by
+// the same functions in the same order as by the separate sweeps, so the
+// results are theirs bit for bit.
+//
+// Against the y march and the x sweep it neither writes nor reads back the
+// y differences and reads the state once: on 512^3 21.5 GB per launch
+// instead of 16.1 + 21.7, which those two moved at the rate of a large copy
+// (3.68 + 4.77 ms); bound by FP64 issue at three waves per SIMD (two for
+// WENO7, whose ring is 17 KB).  yx_shape chooses the rows and columns.
+// ---------------------------------------------------------------------------
+constexpr int kYxRows = 32;
+
+// Orders the LDS accesses of a wave's lanes among themselves: the hardware
+// performs a wave's LDS operations in order, so only the compiler has to
+// keep them so.
+__device__ __forceinline__ void wave_lds_order() {
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+struct YxShape {
+    int cols;      // columns a block advances: 64, or 63 with a helper lane
+    int rows;      // rows a block advances (at most kYxRows)
+    int nx, ny;    // blocks along x and along y
+    unsigned blocks;
+};
+
+template <int SCHEME, int FLUX, int TIME, bool HAS_S>
+__global__ __launch_bounds__(kXBlock)
+__attribute__((amdgpu_waves_per_eu(SCHEME == 3 ? 2 : 3, 8))) void k_stage_yx(SweepArgs W,
+                                                                             YxShape sh) {
+    constexpr int NS = Stencil<SCHEME>::ns;
+    constexpr int H = NS / 2;
+    constexpr int R = NS - 2;             // ring rows a+1-H .. a+H-2
+    constexpr int WID = kXBlock + NS;     // a row: H-1 halo columns, 64, H halo, 1 pad
+    constexpr int HC = NS - 1;            // halo columns per row and variable
+    static_assert(5 * HC <= kXBlock, "one lane per halo value");
+    __shared__ double win[R][5][WID];
+    __shared__ double first[5][kYxRows];
+    if (*W.A.flags) return;   // a fault was raised: keep the step-start state
+    // blocks of one XCD take consecutive numbers (x fastest), so that they
+    // share the halo lines in its L2
+    const unsigned chunk = gridDim.x >> 3;
+    const unsigned bid = (blockIdx.x & 7u) * chunk + (blockIdx.x >> 3);
+    if (bid >= sh.blocks) return;
+    const int t = threadIdx.x;
+    const unsigned bx = bid % (unsigned)sh.nx, br = bid / (unsigned)sh.nx;
+    const int k = (int)(br / (unsigned)sh.ny);
+    const int a0 = (int)(br % (unsigned)sh.ny) * sh.rows;
+    const int a1 = min(a0 + sh.rows, W.G.n[1]);
+    const int helper = kXBlock - sh.cols;              // 1: lane 0 only evaluates a face
+    const int i0 = (int)bx * sh.cols - helper;         // lane 0's column
+    const int i = i0 + t;
+    const int n0 = W.G.n[0];
+    const bool node = i < n0 && t >= helper;           // this lane advances node i
+    const int last = n0 - 1 + H;                       // the last ghost column
+    unsigned flags = 0;
+    double dt_local = INFINITY;
+    const double dt_step = *W.A.dt;   // the step's dt, read once
+    const double lwx = (FLUX == 5) ? *W.A.dt / W.G.d[0] : 0.0;   // Lax-Wendroff dt / spacing
+    const double lwy = (FLUX == 5) ? *W.A.dt / W.G.d[1] : 0.0;
+
+    // the block's first x faces (lower face of lane 0's node), lane r for
+    // row a0 + r
+    if (helper == 0 && a0 + t < a1) {
+        const long long id = node_index(W.G, i0 - 1, a0 + t, k);
+        double st[NS][5];
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+#pragma unroll
+            for (int v = 0; v < 5; ++v) st[s][v] = W.q[v * W.G.P + id + (s + 1 - H)];
+        double f5[5];
+        face_flux<0, SCHEME, FLUX>(st, W.G.gamma, W.G.area[0], f5, flags, lwx);
+        if (!finite_sum5(f5)) flags |= kFlagFlux;
+#pragma unroll
+        for (int v = 0; v < 5; ++v) first[v][t] = f5[v];
+    }
+
+    // Loads address a lane's column by a 32-bit byte offset from the row's
+    // column i0 (i0 >= -1 lies in every row).  Lanes past the grid load its
+    // last ghost column again, which the x faces before them read, and form
+    // faces that nothing takes.
+    const unsigned off = (unsigned)(min(i, last) - i0) * 8u;
+    // halo: lane l < 5 HC loads variable l / HC, halo column l % HC
+    const int hv = t / HC, hc = t % HC;
+    const bool halo = hv < 5;
+    const int hcol = hc < H - 1 ? hc - (H - 1) : kXBlock + hc - (H - 1);   // from i0
+    const int hcl = min(i0 + hcol, last);   // at least -H, the first ghost column
+    const long long step = W.G.stride[1];
+    const long long row0 = node_index(W.G, i0, a0, k);
+    const double* hsrc = W.q + (halo ? hv : 0) * W.G.P + row0 + (hcl - i0);
+    const int hpos = hcol + H - 1;
+
+    {
+        long long id = row0 - H * step;   // row a0 - H
+        for (int s = 0; s < R; ++s, id += step)
+#pragma unroll
+            for (int v = 0; v < 5; ++v) win[s][v][t + H - 1] = at(W.q + v * W.G.P + id, off);
+    }
+    double carried[5];
+#pragma unroll
+    for (int v = 0; v < 5; ++v) carried[v] = at(W.q + v * W.G.P + row0 + (H - 2) * step, off);
+#pragma unroll
+    for (int v = 0; v < 5; ++v) asm volatile("" : "+v"(carried[v]));
+    double hnext = 0.0;
+    int head = 0;
+    double fprev[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
+    long long id = row0 - step;           // row a
+    wave_lds_order();
+#pragma clang loop unroll(disable)
+    for (int a = a0 - 1; a < a1; ++a, id += step) {
+        const SweepArgs& T = sweep_args();
+        // the halo columns of row a join the ring; those of row a + 1 are
+        // requested
+        const auto slot = [&](int s) { return (head + s >= R) ? head + s - R : head + s; };
+        if (halo) {
+            win[slot(H - 1)][hv][hpos] = hnext;
+            hnext = hsrc[(a + 1 - a0) * step];
+        }
+        double st[NS][5];
+#pragma unroll
+        for (int v = 0; v < 5; ++v) st[NS - 1][v] = at(T.q + v * T.G.P + id + H * step, off);
+#pragma unroll
+        for (int s = 0; s < R; ++s)
+#pragma unroll
+            for (int v = 0; v < 5; ++v) st[s][v] = win[slot(s)][v][t + H - 1];
+#pragma unroll
+        for (int v = 0; v < 5; ++v) {
+            st[NS - 2][v] = carried[v];
+            win[head][v][t + H - 1] = carried[v];
+            carried[v] = st[NS - 1][v];
+        }
+        head = (head == R - 1) ? 0 : head + 1;
+        wave_lds_order();
+        // rows a and a + 1 are now at H - 2 and H - 1 from the head
+        const int ra = slot(H - 2), rb = slot(H - 1);
+        unsigned fy = 0;
+        double s5[5];
+        {
+            double f[5];
+            face_flux_from<1, SCHEME, FLUX>(
+                st,
+                [&](int side, double (&b)[5]) {
+#pragma unroll
+                    for (int v = 0; v < 5; ++v) b[v] = win[side ? rb : ra][v][t + H - 1];
+                },
+                T.G.gamma, T.G.area[1], f, fy, lwy);
+            if (!finite_sum5(f)) fy |= kFlagFlux;
+#pragma unroll
+            for (int v = 0; v < 5; ++v) {
+                s5[v] = f[v] - fprev[v];
+                fprev[v] = f[v];
+            }
+        }
+        if (node) flags |= fy;
+        if (a < a0) continue;
+        // the x face; the stage operands are requested before its Riemann
+        // solver, which hides their latency
+        double sx[NS][5], ps[5], pq0[5], f5[5];
+#pragma unroll
+        for (int s = 0; s < NS; ++s)
+#pragma unroll
+            for (int v = 0; v < 5; ++v) sx[s][v] = win[ra][v][t + s];
+        unsigned fx = 0;
+        face_flux_from<0, SCHEME, FLUX>(
+            sx,
+            [&](int side, double (&b)[5]) {
+                if (side == 0) {
+                    const SweepArgs& U = sweep_args();
+#pragma unroll
+                    for (int v = 0; v < 5; ++v) {
+                        if (HAS_S) ps[v] = at(U.S + v * U.G.P + id, off);
+                        pq0[v] = at(U.A.q0 + v * U.G.P + id, off);
+                    }
+                }
+#pragma unroll
+                for (int v = 0; v < 5; ++v) b[v] = win[ra][v][t + H - 1 + side];
+            },
+            T.G.gamma, T.G.area[0], f5, fx, lwx);
+        if (!finite_sum5(f5)) fx |= kFlagFlux;
+        if (i < n0) flags |= fx;
+        double lower[5];
+#pragma unroll
+        for (int v = 0; v < 5; ++v) {
+            const double up = lane_shift_up1(f5[v]);
+            lower[v] = t == 0 ? first[v][a - a0] : up;
+        }
+        if (node) {
+            const SweepArgs& U = sweep_args();
+            double pq[5];
+#pragma unroll
+            for (int v = 0; v < 5; ++v) {
+                pq[v] = win[ra][v][t + H - 1];
+                if (HAS_S) s5[v] = ps[v] + s5[v];
+                s5[v] = s5[v] + (f5[v] - lower[v]);
+            }
+            double dl = INFINITY;
+            double qn[5];
+            const long long nid = id + t;
+            if (solved_node(U.G, i, a, k)) {
+                stage_update_dt<TIME>(U.G, U.A, nid, pq, pq0, s5, dt_step, flags, dl, qn);
+            } else {
+#pragma unroll
+                for (int v = 0; v < 5; ++v) {
+                    qn[v] = pq[v];   // carry_node
+                    U.A.qout[v * U.G.P + nid] = qn[v];
+                }
+            }
+            const SweepArgs& V = sweep_args();
+            if (V.G.images) write_images(V.G, V.A.qout, i, a, k, nid, qn);
+            dt_local = fmin(dt_local, dl);
+        }
+    }
+    raise_fault(flags, W.A.flags, W.A.fault_tag, W.A.tag);
+    if (W.A.reduce_dt) wave_min_atomic(dt_local, W.A.dtmin);
+}
+
 }  // namespace sfamd
