@@ -33,6 +33,23 @@
 namespace sfamd {
 void set_last_error(const std::string& message);
 
+__device__ __forceinline__ double pressure_of(const double* q, long long P, long long id,
+                                              double gamma) {
+    double qq[5];
+#pragma unroll
+    for (int v = 0; v < 5; ++v) qq[v] = q[v * P + id];
+    return close_state(qq, gamma).p;
+}
+
+// totalEnergyFromPressure (SF_singleFluidStateModel.cpp:73-109).
+__device__ __forceinline__ double energy_from_pressure(const double* q, long long P, long long id,
+                                                       double gamma, double p) {
+    const double r = q[id], m1 = q[P + id], m2 = q[2 * P + id], m3 = q[3 * P + id];
+    const double e = p / ((gamma - 1.0) * r);
+    const double kinetic = 0.5 * (1.0 / r) * fma(m3, m3, fma(m2, m2, m1 * m1));
+    return fma(r, e, kinetic);
+}
+
 struct BatchItemDev {
     long long off;      // start of the padded block in the arena
     int n0, n1, m0, gy;

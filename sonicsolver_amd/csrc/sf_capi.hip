@@ -74,7 +74,10 @@ struct sf_grid {
     double* stage_io = nullptr;  // unique-node staging for transfers
     size_t bytes = 0;
     int cur = 0;                 // buffer holding the current state
-    int ghosts_valid = 0;        // ghost layers of buf[cur] are up to date
+    int ghosts_valid = 0;        // buf[cur]'s boundary is prepared as far as map_node needs it
+    int stored = 0;              // buf[cur] holds all boundary nodes and ghosts (k_fill)
+    int separate = 0;            // the last stage ran the separate x sweep
+    int raw = 0;                 // buf[cur] is an upload whose boundary is not prepared yet
     int dtmin_valid = 0;         // clock->dtmin holds the scan of buf[cur]
     double dtmin_cfl = 0.0;      // CFL number the folded scan used
     int step_open = 0;
@@ -157,45 +160,19 @@ void prof_stop(sf_grid* g, int idx) {
     if (idx >= 0) (void)hipEventRecord(g->ev_pool[idx + 1], g->stream);
 }
 
-// Ghost fill in the order of Boundary::Applicator::apply (density and
-// momentum for every transmissive set, then energy from pressure, axis by
-// axis), then the periodic axes.  `all` = 0 skips the periodic axes whose
-// ghosts the final sweep keeps as copies of the interior (G.images): a
-// buffer written by a stage needs no fill for them.
-int fill_ghosts(sf_grid* g, double* q, int all, long long tag) {
+// Stores the boundary nodes and ghosts of q (k_fill).
+int fill_ghosts(sf_grid* g, double* q, long long tag) {
     const GridDev& G = g->G;
+    FillCount F{};
+    long long n = 0;
+    for (int a = 0; a < 3; ++a) {
+        if (G.active[a] && (G.wrap[a] || zg_end(G, a, 0) || zg_end(G, a, 1)))
+            n += 2LL * (G.g[a] + 1) * G.n[(a + 1) % 3] * G.n[(a + 2) % 3];
+        F.end[a] = n;
+    }
+    if (n == 0) return 0;
     const int ev = prof_start(g, SF_KERNEL_GHOST);
-    auto plane = [&](int a) {
-        return 2LL * G.n[(a + 1) % 3] * G.n[(a + 2) % 3];
-    };
-    auto zero_gradient = [&](int a) {
-        return G.active[a] && (G.bc[a] == SF_BC_TRANSMISSIVE || G.bc[a] == SF_BC_NONE_LO ||
-                               G.bc[a] == SF_BC_NONE_HI);
-    };
-    for (int a = 0; a < 3; ++a) {
-        if (!zero_gradient(a)) continue;
-        const int per = a == 0 ? fill_lanes<0>(G, true) : 1;
-        const unsigned nb = blocks_for(plane(a) * per, 256);
-        if (a == 0) k_bc_copy4<0><<<nb, 256, 0, g->stream>>>(G, q, g->flags);
-        if (a == 1) k_bc_copy4<1><<<nb, 256, 0, g->stream>>>(G, q, g->flags);
-        if (a == 2) k_bc_copy4<2><<<nb, 256, 0, g->stream>>>(G, q, g->flags);
-    }
-    for (int a = 0; a < 3; ++a) {
-        if (!zero_gradient(a)) continue;
-        const int per = a == 0 ? fill_lanes<0>(G, false) : 1;
-        const unsigned nb = blocks_for(plane(a) * per, 256);
-        if (a == 0) k_bc_energy<0><<<nb, 256, 0, g->stream>>>(G, q, g->fault, tag);
-        if (a == 1) k_bc_energy<1><<<nb, 256, 0, g->stream>>>(G, q, g->fault, tag);
-        if (a == 2) k_bc_energy<2><<<nb, 256, 0, g->stream>>>(G, q, g->fault, tag);
-    }
-    for (int a = 0; a < 3; ++a) {
-        if (!G.active[a] || G.bc[a] != SF_BC_PERIODIC) continue;
-        if (!all && (G.images & (1 << a))) continue;
-        const unsigned nb = blocks_for(plane(a), 256);
-        if (a == 0) k_bc_periodic<0><<<nb, 256, 0, g->stream>>>(G, q, g->flags);
-        if (a == 1) k_bc_periodic<1><<<nb, 256, 0, g->stream>>>(G, q, g->flags);
-        if (a == 2) k_bc_periodic<2><<<nb, 256, 0, g->stream>>>(G, q, g->flags);
-    }
+    k_fill<<<blocks_for(n, 256), 256, 0, g->stream>>>(G, q, F, g->fault, tag);
     prof_stop(g, ev);
     SF_HIP(hipGetLastError());
     return 0;
@@ -206,7 +183,8 @@ int fill_ghosts(sf_grid* g, double* q, int all, long long tag) {
 // update adds to it.  The flux differences are therefore summed as
 // (dz + dy) + dx rather than the reference's (dx + dy) + dz, which changes
 // the last bit at most.
-int run_sweeps(sf_grid* g, const double* q, const StageArgs& A) {
+// The separate x sweeps read stored ghosts: `stored` says that q has them.
+int run_sweeps(sf_grid* g, double* q, const StageArgs& A, bool stored) {
     SweepCall c{g->G, q, g->S, A, g->stream, g->march_seg, g->cus, g->x_walk};
     auto sweep = [&](int axis, int mode) {
         switch (g->desc.scheme) {
@@ -225,6 +203,9 @@ int run_sweeps(sf_grid* g, const double* q, const StageArgs& A) {
         }
     };
     const YxShape yx = yx_shape(c);
+    g->separate = yx.blocks == 0;
+    if (g->separate && !stored)
+        if (int rc = fill_ghosts(g, q, A.tag)) return rc;
     int axes[3], na = 0;
     for (int a = 2; a >= 0; --a)
         if (g->G.active[a] && !(a == 1 && yx.blocks)) axes[na++] = a;
@@ -261,7 +242,6 @@ int rotation(int time) { return time == SF_TIME_RK4 ? 2 : 1; }
 // fills, the fill that prepares or commits a step, the CFL scan before it.
 long long stage_tag(const sf_grid* g, int s) { return (g->seq - 1) * 8 + s; }
 long long next_tag(const sf_grid* g, int phase) { return g->seq * 8 + phase; }
-long long open_tag(const sf_grid* g, int phase) { return (g->seq - 1) * 8 + phase; }
 
 // Wait for the grid's work and read its fault record.  With flags raised,
 // every launch after the faulting one returned at entry, so the buffer that
@@ -292,6 +272,7 @@ int check_flags(sf_grid* g, const char* where, uint32_t* flags_out = nullptr,
     g->base_cur = g->cur;
     g->step_open = 0;
     g->ghosts_valid = 0;
+    g->stored = 0;
     g->dtmin_valid = 0;
     char what[32];
     if (phase < 4) std::snprintf(what, sizeof what, "stage %d", phase + 1);
@@ -333,10 +314,9 @@ int set_limits(sf_grid* g, double max_dt, double limit) {
 int do_stage(sf_grid* g, int s, int fold_dt) {
     const int in = g->stage_in[s], out = g->stage_out[s];
     if (s == 0 && !g->ghosts_valid) {
-        if (int rc = fill_ghosts(g, g->buf[in], 1, stage_tag(g, s))) return rc;
-    }
-    if (s > 0) {
-        if (int rc = fill_ghosts(g, g->buf[in], 0, stage_tag(g, s))) return rc;
+        if (int rc = fill_ghosts(g, g->buf[in], stage_tag(g, s))) return rc;
+        g->stored = 1;
+        g->raw = 0;
     }
     StageArgs A{};
     A.fault_tag = &g->fault->tag;
@@ -363,7 +343,7 @@ int do_stage(sf_grid* g, int s, int fold_dt) {
     const bool last = s == nstages(g->desc.time) - 1;
     A.reduce_dt = (last && fold_dt) ? 1 : 0;
     A.cfl = g->step_cfl;
-    return run_sweeps(g, g->buf[in], A);
+    return run_sweeps(g, g->buf[in], A, s == 0 && g->stored);
 }
 
 // Stage buffers of a step.  No stage writes the buffer that holds the
@@ -413,36 +393,23 @@ void set_geometry(sf_grid* g, const sf_grid_desc* desc) {
         G.active[a] = desc->active[a];
         G.bc[a] = desc->bc[a];
         G.d[a] = desc->d[a];
-        // A node has at most one periodic copy in the ghost layers only
-        // where n >= 2g; thinner periodic axes are filled between stages
-        // (k_bc_periodic takes the node index modulo n).
-        G.images |= (desc->active[a] && desc->bc[a] == SF_BC_PERIODIC && G.n[a] >= 2 * G.g[a])
-                        ? (1 << a) : 0;
     }
     G.div_line = make_fastdiv((unsigned)G.n[0] + 1u);
     G.div_n1 = make_fastdiv((unsigned)G.n[1]);
-    // A zeroGradient end rewrites the boundary nodes of its axis in the
-    // ghost fill after the stage; copies written by the stage would miss
-    // that, so the copies are used only where no axis has such an end.
-    for (int a = 0; a < 3; ++a)
-        if (desc->active[a] && (desc->bc[a] == SF_BC_TRANSMISSIVE ||
-                                desc->bc[a] == SF_BC_NONE_LO || desc->bc[a] == SF_BC_NONE_HI))
-            G.images = 0;
     for (int a = 0; a < 3; ++a) {
         G.solved_lo[a] = zg_end(G, a, 0) ? 1 : 0;
         G.solved_hi[a] = G.n[a] - 1 - (zg_end(G, a, 1) ? 1 : 0);
+        G.zg_lo[a] = zg_end(G, a, 0) ? 1 : 0;
+        G.zg_hi[a] = zg_end(G, a, 1) ? 1 : 0;
+        G.map_lo[a] = G.zg_lo[a] ? -1 : std::numeric_limits<int>::min();
+        G.map_hi[a] = G.zg_hi[a] ? G.n[a] : std::numeric_limits<int>::max();
+        G.wrap[a] = desc->active[a] && desc->bc[a] == SF_BC_PERIODIC ? G.n[a] : 0;
     }
     G.stride[0] = 1;
     G.stride[1] = G.m[0];
     G.stride[2] = (long long)G.m[0] * G.m[1];
     G.P = (long long)G.m[0] * G.m[1] * G.m[2];
     for (int a = 0; a < 3; ++a) G.ustride[a] = (unsigned)G.stride[a];
-    for (int a = 0; a < 3; ++a) {
-        const bool img = (G.images >> a) & 1;
-        G.img_lo[a] = img ? G.g[a] : 0;
-        G.img_span[a] = img ? (unsigned)(G.n[a] - 2 * G.g[a]) : 0xFFFFFFFFu;
-        G.img_off[a] = img ? (long long)G.n[a] * G.stride[a] : 0;
-    }
     G.gamma = desc->gamma;
     // Uniform Cartesian metrics exactly as the reference forms them:
     // Jac = 1/J, metric = 1/d, face cofactor = 0.5*(metric/Jac + metric/Jac),
@@ -582,7 +549,7 @@ static int upload_from(sf_grid* g, const double* dsrc) {
     k_clear_fault<<<1, 64, 0, g->stream>>>(g->fault);
     g->base_seq = g->seq;
     g->base_cur = g->cur;
-    k_pack<<<nb, 256, 0, g->stream>>>(G, dsrc, g->buf[g->cur], 1);
+    k_pack<<<nb, 256, 0, g->stream>>>(G, dsrc, g->buf[g->cur], 1, 0);
     // ends without a condition: every state buffer's ghost layers there hold
     // the uploaded end nodes from now on
     for (int a = 0; a < 3; ++a) {
@@ -596,6 +563,8 @@ static int upload_from(sf_grid* g, const double* dsrc) {
     }
     SF_HIP(hipGetLastError());
     g->ghosts_valid = 0;
+    g->stored = 0;
+    g->raw = 1;
     g->dtmin_valid = 0;
     g->step_open = 0;
     return 0;
@@ -621,7 +590,7 @@ int sf_state_upload_device(sf_grid* g, const double* soa_device) {
 static int download_to(sf_grid* g, double* ddst) {
     const long long N = (long long)g->G.n[0] * g->G.n[1] * g->G.n[2];
     const unsigned nb = std::min<unsigned>(blocks_for(N, 256), 65535u);
-    k_pack<<<nb, 256, 0, g->stream>>>(g->G, g->buf[g->cur], ddst, 0);
+    k_pack<<<nb, 256, 0, g->stream>>>(g->G, g->buf[g->cur], ddst, 0, !g->raw);
     SF_HIP(hipGetLastError());
     return 0;
 }
@@ -648,8 +617,10 @@ int sf_step_prepare(sf_grid* g) {
     if (int rc = set_device(g)) return rc;
     if (g->step_open) return fail(SF_E_STATE, "sf_step_prepare: a step is open");
     if (!g->ghosts_valid) {
-        if (int rc = fill_ghosts(g, g->buf[g->cur], 1, next_tag(g, kPhaseFill))) return rc;
+        if (int rc = fill_ghosts(g, g->buf[g->cur], next_tag(g, kPhaseFill))) return rc;
         g->ghosts_valid = 1;
+        g->stored = 1;
+        g->raw = 0;
     }
     return 0;
 }
@@ -717,10 +688,12 @@ int sf_step_commit(sf_grid* g) {
         return fail(SF_E_STATE, "sf_step_commit: stages incomplete");
     if (int rc = set_device(g)) return rc;
     g->cur = g->stage_out[nstages(g->desc.time) - 1];
-    if (int rc = fill_ghosts(g, g->buf[g->cur], 0, open_tag(g, kPhaseFill))) return rc;
+    if (g->separate)
+        if (int rc = fill_ghosts(g, g->buf[g->cur], (g->seq - 1) * 8 + kPhaseFill)) return rc;
     k_commit_clock<<<1, 64, 0, g->stream>>>(g->clock, g->flags);
     SF_HIP(hipGetLastError());
     g->ghosts_valid = 1;
+    g->stored = g->separate;
     g->dtmin_valid = g->fold_cfl;
     g->dtmin_cfl = g->step_cfl;
     g->step_open = 0;
@@ -792,10 +765,10 @@ int sf_residual(sf_grid* g, double* soa_out) {
     A.dtmin = &g->clock->dtmin;
     A.fault_tag = &g->fault->tag;
     A.tag = next_tag(g, 0);
-    if (int rc = run_sweeps(g, g->buf[g->cur], A)) return rc;
+    if (int rc = run_sweeps(g, g->buf[g->cur], A, g->stored != 0)) return rc;
     const long long N = (long long)g->G.n[0] * g->G.n[1] * g->G.n[2];
     const unsigned nb = std::min<unsigned>(blocks_for(N, 256), 65535u);
-    k_pack<<<nb, 256, 0, g->stream>>>(g->G, g->buf[scratch], g->stage_io, 0);
+    k_pack<<<nb, 256, 0, g->stream>>>(g->G, g->buf[scratch], g->stage_io, 0, 0);
     SF_HIP(hipGetLastError());
     SF_HIP(hipMemcpyAsync(soa_out, g->stage_io, sizeof(double) * 5 * (size_t)N,
                           hipMemcpyDeviceToHost, g->stream));

@@ -46,17 +46,12 @@ struct GridDev {
     double jac, area[3], gamma;
     double metric[3];   // 1 / spacing on active axes, 0 on inactive ones
     double d[3];        // node spacing (the Lax-Wendroff flux's face spacing)
-    // Bit a set: the final sweep writes every node it updates also into the
-    // periodic ghost positions of axis a that hold its copies, so no ghost
-    // fill is needed for that axis between stages.  A node c of such an axis
-    // has a copy unless g <= c < n - g, i.e. when (unsigned)(c - img_lo[a])
-    // >= img_span[a] (img_lo = g, img_span = n - 2g): at c + n (img_off =
-    // n * stride) if c < g, at c - n otherwise.  On other axes img_lo = 0
-    // and img_span = UINT_MAX, so no node has a copy.
-    int images;
-    int img_lo[3];
-    unsigned img_span[3];
-    long long img_off[3];
+    // Where the value of a ghost is read from, per axis (map_node): beyond a
+    // zeroGradient end from its first ghost layer, which every layer equals,
+    // beyond a periodic one from the node a period away; an end without a
+    // condition keeps its stored ghosts.
+    int map_lo[3], map_hi[3], wrap[3];
+    int zg_lo[3], zg_hi[3];   // 1 where the end carries zeroGradient
     // Nodes the stage advances along each axis: solved_lo[a] .. solved_hi[a]
     // (a zeroGradient end's node is excluded; see solved_node).
     int solved_lo[3], solved_hi[3];
@@ -205,37 +200,43 @@ __device__ __forceinline__ void raise_fault(unsigned f, unsigned* flags, long lo
     if (f && atomicOr(flags, f) == 0u && tag_out) *tag_out = tag;
 }
 
-// Node (i, j, k) at `id` was just written with qn: copy it into the ghost
-// positions of the axes in G.images that hold its periodic copies (node c
-// of an axis with n nodes and g ghost layers is ghost c + n if c < g and
-// ghost c - n if c >= n - g; the host sets an axis's bit only where
-// n >= 2g, so there is at most one copy per axis).  The sweeps read ghosts
-// only along their own axis, so no corner copies are needed.
-__device__ __forceinline__ void write_images(const GridDev& G, double* __restrict__ out, int i,
-                                             int j, int k, long long id, const double qn[5]) {
-    const int c[3] = {i, j, k};
-#pragma unroll
-    for (int a = 0; a < 3; ++a) {
-        if ((unsigned)(c[a] - G.img_lo[a]) < G.img_span[a]) continue;
-        const long long off = c[a] < G.img_lo[a] ? G.img_off[a] : -G.img_off[a];
-#pragma unroll
-        for (int v = 0; v < 5; ++v) out[v * G.P + id + off] = qn[v];
-    }
+// The coordinate along axis a whose stored value stands for coordinate c, a
+// node or ghost within the halo.
+__device__ __forceinline__ int map_node(const GridDev& G, int a, int c) {
+    c = min(max(c, G.map_lo[a]), G.map_hi[a]);
+    c += c < 0 ? G.wrap[a] : 0;
+    return c - (c >= G.n[a] ? G.wrap[a] : 0);
 }
 
-// The reference updates the state in place, so a node that the stage does
-// not advance (a solver-boundary node) keeps the value of the last ghost
-// fill; with separate input and output buffers it is copied across.
-template <int TIME = -1, class GT>
-__device__ __forceinline__ void carry_node(const GT& G, const StageArgs& A, long long id,
-                                           const double* __restrict__ q, double qn[5]) {
-    const int time = TIME >= 0 ? TIME : A.time;
-    if (time == 3) return;
-#pragma unroll
-    for (int v = 0; v < 5; ++v) {
-        qn[v] = q[v * G.P + id];
-        A.qout[v * G.P + id] = qn[v];
-    }
+// Energies of a zeroGradient end whose inner neighbour holds q: density and
+// momentum are the neighbour's, the boundary node's energy is rebuilt from
+// the neighbour's pressure and the ghosts' from the boundary node's
+// (SF_zeroGradient.cpp:88-130, SF_thermodynamicClosure.cpp:219-281), in the
+// reference's own order of operations: both equal q[4] up to rounding, and a
+// run that amplifies rounding at an outflow end follows the reference only
+// if that is rounded as there.  ok: both pressures are positive.
+struct EndEnergy {
+    double node, ghost;
+    bool ok;
+};
+
+__device__ __forceinline__ EndEnergy end_energy(const double q[5], double gamma) {
+    const double r = q[0], inv = frcp(r);
+    const double u = q[1] * inv, v = q[2] * inv, w = q[3] * inv;
+    const double kin = 0.5 * r * (u * u + v * v + w * w);
+    const double kinetic = 0.5 * inv * (q[1] * q[1] + q[2] * q[2] + q[3] * q[3]);
+    const double d = (gamma - 1.0) * r, rd = frcp(d);
+    const auto rebuilt = [&](double p) {
+        const double x = p * rd;
+        return r * fma(fma(-d, x, p), rd, x) + kinetic;
+    };
+    const double ps = d * ((q[4] - kin) * inv);
+    EndEnergy e;
+    e.node = rebuilt(ps);
+    const double pb = d * ((e.node - kin) * inv);
+    e.ghost = rebuilt(pb);
+    e.ok = ps > 0.0 && pb > 0.0;
+    return e;
 }
 
 // Stage update of one node from its current value qc and (SSPRK3 after
@@ -283,38 +284,6 @@ __device__ __forceinline__ void stage_update_dt(const GT& G, const StageArgs& A,
     if (A.reduce_dt) dt_local = local_dt(G, qn, A.cfl, flags);
 }
 
-// stage_update_dt with the step's dt read from *A.dt.
-template <int TIME = -1, class GT>
-__device__ __forceinline__ void stage_update_values(const GT& G, const StageArgs& A,
-                                                    long long id, const double qc[5],
-                                                    const double q0v[5], const double S[5],
-                                                    unsigned& flags, double& dt_local,
-                                                    double qn[5]) {
-    const int time = TIME >= 0 ? TIME : A.time;
-    const double dt = time == 3 ? 0.0 : *A.dt;
-    stage_update_dt<TIME>(G, A, id, qc, q0v, S, dt, flags, dt_local, qn);
-}
-
-// Whether a stage of recipe `time` reads the step-start state q0.
-__device__ __forceinline__ bool stage_reads_q0(int time, int stage) {
-    return (time == 1 && stage > 0) || time == 2;
-}
-
-// stage_update_values with qc and q0v read here.
-template <int TIME = -1, class GT>
-__device__ __forceinline__ void stage_update(const GT& G, const StageArgs& A, long long id,
-                                             const double* __restrict__ q, const double S[5],
-                                             unsigned& flags, double& dt_local, double qn[5]) {
-    const int time = TIME >= 0 ? TIME : A.time;
-    double qc[5], q0v[5];
-#pragma unroll
-    for (int v = 0; v < 5; ++v) {
-        qc[v] = time == 3 ? 0.0 : q[v * G.P + id];
-        q0v[v] = stage_reads_q0(time, A.stage) ? A.q0[v * G.P + id] : 0.0;
-    }
-    stage_update_values<TIME>(G, A, id, qc, q0v, S, flags, dt_local, qn);
-}
-
 // Block-wide minimum of a positive double into *target (one atomic; every
 // thread of the block calls it).
 __device__ __forceinline__ void block_min_atomic(double v, unsigned long long* target,
@@ -341,22 +310,5 @@ struct Clock {
     double max_dt;
     double limit;
 };
-
-__device__ __forceinline__ double pressure_of(const double* q, long long P, long long id,
-                                              double gamma) {
-    double qq[5];
-#pragma unroll
-    for (int v = 0; v < 5; ++v) qq[v] = q[v * P + id];
-    return close_state(qq, gamma).p;
-}
-
-// totalEnergyFromPressure (SF_singleFluidStateModel.cpp:73-109).
-__device__ __forceinline__ double energy_from_pressure(const double* q, long long P, long long id,
-                                                       double gamma, double p) {
-    const double r = q[id], m1 = q[P + id], m2 = q[2 * P + id], m3 = q[3 * P + id];
-    const double e = p / ((gamma - 1.0) * r);
-    const double kinetic = 0.5 * (1.0 / r) * fma(m3, m3, fma(m2, m2, m1 * m1));
-    return fma(r, e, kinetic);
-}
 
 }  // namespace sfamd

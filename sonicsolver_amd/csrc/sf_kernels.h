@@ -6,7 +6,12 @@
 // halo (2 for WENO3, 3 for WENO5 / TENO5, 4 for WENO7) on every active axis
 // (m_d = n_d + 2 g) and none on an inactive one.  Work per RK stage:
 //
-//   ghost fill (O(surface))      k_bc_copy4 / k_bc_energy / k_bc_periodic
+//   boundary closure             none of its own: k_stage_yx writes the
+//                                boundary node and the first ghost next to a
+//                                node it advances at a zeroGradient end, and
+//                                the marches read the node that stands for a
+//                                ghost (map_node); k_fill stores all ghosts
+//                                after an upload and for the separate x sweeps
 //   z sweep                      k_sweep_march: one lane per (x, column
 //                                               segment), marching along the
 //                                               axis with the stencil window
@@ -89,8 +94,66 @@ __global__ void k_commit_clock(Clock* c, const unsigned* flags) {
 }
 
 // ---------------------------------------------------------------------------
-// Ghost fill.  Thread per boundary-plane point (2 sides x plane).
+// Stores the boundary nodes and ghost layers of q: a thread per (side, layer,
+// point) of every axis with a zeroGradient or periodic end, each taking the
+// advanced node that stands for its own, so no thread reads what another
+// writes.  Layer 0 is the boundary node.  Along x the layers of a row are
+// the adjacent doubles, so they are the fastest index there; on the other
+// axes x is.
 // ---------------------------------------------------------------------------
+struct FillCount {
+    long long end[3];   // threads of axes 0 .. a
+};
+
+__global__ __launch_bounds__(256) void k_fill(GridDev G, double* __restrict__ q, FillCount F,
+                                              Fault* fault, long long tag) {
+    if (fault->flags) return;
+    long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x;
+    if (t >= F.end[2]) return;
+    const int axis = t < F.end[0] ? 0 : t < F.end[1] ? 1 : 2;
+    if (axis > 0) t -= F.end[axis - 1];
+    const int layers = G.g[axis] + 1;
+    int p[3], side, l;
+    if (axis == 0) {
+        l = (int)(t % layers);
+        t /= layers;
+        side = (int)(t & 1);
+        t >>= 1;
+        p[1] = (int)(t % G.n[1]);
+        p[2] = (int)(t / G.n[1]);
+    } else {
+        const int o = 3 - axis;
+        p[0] = (int)(t % G.n[0]);
+        t /= G.n[0];
+        p[o] = (int)(t % G.n[o]);
+        t /= G.n[o];
+        side = (int)(t & 1);
+        l = (int)(t >> 1);
+    }
+    const bool zg = zg_end(G, axis, side);
+    if (!zg && (G.wrap[axis] == 0 || l == 0)) return;
+    p[axis] = side ? G.n[axis] - 1 + l : -l;
+    const long long dst = node_index(G, p[0], p[1], p[2]);
+#pragma unroll
+    for (int a = 0; a < 3; ++a) {   // the advanced node
+        p[a] = map_node(G, a, p[a]);
+        if (G.zg_lo[a]) p[a] = max(p[a], G.solved_lo[a]);
+        if (G.zg_hi[a]) p[a] = min(p[a], G.solved_hi[a]);
+    }
+    const long long src = node_index(G, p[0], p[1], p[2]);
+    double v5[5];
+#pragma unroll
+    for (int v = 0; v < 5; ++v) v5[v] = q[v * G.P + src];
+    if (zg) {
+        const EndEnergy e = end_energy(v5, G.gamma);
+        if (l == 0 && !e.ok) raise_fault(kFlagState, &fault->flags, &fault->tag, tag);
+        v5[4] = l == 0 ? e.node : e.ghost;
+    }
+#pragma unroll
+    for (int v = 0; v < 5; ++v) q[v * G.P + dst] = v5[v];
+}
+
+// Thread per boundary-plane point (2 sides x plane).
 template <int AXIS>
 __device__ __forceinline__ bool plane_point(const GridDev& G, long long t, int p[3], int& side) {
     constexpr int e1 = (AXIS + 1) % 3, e2 = (AXIS + 2) % 3;
@@ -102,83 +165,6 @@ __device__ __forceinline__ bool plane_point(const GridDev& G, long long t, int p
     p[e2] = (int)(r / G.n[e1]);
     p[AXIS] = side ? G.n[AXIS] - 1 : 0;
     return true;
-}
-
-// Threads per boundary point of a fill along AXIS: along y and z one per
-// point (a point's neighbours on the plane are adjacent in memory); along
-// x, where the boundary node and its ghosts are the adjacent doubles of one
-// row and the plane's points lie a row apart, one per (variable, node) for
-// the copy and one per node for the energy, so that neighbouring lanes
-// write neighbouring doubles.
-template <int AXIS>
-__host__ __device__ __forceinline__ int fill_lanes(const GridDev& G, bool copy) {
-    return AXIS == 0 ? (copy ? 4 : 1) * (G.g[0] + 1) : 1;
-}
-
-// zeroGradient density + momentum (SF_zeroGradient.cpp:88-130) on the
-// zeroGradient ends of the axis; the ghost depth is G.g[AXIS].
-template <int AXIS>
-__global__ __launch_bounds__(256) void k_bc_copy4(GridDev G, double* __restrict__ q,
-                                                  const unsigned* flags) {
-    if (*flags) return;
-    int p[3], side;
-    const long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-    const int per = fill_lanes<AXIS>(G, true);
-    if (!plane_point<AXIS>(G, t / per, p, side)) return;
-    if (!zg_end(G, AXIS, side)) return;
-    const long long step = G.stride[AXIS];
-    const long long b = node_index(G, p[0], p[1], p[2]);
-    const long long s = side ? b - step : b + step;
-    const long long dir = side ? step : -step;
-    if (AXIS == 0) {
-        const int u = (int)(t % per), v = u / (G.g[0] + 1), l = u % (G.g[0] + 1);
-        q[v * G.P + b + l * dir] = q[v * G.P + s];   // l = 0: the boundary node
-        return;
-    }
-#pragma unroll
-    for (int v = 0; v < 4; ++v) {
-        const double val = q[v * G.P + s];
-        q[v * G.P + b] = val;
-        for (int l = 1; l <= G.g[AXIS]; ++l) q[v * G.P + b + l * dir] = val;
-    }
-}
-
-// zeroGradient pressure -> energy (SF_thermodynamicClosure.cpp:219-281).
-template <int AXIS>
-__global__ __launch_bounds__(256) void k_bc_energy(GridDev G, double* __restrict__ q,
-                                                   Fault* fault, long long tag) {
-    if (fault->flags) return;
-    int p[3], side;
-    const long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-    const int per = fill_lanes<AXIS>(G, false);
-    if (!plane_point<AXIS>(G, t / per, p, side)) return;
-    if (!zg_end(G, AXIS, side)) return;
-    const long long step = G.stride[AXIS];
-    const long long b = node_index(G, p[0], p[1], p[2]);
-    const long long s = side ? b - step : b + step;
-    const long long dir = side ? step : -step;
-    const double ps = pressure_of(q, G.P, s, G.gamma);
-    if (AXIS == 0) {
-        // each lane of the point forms the boundary node's energy and
-        // pressure from the same values; lane 0 stores it, lane l >= 1
-        // fills ghost l
-        const int u = (int)(t % per);
-        const double eb = energy_from_pressure(q, G.P, b, G.gamma, ps);
-        double qb[5] = {q[b], q[G.P + b], q[2 * G.P + b], q[3 * G.P + b], eb};
-        const double pb = close_state(qb, G.gamma).p;
-        if (u == 0) {
-            q[4 * G.P + b] = eb;
-            if (!(ps > 0.0) || !(pb > 0.0)) raise_fault(kFlagState, &fault->flags, &fault->tag, tag);
-        } else {
-            q[4 * G.P + b + u * dir] = energy_from_pressure(q, G.P, b + u * dir, G.gamma, pb);
-        }
-        return;
-    }
-    q[4 * G.P + b] = energy_from_pressure(q, G.P, b, G.gamma, ps);
-    const double pb = pressure_of(q, G.P, b, G.gamma);
-    if (!(ps > 0.0) || !(pb > 0.0)) raise_fault(kFlagState, &fault->flags, &fault->tag, tag);
-    for (int l = 1; l <= G.g[AXIS]; ++l)
-        q[4 * G.P + b + l * dir] = energy_from_pressure(q, G.P, b + l * dir, G.gamma, pb);
 }
 
 // An end without a condition: its ghost layers take the end node's state
@@ -200,28 +186,6 @@ __global__ __launch_bounds__(256) void k_bc_hold(GridDev G, const double* __rest
     }
 }
 
-// Periodic: ghost layer l on either side takes the node (index mod n).
-template <int AXIS>
-__global__ __launch_bounds__(256) void k_bc_periodic(GridDev G, double* __restrict__ q,
-                                                     const unsigned* flags) {
-    if (*flags) return;
-    int p[3], side;
-    const long long t = blockIdx.x * (long long)blockDim.x + threadIdx.x;
-    if (!plane_point<AXIS>(G, t, p, side)) return;
-    const long long step = G.stride[AXIS];
-    const int n = G.n[AXIS];
-    p[AXIS] = 0;
-    const long long base = node_index(G, p[0], p[1], p[2]);  // node 0 on the axis
-    for (int l = 1; l <= G.g[AXIS]; ++l) {
-        // low side: ghost -l <- node n-l ; high side: ghost n-1+l <- node l-1
-        const long long dst = side ? base + (long long)(n - 1 + l) * step : base - l * step;
-        const long long src = side ? base + (long long)((l - 1) % n) * step
-                                   : base + (long long)(((n - l) % n + n) % n) * step;
-#pragma unroll
-        for (int v = 0; v < 5; ++v) q[v * G.P + dst] = q[v * G.P + src];
-    }
-}
-
 // Clear a fault record (a kernel rather than a memset, so that the clear
 // can also be captured in a graph).
 __global__ void k_clear_fault(Fault* fault) {
@@ -232,16 +196,30 @@ __global__ void k_clear_fault(Fault* fault) {
     }
 }
 
-// Copy between the caller's unique-node SoA and the padded layout.
+// Copy between the caller's unique-node SoA and the padded layout.  A stage
+// writes the boundary nodes next to advanced ones only: with `ends` set, a
+// node on two or three zeroGradient ends takes the value of the one on the
+// first of them.
 __global__ __launch_bounds__(256) void k_pack(GridDev G, const double* __restrict__ src,
-                                              double* __restrict__ dst, int to_padded) {
+                                              double* __restrict__ dst, int to_padded,
+                                              int ends) {
     const long long N = (long long)G.n[0] * G.n[1] * G.n[2];
     for (long long u = blockIdx.x * (long long)blockDim.x + threadIdx.x; u < N;
          u += (long long)gridDim.x * blockDim.x) {
         const int i = (int)(u % G.n[0]);
         const int j = (int)((u / G.n[0]) % G.n[1]);
         const int k = (int)(u / ((long long)G.n[0] * G.n[1]));
-        const long long id = node_index(G, i, j, k);
+        int p[3] = {i, j, k};
+        if (ends) {
+            bool on = false;
+#pragma unroll
+            for (int a = 0; a < 3; ++a) {
+                const int c = min(max(p[a], G.solved_lo[a]), G.solved_hi[a]);
+                if (on) p[a] = c;
+                on |= p[a] != c;
+            }
+        }
+        const long long id = node_index(G, p[0], p[1], p[2]);
 #pragma unroll
         for (int v = 0; v < 5; ++v) {
             if (to_padded) dst[v * G.P + id] = src[v * N + u];

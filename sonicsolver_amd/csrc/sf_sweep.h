@@ -124,7 +124,9 @@ int launch_sweep_fm(const SweepCall& c, int axis) {
     if constexpr (MODE == kFinal) {
         return -1;
     } else {
-        const unsigned other = (unsigned)(axis == 1 ? G.n[2] : G.n[1]);
+        // the advanced nodes along each axis
+        const auto span = [&](int a) { return G.solved_hi[a] - G.solved_lo[a] + 1; };
+        const unsigned other = (unsigned)span(3 - axis);
         const unsigned cols = (unsigned)((G.n[0] + kMarchBlock - 1) / kMarchBlock);
         // Each segment re-reads the stencil window and evaluates one extra
         // face at its start; march_cost weighs that against filling the
@@ -134,14 +136,14 @@ int launch_sweep_fm(const SweepCall& c, int axis) {
         if (seg <= 0) {
             double least = 0.0;
             for (int s = 1; s <= 64; ++s) {
-                const long long blocks = (long long)cols * other * ((G.n[axis] + s - 1) / s);
+                const long long blocks = (long long)cols * other * ((span(axis) + s - 1) / s);
                 const double cost = march_cost(blocks, s + 1.0, c.cus);
                 if (seg > 0 && cost >= least) continue;
                 least = cost;
                 seg = s;
             }
         }
-        const dim3 grid(cols, other, (unsigned)((G.n[axis] + seg - 1) / seg));
+        const dim3 grid(cols, other, (unsigned)((span(axis) + seg - 1) / seg));
         if (axis == 1)
             k_sweep_march<1, SCHEME, FLUX, MODE><<<grid, kMarchBlock, 0, c.stream>>>(
                 G, c.q, c.S, c.A, seg);
@@ -231,18 +233,20 @@ inline YxShape yx_shape(const SweepCall& c) {
     YxShape best{};
     const GridDev& G = c.G;
     if (!G.active[1] || c.x_walk >= 0 || c.A.time == 3) return best;
+    const int nx = G.solved_hi[0] - G.solved_lo[0] + 1, ny = G.solved_hi[1] - G.solved_lo[1] + 1;
+    const int nz = G.solved_hi[2] - G.solved_lo[2] + 1;
     double least = 0.0;
     // columns a block advances: 64 with its first x faces evaluated
     // beforehand, or 63 with lane 0 evaluating them
     for (int cols = kXBlock; cols >= kXBlock - 1; --cols) {
         YxShape sh{};
         sh.cols = cols;
-        sh.nx = (G.n[0] + cols - 1) / cols;
+        sh.nx = (nx + cols - 1) / cols;
         for (int rows = 1; rows <= kYxRows; ++rows) {
             if (c.seg > 0 && rows != std::min(c.seg, kYxRows)) continue;
             sh.rows = rows;
-            sh.ny = (G.n[1] + rows - 1) / rows;
-            const long long blocks = (long long)sh.nx * sh.ny * G.n[2];
+            sh.ny = (ny + rows - 1) / rows;
+            const long long blocks = (long long)sh.nx * sh.ny * nz;
             const double cost =
                 march_cost(blocks, 2.0 * rows + 1.0 + (cols == kXBlock ? 1.0 : 0.0), c.cus);
             if (best.blocks && cost >= least) continue;

@@ -171,13 +171,9 @@ __attribute__((amdgpu_waves_per_eu(3, 8))) void k_sweep_x(SweepArgs W) {
             } else if (TIME != 3) {
 #pragma unroll
                 for (int v = 0; v < 5; ++v) {
-                    qn[v] = pq[v];   // carry_node
+                    qn[v] = pq[v];   // not advanced: carried over
                     U.A.qout[v * U.G.P + id] = qn[v];
                 }
-            }
-            if (TIME != 3) {
-                const SweepArgs& V = sweep_args();
-                if (V.G.images) write_images(V.G, V.A.qout, a, j, k, id, qn);
             }
             dt_local = fmin(dt_local, dl);
         }
@@ -382,13 +378,9 @@ __attribute__((amdgpu_waves_per_eu(3, 8))) void k_sweep_xl(SweepArgs W) {
                     } else if (TIME != 3) {
 #pragma unroll
                         for (int v = 0; v < 5; ++v) {
-                            qn[v] = pq[v];   // carry_node
+                            qn[v] = pq[v];   // not advanced: carried over
                             U.A.qout[v * U.G.P + id] = qn[v];
                         }
-                    }
-                    if (TIME != 3) {
-                        const SweepArgs& V = sweep_args();
-                        if (V.G.images) write_images(V.G, V.A.qout, a, j, k, id, qn);
                     }
                     dt_local = fmin(dt_local, dl);
                 }
@@ -403,8 +395,9 @@ __attribute__((amdgpu_waves_per_eu(3, 8))) void k_sweep_xl(SweepArgs W) {
 }
 
 // ---------------------------------------------------------------------------
-// y / z sweep: lane = x index, blockIdx.y = the remaining transverse index,
-// blockIdx.z = segment of SEG nodes along the sweep axis.  Each lane marches
+// y / z sweep over the advanced nodes: lane = x index, blockIdx.y = the
+// remaining transverse index, blockIdx.z = segment of SEG nodes along the
+// sweep axis.  Each lane marches
 // along its column; the NS-node stencil window lives in LDS (one private
 // slot set per lane, a ring indexed by `head`), so between faces only the
 // previous face flux stays in registers.  Lanes never read each other's
@@ -433,17 +426,21 @@ void k_sweep_march(GridDev G,
     constexpr int W = NS - 2;    // LDS ring slots: nodes a+1-H .. a+H-2
     __shared__ double win[W][5][kMarchBlock];
     const int lane = threadIdx.x;
+    // Only advanced nodes need a sum, so the march covers their ranges; along
+    // x a boundary node takes the sum of the node next to it, because S has
+    // to be written without holes: with node 0 of every row left out, the
+    // 201 x 87 x 45 z march took 80 us instead of 38.  Blocks start on
+    // 128-byte lines.
     const int i = blockIdx.x * kMarchBlock + lane;
-    const int o = blockIdx.y;
-    const int a0 = blockIdx.z * seg;
-    const int a1 = min(a0 + seg, G.n[AXIS]);
+    const int ic = min(max(i, G.solved_lo[0]), G.solved_hi[0]);
+    const int o = G.solved_lo[3 - AXIS] + blockIdx.y;
+    const int a0 = G.solved_lo[AXIS] + blockIdx.z * seg;
+    const int a1 = min(a0 + seg, G.solved_hi[AXIS] + 1);
     static_assert(MODE == kCopyS || MODE == kAccumS, "a march writes or accumulates S; the x sweep applies the update");
     if (*A.flags) return;   // a fault was raised: keep the step-start state
     unsigned flags = 0;
     const double lw = (FLUX == 5) ? *A.dt / G.d[AXIS] : 0.0;   // Lax-Wendroff dt / spacing
     if (i < G.n[0]) {
-        const int j0 = (AXIS == 1) ? a0 : o;
-        const int k0 = (AXIS == 2) ? a0 : o;
         const long long step = G.stride[AXIS];
         // The face a+1/2 reads its NS nodes as W from the lane's LDS ring
         // (nodes a+1-H .. a+H-2), node a+H-1 carried in registers from the
@@ -451,14 +448,15 @@ void k_sweep_march(GridDev G,
         // one node early (a = a0-1) so that face a0-1/2 is evaluated by the
         // same instructions as every other face: a face's rounding then does
         // not depend on where a segment starts.
-        long long id = node_index(G, i, j0, k0) - H * step;  // node a0-H
+        const long long col = node_index(G, ic, AXIS == 1 ? 0 : o, AXIS == 2 ? 0 : o);
+        const auto node = [&](int a) { return col + map_node(G, AXIS, a) * step; };
+        long long id = col + (i - ic) + (a0 - 1) * step;   // node a
         for (int s = 0; s < W; ++s)
 #pragma unroll
-            for (int v = 0; v < 5; ++v) win[s][v][lane] = q[v * G.P + id + s * step];
+            for (int v = 0; v < 5; ++v) win[s][v][lane] = q[v * G.P + node(a0 - H + s)];
         double carried[5];
 #pragma unroll
-        for (int v = 0; v < 5; ++v) carried[v] = q[v * G.P + id + W * step];  // node a0+H-2
-        id += (H - 1) * step;  // node a0 - 1
+        for (int v = 0; v < 5; ++v) carried[v] = q[v * G.P + node(a0 + H - 2)];
         int head = 0;          // slot of the oldest node
         double fprev[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
         // Pinned, so that the wait for the carried node stands here and not at
@@ -470,7 +468,7 @@ void k_sweep_march(GridDev G,
         for (int a = a0 - 1; a < a1; ++a, id += step) {
             double st[NS][5];
 #pragma unroll
-            for (int v = 0; v < 5; ++v) st[NS - 1][v] = q[v * G.P + id + H * step];
+            for (int v = 0; v < 5; ++v) st[NS - 1][v] = q[v * G.P + node(a + H)];
 #pragma unroll
             for (int s = 0; s < W; ++s) {
                 const int slot = (head + s >= W) ? head + s - W : head + s;
@@ -529,8 +527,12 @@ void k_sweep_march(GridDev G,
 }
 
 // ---------------------------------------------------------------------------
-// y and x faces and the stage update in one march along y: a block (one
-// wave) takes 64 columns of one z plane and up to kYxRows rows.  At row a
+// y and x faces and the stage update of the advanced nodes in one march along
+// y: a block (one wave) takes 64 columns of one z plane and up to kYxRows
+// rows.  Ghosts are read through map_node (a lane's column and a row's
+// number are mapped once each), and next to a zeroGradient end the launch
+// writes the boundary node and first ghost of what it advances, so no ghost
+// fill is needed between stages.  At row a
 // every lane evaluates its upper y face from its own column, as
 // k_sweep_march does, and its upper x face from the same row of the LDS
 // ring, whose rows carry the NS - 1 halo columns the x stencils reach; the
@@ -548,6 +550,37 @@ void k_sweep_march(GridDev G,
 // WENO7, whose ring is 17 KB).  yx_shape chooses the rows and columns.
 // ---------------------------------------------------------------------------
 constexpr int kYxRows = 32;
+
+// Node (i, j, k) at id was advanced to qn: next to a zeroGradient end, write
+// the boundary node and the first ghost layer (which stands for the others,
+// map_node).
+// Filling the ghosts by launches of their own took four 4-5 us launches per
+// stage in 2D and six in 3D, latency alone: a pass of 20 steps on 853^2 takes
+// 3.51 ms without them and 4.31 with, on 193 x 97 0.83 and 1.87.
+__device__ __forceinline__ void write_ends(const GridDev& G, double* __restrict__ out, int i,
+                                           int j, int k, long long id, const double qn[5]) {
+    const int c[3] = {i, j, k};
+    bool at_end = false;
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+        at_end |= (G.zg_lo[a] && c[a] == G.solved_lo[a]) || (G.zg_hi[a] && c[a] == G.solved_hi[a]);
+    if (!at_end) return;
+    const EndEnergy e = end_energy(qn, G.gamma);
+#pragma unroll
+    for (int a = 0; a < 3; ++a)
+#pragma unroll
+        for (int side = 0; side < 2; ++side) {
+            const bool here = side ? G.zg_hi[a] && c[a] == G.solved_hi[a]
+                                   : G.zg_lo[a] && c[a] == G.solved_lo[a];
+            if (!here) continue;
+            const long long dir = side ? G.stride[a] : -G.stride[a];
+#pragma unroll
+            for (int v = 0; v < 5; ++v) {
+                out[v * G.P + id + dir] = v == 4 ? e.node : qn[v];
+                out[v * G.P + id + 2 * dir] = v == 4 ? e.ghost : qn[v];
+            }
+        }
+}
 
 // Orders the LDS accesses of a wave's lanes among themselves: the hardware
 // performs a wave's LDS operations in order, so only the compiler has to
@@ -585,30 +618,38 @@ __attribute__((amdgpu_waves_per_eu(SCHEME == 3 ? 2 : 3, 8))) void k_stage_yx(Swe
     if (bid >= sh.blocks) return;
     const int t = threadIdx.x;
     const unsigned bx = bid % (unsigned)sh.nx, br = bid / (unsigned)sh.nx;
-    const int k = (int)(br / (unsigned)sh.ny);
-    const int a0 = (int)(br % (unsigned)sh.ny) * sh.rows;
-    const int a1 = min(a0 + sh.rows, W.G.n[1]);
+    const int k = W.G.solved_lo[2] + (int)(br / (unsigned)sh.ny);
+    const int a0 = W.G.solved_lo[1] + (int)(br % (unsigned)sh.ny) * sh.rows;
+    const int a1 = min(a0 + sh.rows, W.G.solved_hi[1] + 1);
     const int helper = kXBlock - sh.cols;              // 1: lane 0 only evaluates a face
-    const int i0 = (int)bx * sh.cols - helper;         // lane 0's column
+    const int i0 = W.G.solved_lo[0] + (int)bx * sh.cols - helper;   // lane 0's column
     const int i = i0 + t;
-    const int n0 = W.G.n[0];
-    const bool node = i < n0 && t >= helper;           // this lane advances node i
-    const int last = n0 - 1 + H;                       // the last ghost column
+    const int hi0 = W.G.solved_hi[0];
+    const bool node = i <= hi0 && t >= helper;         // this lane advances node i
+    const int last = hi0 + H;                          // the last column a face reads
     unsigned flags = 0;
     double dt_local = INFINITY;
     const double dt_step = *W.A.dt;   // the step's dt, read once
     const double lwx = (FLUX == 5) ? *W.A.dt / W.G.d[0] : 0.0;   // Lax-Wendroff dt / spacing
     const double lwy = (FLUX == 5) ? *W.A.dt / W.G.d[1] : 0.0;
+    // Rows are addressed from their first double (column -xo) by a lane's
+    // 32-bit byte offset.
+    const int xo = W.G.xo;
+    const auto row_of = [&](const GridDev& G, int a) {
+        return node_index(G, -xo, map_node(G, 1, a), k);
+    };
 
     // the block's first x faces (lower face of lane 0's node), lane r for
     // row a0 + r
     if (helper == 0 && a0 + t < a1) {
-        const long long id = node_index(W.G, i0 - 1, a0 + t, k);
+        const long long row = row_of(W.G, a0 + t);
         double st[NS][5];
 #pragma unroll
-        for (int s = 0; s < NS; ++s)
+        for (int s = 0; s < NS; ++s) {
+            const int c = map_node(W.G, 0, i0 - H + s) + xo;
 #pragma unroll
-            for (int v = 0; v < 5; ++v) st[s][v] = W.q[v * W.G.P + id + (s + 1 - H)];
+            for (int v = 0; v < 5; ++v) st[s][v] = W.q[v * W.G.P + row + c];
+        }
         double f5[5];
         face_flux<0, SCHEME, FLUX>(st, W.G.gamma, W.G.area[0], f5, flags, lwx);
         if (!finite_sum5(f5)) flags |= kFlagFlux;
@@ -616,36 +657,32 @@ __attribute__((amdgpu_waves_per_eu(SCHEME == 3 ? 2 : 3, 8))) void k_stage_yx(Swe
         for (int v = 0; v < 5; ++v) first[v][t] = f5[v];
     }
 
-    // Loads address a lane's column by a 32-bit byte offset from the row's
-    // column i0 (i0 >= -1 lies in every row).  Lanes past the grid load its
-    // last ghost column again, which the x faces before them read, and form
-    // faces that nothing takes.
-    const unsigned off = (unsigned)(min(i, last) - i0) * 8u;
+    // Lanes past the last column load it again and form faces that nothing
+    // takes.
+    const unsigned off = (unsigned)(map_node(W.G, 0, min(i, last)) + xo) * 8u;
     // halo: lane l < 5 HC loads variable l / HC, halo column l % HC
     const int hv = t / HC, hc = t % HC;
     const bool halo = hv < 5;
     const int hcol = hc < H - 1 ? hc - (H - 1) : kXBlock + hc - (H - 1);   // from i0
-    const int hcl = min(i0 + hcol, last);   // at least -H, the first ghost column
-    const long long step = W.G.stride[1];
-    const long long row0 = node_index(W.G, i0, a0, k);
-    const double* hsrc = W.q + (halo ? hv : 0) * W.G.P + row0 + (hcl - i0);
+    const double* hsrc =
+        W.q + (halo ? hv : 0) * W.G.P + (map_node(W.G, 0, min(i0 + hcol, last)) + xo);
     const int hpos = hcol + H - 1;
-
-    {
-        long long id = row0 - H * step;   // row a0 - H
-        for (int s = 0; s < R; ++s, id += step)
+    const long long step = W.G.stride[1];
+    const unsigned own = (unsigned)(i + xo) * 8u;   // the lane's own node, where it has one
+    for (int s = 0; s < R; ++s) {
+        const long long row = row_of(W.G, a0 - H + s);
 #pragma unroll
-            for (int v = 0; v < 5; ++v) win[s][v][t + H - 1] = at(W.q + v * W.G.P + id, off);
+        for (int v = 0; v < 5; ++v) win[s][v][t + H - 1] = at(W.q + v * W.G.P + row, off);
     }
     double carried[5];
 #pragma unroll
-    for (int v = 0; v < 5; ++v) carried[v] = at(W.q + v * W.G.P + row0 + (H - 2) * step, off);
+    for (int v = 0; v < 5; ++v) carried[v] = at(W.q + v * W.G.P + row_of(W.G, a0 + H - 2), off);
 #pragma unroll
     for (int v = 0; v < 5; ++v) asm volatile("" : "+v"(carried[v]));
     double hnext = 0.0;
     int head = 0;
     double fprev[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-    long long id = row0 - step;           // row a
+    long long id = node_index(W.G, -xo, a0 - 1, k);   // row a
     wave_lds_order();
 #pragma clang loop unroll(disable)
     for (int a = a0 - 1; a < a1; ++a, id += step) {
@@ -655,11 +692,11 @@ __attribute__((amdgpu_waves_per_eu(SCHEME == 3 ? 2 : 3, 8))) void k_stage_yx(Swe
         const auto slot = [&](int s) { return (head + s >= R) ? head + s - R : head + s; };
         if (halo) {
             win[slot(H - 1)][hv][hpos] = hnext;
-            hnext = hsrc[(a + 1 - a0) * step];
+            hnext = hsrc[row_of(T.G, a + 1)];
         }
         double st[NS][5];
 #pragma unroll
-        for (int v = 0; v < 5; ++v) st[NS - 1][v] = at(T.q + v * T.G.P + id + H * step, off);
+        for (int v = 0; v < 5; ++v) st[NS - 1][v] = at(T.q + v * T.G.P + row_of(T.G, a + H), off);
 #pragma unroll
         for (int s = 0; s < R; ++s)
 #pragma unroll
@@ -709,8 +746,8 @@ __attribute__((amdgpu_waves_per_eu(SCHEME == 3 ? 2 : 3, 8))) void k_stage_yx(Swe
                     const SweepArgs& U = sweep_args();
 #pragma unroll
                     for (int v = 0; v < 5; ++v) {
-                        if (HAS_S) ps[v] = at(U.S + v * U.G.P + id, off);
-                        pq0[v] = at(U.A.q0 + v * U.G.P + id, off);
+                        if (HAS_S) ps[v] = at(U.S + v * U.G.P + id, node ? own : off);
+                        pq0[v] = at(U.A.q0 + v * U.G.P + id, node ? own : off);
                     }
                 }
 #pragma unroll
@@ -718,7 +755,7 @@ __attribute__((amdgpu_waves_per_eu(SCHEME == 3 ? 2 : 3, 8))) void k_stage_yx(Swe
             },
             T.G.gamma, T.G.area[0], f5, fx, lwx);
         if (!finite_sum5(f5)) fx |= kFlagFlux;
-        if (i < n0) flags |= fx;
+        if (i <= hi0) flags |= fx;
         double lower[5];
 #pragma unroll
         for (int v = 0; v < 5; ++v) {
@@ -736,18 +773,10 @@ __attribute__((amdgpu_waves_per_eu(SCHEME == 3 ? 2 : 3, 8))) void k_stage_yx(Swe
             }
             double dl = INFINITY;
             double qn[5];
-            const long long nid = id + t;
-            if (solved_node(U.G, i, a, k)) {
-                stage_update_dt<TIME>(U.G, U.A, nid, pq, pq0, s5, dt_step, flags, dl, qn);
-            } else {
-#pragma unroll
-                for (int v = 0; v < 5; ++v) {
-                    qn[v] = pq[v];   // carry_node
-                    U.A.qout[v * U.G.P + nid] = qn[v];
-                }
-            }
+            const long long nid = id + i + xo;
+            stage_update_dt<TIME>(U.G, U.A, nid, pq, pq0, s5, dt_step, flags, dl, qn);
             const SweepArgs& V = sweep_args();
-            if (V.G.images) write_images(V.G, V.A.qout, i, a, k, nid, qn);
+            write_ends(V.G, V.A.qout, i, a, k, nid, qn);
             dt_local = fmin(dt_local, dl);
         }
     }

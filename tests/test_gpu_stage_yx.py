@@ -40,3 +40,30 @@ def test_fused_launch_equals_separate_sweeps(n, bc, scheme, flux, time):
     for state, dts in out[1:]:
         assert np.array_equal(state, out[0][0])
         assert np.array_equal(dts, out[0][1])
+
+
+@pytest.mark.parametrize("n", [(70, 33), (40, 20, 9)])
+def test_boundary_nodes_follow_the_path_taken(n):
+    """An upload is handed back as it is until the boundary is prepared;
+    then every zeroGradient boundary node holds its inner neighbour.  Steps
+    may change between the fused launch and the separate sweeps, whose
+    ghosts are stored."""
+    q = wl.smooth_field(n)
+    desc = make_desc(n=n, bc=("transmissive", "none_hi", "periodic"),
+                     d=tuple(1.0 / x for x in n) + (1.0,) * (3 - len(n)))
+    shape = (5,) + tuple(reversed(n + (1,) * (3 - len(n))))
+    with Grid(desc) as g:
+        g.upload(q)
+        assert np.array_equal(g.download(), q)
+        g.prepare()
+        s = g.download().reshape(shape)
+        assert np.array_equal(s[:4, :, 1:, 0], q.reshape(shape)[:4, :, 1:, 1])
+        assert np.array_equal(s[:4, :, 0, :], s[:4, :, 1, :])
+        np.testing.assert_allclose(s[4, :, 1:, -1], q.reshape(shape)[4, :, 1:, -2], rtol=1e-15)
+        g.run(6, 0.3)
+        ref = g.download()
+        g.upload(q)
+        for walk in (-1, 0, -1):
+            g.set_x_walk(walk)
+            g.run(2, 0.3)
+        assert np.array_equal(g.download(), ref)
