@@ -45,7 +45,8 @@ void set_last_error(const std::string& message) { g_last_error = message; }
 
 namespace {
 
-constexpr unsigned long long kInfBits = 0x7FF0000000000000ull;
+constexpr size_t kDtBytes = sizeof(unsigned long long) * kDtSlots * kDtStride;
+constexpr int kPinnedDts = 480;   // dt values that come back through pinned memory
 
 }  // namespace
 
@@ -56,9 +57,16 @@ struct sf_grid {
     double* buf[3] = {nullptr, nullptr, nullptr};
     double* S = nullptr;
     double* k[3] = {nullptr, nullptr, nullptr};
-    Clock* clock = nullptr;
-    Fault* fault = nullptr;      // device fault record
-    unsigned* flags = nullptr;   // &fault->flags
+    Control* ctl = nullptr;      // device clock and fault record
+    Clock* clock = nullptr;      // &ctl->clock
+    Fault* fault = nullptr;      // &ctl->fault
+    unsigned* flags = nullptr;   // &ctl->fault.flags
+    unsigned long long* slots = nullptr;   // CFL accumulator
+    // Pinned host memory (null for sf_run_static): what k_clock last wrote
+    // there, followed by kPinnedDts doubles.  snapped: it is up to date once
+    // the stream has been waited for.
+    Control* host = nullptr;
+    int snapped = 0;
     long long seq = 0;           // sequence number of the next step to begin
     // The step with sequence number base_seq starts from buffer base_cur;
     // each step moves the current state by a fixed rotation of the three
@@ -78,7 +86,7 @@ struct sf_grid {
     int stored = 0;              // buf[cur] holds all boundary nodes and ghosts (k_fill)
     int separate = 0;            // the last stage ran the separate x sweep
     int raw = 0;                 // buf[cur] is an upload whose boundary is not prepared yet
-    int dtmin_valid = 0;         // clock->dtmin holds the scan of buf[cur]
+    int dtmin_valid = 0;         // the CFL accumulator holds the scan of buf[cur]
     double dtmin_cfl = 0.0;      // CFL number the folded scan used
     int step_open = 0;
     int next_stage = 0;
@@ -171,6 +179,7 @@ int fill_ghosts(sf_grid* g, double* q, long long tag) {
         F.end[a] = n;
     }
     if (n == 0) return 0;
+    g->snapped = 0;
     const int ev = prof_start(g, SF_KERNEL_GHOST);
     k_fill<<<blocks_for(n, 256), 256, 0, g->stream>>>(G, q, F, g->fault, tag);
     prof_stop(g, ev);
@@ -204,6 +213,7 @@ int run_sweeps(sf_grid* g, double* q, const StageArgs& A, bool stored) {
     };
     const YxShape yx = yx_shape(c);
     g->separate = yx.blocks == 0;
+    g->snapped = 0;
     if (g->separate && !stored)
         if (int rc = fill_ghosts(g, q, A.tag)) return rc;
     int axes[3], na = 0;
@@ -243,6 +253,13 @@ int rotation(int time) { return time == SF_TIME_RK4 ? 2 : 1; }
 long long stage_tag(const sf_grid* g, int s) { return (g->seq - 1) * 8 + s; }
 long long next_tag(const sf_grid* g, int phase) { return g->seq * 8 + phase; }
 
+// k_clock on the grid's stream; `snap` takes a snapshot for the host.
+void launch_clock(sf_grid* g, double* hist, int slot, int commit, int next_dt, bool snap) {
+    k_clock<<<1, kDtSlots, 0, g->stream>>>(g->ctl, g->slots, hist, slot, commit, next_dt,
+                                           snap ? g->host : nullptr);
+    g->snapped = snap && g->host;
+}
+
 // Wait for the grid's work and read its fault record.  With flags raised,
 // every launch after the faulting one returned at entry, so the buffer that
 // held the state at the start of the faulting step still holds it: it
@@ -251,11 +268,18 @@ long long next_tag(const sf_grid* g, int phase) { return g->seq * 8 + phase; }
 // 1-based number of the faulting step on the clock and its phase.
 int check_flags(sf_grid* g, const char* where, uint32_t* flags_out = nullptr,
                 long long* step_out = nullptr, int* phase_out = nullptr) {
-    Fault h{};
-    Clock c{};
-    SF_HIP(hipMemcpyAsync(&h, g->fault, sizeof h, hipMemcpyDeviceToHost, g->stream));
-    SF_HIP(hipMemcpyAsync(&c, g->clock, sizeof c, hipMemcpyDeviceToHost, g->stream));
-    SF_HIP(hipStreamSynchronize(g->stream));
+    Control ctl{};
+    if (g->host) {
+        if (!g->snapped) launch_clock(g, nullptr, 0, 0, 0, true);
+        SF_HIP(hipGetLastError());
+        SF_HIP(hipStreamSynchronize(g->stream));
+        ctl = *g->host;
+    } else {
+        SF_HIP(hipMemcpyAsync(&ctl, g->ctl, sizeof ctl, hipMemcpyDeviceToHost, g->stream));
+        SF_HIP(hipStreamSynchronize(g->stream));
+    }
+    const Fault& h = ctl.fault;
+    const Clock& c = ctl.clock;
     if (flags_out) *flags_out = h.flags;
     if (step_out) *step_out = h.flags ? c.steps + 1 : 0;
     if (phase_out) *phase_out = h.flags ? (int)(h.tag & 7) : -1;
@@ -286,28 +310,26 @@ int check_flags(sf_grid* g, const char* where, uint32_t* flags_out = nullptr,
     return fail(SF_E_NUMERIC, msg);
 }
 
-// The next step's CFL scan: folded into the last stage's update when
-// possible, otherwise a standalone pass.
-int scan_dt(sf_grid* g, double cfl) {
-    if (!(g->dtmin_valid && g->dtmin_cfl == cfl)) {
-        k_set_limits<<<1, 64, 0, g->stream>>>(g->clock, g->max_dt, g->limit, 1);
+// The dt limits of the steps that follow and, unless the last stage's update
+// folded it in, the CFL scan of the current state.
+int scan_dt(sf_grid* g, double cfl, double max_dt, double limit) {
+    const bool scan = !(g->dtmin_valid && g->dtmin_cfl == cfl);
+    if (scan || g->max_dt != max_dt || g->limit != limit) {
+        g->max_dt = max_dt;
+        g->limit = limit;
+        k_set_limits<<<1, kDtSlots, 0, g->stream>>>(g->clock, g->slots, max_dt, limit, scan);
+    }
+    if (scan) {
         const long long N = (long long)g->G.n[0] * g->G.n[1] * g->G.n[2];
         const unsigned nb = std::min<unsigned>(blocks_for(N, 256), 8192u);
         const int ev = prof_start(g, SF_KERNEL_CFL);
-        k_cfl<<<nb, 256, 0, g->stream>>>(g->G, g->buf[g->cur], cfl, &g->clock->dtmin, g->fault,
+        k_cfl<<<nb, 256, 0, g->stream>>>(g->G, g->buf[g->cur], cfl, g->slots, g->fault,
                                          next_tag(g, kPhaseScan));
         prof_stop(g, ev);
-        SF_HIP(hipGetLastError());
+        g->snapped = 0;
     }
-    g->dtmin_valid = 0;
-    return 0;
-}
-
-int set_limits(sf_grid* g, double max_dt, double limit) {
-    g->max_dt = max_dt;
-    g->limit = limit;
-    k_set_limits<<<1, 64, 0, g->stream>>>(g->clock, max_dt, limit, 0);
     SF_HIP(hipGetLastError());
+    g->dtmin_valid = 0;
     return 0;
 }
 
@@ -325,7 +347,7 @@ int do_stage(sf_grid* g, int s, int fold_dt) {
     A.qout = g->buf[out];
     for (int i = 0; i < 3; ++i) A.k[i] = g->k[i];
     A.dt = &g->clock->dt;
-    A.dtmin = &g->clock->dtmin;
+    A.dtmin = g->slots;
     A.flags = g->flags;
     A.time = g->desc.time;
     A.stage = s;
@@ -430,8 +452,8 @@ int grid_free(sf_grid* g) {
     for (double* p : g->buf) if (p) (void)hipFree(p);
     for (double* p : g->k) if (p) (void)hipFree(p);
     if (g->S) (void)hipFree(g->S);
-    if (g->clock) (void)hipFree(g->clock);
-    if (g->fault) (void)hipFree(g->fault);
+    if (g->slots) (void)hipFree(g->slots);   // and ctl, behind it
+    if (g->host) (void)hipHostFree(g->host);
     if (g->dt_hist) (void)hipFree(g->dt_hist);
     if (g->stage_io) (void)hipFree(g->stage_io);
     for (hipEvent_t e : g->ev_pool) (void)hipEventDestroy(e);
@@ -491,27 +513,32 @@ int sf_grid_create(const sf_grid_desc* desc, sf_grid** out) {
     if (!rc && desc->time == SF_TIME_RK4)
         for (int i = 0; i < 3 && !rc; ++i) rc = alloc(&g->k[i], state);
     if (!rc) rc = alloc(&g->stage_io, sizeof(double) * 5 * N);
-    if (!rc && hipMalloc(&g->clock, sizeof(Clock)) != hipSuccess)
+    void* ctl = nullptr;
+    if (!rc && hipMalloc(&ctl, kDtBytes + sizeof(Control)) != hipSuccess)
         rc = fail(SF_E_MEMORY, "sf_grid_create: clock allocation failed");
-    if (!rc && hipMalloc(&g->fault, sizeof(Fault)) != hipSuccess)
-        rc = fail(SF_E_MEMORY, "sf_grid_create: fault record allocation failed");
-    if (!rc) g->flags = &g->fault->flags;
+    if (!rc) {
+        g->slots = static_cast<unsigned long long*>(ctl);
+        g->ctl = reinterpret_cast<Control*>(static_cast<char*>(ctl) + kDtBytes);
+        g->clock = &g->ctl->clock;
+        g->fault = &g->ctl->fault;
+        g->flags = &g->fault->flags;
+    }
+    if (!rc && hipHostMalloc((void**)&g->host, sizeof(Control) + sizeof(double) * kPinnedDts,
+                             hipHostMallocDefault) != hipSuccess)
+        rc = fail(SF_E_MEMORY, "sf_grid_create: pinned host allocation failed");
     if (!rc && hipStreamCreateWithFlags(&g->stream, hipStreamNonBlocking) != hipSuccess)
         rc = fail(SF_E_HIP, "sf_grid_create: stream creation failed");
     if (rc) {
         grid_free(g);
         return rc;
     }
-    Clock c{};
-    c.dt = 0.0;
-    c.time = 0.0;
-    c.steps = 0;
-    c.dtmin = kInfBits;
-    c.max_dt = std::numeric_limits<double>::max();
-    c.limit = std::numeric_limits<double>::max();
-    Fault f{0u, 0u, -1};
-    if (hipMemcpy(g->clock, &c, sizeof c, hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(g->fault, &f, sizeof f, hipMemcpyHostToDevice) != hipSuccess ||
+    Control c{};
+    c.clock.max_dt = g->max_dt;
+    c.clock.limit = g->limit;
+    c.fault.tag = -1;
+    const std::vector<unsigned long long> inf(kDtSlots * kDtStride, 0x7FF0000000000000ull);
+    if (hipMemcpy(g->ctl, &c, sizeof c, hipMemcpyHostToDevice) != hipSuccess ||
+        hipMemcpy(g->slots, inf.data(), kDtBytes, hipMemcpyHostToDevice) != hipSuccess ||
         hipMemset(g->buf[0], 0, state) != hipSuccess ||
         hipMemset(g->buf[1], 0, state) != hipSuccess ||
         hipMemset(g->buf[2], 0, state) != hipSuccess ||
@@ -546,6 +573,7 @@ static int upload_from(sf_grid* g, const double* dsrc) {
     const GridDev& G = g->G;
     const long long N = (long long)G.n[0] * G.n[1] * G.n[2];
     const unsigned nb = std::min<unsigned>(blocks_for(N, 256), 65535u);
+    g->snapped = 0;
     k_clear_fault<<<1, 64, 0, g->stream>>>(g->fault);
     g->base_seq = g->seq;
     g->base_cur = g->cur;
@@ -632,16 +660,14 @@ int sf_compute_dt(sf_grid* g, double cfl, double max_dt, double limit, double* d
         return fail(SF_E_ARG, "sf_compute_dt: limits must be positive");
     if (int rc = set_device(g)) return rc;
     if (g->step_open) return fail(SF_E_STATE, "sf_compute_dt: a step is open");
-    if (int rc = set_limits(g, max_dt, limit)) return rc;
-    if (int rc = scan_dt(g, cfl)) return rc;
-    k_finalize_dt<<<1, 64, 0, g->stream>>>(g->clock, nullptr, 0, g->flags);
+    if (int rc = scan_dt(g, cfl, max_dt, limit)) return rc;
+    launch_clock(g, nullptr, 0, 0, 1, dt_out != nullptr);
     SF_HIP(hipGetLastError());
     g->step_cfl = cfl;
     if (dt_out) {
-        SF_HIP(hipMemcpyAsync(dt_out, &g->clock->dt, sizeof(double), hipMemcpyDeviceToHost,
-                              g->stream));
-        SF_HIP(hipStreamSynchronize(g->stream));
-        if (int rc = check_flags(g, "sf_compute_dt")) return rc;
+        const int rc = check_flags(g, "sf_compute_dt");
+        if (g->snapped) *dt_out = g->host->clock.dt;
+        return rc;
     }
     return 0;
 }
@@ -651,6 +677,7 @@ int sf_set_dt(sf_grid* g, double dt) {
     if (!(dt > 0.0) || !std::isfinite(dt)) return fail(SF_E_ARG, "sf_set_dt: invalid dt");
     if (int rc = set_device(g)) return rc;
     if (g->step_open) return fail(SF_E_STATE, "sf_set_dt: a step is open");
+    g->snapped = 0;
     k_set_dt<<<1, 64, 0, g->stream>>>(g->clock, dt);
     SF_HIP(hipGetLastError());
     return 0;
@@ -682,16 +709,11 @@ int sf_stage(sf_grid* g, int stage) {
     return 0;
 }
 
-int sf_step_commit(sf_grid* g) {
-    if (!g) return fail(SF_E_ARG, "sf_step_commit: null grid");
-    if (!g->step_open || g->next_stage != nstages(g->desc.time))
-        return fail(SF_E_STATE, "sf_step_commit: stages incomplete");
-    if (int rc = set_device(g)) return rc;
+// The step's result becomes the current state (the clock is the caller's).
+static int commit_state(sf_grid* g) {
     g->cur = g->stage_out[nstages(g->desc.time) - 1];
     if (g->separate)
         if (int rc = fill_ghosts(g, g->buf[g->cur], (g->seq - 1) * 8 + kPhaseFill)) return rc;
-    k_commit_clock<<<1, 64, 0, g->stream>>>(g->clock, g->flags);
-    SF_HIP(hipGetLastError());
     g->ghosts_valid = 1;
     g->stored = g->separate;
     g->dtmin_valid = g->fold_cfl;
@@ -700,22 +722,34 @@ int sf_step_commit(sf_grid* g) {
     return 0;
 }
 
+int sf_step_commit(sf_grid* g) {
+    if (!g) return fail(SF_E_ARG, "sf_step_commit: null grid");
+    if (!g->step_open || g->next_stage != nstages(g->desc.time))
+        return fail(SF_E_STATE, "sf_step_commit: stages incomplete");
+    if (int rc = set_device(g)) return rc;
+    if (int rc = commit_state(g)) return rc;
+    launch_clock(g, nullptr, 0, 1, 0, true);
+    SF_HIP(hipGetLastError());
+    return 0;
+}
+
 // nsteps whole steps queued on the grid's stream, dt = min(CFL dt, max_dt)
 // each; hist (device memory, may be null) receives the dt values.
 static int queue_steps(sf_grid* g, int nsteps, double cfl, double max_dt, double* hist) {
-    if (int rc = set_limits(g, max_dt, std::numeric_limits<double>::max())) return rc;
     g->fold_cfl = 1;
     g->step_cfl = cfl;
     for (int s = 0; s < nsteps; ++s) {
         if (int rc = sf_step_prepare(g)) return rc;
-        if (int rc = scan_dt(g, cfl)) return rc;
-        k_finalize_dt<<<1, 64, 0, g->stream>>>(g->clock, hist, s, g->flags);
-        SF_HIP(hipGetLastError());
+        if (int rc = scan_dt(g, cfl, max_dt, std::numeric_limits<double>::max())) return rc;
+        // one launch commits the step before and starts this one
+        launch_clock(g, hist, s, s > 0, 1, false);
         if (int rc = sf_step_begin(g)) return rc;
         for (int st = 0; st < nstages(g->desc.time); ++st)
             if (int rc = sf_stage(g, st)) return rc;
-        if (int rc = sf_step_commit(g)) return rc;
+        if (int rc = commit_state(g)) return rc;
     }
+    if (nsteps > 0) launch_clock(g, nullptr, 0, 1, 0, true);
+    SF_HIP(hipGetLastError());
     g->fold_cfl = 0;
     return 0;
 }
@@ -731,11 +765,16 @@ int sf_run(sf_grid* g, int nsteps, double cfl, double max_dt, double* dt_seq) {
         if (int rc = ensure_hist(g, nsteps)) return rc;
     }
     if (int rc = queue_steps(g, nsteps, cfl, max_dt, dt_seq ? g->dt_hist : nullptr)) return rc;
-    if (dt_seq && nsteps > 0) {
-        SF_HIP(hipMemcpyAsync(dt_seq, g->dt_hist, sizeof(double) * (size_t)nsteps,
+    // the dt values come back with the status, through pinned memory where
+    // they fit
+    const bool pinned = dt_seq && nsteps <= kPinnedDts;
+    double* const to = pinned ? reinterpret_cast<double*>(g->host + 1) : dt_seq;
+    if (dt_seq && nsteps > 0)
+        SF_HIP(hipMemcpyAsync(to, g->dt_hist, sizeof(double) * (size_t)nsteps,
                               hipMemcpyDeviceToHost, g->stream));
-    }
-    return check_flags(g, "sf_run");
+    const int rc = check_flags(g, "sf_run");
+    if (pinned) std::copy(to, to + nsteps, dt_seq);
+    return rc;
 }
 
 int sf_clock(sf_grid* g, double* time, long long* steps) {
@@ -762,7 +801,7 @@ int sf_residual(sf_grid* g, double* soa_out) {
     A.flags = g->flags;
     A.time = 3;  // residual only
     A.dt = &g->clock->dt;
-    A.dtmin = &g->clock->dtmin;
+    A.dtmin = g->slots;
     A.fault_tag = &g->fault->tag;
     A.tag = next_tag(g, 0);
     if (int rc = run_sweeps(g, g->buf[g->cur], A, g->stored != 0)) return rc;
@@ -784,6 +823,7 @@ int sf_error_flags(sf_grid* g, uint32_t* flags, int clear) {
     SF_HIP(hipStreamSynchronize(g->stream));
     *flags = h;
     if (clear) {
+        g->snapped = 0;
         k_clear_fault<<<1, 64, 0, g->stream>>>(g->fault);
         SF_HIP(hipGetLastError());
         SF_HIP(hipStreamSynchronize(g->stream));
@@ -858,14 +898,16 @@ namespace {
 
 constexpr size_t kStaticBytes = size_t(64) << 20;
 __device__ __align__(256) unsigned char scratch[kStaticBytes];
+__device__ __align__(128) unsigned long long scratch_slots[kDtSlots * kDtStride];
 
 // Device address of `scratch` on each device (its name is only a host-side
 // stand-in), taken once per device with that device current.
 constexpr int kMaxDevices = 64;
 unsigned char* g_scratch[kMaxDevices] = {};
+unsigned long long* g_scratch_slots[kMaxDevices] = {};
 std::mutex g_scratch_mutex;
 
-int static_scratch(int device, unsigned char** out) {
+int static_scratch(int device, unsigned char** out, unsigned long long** slots) {
     if (device < 0 || device >= kMaxDevices)
         return fail(SF_E_ARG, "sf_run_static: device ordinal out of range");
     std::lock_guard<std::mutex> lock(g_scratch_mutex);
@@ -875,9 +917,16 @@ int static_scratch(int device, unsigned char** out) {
         if (e != hipSuccess || !p)
             return fail(SF_E_HIP, std::string("sf_run_static: hipGetSymbolAddress: ") +
                                       hipGetErrorString(e));
+        void* ps = nullptr;
+        const hipError_t es = hipGetSymbolAddress(&ps, HIP_SYMBOL(scratch_slots));
+        if (es != hipSuccess || !ps)
+            return fail(SF_E_HIP, std::string("sf_run_static: hipGetSymbolAddress: ") +
+                                      hipGetErrorString(es));
         g_scratch[device] = static_cast<unsigned char*>(p);
+        g_scratch_slots[device] = static_cast<unsigned long long*>(ps);
     }
     *out = g_scratch[device];
+    *slots = g_scratch_slots[device];
     return 0;
 }
 
@@ -889,12 +938,12 @@ __global__ __launch_bounds__(256) void k_zero(double* __restrict__ p, long long 
         p[u] = 0.0;
 }
 
-__global__ void k_init_clock(Clock* c) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
+__global__ __launch_bounds__(kDtSlots) void k_init_clock(Clock* c, unsigned long long* slots) {
+    slots[threadIdx.x * kDtStride] = 0x7FF0000000000000ull;
+    if (threadIdx.x == 0) {
         c->dt = 0.0;
         c->time = 0.0;
         c->steps = 0;
-        c->dtmin = kInfBits;
         c->max_dt = std::numeric_limits<double>::max();
         c->limit = std::numeric_limits<double>::max();
     }
@@ -919,11 +968,11 @@ extern "C" int sf_run_static(const sf_grid_desc* desc, double* soa_device, int n
     if (hipDeviceGetAttribute(&g.cus, hipDeviceAttributeMultiprocessorCount, desc->device) !=
             hipSuccess || g.cus <= 0)
         g.cus = 256;
-    // scratch layout: clock, fault record, then the state buffers, the flux
+    // scratch layout: clock and fault record (512 bytes), then the state buffers, the flux
     // accumulator and (RK4) the three stage residuals
     const size_t state = round256(sizeof(double) * 5 * (size_t)g.G.P);
     const int nbuf = desc->time == SF_TIME_RK4 ? 7 : 4;
-    const size_t head = round256(sizeof(Clock)) + round256(sizeof(Fault));
+    const size_t head = 512;
     const size_t need = head + state * nbuf;
     if (scratch_bytes) *scratch_bytes = need;
     if (need > kStaticBytes) {
@@ -936,10 +985,12 @@ extern "C" int sf_run_static(const sf_grid_desc* desc, double* soa_device, int n
     }
     SF_HIP(hipSetDevice(desc->device));
     unsigned char* base = nullptr;
-    if (int rc = static_scratch(desc->device, &base)) return rc;
+    if (int rc = static_scratch(desc->device, &base, &g.slots)) return rc;
     g.stream = static_cast<hipStream_t>(stream);
-    g.clock = reinterpret_cast<Clock*>(base);
-    g.fault = reinterpret_cast<Fault*>(base + round256(sizeof(Clock)));
+    static_assert(sizeof(Control) <= 512, "the head of the scratch layout");
+    g.ctl = reinterpret_cast<Control*>(base);
+    g.clock = &g.ctl->clock;
+    g.fault = &g.ctl->fault;
     g.flags = &g.fault->flags;
     double* bufs[7];
     for (int i = 0; i < nbuf; ++i) bufs[i] = reinterpret_cast<double*>(base + head + state * i);
@@ -949,7 +1000,7 @@ extern "C" int sf_run_static(const sf_grid_desc* desc, double* soa_device, int n
         for (int i = 0; i < 3; ++i) g.k[i] = bufs[4 + i];
     // Every call on this device shares the array and finds the last call's
     // contents: the clock, the fault record and the buffers start cleared.
-    k_init_clock<<<1, 64, 0, g.stream>>>(g.clock);
+    k_init_clock<<<1, kDtSlots, 0, g.stream>>>(g.clock, g.slots);
     k_clear_fault<<<1, 64, 0, g.stream>>>(g.fault);
     const long long words = (long long)(state * nbuf / sizeof(double));
     k_zero<<<std::min<unsigned>(blocks_for(words, 256), 4096u), 256, 0, g.stream>>>(bufs[0], words);

@@ -42,17 +42,18 @@ namespace sfamd {
 // Standalone CFL scan (first step, or sf_compute_dt).
 // ---------------------------------------------------------------------------
 __global__ __launch_bounds__(256) void k_cfl(GridDev G, const double* __restrict__ q, double cfl,
-                                             unsigned long long* dtmin, Fault* fault,
+                                             unsigned long long* slots, Fault* fault,
                                              long long tag) {
     if (fault->flags) return;
-    const long long N = (long long)G.n[0] * G.n[1] * G.n[2];
+    const unsigned N = (unsigned)G.n[0] * G.n[1] * G.n[2];   // at most 2^31
     unsigned flags = 0;
     double best = INFINITY;
-    for (long long u = blockIdx.x * (long long)blockDim.x + threadIdx.x; u < N;
-         u += (long long)gridDim.x * blockDim.x) {
-        const int i = (int)(u % G.n[0]);
-        const int j = (int)((u / G.n[0]) % G.n[1]);
-        const int k = (int)(u / ((long long)G.n[0] * G.n[1]));
+    for (unsigned long long u = blockIdx.x * blockDim.x + threadIdx.x; u < N;
+         u += gridDim.x * blockDim.x) {
+        const unsigned line = (unsigned)u / (unsigned)G.n[0];
+        const int i = (int)((unsigned)u - line * (unsigned)G.n[0]);
+        const unsigned kz = fast_div(line, G.div_n1);
+        const int j = (int)(line - kz * (unsigned)G.n[1]), k = (int)kz;
         if (!solved_node(G, i, j, k)) continue;
         const long long id = node_index(G, i, j, k);
         double qq[5];
@@ -61,36 +62,49 @@ __global__ __launch_bounds__(256) void k_cfl(GridDev G, const double* __restrict
         best = fmin(best, local_dt(G, qq, cfl, flags));
     }
     raise_fault(flags, &fault->flags, &fault->tag, tag);
-    wave_min_atomic(best, dtmin);
+    wave_min_atomic(best, slots);
 }
 
-__global__ void k_finalize_dt(Clock* c, double* dt_hist, int slot, const unsigned* flags) {
-    if (threadIdx.x != 0 || blockIdx.x != 0 || *flags) return;
-    double dt = __longlong_as_double((long long)c->dtmin);
-    dt = fmin(dt, c->max_dt);
-    dt = fmin(dt, c->limit);
-    c->dt = dt;
-    c->dtmin = 0x7FF0000000000000ull;
-    if (dt_hist) dt_hist[slot] = dt;
+// The clock between two steps, by one wave: commit the step just taken, then
+// form the next step's dt from the CFL accumulator, which is reset for the
+// scan after it.  Nothing once a fault is raised.  snap (host memory, may be
+// null) receives the clock and the fault record as they are afterwards.
+__global__ __launch_bounds__(kDtSlots) void k_clock(Control* c, unsigned long long* slots,
+                                                    double* dt_hist, int slot, int commit,
+                                                    int next_dt, Control* snap) {
+    const int t = threadIdx.x;
+    if (!c->fault.flags) {
+        if (commit && t == 0) {
+            c->clock.time += c->clock.dt;
+            c->clock.steps += 1;
+        }
+        if (next_dt) {
+            const unsigned long long b = wave_min_bits(slots[t * kDtStride]);
+            slots[t * kDtStride] = 0x7FF0000000000000ull;
+            if (t == 0) {
+                double dt = __longlong_as_double((long long)b);
+                dt = fmin(dt, c->clock.max_dt);
+                dt = fmin(dt, c->clock.limit);
+                c->clock.dt = dt;
+                if (dt_hist) dt_hist[slot] = dt;
+            }
+        }
+    }
+    if (snap && t == 0) *snap = *c;
 }
 
 __global__ void k_set_dt(Clock* c, double dt) {
     if (threadIdx.x == 0 && blockIdx.x == 0) c->dt = dt;
 }
 
-__global__ void k_set_limits(Clock* c, double max_dt, double limit, int reset_scan) {
-    if (threadIdx.x == 0 && blockIdx.x == 0) {
+__global__ __launch_bounds__(kDtSlots) void k_set_limits(Clock* c, unsigned long long* slots,
+                                                         double max_dt, double limit,
+                                                         int reset_scan) {
+    if (threadIdx.x == 0) {
         c->max_dt = max_dt;
         c->limit = limit;
-        if (reset_scan) c->dtmin = 0x7FF0000000000000ull;
     }
-}
-
-__global__ void k_commit_clock(Clock* c, const unsigned* flags) {
-    if (threadIdx.x == 0 && blockIdx.x == 0 && !*flags) {
-        c->time += c->dt;
-        c->steps += 1;
-    }
+    if (reset_scan) slots[threadIdx.x * kDtStride] = 0x7FF0000000000000ull;
 }
 
 // ---------------------------------------------------------------------------
