@@ -210,8 +210,10 @@ int sf_grid_set_march_segment(sf_grid *grid, int nodes);
  * 0 by tiles of 63 faces over all lines numbered as one sequence, both as a
  * launch of their own after the y march; -1 (the default) in one launch with
  * the y faces on 2D and 3D grids, except on grids narrower than 32 nodes
- * that fill the device anyway.  1D grids, those narrow ones and sf_residual
- * choose between the two walks by the number of lines (lines where nx >= 64
+ * that fill the device anyway; sf_run takes whole steps of 1D grids of up to
+ * 2^20 nodes (2^17 with WENO7 and RK4) in one launch each.  What is left --
+ * larger 1D grids, sf_stage in 1D, those narrow grids and sf_residual --
+ * chooses between the two walks by the number of lines (lines where nx >= 64
  * and there are at least 256 per compute unit).  Grids whose variables exceed
  * 2^32 - 1024 bytes never walk by lines.  No reference counterpart; results
  * do not depend on it. */

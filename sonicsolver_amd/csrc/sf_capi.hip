@@ -45,7 +45,9 @@ void set_last_error(const std::string& message) { g_last_error = message; }
 
 namespace {
 
-constexpr size_t kDtBytes = sizeof(unsigned long long) * kDtSlots * kDtStride;
+// the grid's CFL accumulator and the three that k_step_1d uses in turn
+constexpr size_t kDtWords = (size_t)(1 + kStepSets) * kDtSlots * kDtStride;
+constexpr size_t kDtBytes = sizeof(unsigned long long) * kDtWords;
 constexpr int kPinnedDts = 480;   // dt values that come back through pinned memory
 
 }  // namespace
@@ -536,9 +538,10 @@ int sf_grid_create(const sf_grid_desc* desc, sf_grid** out) {
     c.clock.max_dt = g->max_dt;
     c.clock.limit = g->limit;
     c.fault.tag = -1;
-    const std::vector<unsigned long long> inf(kDtSlots * kDtStride, 0x7FF0000000000000ull);
-    if (hipMemcpy(g->ctl, &c, sizeof c, hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemcpy(g->slots, inf.data(), kDtBytes, hipMemcpyHostToDevice) != hipSuccess ||
+    std::vector<unsigned long long> init(kDtWords + sizeof c / 8, 0x7FF0000000000000ull);
+    static_assert(sizeof c % 8 == 0, "copied behind the accumulators");
+    std::memcpy(init.data() + kDtWords, &c, sizeof c);
+    if (hipMemcpy(g->slots, init.data(), init.size() * 8, hipMemcpyHostToDevice) != hipSuccess ||
         hipMemset(g->buf[0], 0, state) != hipSuccess ||
         hipMemset(g->buf[1], 0, state) != hipSuccess ||
         hipMemset(g->buf[2], 0, state) != hipSuccess ||
@@ -733,9 +736,57 @@ int sf_step_commit(sf_grid* g) {
     return 0;
 }
 
+// Whether a 1D grid's whole steps run in one launch each (k_step_1d), us per
+// step against a launch per stage: WENO5/SSPRK3 10 / 29 at 1000 nodes, 16 /
+// 34 at 65,000, 30 / 48 at 200,000, 121 / 141 at a million (TENO5 171 / 179);
+// with WENO7 and RK4, whose blocks advance 32 nodes on 64 lanes, 16 / 42 at
+// 1000, 45 / 56 at 100,000, 76 / 76 at 200,000, 304 / 273 at a million.
+static bool whole_steps(const sf_grid* g) {
+    const int advanced = 64 - 2 * g->G.g[0] * nstages(g->desc.time);
+    return !g->G.active[1] && g->x_walk < 0 && g->G.n[0] <= (advanced > 32 ? 1 << 20 : 1 << 17);
+}
+
+// queue_steps for a grid that takes whole steps.
+static int queue_steps_1d(sf_grid* g, int nsteps, double cfl, double max_dt, double* hist) {
+    if (int rc = sf_step_prepare(g)) return rc;
+    if (int rc = scan_dt(g, cfl, max_dt, std::numeric_limits<double>::max())) return rc;
+    launch_clock(g, hist, 0, 0, 1, false);
+    unsigned long long* const sets = g->slots + kDtSlots * kDtStride;
+    const auto set = [&](int s) { return sets + (s % kStepSets) * kDtSlots * kDtStride; };
+    for (int s = 0; s < nsteps; ++s) {
+        if (int rc = sf_step_begin(g)) return rc;
+        const int to = g->stage_out[nstages(g->desc.time) - 1];
+        const Step1dArgs W{g->G, g->buf[g->cur], g->buf[to], g->ctl,
+                           s ? set(s - 1) : nullptr, set(s), set(s + 1), hist, s, cfl,
+                           stage_tag(g, 0)};
+        const int ev = prof_start(g, SF_KERNEL_SWEEP_X);
+        int rc;
+        switch (g->desc.scheme) {
+        case SF_SCHEME_TENO5: rc = launch_step1d<1>(W, g->desc.flux, g->desc.time, g->stream); break;
+        case SF_SCHEME_WENO3: rc = launch_step1d<2>(W, g->desc.flux, g->desc.time, g->stream); break;
+        case SF_SCHEME_WENO7: rc = launch_step1d<3>(W, g->desc.flux, g->desc.time, g->stream); break;
+        default: rc = launch_step1d<0>(W, g->desc.flux, g->desc.time, g->stream); break;
+        }
+        prof_stop(g, ev);
+        if (rc) return fail(SF_E_STATE, "sf_run: no kernel for this recipe");
+        g->cur = to;
+        g->stored = 0;
+        g->step_open = 0;
+    }
+    k_close_1d<<<1, kDtSlots, 0, g->stream>>>(g->ctl, g->slots, set(nsteps - 1), sets, g->host);
+    g->snapped = g->host != nullptr;
+    g->step_cfl = cfl;
+    g->dtmin_valid = 1;
+    g->dtmin_cfl = cfl;
+    SF_HIP(hipGetLastError());
+    return 0;
+}
+
 // nsteps whole steps queued on the grid's stream, dt = min(CFL dt, max_dt)
 // each; hist (device memory, may be null) receives the dt values.
 static int queue_steps(sf_grid* g, int nsteps, double cfl, double max_dt, double* hist) {
+    if (nsteps > 0 && whole_steps(g))
+        return queue_steps_1d(g, nsteps, cfl, max_dt, hist);
     g->fold_cfl = 1;
     g->step_cfl = cfl;
     for (int s = 0; s < nsteps; ++s) {
@@ -898,7 +949,7 @@ namespace {
 
 constexpr size_t kStaticBytes = size_t(64) << 20;
 __device__ __align__(256) unsigned char scratch[kStaticBytes];
-__device__ __align__(128) unsigned long long scratch_slots[kDtSlots * kDtStride];
+__device__ __align__(128) unsigned long long scratch_slots[kDtWords];
 
 // Device address of `scratch` on each device (its name is only a host-side
 // stand-in), taken once per device with that device current.
@@ -939,7 +990,8 @@ __global__ __launch_bounds__(256) void k_zero(double* __restrict__ p, long long 
 }
 
 __global__ __launch_bounds__(kDtSlots) void k_init_clock(Clock* c, unsigned long long* slots) {
-    slots[threadIdx.x * kDtStride] = 0x7FF0000000000000ull;
+    for (int s = 0; s <= kStepSets; ++s)
+        slots[(s * kDtSlots + threadIdx.x) * kDtStride] = 0x7FF0000000000000ull;
     if (threadIdx.x == 0) {
         c->dt = 0.0;
         c->time = 0.0;

@@ -88,7 +88,7 @@ struct StageArgs {
 // stays as it was.
 struct Fault {
     unsigned flags;
-    unsigned pad;
+    unsigned stages;   // k_step_1d: the flags raised by stage s at bits 8 s
     long long tag;
 };
 enum { kPhaseFill = 6, kPhaseScan = 7 };
@@ -247,6 +247,16 @@ __device__ __forceinline__ EndEnergy end_energy(const double q[5], double gamma)
     return e;
 }
 
+// validateEquationState (SF_equationState.h:25-57): rho, p > 0, finite (p has
+// the sign of the internal energy; with the refined reciprocal of the
+// density instead of a division, that sign can differ only where the internal
+// energy is within an ulp of the kinetic energy).
+__device__ __forceinline__ void check_state(const double q[5], unsigned& flags) {
+    const double ke = 0.5 * dot3(q + 1, q + 1);
+    const double eint = fma(-ke, frcp(q[0]), q[4]);
+    if (!(q[0] > 0.0) || !(eint > 0.0) || !isfinite(eint)) flags |= kFlagState;
+}
+
 // Stage update of one node from its current value qc and (SSPRK3 after
 // the first stage, RK4) its step-start value q0v; S is the accumulated flux
 // difference and dt the step's dt (*A.dt, which no kernel of a stage
@@ -282,13 +292,7 @@ __device__ __forceinline__ void stage_update_dt(const GT& G, const StageArgs& A,
         }
         A.qout[v * G.P + id] = qn[v];
     }
-    // validateEquationState (SF_equationState.h:25-57): rho, p > 0, finite
-    // (p has the sign of the internal energy; with the refined reciprocal
-    // of the density instead of a division, that sign can differ only where
-    // the internal energy is within an ulp of the kinetic energy)
-    const double ke = 0.5 * dot3(qn + 1, qn + 1);
-    const double eint = fma(-ke, frcp(qn[0]), qn[4]);
-    if (!(qn[0] > 0.0) || !(eint > 0.0) || !isfinite(eint)) flags |= kFlagState;
+    check_state(qn, flags);
     if (A.reduce_dt) dt_local = local_dt(G, qn, A.cfl, flags);
 }
 

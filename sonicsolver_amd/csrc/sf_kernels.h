@@ -34,6 +34,7 @@
 // (SF_residualAssembly.h:12-32).
 #pragma once
 
+#include "sf_step1d.h"
 #include "sf_sweep_kernels.h"
 
 namespace sfamd {
@@ -90,6 +91,30 @@ __global__ __launch_bounds__(kDtSlots) void k_clock(Control* c, unsigned long lo
             }
         }
     }
+    if (snap && t == 0) *snap = *c;
+}
+
+// After the last k_step_1d of a run: commit it, hand the CFL scan it folded to
+// the grid's accumulator and clear the three that the steps used in turn.
+__global__ __launch_bounds__(kDtSlots) void k_close_1d(Control* c, unsigned long long* slots,
+                                                       const unsigned long long* scan,
+                                                       unsigned long long* sets, Control* snap) {
+    const int t = threadIdx.x;
+    if (!c->fault.flags) {
+        if (t == 0) {
+            c->clock.time += c->clock.dt;
+            c->clock.steps += 1;
+        }
+        slots[t * kDtStride] = scan[t * kDtStride];
+    } else if (t == 0 && c->fault.stages) {
+        // tiles run their stages independently: the record is the earliest
+        // stage's, whose flags a launch per stage would have stopped at
+        const int s = (__ffs((int)c->fault.stages) - 1) / 8;
+        c->fault.flags = (c->fault.stages >> (8 * s)) & 0xffu;
+        c->fault.stages = 0u;
+    }
+    for (int s = 0; s < kStepSets; ++s)
+        sets[(s * kDtSlots + t) * kDtStride] = 0x7FF0000000000000ull;
     if (snap && t == 0) *snap = *c;
 }
 
@@ -205,7 +230,7 @@ __global__ __launch_bounds__(256) void k_bc_hold(GridDev G, const double* __rest
 __global__ void k_clear_fault(Fault* fault) {
     if (threadIdx.x == 0 && blockIdx.x == 0) {
         fault->flags = 0u;
-        fault->pad = 0u;
+        fault->stages = 0u;
         fault->tag = -1;
     }
 }
