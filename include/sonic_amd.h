@@ -283,8 +283,9 @@ typedef struct {
 typedef struct sf_batch sf_batch;
 
 /* Padded device nodes a problem occupies in the arena (per variable); the
- * arena holds 4 values of 5 variables per node (three state buffers and the
- * flux accumulator), 160 bytes. */
+ * arena holds 3 values of 5 variables per node (three state buffers).
+ * Budgets in bytes count 160 per node, which leaves room for the tables and
+ * staging beside it. */
 int sf_batch_item_nodes(const sf_batch_item *item, size_t *nodes);
 /* A batch with an arena of node_capacity padded nodes and up to
  * item_capacity problems. */
@@ -312,17 +313,20 @@ int sf_batch_steps(sf_batch *batch, long long *steps);
 /* Arena occupancy in padded nodes, and the number of admitted problems. */
 int sf_batch_memory(const sf_batch *batch, size_t *used_nodes, size_t *free_nodes,
                     int *items);
-/* Tile shape of the persistent sweeps: x tiles of xlen nodes of one line
- * (63, 127 or 255), y tiles of 64 columns by ylen nodes (4..4096).  Takes
- * effect at the next step; results do not depend on it. */
+/* Tile shape of the stages: tiles of 1D problems of xlen nodes (63, 127 or
+ * 255, in strips of 63), of 2D problems of 63 or 64 columns by ylen rows
+ * (4..4096; more than 32 count as 32).  Until it is called, both are chosen
+ * by cost for the problems that the batch holds.  Takes effect at the next
+ * step; results do not depend on it. */
 int sf_batch_set_tiles(sf_batch *batch, int xlen, int ylen);
-/* Persistent grid size of the sweeps in workgroups per compute unit
- * (1..64), or 0 for as many as each sweep kernel keeps resident (the
- * runtime's occupancy figure).  Results do not depend on it. */
+/* Persistent grid size of the stages in workgroups per compute unit
+ * (1..64), or 0 for as many as each stage kernel keeps resident (the
+ * runtime's occupancy figure).  Until it is called, every tile has a
+ * workgroup of its own.  Results do not depend on it. */
 int sf_batch_set_occupancy(sf_batch *batch, int blocks_per_cu);
-/* Sweep schedule: fused != 0 runs one launch per sweep for every
- * (scheme, flux) variant (workgroup ranges assigned per variant); 0 runs one
- * launch per variant present (fewer registers per kernel).  Results do not
+/* Stage schedule: fused != 0 runs one launch per stage for every
+ * (scheme, flux) variant (workgroup ranges assigned per variant; one launch
+ * each for 1D and for 2D problems); 0 runs one launch per variant present.  Results do not
  * depend on it. */
 int sf_batch_set_schedule(sf_batch *batch, int fused);
 /* Per-problem device fault flags (SF_FLAG_*), item_capacity entries (0 for

@@ -68,8 +68,9 @@ int sf_server_result(sf_server *server, long long ticket, double *soa, double *t
 int sf_server_drain(sf_server *server, double timeout_s);
 int sf_server_stats(sf_server *server, sf_serve_stats *stats);
 /* Launch shape of the batch (as sf_batch_set_tiles / _occupancy /
- * _schedule); applied before the loop's next pass.  The default is
- * xlen 255, ylen 32, 16 workgroups per CU, one launch per variant. */
+ * _schedule); applied before the loop's next pass.  Without a call the
+ * batch's defaults hold: tile lengths chosen by cost for the problems it
+ * holds, a workgroup per tile, one launch for every variant. */
 int sf_server_set_shape(sf_server *server, int xlen, int ylen, int blocks_per_cu, int fused);
 /* How each pass launches its steps, as sf_batch_step's use_graph: 0 direct
  * launches, 1 one replayed hipGraph per step, 2 (the default) a graph when

@@ -3,7 +3,7 @@ entry points of include/sonic_amd.h).
 
 Every problem has its own size, scheme, flux, CFL number, dt and clock;
 one call of :meth:`Batch.step` advances every live problem by SSPRK3 steps
-with persistent kernels over a tile table, optionally replaying a captured
+with one launch per stage over a tile table, optionally replaying a captured
 hipGraph.  Boundaries are transmissive on every side.
 """
 from __future__ import annotations
@@ -17,7 +17,7 @@ from ._native import FLUXES, SCHEMES, _check, load
 _P = ctypes.POINTER(ctypes.c_double)
 _VP = ctypes.c_void_p
 
-BYTES_PER_NODE = 4 * 5 * 8  # three state buffers + flux accumulator, 5 FP64 each
+BYTES_PER_NODE = 4 * 5 * 8  # three state buffers of 5 FP64, and room for tables and staging
 
 
 class Tuning(ctypes.Structure):

@@ -1,22 +1,24 @@
 // sf_batch.hip -- batched solves of independent 1D / 2D problems of uneven
 // size.  One device arena holds every admitted problem's padded SoA state;
-// persistent kernels walk a tile table, so one launch per sweep advances all
-// problems by one RK stage; each problem keeps its own CFL dt and clock, and
-// its result does not depend on which other problems share the batch (no
-// cross-problem arithmetic; the per-problem dt is a minimum, which does not
-// depend on the order of the atomics).  The launch sequence of a step is
-// captured in a hipGraph and replayed while the set of problems is
-// unchanged.
+// a stage kernel walks a table of tiles, so one launch advances all problems
+// by one RK stage (two where 1D and 2D problems share the batch); each
+// problem keeps its own CFL dt and clock, and its result does not depend on
+// which other problems share the batch (no cross-problem arithmetic; the
+// per-problem dt is a minimum, which does not depend on the order of the
+// atomics).  The launch sequence of a step is captured in a hipGraph and
+// replayed while the set of problems is unchanged.
 //
 // Boundaries are transmissive (the reference's zeroGradient sets, applied
 // axis by axis as Boundary::Applicator::apply does,
-// solver/boundary/SF_applicator.h:51-83); the time recipe is SSPRK3
+// solver/boundary/SF_applicator.h:51-83), written in place by the stage that
+// advances the nodes next to them (write_ends); the time recipe is SSPRK3
 // (SF_builtinProviders.cpp:98-121).  Layout of problem p in the arena:
 // q[v*P + off_p + (j+gy)*m0 + i+3] with m0 = nx + 6, gy = 3 for a 2D
 // problem and 0 for a 1D one.
 #include "sonic_amd.h"
 #include "sf_batch_copy.h"
-#include "sf_device.h"
+#include "sf_batch_stage.h"
+#include "sf_sweep.h"
 
 #include <hip/hip_runtime.h>
 
@@ -24,6 +26,7 @@
 #include <climits>
 #include <cmath>
 #include <cstdio>
+#include <limits>
 #include <map>
 #include <mutex>
 #include <new>
@@ -33,43 +36,12 @@
 namespace sfamd {
 void set_last_error(const std::string& message);
 
-__device__ __forceinline__ double pressure_of(const double* q, long long P, long long id,
-                                              double gamma) {
-    double qq[5];
-#pragma unroll
-    for (int v = 0; v < 5; ++v) qq[v] = q[v * P + id];
-    return close_state(qq, gamma).p;
-}
-
-// totalEnergyFromPressure (SF_singleFluidStateModel.cpp:73-109).
-__device__ __forceinline__ double energy_from_pressure(const double* q, long long P, long long id,
-                                                       double gamma, double p) {
-    const double r = q[id], m1 = q[P + id], m2 = q[2 * P + id], m3 = q[3 * P + id];
-    const double e = p / ((gamma - 1.0) * r);
-    const double kinetic = 0.5 * (1.0 / r) * fma(m3, m3, fma(m2, m2, m1 * m1));
-    return fma(r, e, kinetic);
-}
-
-struct BatchItemDev {
-    long long off;      // start of the padded block in the arena
-    int n0, n1, m0, gy;
-    int scheme, flux;
-    double jac, area0, area1, metric0, metric1, cfl;
-};
-
 struct BatchDev {
-    const BatchItemDev* items;
-    long long P;        // arena capacity in padded nodes (per variable)
-    double gamma;
-    const int4* xtiles;  // (slot, first face f0, -, -)
-    int nxt;
-    const int4* ytiles;  // (slot, first (segment, column) index, -, -)
-    int nyt;
-    int yseg;            // nodes per y tile
+    const ItemArgs* items;
     const int* active;   // admitted slots
     int nactive;
     double* dt;
-    unsigned long long* dtmin;
+    unsigned long long* dtmin;   // kItemDtSlots partial minima per slot
     double* time;
     long long* steps;
     const long long* target;  // a problem is live while steps < target ...
@@ -77,463 +49,97 @@ struct BatchDev {
     int* live;                // liveness fixed for the current step
 };
 
-struct BatchStage {
-    const double* q0;
-    double* qout;
-    double base, incr;
-    int stage;
-    int reduce_dt;
-};
+constexpr int kItemDtWords = kItemDtSlots * kDtStride;
 
-// per-problem view with the fields local_dt / stage_update / carry_node read
-struct ItemView {
-    long long P;
-    double jac, gamma;
-    int active[3];
-    double metric[3];
-};
-
-__device__ __forceinline__ ItemView item_view(const BatchDev& B, const BatchItemDev& it) {
-    ItemView v;
-    v.P = B.P;
-    v.jac = it.jac;
-    v.gamma = B.gamma;
-    v.active[0] = 1;
-    v.active[1] = it.n1 > 1;
-    v.active[2] = 0;
-    v.metric[0] = it.metric0;
-    v.metric[1] = it.metric1;
-    v.metric[2] = 1.0;
-    return v;
-}
-
-__device__ __forceinline__ bool item_live(const BatchDev& B, int slot) {
-    return B.steps[slot] < B.target[slot] && B.flags[slot] == 0;
-}
-
-// Liveness for the kernels of one step: fixed by k_batch_finalize at the
-// start of the step, so every wave of every kernel of the step takes the
-// same decision for a problem, even while another block raises its flags
-// (a multi-wave x tile must agree, since its waves meet at barriers).  A
-// problem that faults during a step finishes that step's stages on its own
-// nodes, is not committed, and is frozen from the next step on.
-__device__ __forceinline__ bool step_live(const BatchDev& B, int slot) {
-    return B.live[slot] != 0;
-}
-
-__device__ __forceinline__ long long item_index(const BatchItemDev& it, int i, int j) {
-    return it.off + (long long)(j + it.gy) * it.m0 + (i + 3);
-}
-
-__device__ __forceinline__ bool item_solved(const BatchItemDev& it, int i, int j) {
-    if (i == 0 || i == it.n0 - 1) return false;
-    if (it.n1 > 1 && (j == 0 || j == it.n1 - 1)) return false;
-    return true;
-}
-
-// x faces + SSPRK3 stage update over tiles [t0, t1) of one (scheme, flux)
-// variant.  A problem's x faces are numbered line by line, f = j*(nx+1) +
-// (i+1) for face i+1/2, i = -1..nx-1, and a tile is BS consecutive faces
-// starting at f0 (tiles overlap by one face): lane t evaluates face f0+t,
-// and lanes 1..BS-1 whose face is not the first of its line difference it
-// with their left neighbour's face through LDS and update that node.  Short
-// lines therefore share a block and long ones span several.  Block b0 of nb
-// takes tiles t0+b0, t0+b0+nb, ... (persistent).
-__device__ __forceinline__ void batch_operands(const BatchDev& B, const BatchItemDev& it,
-                                               const BatchStage& st,
-                                               const double* __restrict__ q,
-                                               const double* __restrict__ S, long long id,
-                                               double (&pq)[5], double (&ps)[5],
-                                               double (&pq0)[5]) {
-#pragma unroll
-    for (int v = 0; v < 5; ++v) {
-        pq[v] = q[v * B.P + id];
-        ps[v] = it.n1 > 1 ? S[v * B.P + id] : 0.0;
-        pq0[v] = st.stage > 0 ? st.q0[v * B.P + id] : 0.0;
-    }
-}
-
-template <int BS, int SCHEME, int FLUX, bool EARLY>
-__device__ __forceinline__ void x_tiles(const BatchDev& B, const double* __restrict__ q,
-                                        const double* __restrict__ S, const BatchStage& st,
-                                        int t0, int t1, int b0, int nb, double (*sh)[BS],
-                                        unsigned long long* red) {
-    const int t = threadIdx.x;
-    unsigned flags = 0;
-    for (int tile = t0 + b0; tile < t1; tile += nb) {
-        const int4 T = B.xtiles[tile];
-        if (!step_live(B, T.x)) continue;  // uniform over the block
-        const BatchItemDev it = B.items[T.x];
-        // the problem's dt, fixed during a stage: read before the face
-        // arithmetic, whose duration hides the load (after the tile's
-        // stores, which might alias it, it would be read again)
-        const double dt_item = B.dt[T.x];
-        const int per_line = it.n0 + 1;
-        const int f = T.y + t;
-        const bool face = f < per_line * it.n1;
-        const int j = face ? f / per_line : 0;
-        const int a = f - j * per_line - 1;  // lower node of the face
-        // The stage operands of the node this lane updates.  With EARLY they
-        // are loaded before the face arithmetic, so that their latency hides
-        // behind it.  For WENO5 that costs the registers of a fourth wave
-        // per SIMD, which pays where 2D problems read S and not for 1D-only
-        // batches; TENO5 runs at three waves either way and always loads
-        // early.
-        const bool upd = t >= 1 && face && a >= 0;
-        double pq[5] = {0.0, 0.0, 0.0, 0.0, 0.0}, ps[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-        double pq0[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-        if (EARLY && upd) batch_operands(B, it, st, q, S, item_index(it, a, j), pq, ps, pq0);
-        if (face) {
-            const long long base = item_index(it, a, j);
-            double stc[6][5];
-#pragma unroll
-            for (int s = 0; s < 6; ++s)
-#pragma unroll
-                for (int v = 0; v < 5; ++v) stc[s][v] = q[v * B.P + base + (s - 2)];
-            double f5[5];
-            face_flux<0, SCHEME, FLUX>(stc, B.gamma, it.area0, f5, flags);
-            if (!finite_sum5(f5)) flags |= kFlagFlux;
-#pragma unroll
-            for (int v = 0; v < 5; ++v) sh[v][t] = f5[v];
-        }
-        __syncthreads();
-        double dl = INFINITY;
-        if (upd) {
-            const long long id = item_index(it, a, j);
-            if (!EARLY) batch_operands(B, it, st, q, S, id, pq, ps, pq0);
-            double s5[5];
-#pragma unroll
-            for (int v = 0; v < 5; ++v) {
-                const double d = sh[v][t] - sh[v][t - 1];
-                s5[v] = (it.n1 > 1) ? ps[v] + d : d;
-            }
-            StageArgs A{};
-            A.q0 = st.q0;
-            A.qout = st.qout;
-            A.dt = &B.dt[T.x];
-            A.flags = &B.flags[T.x];
-            A.base = st.base;
-            A.incr = st.incr;
-            A.cfl = it.cfl;
-            A.time = SF_TIME_SSPRK3;
-            A.stage = st.stage;
-            A.reduce_dt = st.reduce_dt;
-            const ItemView G = item_view(B, it);
-            double qn[5];
-            if (item_solved(it, a, j)) {
-                stage_update_dt<SF_TIME_SSPRK3>(G, A, id, pq, pq0, s5, dt_item, flags, dl, qn);
-            } else {
-#pragma unroll
-                for (int v = 0; v < 5; ++v) {
-                    qn[v] = pq[v];   // carry_node
-                    A.qout[v * B.P + id] = qn[v];
-                }
-            }
-        }
-        if (st.reduce_dt) block_min_atomic(dl, &B.dtmin[T.x], red);
-        if (flags) {
-            atomicOr(&B.flags[T.x], flags);
-            flags = 0;
-        }
-        __syncthreads();
-    }
-}
-
-// Tile ranges and block ranges of the four (scheme, flux) variants,
-// variant v = 2*scheme + flux.
-struct Split {
-    int tile[5];
-    int block[5];
-};
-
-// One launch for every variant: block ranges are assigned to variants.
-template <int BS>
-__global__ __launch_bounds__(BS) void k_batch_x_fused(BatchDev B, const double* __restrict__ q,
-                                                      const double* __restrict__ S,
-                                                      BatchStage st, Split sp) {
-    __shared__ double sh[5][BS];
-    __shared__ unsigned long long red[BS / 64];
-    const int bid = blockIdx.x;
-    int v = 0;
-    while (v < 3 && bid >= sp.block[v + 1]) ++v;
-    const int b0 = bid - sp.block[v], nb = sp.block[v + 1] - sp.block[v];
-    switch (v) {
-        case 0: x_tiles<BS, 0, 0, true>(B, q, S, st, sp.tile[0], sp.tile[1], b0, nb, sh, red); break;
-        case 1: x_tiles<BS, 0, 1, true>(B, q, S, st, sp.tile[1], sp.tile[2], b0, nb, sh, red); break;
-        case 2: x_tiles<BS, 1, 0, true>(B, q, S, st, sp.tile[2], sp.tile[3], b0, nb, sh, red); break;
-        default: x_tiles<BS, 1, 1, true>(B, q, S, st, sp.tile[3], sp.tile[4], b0, nb, sh, red); break;
-    }
-}
-
-// One launch per variant (fewer registers than the fused form).  Three waves
-// per SIMD fit without spilling except for TENO5 + HLLC, which keeps two.
-template <int BS, int SCHEME, int FLUX, bool EARLY>
-__global__ __launch_bounds__(BS)
-__attribute__((amdgpu_waves_per_eu((SCHEME == 1 && FLUX == 1) ? 2 : 3, 8))) void k_batch_x(BatchDev B, const double* __restrict__ q,
-                                                const double* __restrict__ S, BatchStage st,
-                                                int t0, int t1) {
-    __shared__ double sh[5][BS];
-    __shared__ unsigned long long red[BS / 64];
-    x_tiles<BS, SCHEME, FLUX, EARLY>(B, q, S, st, t0, t1, blockIdx.x, gridDim.x, sh, red);
-}
-
-// y faces of the 2D problems over tiles [t0, t1) of one variant.  A
-// problem's y work is numbered (segment, column) = k -> (k / nx, k % nx),
-// segments of yseg nodes; a tile is 64 consecutive k, one per lane, so
-// narrow problems fill whole waves.  Each lane marches up its column
-// segment with the stencil window in LDS and registers (one load per node)
-// and writes S = F(j+1/2) - F(j-1/2).
-template <int SCHEME, int FLUX>
-__device__ __forceinline__ void y_tiles(const BatchDev& B, const double* __restrict__ q,
-                                        double* __restrict__ S, int t0, int t1, int b0, int nb,
-                                        double (*win)[5][64]) {
-    const int lane = threadIdx.x;
-    unsigned flags = 0;
-    for (int tile = t0 + b0; tile < t1; tile += nb) {
-        const int4 T = B.ytiles[tile];
-        if (!step_live(B, T.x)) continue;
-        const BatchItemDev it = B.items[T.x];
-        const int k = T.y + lane;
-        const int nseg = (it.n1 + B.yseg - 1) / B.yseg;
-        if (k >= nseg * it.n0) continue;  // per lane; no barrier below
-        const int seg = k / it.n0;
-        const int i = k - seg * it.n0;
-        const int a0 = seg * B.yseg;
-        const int a1 = min(a0 + B.yseg, it.n1);
-        const long long step = it.m0;
-        // the face a+1/2 reads nodes a-2 .. a+1 from the lane's 4-slot LDS
-        // ring, node a+2 carried in registers, node a+3 loaded for it; the
-        // march starts at a0-1 so every face is evaluated by the same
-        // instructions (see k_sweep_march)
-        long long id = item_index(it, i, a0) - 3 * step;  // node a0-3
-        for (int s = 0; s < 4; ++s)
-#pragma unroll
-            for (int v = 0; v < 5; ++v) win[s][v][lane] = q[v * B.P + id + s * step];
-        double carried[5];
-#pragma unroll
-        for (int v = 0; v < 5; ++v) carried[v] = q[v * B.P + id + 4 * step];
-        id += 2 * step;
-        int head = 0;
-        double fprev[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
-#pragma clang loop unroll(disable)
-        for (int a = a0 - 1; a < a1; ++a, id += step) {
-            double stc[6][5];
-#pragma unroll
-            for (int v = 0; v < 5; ++v) stc[5][v] = q[v * B.P + id + 3 * step];
-#pragma unroll
-            for (int s = 0; s < 4; ++s) {
-                const int slot = (head + s) & 3;
-#pragma unroll
-                for (int v = 0; v < 5; ++v) stc[s][v] = win[slot][v][lane];
-            }
-#pragma unroll
-            for (int v = 0; v < 5; ++v) {
-                stc[4][v] = carried[v];
-                win[head][v][lane] = carried[v];
-                carried[v] = stc[5][v];
-            }
-            head = (head + 1) & 3;
-            double f[5];
-            face_flux<1, SCHEME, FLUX>(stc, B.gamma, it.area1, f, flags);
-            double d[5];
-            if (!finite_sum5(f)) flags |= kFlagFlux;
-#pragma unroll
-            for (int v = 0; v < 5; ++v) {
-                d[v] = f[v] - fprev[v];
-                fprev[v] = f[v];
-            }
-            if (a < a0) continue;
-#pragma unroll
-            for (int v = 0; v < 5; ++v) S[v * B.P + id] = d[v];
-        }
-        if (flags) {
-            atomicOr(&B.flags[T.x], flags);
-            flags = 0;
-        }
-    }
-}
-
-__global__ __launch_bounds__(64) void k_batch_y_fused(BatchDev B, const double* __restrict__ q,
-                                                      double* __restrict__ S, Split sp) {
-    __shared__ double win[4][5][64];
-    const int bid = blockIdx.x;
-    int v = 0;
-    while (v < 3 && bid >= sp.block[v + 1]) ++v;
-    const int b0 = bid - sp.block[v], nb = sp.block[v + 1] - sp.block[v];
-    switch (v) {
-        case 0: y_tiles<0, 0>(B, q, S, sp.tile[0], sp.tile[1], b0, nb, win); break;
-        case 1: y_tiles<0, 1>(B, q, S, sp.tile[1], sp.tile[2], b0, nb, win); break;
-        case 2: y_tiles<1, 0>(B, q, S, sp.tile[2], sp.tile[3], b0, nb, win); break;
-        default: y_tiles<1, 1>(B, q, S, sp.tile[3], sp.tile[4], b0, nb, win); break;
-    }
-}
-
-// The WENO5 variants fit four waves per SIMD (128 VGPRs) when asked to.
-template <int SCHEME, int FLUX>
-__global__ __launch_bounds__(64)
-__attribute__((amdgpu_waves_per_eu((SCHEME == 0) ? 4 : 3, 8))) void k_batch_y(BatchDev B, const double* __restrict__ q,
-                                                double* __restrict__ S, int t0, int t1) {
-    __shared__ double win[4][5][64];
-    y_tiles<SCHEME, FLUX>(B, q, S, t0, t1, blockIdx.x, gridDim.x, win);
-}
-
-// Transmissive fill along AXIS of every live problem (blockIdx.x = the
-// problem, blockIdx.y = a share of its boundary points, so a large problem's
-// accesses are spread over several blocks).
-// PHASE 0 copies density and momentum from the inner neighbour into the
-// boundary node and its ghosts (SF_zeroGradient.cpp:88-130); PHASE 1
-// rebuilds energy from the neighbour's pressure
-// (SF_thermodynamicClosure.cpp:219-281).  The phases run x then y each, as
-// the grid fill does.
-//
-// Along y a boundary row is contiguous, so a thread per row point writes
-// coalesced.  Along x the boundary node and its ghosts of one row are four
-// adjacent doubles per variable while rows lie a row pitch apart, so there
-// the work is split finer: PHASE 0 gives each (row, variable, node) a
-// thread, PHASE 1 each (row, node) -- every thread of a row forms the
-// boundary node's energy and pressure itself, from the same values, so the
-// ghosts take exactly the pressure the boundary node holds -- and
-// neighbouring lanes write neighbouring doubles.
-template <int AXIS, int PHASE>
-__global__ __launch_bounds__(256) void k_batch_fill(BatchDev B, double* __restrict__ q) {
-    const int slot = B.active[blockIdx.x];
-    if (!step_live(B, slot)) return;
-    const BatchItemDev it = B.items[slot];
-    if (AXIS == 1 && it.n1 <= 1) return;
-    if (AXIS == 0) {
-        constexpr int per = PHASE == 0 ? 16 : 4;   // threads per boundary row
-        const int nrow = it.n1;
-        for (int t = blockIdx.y * blockDim.x + threadIdx.x; t < 2 * nrow * per;
-             t += gridDim.y * blockDim.x) {
-            const int pr = t / per, u = t % per;
-            const int side = pr / nrow, r = pr % nrow;
-            const long long b = item_index(it, side ? it.n0 - 1 : 0, r);
-            const long long s = side ? b - 1 : b + 1;
-            const long long dir = side ? 1 : -1;
-            if (PHASE == 0) {
-                const int v = u >> 2, l = u & 3;   // l = 0: the boundary node
-                q[v * B.P + b + l * dir] = q[v * B.P + s];
-            } else {
-                // every thread of the row forms the boundary node's energy
-                // and pressure from the same values; thread 0 stores the
-                // energy, thread l >= 1 fills ghost l
-                const double ps = pressure_of(q, B.P, s, B.gamma);
-                const double eb = energy_from_pressure(q, B.P, b, B.gamma, ps);
-                double qb[5] = {q[b], q[B.P + b], q[2 * B.P + b], q[3 * B.P + b], eb};
-                const double pb = close_state(qb, B.gamma).p;
-                if (u == 0) {
-                    q[4 * B.P + b] = eb;
-                    if (!(ps > 0.0) || !(pb > 0.0)) atomicOr(&B.flags[slot], (unsigned)kFlagState);
-                } else {
-                    q[4 * B.P + b + u * dir] = energy_from_pressure(q, B.P, b + u * dir, B.gamma, pb);
-                }
-            }
-        }
-        return;
-    }
-    const int nother = AXIS == 0 ? it.n1 : it.n0;
-    const int nax = AXIS == 0 ? it.n0 : it.n1;
-    const long long step = AXIS == 0 ? 1 : it.m0;
-    for (int t = blockIdx.y * blockDim.x + threadIdx.x; t < 2 * nother;
-         t += gridDim.y * blockDim.x) {
-        const int side = t / nother, r = t % nother;
-        const int bnode = side ? nax - 1 : 0;
-        const long long b = AXIS == 0 ? item_index(it, bnode, r) : item_index(it, r, bnode);
-        const long long s = side ? b - step : b + step;
-        const long long dir = side ? step : -step;
-        if (PHASE == 0) {
-#pragma unroll
-            for (int v = 0; v < 4; ++v) {
-                const double val = q[v * B.P + s];
-                q[v * B.P + b] = val;
-#pragma unroll
-                for (int l = 1; l <= 3; ++l) q[v * B.P + b + l * dir] = val;
-            }
-        } else {
-            const double ps = pressure_of(q, B.P, s, B.gamma);
-            q[4 * B.P + b] = energy_from_pressure(q, B.P, b, B.gamma, ps);
-            const double pb = pressure_of(q, B.P, b, B.gamma);
-            if (!(ps > 0.0) || !(pb > 0.0)) atomicOr(&B.flags[slot], (unsigned)kFlagState);
-#pragma unroll
-            for (int l = 1; l <= 3; ++l)
-                q[4 * B.P + b + l * dir] = energy_from_pressure(q, B.P, b + l * dir, B.gamma, pb);
-        }
-    }
-}
-
-// CFL scan of the listed problems (blockIdx.x = list entry, blockIdx.y
-// splits the nodes) folded into dtmin[slot] (RusanovEOS::deltaT,
-// SF_rusanovEOS.cpp:110-147).
-__global__ __launch_bounds__(256) void k_batch_cfl(BatchDev B, const int* __restrict__ list,
-                                                   const double* __restrict__ q) {
-    __shared__ unsigned long long red[4];
+// The problems admitted since the last step (blockIdx.x = list entry,
+// blockIdx.y splits the nodes): their ends are written and their CFL scan
+// (RusanovEOS::deltaT, SF_rusanovEOS.cpp:110-147) goes to dtmin.
+__global__ __launch_bounds__(256) void k_batch_prepare(BatchDev B, const int* __restrict__ list) {
     const int slot = list[blockIdx.x];
-    const BatchItemDev it = B.items[slot];
-    const ItemView G = item_view(B, it);
-    const long long N = (long long)it.n0 * it.n1;
+    const SweepArgs& W = B.items[slot].stage[0];
+    const GridDev& G = W.G;
+    double* const q = const_cast<double*>(W.q);
+    const int nx = G.solved_hi[0] - G.solved_lo[0] + 1;
+    const long long N = (long long)nx * (G.solved_hi[1] - G.solved_lo[1] + 1);
     unsigned flags = 0;
     double best = INFINITY;
     for (long long u = blockIdx.y * (long long)blockDim.x + threadIdx.x; u < N;
          u += (long long)gridDim.y * blockDim.x) {
-        const int i = (int)(u % it.n0), j = (int)(u / it.n0);
-        if (!item_solved(it, i, j)) continue;
-        const long long id = item_index(it, i, j);
+        const int i = G.solved_lo[0] + (int)(u % nx), j = G.solved_lo[1] + (int)(u / nx);
+        const long long id = node_index(G, i, j, 0);
         double qq[5];
 #pragma unroll
-        for (int v = 0; v < 5; ++v) qq[v] = q[v * B.P + id];
-        best = fmin(best, local_dt(G, qq, it.cfl, flags));
+        for (int v = 0; v < 5; ++v) qq[v] = q[v * G.P + id];
+        best = fmin(best, local_dt(G, qq, W.A.cfl, flags));
+        if (!write_ends<true>(G, q, i, j, 0, id, qq)) flags |= kFlagState;
     }
     if (flags) atomicOr(&B.flags[slot], flags);
-    block_min_atomic(best, &B.dtmin[slot], red);
+    const unsigned long long b = wave_min_bits(
+        (best > 0.0 && isfinite(best)) ? (unsigned long long)__double_as_longlong(best)
+                                       : 0x7FF0000000000000ull);
+    if ((threadIdx.x & 63) == 0 && b != 0x7FF0000000000000ull)
+        atomicMin(B.dtmin + (long long)slot * kItemDtWords + (blockIdx.y % kItemDtSlots) * kDtStride,
+                  b);
 }
 
-// dt of the step from the folded CFL minimum; the accumulator is reset for
-// the fold of this step's last stage.
-__global__ void k_batch_finalize(BatchDev B) {
+// The clock between two steps: commits the step before (live says which
+// problems took one; a problem that faulted in it is not counted) and, with
+// `next`, starts the following one: its liveness is fixed, so that every
+// wave of every kernel of the step takes the same decision for a problem
+// even while another block raises its flags, dt is the folded CFL minimum,
+// and the accumulator is cleared for the fold of the step's last stage.  A
+// problem that faults during a step finishes that step's stages on its own
+// nodes and is frozen from the next step on.
+__global__ void k_batch_clock(BatchDev B, int next) {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= B.nactive) return;
     const int slot = B.active[k];
-    const bool live = item_live(B, slot);
+    const bool sound = B.flags[slot] == 0;
+    long long steps = B.steps[slot];
+    if (B.live[slot] && sound) {
+        B.time[slot] += B.dt[slot];
+        B.steps[slot] = ++steps;
+    }
+    const bool live = next && sound && steps < B.target[slot];
     B.live[slot] = live ? 1 : 0;
     if (!live) return;
-    B.dt[slot] = __longlong_as_double((long long)B.dtmin[slot]);
-    B.dtmin[slot] = 0x7FF0000000000000ull;
-}
-
-__global__ void k_batch_commit(BatchDev B) {
-    const int k = blockIdx.x * blockDim.x + threadIdx.x;
-    if (k >= B.nactive) return;
-    const int slot = B.active[k];
-    if (!step_live(B, slot) || B.flags[slot] != 0) return;
-    B.time[slot] += B.dt[slot];
-    B.steps[slot] += 1;
+    unsigned long long* const m = B.dtmin + (long long)slot * kItemDtWords;
+    unsigned long long b = m[0];
+#pragma unroll
+    for (int s = 1; s < kItemDtSlots; ++s) b = min(b, m[s * kDtStride]);
+#pragma unroll
+    for (int s = 0; s < kItemDtSlots; ++s) m[s * kDtStride] = 0x7FF0000000000000ull;
+    B.dt[slot] = __longlong_as_double((long long)b);
 }
 
 __global__ void k_batch_reset(BatchDev B, const int* __restrict__ list, int n) {
     const int k = blockIdx.x * blockDim.x + threadIdx.x;
     if (k >= n) return;
     const int slot = list[k];
-    B.dtmin[slot] = 0x7FF0000000000000ull;
+#pragma unroll
+    for (int s = 0; s < kItemDtSlots; ++s)
+        B.dtmin[(long long)slot * kItemDtWords + s * kDtStride] = 0x7FF0000000000000ull;
     B.time[slot] = 0.0;
     B.steps[slot] = 0;
     B.dt[slot] = 0.0;
     B.flags[slot] = 0;
-    B.live[slot] = 1;   // for the fill that prepares the problem
+    B.live[slot] = 0;
 }
 
 // unique-node SoA of one problem <-> its padded block in the arena
-__global__ __launch_bounds__(256) void k_batch_pack(BatchDev B, int slot,
+__global__ __launch_bounds__(256) void k_batch_pack(const ItemArgs* __restrict__ item,
                                                     const double* __restrict__ src,
                                                     double* __restrict__ dst, int to_arena) {
-    const BatchItemDev it = B.items[slot];
-    const long long N = (long long)it.n0 * it.n1;
+    const GridDev& G = item->stage[0].G;
+    double* const q = const_cast<double*>(item->stage[0].q);
+    const long long N = (long long)G.n[0] * G.n[1];
     for (long long u = blockIdx.x * (long long)blockDim.x + threadIdx.x; u < N;
          u += (long long)gridDim.x * blockDim.x) {
-        const long long id = item_index(it, (int)(u % it.n0), (int)(u / it.n0));
+        const long long id = node_index(G, (int)(u % G.n[0]), (int)(u / G.n[0]), 0);
 #pragma unroll
         for (int v = 0; v < 5; ++v) {
-            if (to_arena) dst[v * B.P + id] = src[v * N + u];
-            else dst[v * N + u] = src[v * B.P + id];
+            if (to_arena) q[v * G.P + id] = src[v * N + u];
+            else dst[v * N + u] = q[v * G.P + id];
         }
     }
 }
@@ -565,6 +171,12 @@ long long padded_nodes(const sf_batch_item& it) {
 }  // namespace
 
 struct sf_batch {
+    // placement of a problem in the arena
+    struct Item {
+        long long off = 0;      // start of its padded block
+        int n0 = 0, n1 = 0, m0 = 0, gy = 0;
+        int scheme = 0, flux = 0;
+    };
     int device = 0;
     int cus = 256;
     double gamma = 1.4;
@@ -574,10 +186,9 @@ struct sf_batch {
     hipStream_t copy_stream = nullptr;   // copy-out of finished problems
     hipEvent_t copy_after = nullptr;     // orders copy-outs after the compute stream
     double* buf[3] = {nullptr, nullptr, nullptr};
-    double* S = nullptr;
     double* staging = nullptr;
     long long staging_nodes = 0;
-    BatchItemDev* d_items = nullptr;
+    ItemArgs* d_items = nullptr;
     double* d_dt = nullptr;
     unsigned long long* d_dtmin = nullptr;
     double* d_time = nullptr;
@@ -585,27 +196,25 @@ struct sf_batch {
     long long* d_target = nullptr;
     unsigned* d_flags = nullptr;
     int* d_live = nullptr;
-    int4* d_xt = nullptr;
-    int4* d_yt = nullptr;
+    BatchTile* d_tiles = nullptr;
     int* d_active = nullptr;
     int* d_scan = nullptr;
-    size_t xt_cap = 0, yt_cap = 0;
+    size_t tile_cap = 0;
     // launch shape (tunable)
-    int xbs = 128;              // x block: 64, 128 or 256 lanes (tile = xbs-1 nodes)
-    int yseg = 32;              // y tile length
-    int blocks_per_cu = 8;      // persistent grid size
-    int fused = 1;              // 1: one launch per sweep for all variants
+    int xlen = 0;               // nodes of a 1D tile, in strips of 63 (0: by cost)
+    int ylen = 0;               // rows of a 2D tile (0: by cost)
+    int blocks_per_cu = -1;     // persistent grid size (-1: a block per tile)
+    int fused = 1;              // 1: one launch per stage for all variants
     // host side
-    std::vector<BatchItemDev> items;
+    std::vector<Item> items;
     std::vector<sf_batch_item> desc;
     std::vector<char> used;
     std::map<long long, long long> free_ranges;  // offset -> length
     std::vector<int> pending_scan;               // admitted since the last step
     bool tables_dirty = true;
-    int nxt = 0, nyt = 0, nactive = 0;
-    int xr[5] = {0, 0, 0, 0, 0}, yr[5] = {0, 0, 0, 0, 0};  // tile ranges per variant
+    int nactive = 0;
+    int line[5] = {0, 0, 0, 0, 0}, plane[5] = {0, 0, 0, 0, 0};  // tile ranges per variant
     bool any2d = false;
-    int max_n0 = 1, max_n1 = 1;  // largest n0 / n1 of the admitted problems
     hipGraph_t graph = nullptr;
     hipGraphExec_t graph_exec = nullptr;
 };
@@ -615,13 +224,6 @@ namespace {
 BatchDev view(const sf_batch* b) {
     BatchDev B{};
     B.items = b->d_items;
-    B.P = b->capacity;
-    B.gamma = b->gamma;
-    B.xtiles = b->d_xt;
-    B.nxt = b->nxt;
-    B.ytiles = b->d_yt;
-    B.nyt = b->nyt;
-    B.yseg = b->yseg;
     B.active = b->d_active;
     B.nactive = b->nactive;
     B.dt = b->d_dt;
@@ -634,6 +236,63 @@ BatchDev view(const sf_batch* b) {
     return B;
 }
 
+// Arguments of the three stages of a problem in slot `slot`: stage s reads
+// buf[s] and writes buf[s + 1], the last one buf[0].  Uniform Cartesian
+// metrics are formed as for a grid with unit spacing on the absent axes
+// (SF_mesh.cpp:320-338, SF_canonicalFace.h:87-108).
+ItemArgs item_args(const sf_batch* b, int slot, const sf_batch::Item& it,
+                   const sf_batch_item* item) {
+    SweepArgs W{};
+    GridDev& G = W.G;
+    const int n[3] = {it.n0, it.n1, 1};
+    const int ghosts[3] = {3, it.gy, 0};
+    const double d[3] = {item->d[0], it.n1 > 1 ? item->d[1] : 1.0, 1.0};
+    G.jac = 1.0 / (d[0] * d[1] * d[2]);
+    for (int a = 0; a < 3; ++a) {
+        const int on = n[a] > 1;
+        G.n[a] = n[a];
+        G.g[a] = ghosts[a];
+        G.m[a] = n[a] + 2 * ghosts[a];
+        G.active[a] = on;
+        G.zg_lo[a] = G.zg_hi[a] = on;
+        G.solved_lo[a] = on;
+        G.solved_hi[a] = n[a] - 1 - on;
+        G.map_lo[a] = on ? -1 : std::numeric_limits<int>::min();
+        G.map_hi[a] = on ? n[a] : std::numeric_limits<int>::max();
+        G.d[a] = d[a];
+        const double metric = 1.0 / d[a];
+        const double c = metric / G.jac, f = 0.5 * (c + c);
+        G.area[a] = std::sqrt(f * f + 0.0 * 0.0 + 0.0 * 0.0);
+        G.metric[a] = on ? metric : 0.0;
+    }
+    G.xo = 3;
+    G.P = b->capacity;
+    G.stride[0] = 1;
+    G.stride[1] = it.m0;
+    G.stride[2] = (long long)it.m0 * G.m[1];
+    for (int a = 0; a < 3; ++a) G.ustride[a] = (unsigned)G.stride[a];
+    G.gamma = b->gamma;
+    static const double base[3] = {0.0, 0.75, 1.0 / 3.0};
+    static const double incr[3] = {1.0, 0.25, 2.0 / 3.0};
+    W.A.q0 = b->buf[0] + it.off;
+    W.A.dt = b->d_dt + slot;
+    W.A.dtmin = b->d_dtmin + (size_t)slot * kItemDtWords;
+    W.A.flags = b->d_flags + slot;
+    W.A.cfl = item->cfl;
+    W.A.time = SF_TIME_SSPRK3;
+    ItemArgs args{};
+    for (int s = 0; s < 3; ++s) {
+        W.q = b->buf[s] + it.off;
+        W.A.qout = b->buf[(s + 1) % 3] + it.off;
+        W.A.base = base[s];
+        W.A.incr = incr[s];
+        W.A.stage = s;
+        W.A.reduce_dt = s == 2;
+        args.stage[s] = W;
+    }
+    return args;
+}
+
 void drop_graph(sf_batch* b) {
     if (b->graph_exec) (void)hipGraphExecDestroy(b->graph_exec);
     if (b->graph) (void)hipGraphDestroy(b->graph);
@@ -641,21 +300,32 @@ void drop_graph(sf_batch* b) {
     b->graph = nullptr;
 }
 
-// Tile tables and the active list after admissions / removals.  Tiles are
+// Strips of a 2D problem along x: 63 columns and a lane that evaluates the
+// first face, or 64 with the first faces evaluated beforehand where that
+// saves a strip.
+struct Strips {
+    int cols, count;
+};
+
+Strips strips(int n0) {
+    const int nx = n0 - 2;
+    const Strips s{kXBlock - 1, (nx + kXBlock - 2) / (kXBlock - 1)};
+    const int whole = (nx + kXBlock - 1) / kXBlock;
+    return whole < s.count ? Strips{kXBlock, whole} : s;
+}
+
+// Tile table and the active list after admissions / removals.  Tiles are
 // grouped by (scheme, flux) variant and, within a variant, listed largest
-// problem first, so the persistent blocks start on the big problems and
-// finish on the small ones.
+// problem first, so the blocks start on the big problems and finish on the
+// small ones.  Rows of a 2D tile and strips of a 1D one are the longest that
+// march_cost finds worth while over all problems of the kind: few problems
+// then spread over the whole device, many run long tiles.  A node's
+// arithmetic does not depend on them.
 int rebuild_tables(sf_batch* b) {
-    std::vector<int4> xt, yt;
     std::vector<int> act;
     b->any2d = false;
-    b->max_n0 = b->max_n1 = 1;
     for (int s = 0; s < b->item_capacity; ++s)
-        if (b->used[s]) {
-            act.push_back(s);
-            b->max_n0 = std::max(b->max_n0, b->items[s].n0);
-            b->max_n1 = std::max(b->max_n1, b->items[s].n1);
-        }
+        if (b->used[s]) act.push_back(s);
     std::vector<int> order = act;
     auto variant = [&](int s) { return 2 * b->items[s].scheme + b->items[s].flux; };
     std::stable_sort(order.begin(), order.end(), [&](int x, int y) {
@@ -663,49 +333,70 @@ int rebuild_tables(sf_batch* b) {
         return (long long)b->items[x].n0 * b->items[x].n1 >
                (long long)b->items[y].n0 * b->items[y].n1;
     });
-    const int xstep = b->xbs - 1;
-    int v = 0;
-    b->xr[0] = b->yr[0] = 0;
-    for (int s : order) {
-        while (v < variant(s)) {
-            ++v;
-            b->xr[v] = (int)xt.size();
-            b->yr[v] = (int)yt.size();
+    const auto line_strips = [&](int s) { return (b->items[s].n0 - 2 + kXBlock - 2) / (kXBlock - 1); };
+    // the least cost over tile lengths 1 .. most
+    const auto choose = [&](int most, double faces_per, double extra, auto tiles_of) {
+        int best = 1;
+        double least = 0.0;
+        for (int r = 1; r <= most; ++r) {
+            long long blocks = 0;
+            for (int s : order) blocks += tiles_of(s, r);
+            const double cost = march_cost(blocks, faces_per * r + extra, b->cus);
+            if (r > 1 && cost >= least) continue;
+            least = cost;
+            best = r;
         }
-        const BatchItemDev& it = b->items[s];
-        // x: tiles of xbs consecutive faces, overlapping by one
-        const long long faces = (long long)(it.n0 + 1) * it.n1;
-        for (long long f0 = 0; f0 < faces - 1; f0 += xstep) xt.push_back(make_int4(s, (int)f0, 0, 0));
-        if (it.n1 > 1) {
-            b->any2d = true;
-            const long long work = (long long)((it.n1 + b->yseg - 1) / b->yseg) * it.n0;
-            for (long long k0 = 0; k0 < work; k0 += 64) yt.push_back(make_int4(s, (int)k0, 0, 0));
-        }
-    }
-    while (v < 4) {
-        ++v;
-        b->xr[v] = (int)xt.size();
-        b->yr[v] = (int)yt.size();
-    }
-    auto upload = [&](int4** ptr, size_t* cap, const std::vector<int4>& vec) -> int {
-        if (vec.size() > *cap) {
-            if (*ptr) SF_BHIP(hipFree(*ptr));
-            *ptr = nullptr;
-            *cap = 0;
-            const size_t want = std::max<size_t>(vec.size(), 1024);
-            SF_BHIP(hipMalloc(ptr, want * sizeof(int4)));
-            *cap = want;
-        }
-        if (!vec.empty())
-            SF_BHIP(hipMemcpy(*ptr, vec.data(), vec.size() * sizeof(int4), hipMemcpyHostToDevice));
-        return 0;
+        return best;
     };
-    if (int rc = upload(&b->d_xt, &b->xt_cap, xt)) return rc;
-    if (int rc = upload(&b->d_yt, &b->yt_cap, yt)) return rc;
+    for (int s : order) b->any2d = b->any2d || b->items[s].n1 > 1;
+    int rows = std::min(b->ylen, kYxRows), run = (b->xlen + 1) / kXBlock;
+    if (b->any2d && rows == 0)
+        rows = choose(kYxRows, 2.0, 1.0, [&](int s, int r) -> long long {
+            const sf_batch::Item& it = b->items[s];
+            return it.n1 > 1 ? (long long)strips(it.n0).count * ((it.n1 - 2 + r - 1) / r) : 0;
+        });
+    if (run == 0)
+        run = choose(8, 1.0, 0.0, [&](int s, int r) -> long long {
+            return b->items[s].n1 > 1 ? 0 : (line_strips(s) + r - 1) / r;
+        });
+    std::vector<BatchTile> tiles;
+    const auto fill = [&](bool plane, int (&range)[5]) {
+        int v = 0;
+        range[0] = (int)tiles.size();
+        for (int s : order) {
+            const sf_batch::Item& it = b->items[s];
+            if ((it.n1 > 1) != plane) continue;
+            while (v < variant(s)) range[++v] = (int)tiles.size();
+            if (plane) {
+                const Strips st = strips(it.n0);
+                const int helper = kXBlock - st.cols;
+                for (int a0 = 1; a0 <= it.n1 - 2; a0 += rows)
+                    for (int x = 0; x < st.count; ++x)
+                        tiles.push_back({s, 1 + x * st.cols - helper, a0,
+                                         (int)((unsigned)std::min(a0 + rows, it.n1 - 1) |
+                                               ((unsigned)helper << 31))});
+            } else {
+                for (int x = 0; x < line_strips(s); x += run)
+                    tiles.push_back({s, x * (kXBlock - 1), run, 0});
+            }
+        }
+        while (v < 4) range[++v] = (int)tiles.size();
+    };
+    fill(true, b->plane);
+    fill(false, b->line);
+    if (tiles.size() > b->tile_cap) {
+        if (b->d_tiles) SF_BHIP(hipFree(b->d_tiles));
+        b->d_tiles = nullptr;
+        b->tile_cap = 0;
+        const size_t want = std::max<size_t>(tiles.size(), 1024);
+        SF_BHIP(hipMalloc(&b->d_tiles, want * sizeof(BatchTile)));
+        b->tile_cap = want;
+    }
+    if (!tiles.empty())
+        SF_BHIP(hipMemcpy(b->d_tiles, tiles.data(), tiles.size() * sizeof(BatchTile),
+                          hipMemcpyHostToDevice));
     if (!act.empty())
         SF_BHIP(hipMemcpy(b->d_active, act.data(), act.size() * sizeof(int), hipMemcpyHostToDevice));
-    b->nxt = (int)xt.size();
-    b->nyt = (int)yt.size();
     b->nactive = (int)act.size();
     b->tables_dirty = false;
     drop_graph(b);
@@ -714,13 +405,14 @@ int rebuild_tables(sf_batch* b) {
 
 // Relative cost of a tile of each variant (TENO5 evaluates its three
 // candidate weights with a sixth power; HLLC adds a star state).
-constexpr double kVariantCost[4] = {1.0, 1.03, 1.16, 1.19};
+constexpr double kVariantCost[4] = {1.0, 1.08, 1.52, 1.62};
 
 // Block ranges of a fused launch of `total` blocks over the variant tile
 // ranges r[5]: proportional to the tiles' cost, at least one block for a
 // non-empty variant, never more blocks than tiles.
 Split split_blocks(const int r[5], unsigned total) {
     Split sp{};
+    const unsigned tiles = (unsigned)(r[4] - r[0]);
     double w[4], sum = 0.0;
     for (int v = 0; v < 4; ++v) {
         w[v] = (r[v + 1] - r[v]) * kVariantCost[v];
@@ -731,7 +423,8 @@ Split split_blocks(const int r[5], unsigned total) {
     for (int v = 0; v < 4; ++v) {
         const int n = r[v + 1] - r[v];
         int nb = 0;
-        if (n > 0) nb = std::min(n, std::max(1, (int)std::lround(total * w[v] / sum)));
+        if (total >= tiles) nb = n;
+        else if (n > 0) nb = std::min(n, std::max(1, (int)std::lround(total * w[v] / sum)));
         sp.tile[v + 1] = r[v + 1];
         sp.block[v + 1] = sp.block[v] + nb;
     }
@@ -755,118 +448,57 @@ int resident_per_cu(Kernel kernel, int threads) {
     return n;
 }
 
-// Persistent grid of a sweep over `tiles` tiles: blocks_per_cu blocks per
-// compute unit, or with blocks_per_cu = 0 as many as the device holds at
-// once (`per_cu` = the kernel's resident blocks per unit).
-unsigned persistent_blocks(const sf_batch* b, int tiles, int per_cu = 0) {
-    const int want = b->blocks_per_cu > 0 ? b->blocks_per_cu : std::max(per_cu, 1);
+// Grid of a stage over `tiles` tiles: a block per tile, or persistent
+// blocks, blocks_per_cu per compute unit, or with blocks_per_cu = 0 as many
+// as the device holds at once.  A block per tile is the default: the
+// dispatcher hands the next tile to whichever SIMD is free.
+template <class Kernel>
+unsigned stage_blocks(const sf_batch* b, int tiles, Kernel kernel) {
+    if (b->blocks_per_cu < 0) return (unsigned)tiles;
+    const int want = b->blocks_per_cu > 0 ? b->blocks_per_cu : resident_per_cu(kernel, kXBlock);
     return (unsigned)std::max(1, std::min(tiles, b->cus * want));
 }
 
-// ghost fill of every live problem: copy x, copy y, energy x, energy y;
-// blocks per problem sized so each thread takes about four work items of
-// the largest problem (at most 32)
-void enqueue_fill(sf_batch* b, double* q) {
-    const BatchDev B = view(b);
-    auto grid = [&](long long items) {
-        return dim3((unsigned)b->nactive,
-                    (unsigned)std::min<long long>(32, std::max<long long>(1, (items + 1023) / 1024)));
-    };
-    k_batch_fill<0, 0><<<grid(32LL * b->max_n1), 256, 0, b->stream>>>(B, q);
-    if (b->any2d) k_batch_fill<1, 0><<<grid(2LL * b->max_n0), 256, 0, b->stream>>>(B, q);
-    k_batch_fill<0, 1><<<grid(8LL * b->max_n1), 256, 0, b->stream>>>(B, q);
-    if (b->any2d) k_batch_fill<1, 1><<<grid(2LL * b->max_n0), 256, 0, b->stream>>>(B, q);
+template <bool PLANE, int SCHEME, int FLUX>
+void launch_variant(sf_batch* b, const BatchStage& B, const int r[5]) {
+    constexpr int v = 2 * SCHEME + FLUX;
+    if (r[v + 1] == r[v]) return;
+    k_batch_stage<PLANE, SCHEME, FLUX>
+        <<<stage_blocks(b, r[v + 1] - r[v], k_batch_stage<PLANE, SCHEME, FLUX>), kXBlock, 0,
+           b->stream>>>(B, r[v], r[v + 1]);
 }
 
-void launch_x(sf_batch* b, const double* q, BatchStage st) {
-    const BatchDev B = view(b);
-    if (b->fused) {
-#define SF_XF(BS)                                                                            \
-    do {                                                                                     \
-        const Split sp = split_blocks(                                                       \
-            b->xr, persistent_blocks(b, b->nxt, resident_per_cu(k_batch_x_fused<BS>, BS)));  \
-        k_batch_x_fused<BS><<<(unsigned)sp.block[4], BS, 0, b->stream>>>(B, q, b->S, st, sp); \
-    } while (0)
-        switch (b->xbs) {
-            case 64: SF_XF(64); break;
-            case 256: SF_XF(256); break;
-            default: SF_XF(128); break;
-        }
-#undef SF_XF
+// Stage of the 2D (PLANE) or the 1D problems.  With one variant present the
+// kernel of its own is the fused launch, too.
+template <bool PLANE>
+void launch_stage(sf_batch* b, const BatchStage& B, const int r[5]) {
+    int present = 0;
+    for (int v = 0; v < 4; ++v) present += r[v + 1] > r[v];
+    if (b->fused && present > 1) {
+        const Split sp =
+            split_blocks(r, stage_blocks(b, r[4] - r[0], k_batch_stage_mixed<PLANE>));
+        k_batch_stage_mixed<PLANE><<<(unsigned)sp.block[4], kXBlock, 0, b->stream>>>(B, sp);
         return;
     }
-    for (int v = 0; v < 4; ++v) {
-        const int t0 = b->xr[v], t1 = b->xr[v + 1];
-        if (t1 == t0) continue;
-#define SF_XV1(BS, SC, FL, W)                                                              \
-    k_batch_x<BS, SC, FL, W>                                                               \
-        <<<persistent_blocks(b, t1 - t0, resident_per_cu(k_batch_x<BS, SC, FL, W>, BS)),  \
-           BS, 0, b->stream>>>(B, q, b->S, st, t0, t1)
-#define SF_XV(BS, SC, FL)                                   \
-    do {                                                   \
-        if (b->any2d || SC == 1) SF_XV1(BS, SC, FL, true); \
-        else SF_XV1(BS, SC, FL, false);                    \
-    } while (0)
-#define SF_XBS(SC, FL)                        \
-    switch (b->xbs) {                         \
-        case 64: SF_XV(64, SC, FL); break;    \
-        case 256: SF_XV(256, SC, FL); break;  \
-        default: SF_XV(128, SC, FL); break;   \
-    }
-        switch (v) {
-            case 0: SF_XBS(0, 0); break;
-            case 1: SF_XBS(0, 1); break;
-            case 2: SF_XBS(1, 0); break;
-            default: SF_XBS(1, 1); break;
-        }
-#undef SF_XBS
-#undef SF_XV
-#undef SF_XV1
-    }
+    launch_variant<PLANE, 0, 0>(b, B, r);
+    launch_variant<PLANE, 0, 1>(b, B, r);
+    launch_variant<PLANE, 1, 0>(b, B, r);
+    launch_variant<PLANE, 1, 1>(b, B, r);
 }
 
-void launch_y(sf_batch* b, const double* q) {
-    const BatchDev B = view(b);
-    if (b->nyt == 0) return;
-    if (b->fused) {
-        const Split sp = split_blocks(
-            b->yr, persistent_blocks(b, b->nyt, resident_per_cu(k_batch_y_fused, 64)));
-        k_batch_y_fused<<<(unsigned)sp.block[4], 64, 0, b->stream>>>(B, q, b->S, sp);
-        return;
-    }
-    for (int v = 0; v < 4; ++v) {
-        const int t0 = b->yr[v], t1 = b->yr[v + 1];
-        if (t1 == t0) continue;
-#define SF_YV(SC, FL)                                                                         \
-    k_batch_y<SC, FL><<<persistent_blocks(b, t1 - t0, resident_per_cu(k_batch_y<SC, FL>, 64)), \
-                        64, 0, b->stream>>>(B, q, b->S, t0, t1)
-        switch (v) {
-            case 0: SF_YV(0, 0); break;
-            case 1: SF_YV(0, 1); break;
-            case 2: SF_YV(1, 0); break;
-            default: SF_YV(1, 1); break;
-        }
-#undef SF_YV
-    }
+void launch_clock(sf_batch* b, int next) {
+    k_batch_clock<<<(unsigned)((b->nactive + 63) / 64), 64, 0, b->stream>>>(view(b), next);
 }
 
-// One SSPRK3 step of every live problem (the captured sequence):
-// stage s reads buf[in[s]] and writes buf[out[s]]; the step ends in buf[0].
+// One SSPRK3 step of every live problem (the captured sequence); its commit
+// is the next clock launch.
 void enqueue_step(sf_batch* b) {
-    const BatchDev B = view(b);
-    const unsigned nb = (unsigned)((b->nactive + 255) / 256);
-    k_batch_finalize<<<nb, 256, 0, b->stream>>>(B);
-    static const double base[3] = {0.0, 0.75, 1.0 / 3.0};
-    static const double incr[3] = {1.0, 0.25, 2.0 / 3.0};
-    const int in[3] = {0, 1, 2}, out[3] = {1, 2, 0};
+    launch_clock(b, 1);
     for (int s = 0; s < 3; ++s) {
-        if (s > 0) enqueue_fill(b, b->buf[in[s]]);
-        launch_y(b, b->buf[in[s]]);
-        BatchStage st{b->buf[0], b->buf[out[s]], base[s], incr[s], s, s == 2 ? 1 : 0};
-        launch_x(b, b->buf[in[s]], st);
+        const BatchStage B{b->d_items, b->d_live, b->d_tiles, s};
+        launch_stage<true>(b, B, b->plane);
+        launch_stage<false>(b, B, b->line);
     }
-    enqueue_fill(b, b->buf[0]);
-    k_batch_commit<<<nb, 256, 0, b->stream>>>(B);
 }
 
 int check_item(const sf_batch_item* it) {
@@ -890,7 +522,7 @@ bool valid_slot(const sf_batch* b, int slot) {
     return b && slot >= 0 && slot < b->item_capacity && b->used[slot];
 }
 
-// Fill and CFL-scan the problems admitted since the last step.
+// Boundary nodes and CFL scan of the problems admitted since the last step.
 int prepare_pending(sf_batch* b) {
     if (b->pending_scan.empty()) return 0;
     const int n = (int)b->pending_scan.size();
@@ -898,9 +530,8 @@ int prepare_pending(sf_batch* b) {
                            hipMemcpyHostToDevice, b->stream));
     const BatchDev B = view(b);
     k_batch_reset<<<(n + 255) / 256, 256, 0, b->stream>>>(B, b->d_scan, n);
-    enqueue_fill(b, b->buf[0]);
     const dim3 grid((unsigned)n, 16);
-    k_batch_cfl<<<grid, 256, 0, b->stream>>>(B, b->d_scan, b->buf[0]);
+    k_batch_prepare<<<grid, 256, 0, b->stream>>>(B, b->d_scan);
     SF_BHIP(hipGetLastError());
     SF_BHIP(hipStreamSynchronize(b->stream));
     b->pending_scan.clear();
@@ -928,6 +559,7 @@ int advance(sf_batch* b, int nsteps, int use_graph) {
     } else {
         for (int s = 0; s < nsteps; ++s) enqueue_step(b);
     }
+    launch_clock(b, 0);
     SF_BHIP(hipGetLastError());
     return 0;
 }
@@ -979,10 +611,9 @@ int sf_batch_create(int device, double gamma, size_t node_capacity, int item_cap
     const size_t state = sizeof(double) * 5 * node_capacity;
     bool ok = true;
     for (int i = 0; i < 3 && ok; ++i) ok = hipMalloc(&b->buf[i], state) == hipSuccess;
-    ok = ok && hipMalloc(&b->S, state) == hipSuccess;
-    ok = ok && hipMalloc(&b->d_items, sizeof(BatchItemDev) * item_capacity) == hipSuccess;
+    ok = ok && hipMalloc(&b->d_items, sizeof(ItemArgs) * item_capacity) == hipSuccess;
     ok = ok && hipMalloc(&b->d_dt, sizeof(double) * item_capacity) == hipSuccess;
-    ok = ok && hipMalloc(&b->d_dtmin, sizeof(unsigned long long) * item_capacity) == hipSuccess;
+    ok = ok && hipMalloc(&b->d_dtmin, sizeof(unsigned long long) * kItemDtWords * item_capacity) == hipSuccess;
     ok = ok && hipMalloc(&b->d_time, sizeof(double) * item_capacity) == hipSuccess;
     ok = ok && hipMalloc(&b->d_steps, sizeof(long long) * item_capacity) == hipSuccess;
     ok = ok && hipMalloc(&b->d_target, sizeof(long long) * item_capacity) == hipSuccess;
@@ -999,11 +630,10 @@ int sf_batch_create(int device, double gamma, size_t node_capacity, int item_cap
     ok = ok && hipMemset(b->d_target, 0, sizeof(long long) * item_capacity) == hipSuccess;
     // the arena starts zeroed, so padding that is never written stays finite
     for (int i = 0; i < 3 && ok; ++i) ok = hipMemset(b->buf[i], 0, state) == hipSuccess;
-    ok = ok && hipMemset(b->S, 0, state) == hipSuccess;
     if (!ok) {
         sf_batch_destroy(b);
         return bfail(SF_E_MEMORY, "sf_batch_create: device allocation of " +
-                                      std::to_string(4 * state) + " bytes failed");
+                                      std::to_string(3 * state) + " bytes failed");
     }
     b->items.resize(item_capacity);
     b->desc.resize(item_capacity);
@@ -1021,10 +651,9 @@ int sf_batch_destroy(sf_batch* b) {
     drop_graph(b);
     for (double* p : b->buf)
         if (p) (void)hipFree(p);
-    if (b->S) (void)hipFree(b->S);
     if (b->staging) (void)hipFree(b->staging);
     void* ptrs[] = {b->d_items, b->d_dt,   b->d_dtmin, b->d_time,   b->d_steps, b->d_target,
-                    b->d_flags, b->d_live, b->d_xt,    b->d_yt,     b->d_active, b->d_scan};
+                    b->d_flags, b->d_live, b->d_tiles, b->d_active, b->d_scan};
     for (void* p : ptrs)
         if (p) (void)hipFree(p);
     if (b->stream) (void)hipStreamDestroy(b->stream);
@@ -1067,7 +696,7 @@ int sf_batch_add(sf_batch* b, const sf_batch_item* item, const double* soa, long
         b->staging_nodes = N;
     }
     const long long off = fit->first, len = fit->second;
-    BatchItemDev it{};
+    sf_batch::Item it;
     it.off = off;
     it.n0 = item->n[0];
     it.n1 = std::max(1, item->n[1]);
@@ -1075,26 +704,15 @@ int sf_batch_add(sf_batch* b, const sf_batch_item* item, const double* soa, long
     it.gy = it.n1 > 1 ? 3 : 0;
     it.scheme = item->scheme;
     it.flux = item->flux;
-    it.cfl = item->cfl;
-    // uniform Cartesian metrics formed as for a grid with unit spacing on
-    // the absent axes (SF_mesh.cpp:320-338, SF_canonicalFace.h:87-108)
-    const double dx = item->d[0], dy = it.n1 > 1 ? item->d[1] : 1.0, dz = 1.0;
-    it.jac = 1.0 / (dx * dy * dz);
-    it.metric0 = 1.0 / dx;
-    it.metric1 = 1.0 / dy;
-    const double c0 = it.metric0 / it.jac, c1 = it.metric1 / it.jac;
-    const double f0 = 0.5 * (c0 + c0), f1 = 0.5 * (c1 + c1);
-    it.area0 = std::sqrt(f0 * f0 + 0.0 * 0.0 + 0.0 * 0.0);
-    it.area1 = std::sqrt(f1 * f1 + 0.0 * 0.0 + 0.0 * 0.0);
+    const ItemArgs args = item_args(b, s, it, item);
     const long long target = max_steps > 0 ? max_steps : LLONG_MAX;
-    SF_BHIP(hipMemcpy(b->d_items + s, &it, sizeof it, hipMemcpyHostToDevice));
+    SF_BHIP(hipMemcpy(b->d_items + s, &args, sizeof args, hipMemcpyHostToDevice));
     SF_BHIP(hipMemcpy(b->d_target + s, &target, sizeof target, hipMemcpyHostToDevice));
     SF_BHIP(hipMemcpyAsync(b->staging, soa, sizeof(double) * 5 * (size_t)N, hipMemcpyHostToDevice,
                            b->stream));
     b->items[s] = it;
-    const BatchDev B = view(b);
     const unsigned nb = (unsigned)std::min<long long>((N + 255) / 256, 4096);
-    k_batch_pack<<<nb, 256, 0, b->stream>>>(B, s, b->staging, b->buf[0], 1);
+    k_batch_pack<<<nb, 256, 0, b->stream>>>(b->d_items + s, b->staging, nullptr, 1);
     SF_BHIP(hipGetLastError());
     SF_BHIP(hipStreamSynchronize(b->stream));
     b->free_ranges.erase(fit);
@@ -1137,12 +755,11 @@ int sf_batch_remove(sf_batch* b, int slot) {
 int sf_batch_download(sf_batch* b, int slot, double* soa) {
     if (!soa || !valid_slot(b, slot)) return bfail(SF_E_ARG, "sf_batch_download: invalid slot");
     SF_BHIP(hipSetDevice(b->device));
-    const BatchItemDev& it = b->items[slot];
+    const sf_batch::Item& it = b->items[slot];
     const long long N = (long long)it.n0 * it.n1;
     if (N > b->staging_nodes) return bfail(SF_E_STATE, "sf_batch_download: staging too small");
-    const BatchDev B = view(b);
     const unsigned nb = (unsigned)std::min<long long>((N + 255) / 256, 4096);
-    k_batch_pack<<<nb, 256, 0, b->stream>>>(B, slot, b->buf[0], b->staging, 0);
+    k_batch_pack<<<nb, 256, 0, b->stream>>>(b->d_items + slot, nullptr, b->staging, 0);
     SF_BHIP(hipGetLastError());
     SF_BHIP(hipMemcpyAsync(soa, b->staging, sizeof(double) * 5 * (size_t)N, hipMemcpyDeviceToHost,
                            b->stream));
@@ -1220,8 +837,8 @@ int sf_batch_set_tiles(sf_batch* b, int xlen, int ylen) {
     if (xlen != 63 && xlen != 127 && xlen != 255)
         return bfail(SF_E_ARG, "sf_batch_set_tiles: x tile must be 63, 127 or 255 nodes");
     if (ylen < 4 || ylen > 4096) return bfail(SF_E_ARG, "sf_batch_set_tiles: y tile out of range");
-    b->xbs = xlen + 1;
-    b->yseg = ylen;
+    b->xlen = xlen;
+    b->ylen = ylen;
     b->tables_dirty = true;
     return 0;
 }
@@ -1256,13 +873,13 @@ int snapshot_save(sf_batch* b, Snapshot& sn) {
     const size_t n = (size_t)b->item_capacity;
     sn.dt.resize(n);
     sn.time.resize(n);
-    sn.dtmin.resize(n);
+    sn.dtmin.resize(n * kItemDtWords);
     sn.steps.resize(n);
     sn.flags.resize(n);
     SF_BHIP(hipStreamSynchronize(b->stream));
     SF_BHIP(hipMemcpy(sn.dt.data(), b->d_dt, sizeof(double) * n, hipMemcpyDeviceToHost));
     SF_BHIP(hipMemcpy(sn.time.data(), b->d_time, sizeof(double) * n, hipMemcpyDeviceToHost));
-    SF_BHIP(hipMemcpy(sn.dtmin.data(), b->d_dtmin, 8 * n, hipMemcpyDeviceToHost));
+    SF_BHIP(hipMemcpy(sn.dtmin.data(), b->d_dtmin, 8 * n * kItemDtWords, hipMemcpyDeviceToHost));
     SF_BHIP(hipMemcpy(sn.steps.data(), b->d_steps, 8 * n, hipMemcpyDeviceToHost));
     SF_BHIP(hipMemcpy(sn.flags.data(), b->d_flags, 4 * n, hipMemcpyDeviceToHost));
     return 0;
@@ -1276,7 +893,7 @@ int snapshot_restore(sf_batch* b, const Snapshot& sn) {
     const size_t n = (size_t)b->item_capacity;
     SF_BHIP(hipMemcpy(b->d_dt, sn.dt.data(), sizeof(double) * n, hipMemcpyHostToDevice));
     SF_BHIP(hipMemcpy(b->d_time, sn.time.data(), sizeof(double) * n, hipMemcpyHostToDevice));
-    SF_BHIP(hipMemcpy(b->d_dtmin, sn.dtmin.data(), 8 * n, hipMemcpyHostToDevice));
+    SF_BHIP(hipMemcpy(b->d_dtmin, sn.dtmin.data(), 8 * n * kItemDtWords, hipMemcpyHostToDevice));
     SF_BHIP(hipMemcpy(b->d_steps, sn.steps.data(), 8 * n, hipMemcpyHostToDevice));
     SF_BHIP(hipMemcpy(b->d_flags, sn.flags.data(), 4 * n, hipMemcpyHostToDevice));
     return 0;
@@ -1317,21 +934,22 @@ extern "C" int sf_batch_autotune(sf_batch* b, int trial_steps, sf_batch_tuning* 
     if (b->nactive == 0) return bfail(SF_E_STATE, "sf_batch_autotune: the batch is empty");
     Snapshot sn;
     int rc = snapshot_save(b, sn);
-    const int keep[4] = {b->xbs, b->yseg, b->blocks_per_cu, b->fused};
+    const int keep[4] = {b->xlen, b->ylen, b->blocks_per_cu, b->fused};
     sf_batch_tuning best{};
     best.ms_per_step = 1e300;
     int tried = 0;
     const int xlens[3] = {63, 127, 255};
     const int occs[5] = {0, 2, 4, 8, 16};   // 0: as many as stay resident
-    std::vector<int> ysegs = b->any2d ? std::vector<int>{16, 32, 64} : std::vector<int>{b->yseg};
+    std::vector<int> ysegs = b->any2d ? std::vector<int>{8, 16, 32}
+                                     : std::vector<int>{std::max(b->ylen, 4)};
     for (int fused = 0; fused < 2 && !rc; ++fused)
         for (int xl : xlens)
             for (int ys : ysegs)
                 for (int oc : occs) {
                     if (rc) break;
                     b->fused = fused;
-                    b->xbs = xl + 1;
-                    b->yseg = ys;
+                    b->xlen = xl;
+                    b->ylen = ys;
                     b->blocks_per_cu = oc;
                     b->tables_dirty = true;
                     double ms = 0.0;
@@ -1349,16 +967,16 @@ extern "C" int sf_batch_autotune(sf_batch* b, int trial_steps, sf_batch_tuning* 
                 }
     if (sn.q) (void)hipFree(sn.q);
     if (rc) {
-        b->xbs = keep[0];
-        b->yseg = keep[1];
+        b->xlen = keep[0];
+        b->ylen = keep[1];
         b->blocks_per_cu = keep[2];
         b->fused = keep[3];
         b->tables_dirty = true;
         return rc;
     }
     best.candidates = tried;
-    b->xbs = best.xlen + 1;
-    b->yseg = best.ylen;
+    b->xlen = best.xlen;
+    b->ylen = best.ylen;
     b->blocks_per_cu = best.blocks_per_cu;
     b->fused = best.fused;
     b->tables_dirty = true;
@@ -1387,14 +1005,14 @@ extern "C" int sf_batch_set_occupancy(sf_batch* b, int blocks_per_cu) {
 namespace sfamd {
 
 long long batch_copy_doubles(const sf_batch* b, int slot) {
-    const BatchItemDev& it = b->items[(size_t)slot];
+    const sf_batch::Item& it = b->items[(size_t)slot];
     return 5LL * it.m0 * (it.n1 + 2 * it.gy) + 1;
 }
 
 int batch_copy_out_async(sf_batch* b, int slot, double* dst, hipEvent_t done) {
     if (!valid_slot(b, slot)) return bfail(SF_E_ARG, "batch copy-out: invalid slot");
     SF_BHIP(hipSetDevice(b->device));
-    const BatchItemDev& it = b->items[(size_t)slot];
+    const sf_batch::Item& it = b->items[(size_t)slot];
     const long long extent = (long long)it.m0 * (it.n1 + 2 * it.gy);
     SF_BHIP(hipEventRecord(b->copy_after, b->stream));
     SF_BHIP(hipStreamWaitEvent(b->copy_stream, b->copy_after, 0));
@@ -1410,7 +1028,7 @@ int batch_copy_out_async(sf_batch* b, int slot, double* dst, hipEvent_t done) {
 }
 
 void batch_unpack(const sf_batch* b, int slot, const double* src, double* soa, double* time) {
-    const BatchItemDev& it = b->items[(size_t)slot];
+    const sf_batch::Item& it = b->items[(size_t)slot];
     const long long extent = (long long)it.m0 * (it.n1 + 2 * it.gy);
     const long long N = (long long)it.n0 * it.n1;
     for (int v = 0; v < 5; ++v)

@@ -182,12 +182,13 @@ constexpr int kDtSlots = 64, kDtStride = 16;
 // Wave-wide minimum of a positive double into the accumulator (one atomic per
 // wave; every lane of the wave calls it).  Positive doubles order like their
 // bit patterns; a lane without a value contributes +infinity.
+template <int SLOTS = kDtSlots>
 __device__ __forceinline__ void wave_min_atomic(double v, unsigned long long* slots) {
     const unsigned long long b = wave_min_bits(
         (v > 0.0 && isfinite(v)) ? (unsigned long long)__double_as_longlong(v)
                                  : 0x7FF0000000000000ull);
     if ((threadIdx.x & 63) == 0 && b != 0x7FF0000000000000ull)
-        atomicMin(slots + (blockIdx.x % kDtSlots) * kDtStride, b);
+        atomicMin(slots + (blockIdx.x % SLOTS) * kDtStride, b);
 }
 
 // Whether all five values are finite, from their sum: a NaN or an infinity

@@ -557,14 +557,15 @@ constexpr int kYxRows = 32;
 // Filling the ghosts by launches of their own took four 4-5 us launches per
 // stage in 2D and six in 3D, latency alone: a pass of 20 steps on 853^2 takes
 // 3.51 ms without them and 4.31 with, on 193 x 97 0.83 and 1.87.
-__device__ __forceinline__ void write_ends(const GridDev& G, double* __restrict__ out, int i,
+template <bool CORNERS = false>
+__device__ __forceinline__ bool write_ends(const GridDev& G, double* __restrict__ out, int i,
                                            int j, int k, long long id, const double qn[5]) {
     const int c[3] = {i, j, k};
     bool at_end = false;
 #pragma unroll
     for (int a = 0; a < 3; ++a)
         at_end |= (G.zg_lo[a] && c[a] == G.solved_lo[a]) || (G.zg_hi[a] && c[a] == G.solved_hi[a]);
-    if (!at_end) return;
+    if (!at_end) return true;
     const EndEnergy e = end_energy(qn, G.gamma);
 #pragma unroll
     for (int a = 0; a < 3; ++a)
@@ -580,6 +581,19 @@ __device__ __forceinline__ void write_ends(const GridDev& G, double* __restrict_
                 out[v * G.P + id + 2 * dir] = v == 4 ? e.ghost : qn[v];
             }
         }
+    if (CORNERS) {   // of a plane whose four ends carry zeroGradient
+#pragma unroll
+        for (int c = 0; c < 4; ++c) {
+            const int sx = c & 1, sy = c >> 1;
+            const bool here = i == (sx ? G.solved_hi[0] : G.solved_lo[0]) &&
+                              j == (sy ? G.solved_hi[1] : G.solved_lo[1]) && G.zg_lo[1];
+            if (!here) continue;
+            const long long at = id + (sx ? 1 : -1) + (sy ? G.stride[1] : -G.stride[1]);
+#pragma unroll
+            for (int v = 0; v < 5; ++v) out[v * G.P + at] = v == 4 ? e.node : qn[v];
+        }
+    }
+    return e.ok;
 }
 
 // Orders the LDS accesses of a wave's lanes among themselves: the hardware
@@ -598,31 +612,31 @@ struct YxShape {
     unsigned blocks;
 };
 
-template <int SCHEME, int FLUX, int TIME, bool HAS_S>
-__global__ __launch_bounds__(kXBlock)
-__attribute__((amdgpu_waves_per_eu(SCHEME == 3 ? 2 : 3, 8))) void k_stage_yx(SweepArgs W,
-                                                                             YxShape sh) {
+// LDS of a block that advances a tile of a y / x stage.
+template <int SCHEME>
+struct YxLds {
+    static constexpr int NS = Stencil<SCHEME>::ns;
+    double win[NS - 2][5][kXBlock + NS];   // ring rows a+1-H .. a+H-2, each
+                                           // H-1 halo columns, 64, H halo, 1 pad
+    double first[5][kYxRows];
+};
+
+// One tile: rows a0 .. a1-1 of plane k; lane t has column i0 + t.  W and
+// args() are the sweep's arguments, args() as sweep_args() reads them.
+// CORNERS: write_ends writes the corners, too; SLOTS: partial minima of the
+// CFL accumulator.
+template <int SCHEME, int FLUX, int TIME, bool HAS_S, bool CORNERS, int SLOTS, class Args>
+__device__ __forceinline__ void stage_yx_tile(const SweepArgs& W, const Args& args,
+                                              YxLds<SCHEME>& lds, int i0, int helper, int a0,
+                                              int a1, int k) {
     constexpr int NS = Stencil<SCHEME>::ns;
     constexpr int H = NS / 2;
-    constexpr int R = NS - 2;             // ring rows a+1-H .. a+H-2
-    constexpr int WID = kXBlock + NS;     // a row: H-1 halo columns, 64, H halo, 1 pad
+    constexpr int R = NS - 2;
     constexpr int HC = NS - 1;            // halo columns per row and variable
     static_assert(5 * HC <= kXBlock, "one lane per halo value");
-    __shared__ double win[R][5][WID];
-    __shared__ double first[5][kYxRows];
-    if (*W.A.flags) return;   // a fault was raised: keep the step-start state
-    // blocks of one XCD take consecutive numbers (x fastest), so that they
-    // share the halo lines in its L2
-    const unsigned chunk = gridDim.x >> 3;
-    const unsigned bid = (blockIdx.x & 7u) * chunk + (blockIdx.x >> 3);
-    if (bid >= sh.blocks) return;
+    auto& win = lds.win;
+    auto& first = lds.first;
     const int t = threadIdx.x;
-    const unsigned bx = bid % (unsigned)sh.nx, br = bid / (unsigned)sh.nx;
-    const int k = W.G.solved_lo[2] + (int)(br / (unsigned)sh.ny);
-    const int a0 = W.G.solved_lo[1] + (int)(br % (unsigned)sh.ny) * sh.rows;
-    const int a1 = min(a0 + sh.rows, W.G.solved_hi[1] + 1);
-    const int helper = kXBlock - sh.cols;              // 1: lane 0 only evaluates a face
-    const int i0 = W.G.solved_lo[0] + (int)bx * sh.cols - helper;   // lane 0's column
     const int i = i0 + t;
     const int hi0 = W.G.solved_hi[0];
     const bool node = i <= hi0 && t >= helper;         // this lane advances node i
@@ -686,7 +700,7 @@ __attribute__((amdgpu_waves_per_eu(SCHEME == 3 ? 2 : 3, 8))) void k_stage_yx(Swe
     wave_lds_order();
 #pragma clang loop unroll(disable)
     for (int a = a0 - 1; a < a1; ++a, id += step) {
-        const SweepArgs& T = sweep_args();
+        const SweepArgs& T = args();
         // the halo columns of row a join the ring; those of row a + 1 are
         // requested
         const auto slot = [&](int s) { return (head + s >= R) ? head + s - R : head + s; };
@@ -743,7 +757,7 @@ __attribute__((amdgpu_waves_per_eu(SCHEME == 3 ? 2 : 3, 8))) void k_stage_yx(Swe
             sx,
             [&](int side, double (&b)[5]) {
                 if (side == 0) {
-                    const SweepArgs& U = sweep_args();
+                    const SweepArgs& U = args();
 #pragma unroll
                     for (int v = 0; v < 5; ++v) {
                         if (HAS_S) ps[v] = at(U.S + v * U.G.P + id, node ? own : off);
@@ -763,7 +777,7 @@ __attribute__((amdgpu_waves_per_eu(SCHEME == 3 ? 2 : 3, 8))) void k_stage_yx(Swe
             lower[v] = t == 0 ? first[v][a - a0] : up;
         }
         if (node) {
-            const SweepArgs& U = sweep_args();
+            const SweepArgs& U = args();
             double pq[5];
 #pragma unroll
             for (int v = 0; v < 5; ++v) {
@@ -775,13 +789,34 @@ __attribute__((amdgpu_waves_per_eu(SCHEME == 3 ? 2 : 3, 8))) void k_stage_yx(Swe
             double qn[5];
             const long long nid = id + i + xo;
             stage_update_dt<TIME>(U.G, U.A, nid, pq, pq0, s5, dt_step, flags, dl, qn);
-            const SweepArgs& V = sweep_args();
-            write_ends(V.G, V.A.qout, i, a, k, nid, qn);
+            const SweepArgs& V = args();
+            write_ends<CORNERS>(V.G, V.A.qout, i, a, k, nid, qn);
             dt_local = fmin(dt_local, dl);
         }
     }
     raise_fault(flags, W.A.flags, W.A.fault_tag, W.A.tag);
-    if (W.A.reduce_dt) wave_min_atomic(dt_local, W.A.dtmin);
+    if (W.A.reduce_dt) wave_min_atomic<SLOTS>(dt_local, W.A.dtmin);
+}
+
+template <int SCHEME, int FLUX, int TIME, bool HAS_S>
+__global__ __launch_bounds__(kXBlock)
+__attribute__((amdgpu_waves_per_eu(SCHEME == 3 ? 2 : 3, 8))) void k_stage_yx(SweepArgs W,
+                                                                             YxShape sh) {
+    __shared__ YxLds<SCHEME> lds;
+    if (*W.A.flags) return;   // a fault was raised: keep the step-start state
+    // blocks of one XCD take consecutive numbers (x fastest), so that they
+    // share the halo lines in its L2
+    const unsigned chunk = gridDim.x >> 3;
+    const unsigned bid = (blockIdx.x & 7u) * chunk + (blockIdx.x >> 3);
+    if (bid >= sh.blocks) return;
+    const unsigned bx = bid % (unsigned)sh.nx, br = bid / (unsigned)sh.nx;
+    const int k = W.G.solved_lo[2] + (int)(br / (unsigned)sh.ny);
+    const int a0 = W.G.solved_lo[1] + (int)(br % (unsigned)sh.ny) * sh.rows;
+    const int a1 = min(a0 + sh.rows, W.G.solved_hi[1] + 1);
+    const int helper = kXBlock - sh.cols;              // 1: lane 0 only evaluates a face
+    const int i0 = W.G.solved_lo[0] + (int)bx * sh.cols - helper;   // lane 0's column
+    stage_yx_tile<SCHEME, FLUX, TIME, HAS_S, false, kDtSlots>(
+        W, [] () -> const SweepArgs& { return sweep_args(); }, lds, i0, helper, a0, a1, k);
 }
 
 }  // namespace sfamd

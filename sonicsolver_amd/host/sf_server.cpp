@@ -379,12 +379,6 @@ int sf_server_create(int device, double gamma, size_t device_bytes, int max_item
         delete s;
         return rc;
     }
-    // the launch shape the autotuner picks for one-variant streams of
-    // mid-size problems: one launch per variant, long x tiles, a deep
-    // persistent grid
-    sf_batch_set_schedule(s->batch, 0);
-    sf_batch_set_tiles(s->batch, 255, 32);
-    sf_batch_set_occupancy(s->batch, 16);
     s->max_items = max_items;
     s->steps_per_tick = steps_per_tick;
     s->arena_nodes = nodes;
