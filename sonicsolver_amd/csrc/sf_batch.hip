@@ -26,6 +26,7 @@
 #include <climits>
 #include <cmath>
 #include <cstdio>
+#include <cstring>
 #include <limits>
 #include <map>
 #include <mutex>
@@ -126,21 +127,50 @@ __global__ void k_batch_reset(BatchDev B, const int* __restrict__ list, int n) {
     B.live[slot] = 0;
 }
 
-// unique-node SoA of one problem <-> its padded block in the arena
-__global__ __launch_bounds__(256) void k_batch_pack(const ItemArgs* __restrict__ item,
-                                                    const double* __restrict__ src,
-                                                    double* __restrict__ dst, int to_arena) {
-    const GridDev& G = item->stage[0].G;
-    double* const q = const_cast<double*>(item->stage[0].q);
-    const long long N = (long long)G.n[0] * G.n[1];
-    for (long long u = blockIdx.x * (long long)blockDim.x + threadIdx.x; u < N;
-         u += (long long)gridDim.x * blockDim.x) {
-        const long long id = node_index(G, (int)(u % G.n[0]), (int)(u / G.n[0]), 0);
+// A problem's arguments as a kernel's first argument, read in place.
+__device__ __forceinline__ const ItemArgs& item_kernarg() {
+    return *(const ItemArgs*)(const __attribute__((address_space(4))) ItemArgs*)
+        __builtin_amdgcn_kernarg_segment_ptr();
+}
+
+// Admission: nodes u0 .. u0+cnt-1 of a problem from pinned host memory
+// (src[v*cnt + u-u0]) into its padded block, and its arguments and step limit
+// into their tables.
+__global__ __launch_bounds__(256) void k_batch_admit(ItemArgs, ItemArgs* __restrict__ item,
+                                                     long long* __restrict__ target,
+                                                     long long limit,
+                                                     const double* __restrict__ src,
+                                                     unsigned u0, unsigned cnt) {
+    const ItemArgs& args = item_kernarg();
+    if (blockIdx.x == 0) {
+        constexpr unsigned words = sizeof(ItemArgs) / 8;
+        for (unsigned w = threadIdx.x; w < words; w += blockDim.x)
+            ((unsigned long long*)item)[w] = ((const unsigned long long*)&args)[w];
+        if (threadIdx.x == 0) *target = limit;
+    }
+    const GridDev& G = args.stage[0].G;
+    double* const q = const_cast<double*>(args.stage[0].q);
+    for (unsigned u = blockIdx.x * blockDim.x + threadIdx.x; u < cnt; u += gridDim.x * blockDim.x) {
+        const unsigned at = u0 + u, n0 = (unsigned)G.n[0];
+        const long long id = node_index(G, (int)(at % n0), (int)(at / n0), 0);
 #pragma unroll
-        for (int v = 0; v < 5; ++v) {
-            if (to_arena) q[v * G.P + id] = src[v * N + u];
-            else dst[v * N + u] = q[v * G.P + id];
-        }
+        for (int v = 0; v < 5; ++v) q[v * G.P + id] = src[(size_t)v * cnt + u];
+    }
+}
+
+// Nodes u0 .. u0+cnt-1 of a problem's state to pinned host memory
+// (dst[v*cnt + u-u0], then its clock time where `time` is given).
+__global__ __launch_bounds__(256) void k_batch_pack(const ItemArgs* __restrict__ item,
+                                                    double* __restrict__ dst, unsigned u0,
+                                                    unsigned cnt, const double* __restrict__ time) {
+    const GridDev& G = item->stage[0].G;
+    const double* const q = item->stage[0].q;
+    if (time && blockIdx.x == 0 && threadIdx.x == 0) dst[5 * (size_t)cnt] = *time;
+    for (unsigned u = blockIdx.x * blockDim.x + threadIdx.x; u < cnt; u += gridDim.x * blockDim.x) {
+        const unsigned at = u0 + u, n0 = (unsigned)G.n[0];
+        const long long id = node_index(G, (int)(at % n0), (int)(at / n0), 0);
+#pragma unroll
+        for (int v = 0; v < 5; ++v) dst[(size_t)v * cnt + u] = q[v * G.P + id];
     }
 }
 
@@ -170,6 +200,10 @@ long long padded_nodes(const sf_batch_item& it) {
 
 }  // namespace
 
+constexpr int kPinChunks = 4;
+constexpr size_t kPinBytes = 2u << 20;                       // of a chunk
+constexpr long long kPinNodes = (long long)(kPinBytes / (5 * sizeof(double)));
+
 struct sf_batch {
     // placement of a problem in the arena
     struct Item {
@@ -186,8 +220,17 @@ struct sf_batch {
     hipStream_t copy_stream = nullptr;   // copy-out of finished problems
     hipEvent_t copy_after = nullptr;     // orders copy-outs after the compute stream
     double* buf[3] = {nullptr, nullptr, nullptr};
-    double* staging = nullptr;
-    long long staging_nodes = 0;
+    // Pinned host memory that kernels read admitted states from and write
+    // downloaded ones to: a ring of chunks, each reused once the work queued
+    // on it has passed.  An admitted problem of 2300 nodes takes 10 us and a
+    // downloaded one 21; three blocking copies from pageable memory and a
+    // wait took 57, a device-side pack and a blocking copy 33.  8 MiB keep
+    // the link busy: a chunk takes 40 us on it and 150 to fill.
+    char* pin = nullptr;
+    hipEvent_t pin_done[kPinChunks] = {};
+    bool pin_busy[kPinChunks] = {};
+    int pin_at = 0;
+    size_t pin_used = 0;
     ItemArgs* d_items = nullptr;
     double* d_dt = nullptr;
     unsigned long long* d_dtmin = nullptr;
@@ -300,6 +343,49 @@ void drop_graph(sf_batch* b) {
     b->graph = nullptr;
 }
 
+int pin_open(sf_batch* b) {
+    if (b->pin) return 0;
+    for (hipEvent_t& e : b->pin_done)
+        if (!e) SF_BHIP(hipEventCreateWithFlags(&e, hipEventDisableTiming));
+    SF_BHIP(hipHostMalloc((void**)&b->pin, kPinChunks * kPinBytes, hipHostMallocDefault));
+    return 0;
+}
+
+// Room for `bytes` (at most a chunk) in the pinned ring.  The work on it has
+// to be queued on the compute stream before the next call.
+int pin_reserve(sf_batch* b, size_t bytes, void** out) {
+    if (int rc = pin_open(b)) return rc;
+    if (b->pin_used + bytes > kPinBytes) {
+        SF_BHIP(hipEventRecord(b->pin_done[b->pin_at], b->stream));
+        b->pin_busy[b->pin_at] = true;
+        b->pin_at = (b->pin_at + 1) % kPinChunks;
+        if (b->pin_busy[b->pin_at]) SF_BHIP(hipEventSynchronize(b->pin_done[b->pin_at]));
+        b->pin_busy[b->pin_at] = false;
+        b->pin_used = 0;
+    }
+    *out = b->pin + b->pin_at * kPinBytes + b->pin_used;
+    b->pin_used += (bytes + 255) & ~(size_t)255;
+    return 0;
+}
+
+// The compute stream is idle: the whole ring is free.
+void pin_reset(sf_batch* b) {
+    for (bool& busy : b->pin_busy) busy = false;
+    b->pin_used = 0;
+}
+
+// Queue a copy of host data that may be changed on return.
+int upload(sf_batch* b, void* dst, const void* src, size_t bytes) {
+    for (size_t o = 0; o < bytes; o += kPinBytes) {
+        const size_t n = std::min(kPinBytes, bytes - o);
+        void* p = nullptr;
+        if (int rc = pin_reserve(b, n, &p)) return rc;
+        std::memcpy(p, (const char*)src + o, n);
+        SF_BHIP(hipMemcpyAsync((char*)dst + o, p, n, hipMemcpyHostToDevice, b->stream));
+    }
+    return 0;
+}
+
 // Strips of a 2D problem along x: 63 columns and a lane that evaluates the
 // first face, or 64 with the first faces evaluated beforehand where that
 // saves a strip.
@@ -392,11 +478,8 @@ int rebuild_tables(sf_batch* b) {
         SF_BHIP(hipMalloc(&b->d_tiles, want * sizeof(BatchTile)));
         b->tile_cap = want;
     }
-    if (!tiles.empty())
-        SF_BHIP(hipMemcpy(b->d_tiles, tiles.data(), tiles.size() * sizeof(BatchTile),
-                          hipMemcpyHostToDevice));
-    if (!act.empty())
-        SF_BHIP(hipMemcpy(b->d_active, act.data(), act.size() * sizeof(int), hipMemcpyHostToDevice));
+    if (int rc = upload(b, b->d_tiles, tiles.data(), tiles.size() * sizeof(BatchTile))) return rc;
+    if (int rc = upload(b, b->d_active, act.data(), act.size() * sizeof(int))) return rc;
     b->nactive = (int)act.size();
     b->tables_dirty = false;
     drop_graph(b);
@@ -526,14 +609,12 @@ bool valid_slot(const sf_batch* b, int slot) {
 int prepare_pending(sf_batch* b) {
     if (b->pending_scan.empty()) return 0;
     const int n = (int)b->pending_scan.size();
-    SF_BHIP(hipMemcpyAsync(b->d_scan, b->pending_scan.data(), sizeof(int) * n,
-                           hipMemcpyHostToDevice, b->stream));
+    if (int rc = upload(b, b->d_scan, b->pending_scan.data(), sizeof(int) * (size_t)n)) return rc;
     const BatchDev B = view(b);
     k_batch_reset<<<(n + 255) / 256, 256, 0, b->stream>>>(B, b->d_scan, n);
     const dim3 grid((unsigned)n, 16);
     k_batch_prepare<<<grid, 256, 0, b->stream>>>(B, b->d_scan);
     SF_BHIP(hipGetLastError());
-    SF_BHIP(hipStreamSynchronize(b->stream));
     b->pending_scan.clear();
     return 0;
 }
@@ -651,7 +732,9 @@ int sf_batch_destroy(sf_batch* b) {
     drop_graph(b);
     for (double* p : b->buf)
         if (p) (void)hipFree(p);
-    if (b->staging) (void)hipFree(b->staging);
+    if (b->pin) (void)hipHostFree(b->pin);
+    for (hipEvent_t e : b->pin_done)
+        if (e) (void)hipEventDestroy(e);
     void* ptrs[] = {b->d_items, b->d_dt,   b->d_dtmin, b->d_time,   b->d_steps, b->d_target,
                     b->d_flags, b->d_live, b->d_tiles, b->d_active, b->d_scan};
     for (void* p : ptrs)
@@ -688,13 +771,6 @@ int sf_batch_add(sf_batch* b, const sf_batch_item* item, const double* soa, long
         return bfail(SF_E_MEMORY, "sf_batch_add: no room in the arena for the problem (" +
                                       std::to_string(need) + " padded nodes)");
     const long long N = (long long)item->n[0] * std::max(1, item->n[1]);
-    if (N > b->staging_nodes) {
-        if (b->staging) SF_BHIP(hipFree(b->staging));
-        b->staging = nullptr;
-        b->staging_nodes = 0;
-        SF_BHIP(hipMalloc(&b->staging, sizeof(double) * 5 * (size_t)N));
-        b->staging_nodes = N;
-    }
     const long long off = fit->first, len = fit->second;
     sf_batch::Item it;
     it.off = off;
@@ -706,15 +782,18 @@ int sf_batch_add(sf_batch* b, const sf_batch_item* item, const double* soa, long
     it.flux = item->flux;
     const ItemArgs args = item_args(b, s, it, item);
     const long long target = max_steps > 0 ? max_steps : LLONG_MAX;
-    SF_BHIP(hipMemcpy(b->d_items + s, &args, sizeof args, hipMemcpyHostToDevice));
-    SF_BHIP(hipMemcpy(b->d_target + s, &target, sizeof target, hipMemcpyHostToDevice));
-    SF_BHIP(hipMemcpyAsync(b->staging, soa, sizeof(double) * 5 * (size_t)N, hipMemcpyHostToDevice,
-                           b->stream));
+    for (long long u0 = 0; u0 < N; u0 += kPinNodes) {
+        const long long cnt = std::min(kPinNodes, N - u0);
+        void* p = nullptr;
+        if (int rc = pin_reserve(b, sizeof(double) * 5 * (size_t)cnt, &p)) return rc;
+        for (int v = 0; v < 5; ++v)
+            std::memcpy((double*)p + v * cnt, soa + v * N + u0, sizeof(double) * (size_t)cnt);
+        k_batch_admit<<<(unsigned)((cnt + 255) / 256), 256, 0, b->stream>>>(
+            args, b->d_items + s, b->d_target + s, target, (const double*)p, (unsigned)u0,
+            (unsigned)cnt);
+        SF_BHIP(hipGetLastError());
+    }
     b->items[s] = it;
-    const unsigned nb = (unsigned)std::min<long long>((N + 255) / 256, 4096);
-    k_batch_pack<<<nb, 256, 0, b->stream>>>(b->d_items + s, b->staging, nullptr, 1);
-    SF_BHIP(hipGetLastError());
-    SF_BHIP(hipStreamSynchronize(b->stream));
     b->free_ranges.erase(fit);
     if (len > need) b->free_ranges[off + need] = len - need;
     b->desc[s] = *item;
@@ -757,13 +836,32 @@ int sf_batch_download(sf_batch* b, int slot, double* soa) {
     SF_BHIP(hipSetDevice(b->device));
     const sf_batch::Item& it = b->items[slot];
     const long long N = (long long)it.n0 * it.n1;
-    if (N > b->staging_nodes) return bfail(SF_E_STATE, "sf_batch_download: staging too small");
-    const unsigned nb = (unsigned)std::min<long long>((N + 255) / 256, 4096);
-    k_batch_pack<<<nb, 256, 0, b->stream>>>(b->d_items + slot, nullptr, b->staging, 0);
-    SF_BHIP(hipGetLastError());
-    SF_BHIP(hipMemcpyAsync(soa, b->staging, sizeof(double) * 5 * (size_t)N, hipMemcpyDeviceToHost,
-                           b->stream));
-    SF_BHIP(hipStreamSynchronize(b->stream));
+    if (int rc = pin_open(b)) return rc;
+    // a chunk of the ring per piece; the pieces after it are written while
+    // one is copied out
+    const long long pieces = (N + kPinNodes - 1) / kPinNodes;
+    const auto count = [&](long long p) { return std::min(kPinNodes, N - p * kPinNodes); };
+    const auto chunk = [&](long long p) {
+        return (double*)(b->pin + (size_t)(p % kPinChunks) * kPinBytes);
+    };
+    for (long long p = 0; p < pieces + kPinChunks; ++p) {
+        const long long out = p - kPinChunks;
+        if (out >= 0 && out < pieces) {
+            if (pieces == 1) SF_BHIP(hipStreamSynchronize(b->stream));
+            else SF_BHIP(hipEventSynchronize(b->pin_done[out % kPinChunks]));
+            for (int v = 0; v < 5; ++v)
+                std::memcpy(soa + v * N + out * kPinNodes, chunk(out) + v * count(out),
+                            sizeof(double) * (size_t)count(out));
+        }
+        if (p < pieces) {
+            k_batch_pack<<<(unsigned)((count(p) + 255) / 256), 256, 0, b->stream>>>(
+                b->d_items + slot, chunk(p), (unsigned)(p * kPinNodes), (unsigned)count(p),
+                nullptr);
+            SF_BHIP(hipGetLastError());
+            if (pieces > 1) SF_BHIP(hipEventRecord(b->pin_done[p % kPinChunks], b->stream));
+        }
+    }
+    pin_reset(b);
     return 0;
 }
 
@@ -777,6 +875,7 @@ int sf_batch_step(sf_batch* b, int nsteps, int use_graph) {
     if (b->nactive == 0 || nsteps == 0) return 0;
     if (int rc = advance(b, nsteps, use_graph)) return rc;
     SF_BHIP(hipStreamSynchronize(b->stream));
+    pin_reset(b);
     std::vector<unsigned> flags((size_t)b->item_capacity);
     int faulted = 0;
     if (int rc = read_faults(b, flags.data(), &faulted)) return rc;
@@ -1006,37 +1105,28 @@ namespace sfamd {
 
 long long batch_copy_doubles(const sf_batch* b, int slot) {
     const sf_batch::Item& it = b->items[(size_t)slot];
-    return 5LL * it.m0 * (it.n1 + 2 * it.gy) + 1;
+    return 5LL * it.n0 * it.n1 + 1;
 }
 
 int batch_copy_out_async(sf_batch* b, int slot, double* dst, hipEvent_t done) {
     if (!valid_slot(b, slot)) return bfail(SF_E_ARG, "batch copy-out: invalid slot");
     SF_BHIP(hipSetDevice(b->device));
     const sf_batch::Item& it = b->items[(size_t)slot];
-    const long long extent = (long long)it.m0 * (it.n1 + 2 * it.gy);
+    const unsigned N = (unsigned)it.n0 * (unsigned)it.n1;
     SF_BHIP(hipEventRecord(b->copy_after, b->stream));
     SF_BHIP(hipStreamWaitEvent(b->copy_stream, b->copy_after, 0));
-    // the state after a whole step is in buf[0]
-    for (int v = 0; v < 5; ++v)
-        SF_BHIP(hipMemcpyAsync(dst + v * extent, b->buf[0] + v * b->capacity + it.off,
-                               sizeof(double) * (size_t)extent, hipMemcpyDeviceToHost,
-                               b->copy_stream));
-    SF_BHIP(hipMemcpyAsync(dst + 5 * extent, b->d_time + slot, sizeof(double),
-                           hipMemcpyDeviceToHost, b->copy_stream));
+    k_batch_pack<<<(N + 255) / 256, 256, 0, b->copy_stream>>>(b->d_items + slot, dst, 0, N,
+                                                              b->d_time + slot);
+    SF_BHIP(hipGetLastError());
     SF_BHIP(hipEventRecord(done, b->copy_stream));
     return 0;
 }
 
 void batch_unpack(const sf_batch* b, int slot, const double* src, double* soa, double* time) {
     const sf_batch::Item& it = b->items[(size_t)slot];
-    const long long extent = (long long)it.m0 * (it.n1 + 2 * it.gy);
-    const long long N = (long long)it.n0 * it.n1;
-    for (int v = 0; v < 5; ++v)
-        for (int j = 0; j < it.n1; ++j) {
-            const double* row = src + v * extent + (long long)(j + it.gy) * it.m0 + 3;
-            std::copy(row, row + it.n0, soa + v * N + (long long)j * it.n0);
-        }
-    *time = src[5 * extent];
+    const size_t N = (size_t)it.n0 * (size_t)it.n1;
+    std::memcpy(soa, src, sizeof(double) * 5 * N);
+    *time = src[5 * N];
 }
 
 }  // namespace sfamd

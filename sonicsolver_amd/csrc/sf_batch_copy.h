@@ -10,8 +10,8 @@ struct sf_batch;
 
 namespace sfamd {
 
-// Doubles of host memory one copy-out of `slot` fills: the padded block of
-// each of the five variables, then the problem's clock time.
+// Doubles of host memory one copy-out of `slot` fills: the unique-node SoA
+// (5 x n0 x n1), then the problem's clock time.
 long long batch_copy_doubles(const sf_batch* b, int slot);
 
 // Enqueue the copy of `slot`'s state and time into pinned host memory

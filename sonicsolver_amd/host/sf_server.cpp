@@ -48,7 +48,7 @@ struct Request {
     sf_batch_item item{};
     long long steps = 0;
     long long nodes = 0;          // unique nodes
-    std::vector<double> state;    // initial state, then the result
+    std::unique_ptr<double[]> state;   // initial state, then the result
     Clock::time_point submit, done;
     int status = 0;               // 0 pending, 1 done, -1 failed
     int slot = -1;
@@ -56,6 +56,8 @@ struct Request {
     double time = 0.0;
     int bypassed = 0;
     std::string error;
+
+    size_t doubles() const { return (size_t)5 * (size_t)nodes; }
 };
 
 using RequestPtr = std::shared_ptr<Request>;
@@ -143,10 +145,10 @@ void admit(sf_server* s) {
     for (auto it = s->waiting.begin(); it != s->waiting.end();) {
         const RequestPtr& r = *it;
         int slot = -1;
-        const int rc = sf_batch_add(s->batch, &r->item, r->state.data(), r->steps, &slot);
+        const int rc = sf_batch_add(s->batch, &r->item, r->state.get(), r->steps, &slot);
         if (rc == 0) {
             r->slot = slot;
-            std::vector<double>().swap(r->state);  // the device holds it now
+            r->state.reset();  // the batch holds it now
             {
                 std::lock_guard<std::mutex> lk(s->mu);
                 ++s->resident;
@@ -225,8 +227,9 @@ void collect(sf_server* s, bool wait) {
         sf_server::Pinned& b = s->pinned[(size_t)it->buffer];
         std::string err;
         if (e == hipSuccess) {
-            r->state.resize((size_t)5 * (size_t)r->nodes);
-            sfamd::batch_unpack(s->batch, r->slot, b.p, r->state.data(), &r->time);
+            r->state.reset(new (std::nothrow) double[r->doubles()]);
+            if (r->state) sfamd::batch_unpack(s->batch, r->slot, b.p, r->state.get(), &r->time);
+            else err = "copy-out: host allocation failed";
         } else {
             err = std::string("copy-out: ") + hipGetErrorString(e);
         }
@@ -422,10 +425,11 @@ int sf_server_submit(sf_server* s, const sf_batch_item* item, const double* soa,
     r->steps = steps;
     r->nodes = (long long)item->n[0] * std::max(1, item->n[1]);
     try {
-        r->state.assign(soa, soa + (size_t)5 * (size_t)r->nodes);
+        r->state.reset(new double[r->doubles()]);
     } catch (...) {
         return fail(SF_E_MEMORY, "sf_server_submit: host allocation failed");
     }
+    std::memcpy(r->state.get(), soa, sizeof(double) * r->doubles());
     r->submit = Clock::now();
     {
         std::lock_guard<std::mutex> lk(s->mu);
@@ -467,20 +471,19 @@ int sf_server_wait(sf_server* s, long long ticket, double timeout_s, int* status
 int sf_server_result(sf_server* s, long long ticket, double* soa, double* time, long long* steps,
                      double* latency_ms) {
     if (!s) return fail(SF_E_ARG, "sf_server_result: null server");
-    std::lock_guard<std::mutex> lk(s->mu);
-    RequestPtr r = find(s, ticket);
-    if (!r) return fail(SF_E_ARG, "sf_server_result: unknown ticket");
-    if (r->status == 0) return fail(SF_E_STATE, "sf_server_result: request still pending");
-    if (r->status < 0) {
-        const std::string msg = "request failed: " + r->error;
-        s->table.erase(ticket);
-        return fail(SF_E_NUMERIC, msg);
+    RequestPtr r;
+    {
+        std::lock_guard<std::mutex> lk(s->mu);
+        r = find(s, ticket);
+        if (!r) return fail(SF_E_ARG, "sf_server_result: unknown ticket");
+        if (r->status == 0) return fail(SF_E_STATE, "sf_server_result: request still pending");
+        s->table.erase(ticket);   // this call owns the finished request
     }
-    if (soa) std::memcpy(soa, r->state.data(), sizeof(double) * r->state.size());
+    if (r->status < 0) return fail(SF_E_NUMERIC, "request failed: " + r->error);
+    if (soa) std::memcpy(soa, r->state.get(), sizeof(double) * r->doubles());
     if (time) *time = r->time;
     if (steps) *steps = r->steps_done;
     if (latency_ms) *latency_ms = std::chrono::duration<double, std::milli>(r->done - r->submit).count();
-    s->table.erase(ticket);
     return 0;
 }
 
