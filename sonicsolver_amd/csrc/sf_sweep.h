@@ -5,7 +5,7 @@
 // parallel.
 #pragma once
 
-#include "sf_sweep_kernels.h"
+#include "sf_block_kernels.h"
 
 #include <algorithm>
 
@@ -37,6 +37,36 @@ inline double march_cost(long long blocks, double faces, int cus) {
     if (w <= 1) return 1.73 * (faces + 5.0);
     if (w == 2) return 2.6 * (faces + 4.0);
     return 1.07 * (double)w * (faces + (w <= 4 ? 3.0 : 1.5));
+}
+
+// Waves on the busiest SIMD when `blocks` blocks of `waves` waves are dealt
+// evenly to the compute units.
+inline long long waves_per_simd(long long blocks, int waves, int cus) {
+    const long long units = std::max(cus, 8);
+    return (blocks + units - 1) / units * ((waves + 3) / 4);
+}
+
+inline long long block_load(const YxShape& sh, int cus) {
+    return waves_per_simd(sh.blocks, block_waves(sh), cus);
+}
+
+// Nodes along z of a block of the z sweep of small grids (k_block_z), whose
+// blocks take `columns` columns of 64 nodes, or 0 where the march takes it:
+// where the device does not hold all blocks at once.  With WENO5/HLLC a pass
+// of 20 steps on 24^3 takes 0.96 ms by the march and 0.86 by blocks, on 48^3
+// 1.75 and 1.50 (three waves per SIMD), on 100 x 40 x 40 2.02 and 1.92 (four);
+// on 64^3, with six, 2.56 and 3.16.
+template <int SCHEME>
+int block_z_nodes(long long columns, int nz, int cus) {
+    int best = 0;
+    long long least = SCHEME == 3 ? 3 : 5;
+    for (int nodes : {7, 3}) {
+        const long long w = waves_per_simd(columns * ((nz + nodes - 1) / nodes), nodes + 1, cus);
+        if (w >= least) continue;
+        least = w;
+        best = nodes;
+    }
+    return best;
 }
 
 // Grid of the x sweep (a multiple of 8 for the XCD mapping): one block per
@@ -133,6 +163,17 @@ int launch_sweep_fm(const SweepCall& c, int axis) {
         // chip.  A face's arithmetic does not depend on the segment length,
         // so neither does the result.  c.seg > 0 fixes the length instead.
         int seg = c.seg;
+        if constexpr (MODE == kCopyS) {
+            const int nodes = axis == 2 && seg <= 0
+                                  ? block_z_nodes<SCHEME>((long long)cols * other, span(2), c.cus)
+                                  : 0;
+            if (nodes > 0) {
+                const dim3 grid(cols, other, (unsigned)((span(2) + nodes - 1) / nodes));
+                k_block_z<SCHEME, FLUX><<<grid, kXBlock * (nodes + 1), 0, c.stream>>>(G, c.q, c.S,
+                                                                                      c.A);
+                return 0;
+            }
+        }
         if (seg <= 0) {
             double least = 0.0;
             for (int s = 1; s <= 64; ++s) {
@@ -167,9 +208,14 @@ template <int SCHEME, int FLUX>
 int launch_yx_f(const SweepCall& c, const YxShape& sh) {
     const SweepArgs W{c.G, c.q, c.S, c.A};
     const unsigned nb = (sh.blocks + 7) & ~7u;
+    const unsigned wg = kXBlock * block_waves(sh);
 #define SF_LAUNCH_YX(T)                                                                       \
     do {                                                                                      \
-        if (c.G.active[2])                                                                    \
+        if (sh.block && c.G.active[2])                                                        \
+            k_block_yx<SCHEME, FLUX, T, true><<<nb, wg, 0, c.stream>>>(W, sh);                \
+        else if (sh.block)                                                                    \
+            k_block_yx<SCHEME, FLUX, T, false><<<nb, wg, 0, c.stream>>>(W, sh);               \
+        else if (c.G.active[2])                                                                    \
             k_stage_yx<SCHEME, FLUX, T, true><<<nb, kXBlock, 0, c.stream>>>(W, sh);           \
         else                                                                                  \
             k_stage_yx<SCHEME, FLUX, T, false><<<nb, kXBlock, 0, c.stream>>>(W, sh);          \
@@ -219,6 +265,28 @@ extern template int launch_yx<1>(const SweepCall&, int, const YxShape&);
 extern template int launch_yx<2>(const SweepCall&, int, const YxShape&);
 extern template int launch_yx<3>(const SweepCall&, int, const YxShape&);
 
+// Shape of a launch of k_block_yx over nx x ny x nz advanced nodes: the rows
+// and columns of a block with the least load.  A block's 2 rows + 1 waves,
+// one more with 64 columns, fill the four SIMDs evenly, or all but one wave,
+// with an odd number of rows.
+inline YxShape block_shape(int nx, int ny, int nz, int cus) {
+    YxShape best{};
+    for (int cols = kXBlock - 1; cols <= kXBlock; ++cols)
+        for (int rows = 1; rows <= kBlockRows; rows += 2) {
+            YxShape sh{};
+            sh.cols = cols;
+            sh.rows = rows;
+            sh.nx = (nx + cols - 1) / cols;
+            sh.ny = (ny + rows - 1) / rows;
+            const long long blocks = (long long)sh.nx * sh.ny * nz;
+            if (blocks > 1LL << 24) continue;
+            sh.blocks = (unsigned)blocks;
+            sh.block = 1;
+            if (!best.blocks || block_load(sh, cus) < block_load(best, cus)) best = sh;
+        }
+    return best;
+}
+
 // Shape of the fused y / x launch of a stage, or blocks = 0 where the
 // separate sweeps take it: the residual-only mode, a chosen x walk, and grids
 // narrower than half a wave that fill the device more than twice over, whose
@@ -229,12 +297,26 @@ extern template int launch_yx<3>(const SweepCall&, int, const YxShape&);
 // TENO5/HLLC 6.39 -> 5.75, 853^2 5.22 -> 4.23, 256^2 TENO5/HLLC 2.40 ->
 // 1.36, 64^3 4.32 -> 2.87, 40^2 1.05 -> 0.76 (the small ones by shorter
 // segments in the z march, too).
+//
+// Small grids take k_block_yx, up to the number of waves per SIMD at which it
+// stays ahead of the march with every scheme: 8 in 2D (400^2, passes of 20
+// steps: WENO5/HLLC 1.11 ms against 1.24, TENO5/HLLC 1.38 against 1.59,
+// WENO3/HLLC 0.86 against 0.98; at 12, 500^2, 1.50 against 1.45, 1.90 against
+// 1.80 and 1.13 against 1.11), 6 in 3D (48^3 with WENO5/HLLC 1.75 against
+// 1.90; at 8, 100 x 40 x 40, 2.16 against 2.02) and 4 with WENO7, of which
+// three waves fit a SIMD (10 RK4 steps on 300^2 0.71 against 0.83; at 8,
+// 400^2, 1.18 against 1.14).
 inline YxShape yx_shape(const SweepCall& c) {
     YxShape best{};
     const GridDev& G = c.G;
     if (!G.active[1] || c.x_walk >= 0 || c.A.time == 3) return best;
     const int nx = G.solved_hi[0] - G.solved_lo[0] + 1, ny = G.solved_hi[1] - G.solved_lo[1] + 1;
     const int nz = G.solved_hi[2] - G.solved_lo[2] + 1;
+    if (c.seg <= 0) {
+        const YxShape sh = block_shape(nx, ny, nz, c.cus);
+        const long long most = G.g[0] == kBlockHalo7 ? 4 : G.active[2] ? 6 : 8;
+        if (block_load(sh, c.cus) <= most) return sh;
+    }
     double least = 0.0;
     // columns a block advances: 64 with its first x faces evaluated
     // beforehand, or 63 with lane 0 evaluating them

@@ -610,6 +610,7 @@ struct YxShape {
     int rows;      // rows a block advances (at most kYxRows)
     int nx, ny;    // blocks along x and along y
     unsigned blocks;
+    int block;     // 1: a wave per face (k_block_yx)
 };
 
 // LDS of a block that advances a tile of a y / x stage.
