@@ -42,7 +42,7 @@ struct BlockLds {
 template <int SCHEME, int FLUX, int TIME, bool HAS_S, bool CORNERS, int SLOTS, class Args>
 __device__ __forceinline__ void block_yx_tile(const SweepArgs& W, const Args& args,
                                               BlockLds<SCHEME>& lds, int i0, int helper, int a0,
-                                              int rows, int k) {
+                                              int rows, int k, bool first_block) {
     constexpr int NS = Stencil<SCHEME>::ns;
     constexpr int H = NS / 2;
     const int t = threadIdx.x & (kXBlock - 1);
@@ -58,9 +58,10 @@ __device__ __forceinline__ void block_yx_tile(const SweepArgs& W, const Args& ar
     // may read it differently while another block raises it, so each drops
     // its own results only.
     const bool raised = *W.A.flags != 0;
-    const double dt_step = *W.A.dt;
-    const double lwx = (FLUX == 5) ? dt_step / W.G.d[0] : 0.0;
-    const double lwy = (FLUX == 5) ? dt_step / W.G.d[1] : 0.0;
+    const StepClock clock(W.A);
+    const double dt_lw = (FLUX == 5) ? clock.get(W.A) : 0.0;
+    const double lwx = (FLUX == 5) ? dt_lw / W.G.d[0] : 0.0;   // Lax-Wendroff dt / spacing
+    const double lwy = (FLUX == 5) ? dt_lw / W.G.d[1] : 0.0;
     const int xo = W.G.xo;
     const auto row_of = [&](const GridDev& G, int a) {
         return node_index(G, -xo, map_node(G, 1, a), k);
@@ -130,6 +131,8 @@ __device__ __forceinline__ void block_yx_tile(const SweepArgs& W, const Args& ar
         for (int v = 0; v < 5; ++v) lds.first[v][t] = f[v];
     }
     __syncthreads();
+    const double dt_step = clock.get(W.A);
+    if (first_block && w == 0) clock.commit(W.A, dt_step);
     if (raised) return;
     if (x_wave) {
         const int r = a - a0;
@@ -171,7 +174,8 @@ __global__ __launch_bounds__(kXBlock * (2 * kBlockRows + 2)) void k_block_yx(Swe
     const int helper = kXBlock - sh.cols;
     const int i0 = W.G.solved_lo[0] + (int)bx * sh.cols - helper;
     block_yx_tile<SCHEME, FLUX, TIME, HAS_S, false, kDtSlots>(
-        W, [] () -> const SweepArgs& { return sweep_args(); }, lds, i0, helper, a0, sh.rows, k);
+        W, [] () -> const SweepArgs& { return sweep_args(); }, lds, i0, helper, a0, sh.rows, k,
+        bid == 0);
 }
 
 // z sweep of small grids (block_z_nodes): wave w of a block evaluates the
@@ -194,7 +198,7 @@ __global__ __launch_bounds__(kXBlock * (kBlockZ + 1)) void k_block_z(
     const int ic = min(max(i, G.solved_lo[0]), G.solved_hi[0]);
     const int j = G.solved_lo[1] + blockIdx.y;
     const int a = G.solved_lo[2] + blockIdx.z * seg + w;   // the face below node a
-    const double lw = (FLUX == 5) ? *A.dt / G.d[2] : 0.0;
+    const double lw = (FLUX == 5) ? StepClock(A).get(A) / G.d[2] : 0.0;
     unsigned flags = 0;
     if (a <= G.solved_hi[2] + 1) {
         double st[NS][5], f[5];

@@ -92,6 +92,8 @@ struct sf_grid {
     double dtmin_cfl = 0.0;      // CFL number the folded scan used
     int step_open = 0;
     int next_stage = 0;
+    int run_step = -1;           // step of a run whose steps keep the clock (StepClock), or -1
+    double* run_hist = nullptr;  // its dt values go here
     int stage_in[4] = {0, 0, 0, 0}, stage_out[4] = {0, 0, 0, 0};
     double step_cfl = 0.5;       // CFL folded into the last stage's update
     int fold_cfl = 0;
@@ -335,6 +337,11 @@ int scan_dt(sf_grid* g, double cfl, double max_dt, double limit) {
     return 0;
 }
 
+// The accumulators of a run's steps (StepClock); step s folds into set s.
+unsigned long long* step_set(const sf_grid* g, int s) {
+    return g->slots + (1 + s % kStepSets) * kDtSlots * kDtStride;
+}
+
 int do_stage(sf_grid* g, int s, int fold_dt) {
     const int in = g->stage_in[s], out = g->stage_out[s];
     if (s == 0 && !g->ghosts_valid) {
@@ -349,10 +356,17 @@ int do_stage(sf_grid* g, int s, int fold_dt) {
     A.qout = g->buf[out];
     for (int i = 0; i < 3; ++i) A.k[i] = g->k[i];
     A.dt = &g->clock->dt;
-    A.dtmin = g->slots;
+    A.dtmin = g->run_step >= 0 ? step_set(g, g->run_step) : g->slots;
     A.flags = g->flags;
     A.time = g->desc.time;
     A.stage = s;
+    if (g->run_step >= 0 && s == 0) {
+        A.ctl = g->ctl;
+        A.scan = g->run_step > 0 ? step_set(g, g->run_step - 1) : nullptr;
+        A.clear = step_set(g, g->run_step + 1);
+        A.dt_hist = g->run_hist;
+        A.slot = g->run_step;
+    }
     if (g->desc.time == SF_TIME_SSPRK3) {
         static const double base[3] = {0.0, 0.75, 1.0 / 3.0};
         static const double incr[3] = {1.0, 0.25, 2.0 / 3.0};
@@ -746,47 +760,73 @@ static bool whole_steps(const sf_grid* g) {
     return !g->G.active[1] && g->x_walk < 0 && g->G.n[0] <= (advanced > 32 ? 1 << 20 : 1 << 17);
 }
 
-// queue_steps for a grid that takes whole steps.
-static int queue_steps_1d(sf_grid* g, int nsteps, double cfl, double max_dt, double* hist) {
+// One step of a grid that takes whole steps.
+static int whole_step(sf_grid* g, int s, double cfl, double* hist) {
+    const int to = g->stage_out[nstages(g->desc.time) - 1];
+    const Step1dArgs W{g->G, g->buf[g->cur], g->buf[to], g->ctl,
+                       s ? step_set(g, s - 1) : nullptr, step_set(g, s), step_set(g, s + 1),
+                       hist, s, cfl, stage_tag(g, 0)};
+    const int ev = prof_start(g, SF_KERNEL_SWEEP_X);
+    int rc;
+    switch (g->desc.scheme) {
+    case SF_SCHEME_TENO5: rc = launch_step1d<1>(W, g->desc.flux, g->desc.time, g->stream); break;
+    case SF_SCHEME_WENO3: rc = launch_step1d<2>(W, g->desc.flux, g->desc.time, g->stream); break;
+    case SF_SCHEME_WENO7: rc = launch_step1d<3>(W, g->desc.flux, g->desc.time, g->stream); break;
+    default: rc = launch_step1d<0>(W, g->desc.flux, g->desc.time, g->stream); break;
+    }
+    prof_stop(g, ev);
+    if (rc) return fail(SF_E_STATE, "sf_run: no kernel for this recipe");
+    g->cur = to;
+    g->ghosts_valid = 1;
+    g->stored = 0;
+    g->step_open = 0;
+    return 0;
+}
+
+// queue_steps for a grid whose steps keep the clock by themselves: whole
+// steps (k_step_1d) or fused stages (StepClock).
+static int queue_run(sf_grid* g, int nsteps, double cfl, double max_dt, double* hist, bool whole) {
     if (int rc = sf_step_prepare(g)) return rc;
     if (int rc = scan_dt(g, cfl, max_dt, std::numeric_limits<double>::max())) return rc;
     launch_clock(g, hist, 0, 0, 1, false);
-    unsigned long long* const sets = g->slots + kDtSlots * kDtStride;
-    const auto set = [&](int s) { return sets + (s % kStepSets) * kDtSlots * kDtStride; };
-    for (int s = 0; s < nsteps; ++s) {
-        if (int rc = sf_step_begin(g)) return rc;
-        const int to = g->stage_out[nstages(g->desc.time) - 1];
-        const Step1dArgs W{g->G, g->buf[g->cur], g->buf[to], g->ctl,
-                           s ? set(s - 1) : nullptr, set(s), set(s + 1), hist, s, cfl,
-                           stage_tag(g, 0)};
-        const int ev = prof_start(g, SF_KERNEL_SWEEP_X);
-        int rc;
-        switch (g->desc.scheme) {
-        case SF_SCHEME_TENO5: rc = launch_step1d<1>(W, g->desc.flux, g->desc.time, g->stream); break;
-        case SF_SCHEME_WENO3: rc = launch_step1d<2>(W, g->desc.flux, g->desc.time, g->stream); break;
-        case SF_SCHEME_WENO7: rc = launch_step1d<3>(W, g->desc.flux, g->desc.time, g->stream); break;
-        default: rc = launch_step1d<0>(W, g->desc.flux, g->desc.time, g->stream); break;
-        }
-        prof_stop(g, ev);
-        if (rc) return fail(SF_E_STATE, "sf_run: no kernel for this recipe");
-        g->cur = to;
-        g->stored = 0;
-        g->step_open = 0;
-    }
-    k_close_1d<<<1, kDtSlots, 0, g->stream>>>(g->ctl, g->slots, set(nsteps - 1), sets, g->host);
-    g->snapped = g->host != nullptr;
     g->step_cfl = cfl;
+    g->run_hist = hist;
+    int rc = 0;
+    for (int s = 0; s < nsteps && !rc; ++s) {
+        rc = sf_step_begin(g);
+        if (rc) break;
+        if (whole) {
+            rc = whole_step(g, s, cfl, hist);
+            continue;
+        }
+        g->run_step = s;
+        for (int st = 0; st < nstages(g->desc.time) && !rc; ++st) rc = do_stage(g, st, 1);
+        g->run_step = -1;
+        if (!rc) rc = commit_state(g);
+    }
+    if (rc) return rc;
+    k_close_run<<<1, kDtSlots, 0, g->stream>>>(g->ctl, g->slots, step_set(g, nsteps - 1),
+                                               step_set(g, 0), g->host);
+    g->snapped = g->host != nullptr;
     g->dtmin_valid = 1;
     g->dtmin_cfl = cfl;
     SF_HIP(hipGetLastError());
     return 0;
 }
 
+// Whether the stages of a step run the fused y / x launch, which keeps the
+// clock in runs of steps.
+static bool fused_stages(const sf_grid* g) {
+    SweepCall c{g->G, nullptr, nullptr, StageArgs{}, g->stream, g->march_seg, g->cus, g->x_walk};
+    c.A.time = g->desc.time;
+    return yx_shape(c).blocks != 0;
+}
+
 // nsteps whole steps queued on the grid's stream, dt = min(CFL dt, max_dt)
 // each; hist (device memory, may be null) receives the dt values.
 static int queue_steps(sf_grid* g, int nsteps, double cfl, double max_dt, double* hist) {
-    if (nsteps > 0 && whole_steps(g))
-        return queue_steps_1d(g, nsteps, cfl, max_dt, hist);
+    if (nsteps > 0 && whole_steps(g)) return queue_run(g, nsteps, cfl, max_dt, hist, true);
+    if (nsteps > 0 && fused_stages(g)) return queue_run(g, nsteps, cfl, max_dt, hist, false);
     g->fold_cfl = 1;
     g->step_cfl = cfl;
     for (int s = 0; s < nsteps; ++s) {

@@ -94,9 +94,9 @@ __global__ __launch_bounds__(kDtSlots) void k_clock(Control* c, unsigned long lo
     if (snap && t == 0) *snap = *c;
 }
 
-// After the last k_step_1d of a run: commit it, hand the CFL scan it folded to
+// After the last step of a run whose steps keep the clock: commit it, hand the CFL scan it folded to
 // the grid's accumulator and clear the three that the steps used in turn.
-__global__ __launch_bounds__(kDtSlots) void k_close_1d(Control* c, unsigned long long* slots,
+__global__ __launch_bounds__(kDtSlots) void k_close_run(Control* c, unsigned long long* slots,
                                                        const unsigned long long* scan,
                                                        unsigned long long* sets, Control* snap) {
     const int t = threadIdx.x;

@@ -437,9 +437,9 @@ void k_sweep_march(GridDev G,
     const int a0 = G.solved_lo[AXIS] + blockIdx.z * seg;
     const int a1 = min(a0 + seg, G.solved_hi[AXIS] + 1);
     static_assert(MODE == kCopyS || MODE == kAccumS, "a march writes or accumulates S; the x sweep applies the update");
-    if (*A.flags) return;   // a fault was raised: keep the step-start state
+    const unsigned raised = *A.flags;   // tested once the window is on its way
     unsigned flags = 0;
-    const double lw = (FLUX == 5) ? *A.dt / G.d[AXIS] : 0.0;   // Lax-Wendroff dt / spacing
+    const double lw = (FLUX == 5) ? StepClock(A).get(A) / G.d[AXIS] : 0.0;   // dt / spacing
     if (i < G.n[0]) {
         const long long step = G.stride[AXIS];
         // The face a+1/2 reads its NS nodes as W from the lane's LDS ring
@@ -464,6 +464,7 @@ void k_sweep_march(GridDev G,
         // the previous node.
 #pragma unroll
         for (int v = 0; v < 5; ++v) asm volatile("" : "+v"(carried[v]));
+        if (raised) return;   // a fault was raised: keep the step-start state
 #pragma clang loop unroll(disable)
         for (int a = a0 - 1; a < a1; ++a, id += step) {
             double st[NS][5];
@@ -629,7 +630,7 @@ struct YxLds {
 template <int SCHEME, int FLUX, int TIME, bool HAS_S, bool CORNERS, int SLOTS, class Args>
 __device__ __forceinline__ void stage_yx_tile(const SweepArgs& W, const Args& args,
                                               YxLds<SCHEME>& lds, int i0, int helper, int a0,
-                                              int a1, int k) {
+                                              int a1, int k, bool first_block, unsigned raised) {
     constexpr int NS = Stencil<SCHEME>::ns;
     constexpr int H = NS / 2;
     constexpr int R = NS - 2;
@@ -644,9 +645,10 @@ __device__ __forceinline__ void stage_yx_tile(const SweepArgs& W, const Args& ar
     const int last = hi0 + H;                          // the last column a face reads
     unsigned flags = 0;
     double dt_local = INFINITY;
-    const double dt_step = *W.A.dt;   // the step's dt, read once
-    const double lwx = (FLUX == 5) ? *W.A.dt / W.G.d[0] : 0.0;   // Lax-Wendroff dt / spacing
-    const double lwy = (FLUX == 5) ? *W.A.dt / W.G.d[1] : 0.0;
+    const StepClock clock(W.A);
+    const double dt_lw = (FLUX == 5) ? clock.get(W.A) : 0.0;
+    const double lwx = (FLUX == 5) ? dt_lw / W.G.d[0] : 0.0;   // Lax-Wendroff dt / spacing
+    const double lwy = (FLUX == 5) ? dt_lw / W.G.d[1] : 0.0;
     // Rows are addressed from their first double (column -xo) by a lane's
     // 32-bit byte offset.
     const int xo = W.G.xo;
@@ -699,6 +701,9 @@ __device__ __forceinline__ void stage_yx_tile(const SweepArgs& W, const Args& ar
     double fprev[5] = {0.0, 0.0, 0.0, 0.0, 0.0};
     long long id = node_index(W.G, -xo, a0 - 1, k);   // row a
     wave_lds_order();
+    const double dt_step = clock.get(W.A);
+    if (first_block) clock.commit(W.A, dt_step);
+    if (raised) return;   // a fault was raised: keep the step-start state
 #pragma clang loop unroll(disable)
     for (int a = a0 - 1; a < a1; ++a, id += step) {
         const SweepArgs& T = args();
@@ -804,7 +809,7 @@ __global__ __launch_bounds__(kXBlock)
 __attribute__((amdgpu_waves_per_eu(SCHEME == 3 ? 2 : 3, 8))) void k_stage_yx(SweepArgs W,
                                                                              YxShape sh) {
     __shared__ YxLds<SCHEME> lds;
-    if (*W.A.flags) return;   // a fault was raised: keep the step-start state
+    const unsigned raised = *W.A.flags;   // tested once the window is on its way
     // blocks of one XCD take consecutive numbers (x fastest), so that they
     // share the halo lines in its L2
     const unsigned chunk = gridDim.x >> 3;
@@ -817,7 +822,8 @@ __attribute__((amdgpu_waves_per_eu(SCHEME == 3 ? 2 : 3, 8))) void k_stage_yx(Swe
     const int helper = kXBlock - sh.cols;              // 1: lane 0 only evaluates a face
     const int i0 = W.G.solved_lo[0] + (int)bx * sh.cols - helper;   // lane 0's column
     stage_yx_tile<SCHEME, FLUX, TIME, HAS_S, false, kDtSlots>(
-        W, [] () -> const SweepArgs& { return sweep_args(); }, lds, i0, helper, a0, a1, k);
+        W, [] () -> const SweepArgs& { return sweep_args(); }, lds, i0, helper, a0, a1, k,
+        bid == 0, raised);
 }
 
 }  // namespace sfamd
