@@ -72,7 +72,7 @@ __device__ __forceinline__ void plane_tiles(const BatchStage& B, YxLds<SCHEME>& 
         if (!B.live[T.slot]) continue;   // fixed during a step
         const ItemArgsAt args{&B.items[T.slot].stage[B.stage]};
         wave_lds_order();   // after the tile before
-        stage_yx_tile<SCHEME, FLUX, SF_TIME_SSPRK3, false, true, kItemDtSlots>(
+        stage_yx_tile<SCHEME, FLUX, SF_TIME_SSPRK3, false, true, kItemDtSlots, 1>(
             args(), args, lds, T.i0, (int)((unsigned)T.a1 >> 31), T.a0, T.a1 & 0x7fffffff, 0,
             false, 0u);
     }

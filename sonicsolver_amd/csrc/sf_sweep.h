@@ -215,10 +215,16 @@ int launch_yx_f(const SweepCall& c, const YxShape& sh) {
             k_block_yx<SCHEME, FLUX, T, true><<<nb, wg, 0, c.stream>>>(W, sh);                \
         else if (sh.block)                                                                    \
             k_block_yx<SCHEME, FLUX, T, false><<<nb, wg, 0, c.stream>>>(W, sh);               \
-        else if (c.G.active[2])                                                                    \
-            k_stage_yx<SCHEME, FLUX, T, true><<<nb, kXBlock, 0, c.stream>>>(W, sh);           \
+        else if (sh.waves > 1 && c.G.active[2])                                               \
+            k_stage_yx<SCHEME, FLUX, T, true, kYxWaves>                                       \
+                <<<nb, kXBlock * kYxWaves, 0, c.stream>>>(W, sh);                             \
+        else if (sh.waves > 1)                                                                \
+            k_stage_yx<SCHEME, FLUX, T, false, kYxWaves>                                      \
+                <<<nb, kXBlock * kYxWaves, 0, c.stream>>>(W, sh);                             \
+        else if (c.G.active[2])                                                               \
+            k_stage_yx<SCHEME, FLUX, T, true, 1><<<nb, kXBlock, 0, c.stream>>>(W, sh);        \
         else                                                                                  \
-            k_stage_yx<SCHEME, FLUX, T, false><<<nb, kXBlock, 0, c.stream>>>(W, sh);          \
+            k_stage_yx<SCHEME, FLUX, T, false, 1><<<nb, kXBlock, 0, c.stream>>>(W, sh);       \
     } while (0)
     switch (c.A.time) {
     case 0: SF_LAUNCH_YX(0); break;
@@ -298,6 +304,11 @@ inline YxShape block_shape(int nx, int ny, int nz, int cus) {
 // 1.36, 64^3 4.32 -> 2.87, 40^2 1.05 -> 0.76 (the small ones by shorter
 // segments in the z march, too).
 //
+// Blocks of four waves: 853^2 2.94 -> 2.83 ms a pass of 20 steps, 600^2 1.82
+// -> 1.71, 64^3 2.49 -> 2.38, 1000^2 (10 steps) 2.03 -> 1.94, 900^2 with
+// TENO5/HLLC 2.45 -> 2.37; with the long tiles of the largest grids there is
+// little to share, and they take one (512^3 71.6 ms, 72.9 with four).
+//
 // Small grids take k_block_yx, up to the number of waves per SIMD at which it
 // stays ahead of the march with every scheme: 8 in 2D (400^2, passes of 20
 // steps: WENO5/HLLC 1.11 ms against 1.24, TENO5/HLLC 1.38 against 1.59,
@@ -319,25 +330,32 @@ inline YxShape yx_shape(const SweepCall& c) {
     }
     double least = 0.0;
     // columns a block advances: 64 with its first x faces evaluated
-    // beforehand, or 63 with lane 0 evaluating them
-    for (int cols = kXBlock; cols >= kXBlock - 1; --cols) {
-        YxShape sh{};
-        sh.cols = cols;
-        sh.nx = (nx + cols - 1) / cols;
-        for (int rows = 1; rows <= kYxRows; ++rows) {
-            if (c.seg > 0 && rows != std::min(c.seg, kYxRows)) continue;
-            sh.rows = rows;
-            sh.ny = (ny + rows - 1) / rows;
-            const long long blocks = (long long)sh.nx * sh.ny * nz;
-            const double cost =
-                march_cost(blocks, 2.0 * rows + 1.0 + (cols == kXBlock ? 1.0 : 0.0), c.cus);
-            if (best.blocks && cost >= least) continue;
-            least = cost;
-            best = sh;
-            best.blocks = (unsigned)blocks;
+    // beforehand, or 63 with lane 0 evaluating them; one wave per block, whose
+    // rows' first y face the block below evaluates, too, or kYxWaves, which
+    // share theirs
+    for (int waves = 1; waves <= kYxWaves; waves += kYxWaves - 1)
+        for (int cols = kXBlock; cols >= kXBlock - 1; --cols) {
+            YxShape sh{};
+            sh.cols = cols;
+            sh.waves = waves;
+            sh.nx = (nx + cols - 1) / cols;
+            const int most = waves > 1 && cols == kXBlock ? kYxWaveRows : kYxRows;
+            for (int rows = 1; rows <= most; ++rows) {
+                if (c.seg > 0 && (waves > 1 || rows != std::min(c.seg, kYxRows))) continue;
+                sh.rows = rows;
+                sh.ny = (ny + rows * waves - 1) / (rows * waves);
+                const long long blocks = (long long)sh.nx * sh.ny * nz;
+                const double faces = 2.0 * rows + 1.0 / waves + (cols == kXBlock ? 1.0 : 0.0);
+                const double cost = march_cost(blocks * waves, faces, c.cus);
+                if (best.blocks && cost >= least) continue;
+                least = cost;
+                best = sh;
+                best.blocks = (unsigned)blocks;
+            }
         }
-    }
-    if (2 * G.n[0] < kXBlock && best.blocks > 8u * (unsigned)std::max(c.cus, 8)) best.blocks = 0;
+    if (2 * G.n[0] < kXBlock &&
+        (long long)best.blocks * best.waves > 8LL * std::max(c.cus, 8))
+        best.blocks = 0;
     return best;
 }
 

@@ -551,6 +551,7 @@ void k_sweep_march(GridDev G,
 // WENO7, whose ring is 17 KB).  yx_shape chooses the rows and columns.
 // ---------------------------------------------------------------------------
 constexpr int kYxRows = 32;
+constexpr int kYxWaves = 4, kYxWaveRows = 8;   // blocks of several waves
 
 // Node (i, j, k) at id was advanced to qn: next to a zeroGradient end, write
 // the boundary node and the first ghost layer (which stands for the others,
@@ -608,40 +609,54 @@ __device__ __forceinline__ void wave_lds_order() {
 
 struct YxShape {
     int cols;      // columns a block advances: 64, or 63 with a helper lane
-    int rows;      // rows a block advances (at most kYxRows)
+    int rows;      // rows a wave advances (at most kYxRows), of a block of
+    int waves;     // this many waves (1 or kYxWaves)
     int nx, ny;    // blocks along x and along y
     unsigned blocks;
     int block;     // 1: a wave per face (k_block_yx)
 };
 
 // LDS of a block that advances a tile of a y / x stage.
-template <int SCHEME>
+template <int SCHEME, int WAVES = 1>
 struct YxLds {
     static constexpr int NS = Stencil<SCHEME>::ns;
-    double win[NS - 2][5][kXBlock + NS];   // ring rows a+1-H .. a+H-2, each
-                                           // H-1 halo columns, 64, H halo, 1 pad
-    double first[5][kYxRows];
+    static constexpr int rows = WAVES > 1 ? kYxWaveRows : kYxRows;
+    double win[WAVES][NS - 2][5][kXBlock + NS];   // ring rows a+1-H .. a+H-2, each
+                                                  // H-1 halo columns, 64, H halo, 1 pad
+    double first[WAVES][5][rows];
+    double edge[WAVES > 1 ? WAVES - 1 : 1][5][WAVES > 1 ? kXBlock : 1];
 };
 
-// One tile: rows a0 .. a1-1 of plane k; lane t has column i0 + t.  W and
-// args() are the sweep's arguments, args() as sweep_args() reads them.
+// One wave's tile: rows a0 .. a1-1 of plane k; lane t has column i0 + t.  W
+// and args() are the sweep's arguments, args() as sweep_args() reads them.
 // CORNERS: write_ends writes the corners, too; SLOTS: partial minima of the
-// CFL accumulator.
-template <int SCHEME, int FLUX, int TIME, bool HAS_S, bool CORNERS, int SLOTS, class Args>
+// CFL accumulator.  The waves of a block (WAVES > 1) lie one above the other:
+// the last y face of each is the first of the next, which is evaluated there,
+// at the start of the march, and passed on in LDS.
+template <int SCHEME, int FLUX, int TIME, bool HAS_S, bool CORNERS, int SLOTS, int WAVES, class Args>
 __device__ __forceinline__ void stage_yx_tile(const SweepArgs& W, const Args& args,
-                                              YxLds<SCHEME>& lds, int i0, int helper, int a0,
-                                              int a1, int k, bool first_block, unsigned raised) {
+                                              YxLds<SCHEME, WAVES>& lds, int i0, int helper,
+                                              int a0, int a1, int k, bool first_block,
+                                              unsigned raised) {
     constexpr int NS = Stencil<SCHEME>::ns;
     constexpr int H = NS / 2;
     constexpr int R = NS - 2;
     constexpr int HC = NS - 1;            // halo columns per row and variable
     static_assert(5 * HC <= kXBlock, "one lane per halo value");
-    auto& win = lds.win;
-    auto& first = lds.first;
-    const int t = threadIdx.x;
+    const int w = WAVES > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x / kXBlock) : 0;
+    auto& win = lds.win[w];
+    auto& first = lds.first[w];
+    const int t = WAVES > 1 ? threadIdx.x & (kXBlock - 1) : threadIdx.x;
     const int i = i0 + t;
     const int hi0 = W.G.solved_hi[0];
-    const bool node = i <= hi0 && t >= helper;         // this lane advances node i
+    if (WAVES > 1 && a0 >= a1) {   // no rows left for this wave
+        __syncthreads();
+        return;
+    }
+    const bool edge = WAVES > 1 && w < WAVES - 1 && a1 <= W.G.solved_hi[1];
+    // this lane advances node i (none of a block's waves leaves early where
+    // a fault was raised, because the others may have read the flags before)
+    const bool node = i <= hi0 && t >= helper && !(WAVES > 1 && raised);
     const int last = hi0 + H;                          // the last column a face reads
     unsigned flags = 0;
     double dt_local = INFINITY;
@@ -703,7 +718,7 @@ __device__ __forceinline__ void stage_yx_tile(const SweepArgs& W, const Args& ar
     wave_lds_order();
     const double dt_step = clock.get(W.A);
     if (first_block) clock.commit(W.A, dt_step);
-    if (raised) return;   // a fault was raised: keep the step-start state
+    if (WAVES == 1 && raised) return;   // a fault was raised: keep the step-start state
 #pragma clang loop unroll(disable)
     for (int a = a0 - 1; a < a1; ++a, id += step) {
         const SweepArgs& T = args();
@@ -735,14 +750,26 @@ __device__ __forceinline__ void stage_yx_tile(const SweepArgs& W, const Args& ar
         double s5[5];
         {
             double f[5];
-            face_flux_from<1, SCHEME, FLUX>(
-                st,
-                [&](int side, double (&b)[5]) {
+            if (edge && a == a1 - 1) {
 #pragma unroll
-                    for (int v = 0; v < 5; ++v) b[v] = win[side ? rb : ra][v][t + H - 1];
-                },
-                T.G.gamma, T.G.area[1], f, fy, lwy);
-            if (!finite_sum5(f)) fy |= kFlagFlux;
+                for (int v = 0; v < 5; ++v) f[v] = lds.edge[WAVES > 1 ? w : 0][v][t];
+            } else {
+                face_flux_from<1, SCHEME, FLUX>(
+                    st,
+                    [&](int side, double (&b)[5]) {
+#pragma unroll
+                        for (int v = 0; v < 5; ++v) b[v] = win[side ? rb : ra][v][t + H - 1];
+                    },
+                    T.G.gamma, T.G.area[1], f, fy, lwy);
+                if (!finite_sum5(f)) fy |= kFlagFlux;
+            }
+            if (WAVES > 1 && a < a0) {
+                if (w > 0) {
+#pragma unroll
+                    for (int v = 0; v < 5; ++v) lds.edge[w - 1][v][t] = f[v];
+                }
+                __syncthreads();
+            }
 #pragma unroll
             for (int v = 0; v < 5; ++v) {
                 s5[v] = f[v] - fprev[v];
@@ -800,15 +827,16 @@ __device__ __forceinline__ void stage_yx_tile(const SweepArgs& W, const Args& ar
             dt_local = fmin(dt_local, dl);
         }
     }
+    if (WAVES > 1 && raised) return;
     raise_fault(flags, W.A.flags, W.A.fault_tag, W.A.tag);
     if (W.A.reduce_dt) wave_min_atomic<SLOTS>(dt_local, W.A.dtmin);
 }
 
-template <int SCHEME, int FLUX, int TIME, bool HAS_S>
-__global__ __launch_bounds__(kXBlock)
+template <int SCHEME, int FLUX, int TIME, bool HAS_S, int WAVES>
+__global__ __launch_bounds__(kXBlock * WAVES)
 __attribute__((amdgpu_waves_per_eu(SCHEME == 3 ? 2 : 3, 8))) void k_stage_yx(SweepArgs W,
                                                                              YxShape sh) {
-    __shared__ YxLds<SCHEME> lds;
+    __shared__ YxLds<SCHEME, WAVES> lds;
     const unsigned raised = *W.A.flags;   // tested once the window is on its way
     // blocks of one XCD take consecutive numbers (x fastest), so that they
     // share the halo lines in its L2
@@ -817,13 +845,15 @@ __attribute__((amdgpu_waves_per_eu(SCHEME == 3 ? 2 : 3, 8))) void k_stage_yx(Swe
     if (bid >= sh.blocks) return;
     const unsigned bx = bid % (unsigned)sh.nx, br = bid / (unsigned)sh.nx;
     const int k = W.G.solved_lo[2] + (int)(br / (unsigned)sh.ny);
-    const int a0 = W.G.solved_lo[1] + (int)(br % (unsigned)sh.ny) * sh.rows;
+    const int wave = WAVES > 1 ? __builtin_amdgcn_readfirstlane((int)threadIdx.x / kXBlock) : 0;
+    const int a0 =
+        W.G.solved_lo[1] + ((int)(br % (unsigned)sh.ny) * WAVES + wave) * sh.rows;
     const int a1 = min(a0 + sh.rows, W.G.solved_hi[1] + 1);
     const int helper = kXBlock - sh.cols;              // 1: lane 0 only evaluates a face
     const int i0 = W.G.solved_lo[0] + (int)bx * sh.cols - helper;   // lane 0's column
-    stage_yx_tile<SCHEME, FLUX, TIME, HAS_S, false, kDtSlots>(
+    stage_yx_tile<SCHEME, FLUX, TIME, HAS_S, false, kDtSlots, WAVES>(
         W, [] () -> const SweepArgs& { return sweep_args(); }, lds, i0, helper, a0, a1, k,
-        bid == 0, raised);
+        bid == 0 && wave == 0, raised);
 }
 
 }  // namespace sfamd

@@ -38,6 +38,28 @@ def test_blocks_equal_march(scheme, flux, time, bc):
             assert np.array_equal(march_dts, dts), n
 
 
+@pytest.mark.parametrize("scheme,flux,time", [("weno5", "hllc", "ssprk3"),
+                                              ("teno5", "rusanov", "rk4"),
+                                              ("weno3", "laxwendroff", "euler"),
+                                              ("weno7", "roe", "ssprk3")])
+@pytest.mark.parametrize("n", [(502, 499), (600, 613), (640, 601), (1000, 333), (65, 61, 70),
+                               (64, 64, 64)])
+def test_stacked_waves_equal_single(n, scheme, flux, time):
+    """Blocks of four waves that share the y faces between them, with the last
+    block's waves full, partly filled and without rows."""
+    h = [1.0 / m for m in n] + [1.0] * (3 - len(n))
+    q = wl.smooth_field(n, seed=5, amp=0.1)
+    for bc in ("transmissive", "periodic"):
+        with Grid(make_desc(n=n, bc=(bc,) * 3, d=h, scheme=scheme, flux=flux, time=time)) as g:
+            g.upload(q)
+            dts = g.run(2, 0.2)
+            stacked = g.download()
+            g.upload(q)
+            g.set_march_segment(7)
+            assert np.array_equal(g.run(2, 0.2), dts)
+            assert np.array_equal(g.download(), stacked)
+
+
 def test_fault_keeps_the_step_start():
     """Two halves that move apart until a near-vacuum turns non-physical in
     some stage: both paths stop at the same step and stage, with the state at
