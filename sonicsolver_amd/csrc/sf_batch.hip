@@ -705,12 +705,17 @@ int sf_batch_create(int device, double gamma, size_t node_capacity, int item_cap
     ok = ok && hipStreamCreateWithFlags(&b->stream, hipStreamNonBlocking) == hipSuccess;
     ok = ok && hipStreamCreateWithFlags(&b->copy_stream, hipStreamNonBlocking) == hipSuccess;
     ok = ok && hipEventCreateWithFlags(&b->copy_after, hipEventDisableTiming) == hipSuccess;
-    ok = ok && hipMemset(b->d_flags, 0, sizeof(unsigned) * item_capacity) == hipSuccess;
-    ok = ok && hipMemset(b->d_live, 0, sizeof(int) * item_capacity) == hipSuccess;
-    ok = ok && hipMemset(b->d_steps, 0, sizeof(long long) * item_capacity) == hipSuccess;
-    ok = ok && hipMemset(b->d_target, 0, sizeof(long long) * item_capacity) == hipSuccess;
+    // cleared on the stream that uses them: the first admission is not waited
+    // for, and the compute stream does not wait for the null stream
+    const auto clear = [&](void* p, size_t bytes) {
+        return hipMemsetAsync(p, 0, bytes, b->stream) == hipSuccess;
+    };
+    ok = ok && clear(b->d_flags, sizeof(unsigned) * item_capacity);
+    ok = ok && clear(b->d_live, sizeof(int) * item_capacity);
+    ok = ok && clear(b->d_steps, sizeof(long long) * item_capacity);
+    ok = ok && clear(b->d_target, sizeof(long long) * item_capacity);
     // the arena starts zeroed, so padding that is never written stays finite
-    for (int i = 0; i < 3 && ok; ++i) ok = hipMemset(b->buf[i], 0, state) == hipSuccess;
+    for (int i = 0; i < 3 && ok; ++i) ok = clear(b->buf[i], state);
     if (!ok) {
         sf_batch_destroy(b);
         return bfail(SF_E_MEMORY, "sf_batch_create: device allocation of " +

@@ -556,10 +556,10 @@ int sf_grid_create(const sf_grid_desc* desc, sf_grid** out) {
     static_assert(sizeof c % 8 == 0, "copied behind the accumulators");
     std::memcpy(init.data() + kDtWords, &c, sizeof c);
     if (hipMemcpy(g->slots, init.data(), init.size() * 8, hipMemcpyHostToDevice) != hipSuccess ||
-        hipMemset(g->buf[0], 0, state) != hipSuccess ||
-        hipMemset(g->buf[1], 0, state) != hipSuccess ||
-        hipMemset(g->buf[2], 0, state) != hipSuccess ||
-        hipMemset(g->S, 0, state) != hipSuccess) {
+        hipMemsetAsync(g->buf[0], 0, state, g->stream) != hipSuccess ||
+        hipMemsetAsync(g->buf[1], 0, state, g->stream) != hipSuccess ||
+        hipMemsetAsync(g->buf[2], 0, state, g->stream) != hipSuccess ||
+        hipMemsetAsync(g->S, 0, state, g->stream) != hipSuccess) {
         grid_free(g);
         return fail(SF_E_HIP, "sf_grid_create: initialisation copy failed");
     }

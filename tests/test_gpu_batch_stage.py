@@ -8,6 +8,7 @@ each variable's largest value, 3 steps times 3 stages times a handful of
 units in the last place."""
 import numpy as np
 import pytest
+import torch
 
 from sonicsolver_amd import workloads as wl
 from sonicsolver_amd._native import Grid, make_desc
@@ -54,3 +55,27 @@ def test_batch_equals_grid(shape, fused):
         tol = 1e-13 * np.abs(ref).max(axis=1, keepdims=True)
         assert (np.abs(out - ref) <= tol).all(), kw
         assert clock[1] == 3 and abs(clock[0] - rclock[0]) <= 1e-13 * rclock[0], kw
+
+
+def test_first_state_of_a_fresh_arena_or_grid():
+    """A state that arrives right after its memory was allocated, while the
+    clearing of some gigabytes is still under way, is not cleared with it."""
+    kw = dict(n=(64, 64), d=(0.01, 0.01), scheme="weno5", flux="hllc", cfl=0.4)
+    q = wl.smooth_field((64, 64), seed=2)
+    ref, _ = _grid_run(kw, q, 2)
+    for _ in range(2):
+        with Batch(60_000_000, 4) as b:
+            slot = b.add(make_item(**kw), q)
+            b.step(2, graph=False)
+            assert np.abs(b.download(slot).reshape(5, -1) - ref).max() <= 1e-13 * np.abs(ref).max()
+    n = (512, 512, 96)
+    desc = make_desc(n=n, bc=("periodic",) * 3, d=(0.01,) * 3)
+    field = torch.rand(5, n[0] * n[1] * n[2], dtype=torch.float64, device="cuda") + 1.0
+    back = torch.empty_like(field)
+    torch.cuda.synchronize()
+    for _ in range(2):
+        with Grid(desc) as g:
+            g.upload_device(field.data_ptr())
+            g.download_device(back.data_ptr())
+            g.synchronize()
+        assert torch.equal(back, field)
