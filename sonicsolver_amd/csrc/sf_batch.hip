@@ -5,7 +5,7 @@
 // problem keeps its own CFL dt and clock, and its result does not depend on
 // which other problems share the batch (no cross-problem arithmetic; the
 // per-problem dt is a minimum, which does not depend on the order of the
-// atomics).  The launch sequence of a step is captured in a hipGraph and
+// atomics).  The launches of a few steps can be captured in a hipGraph and
 // replayed while the set of problems is unchanged.
 //
 // Boundaries are transmissive (the reference's zeroGradient sets, applied
@@ -619,27 +619,30 @@ int prepare_pending(sf_batch* b) {
     return 0;
 }
 
-// Queue nsteps steps (graph replay or direct launches); no wait.
-// Steps from which capturing a new graph pays for itself against direct
-// launches (a capture and instantiation cost about as much as a dozen
-// steps' worth of kernel launches).
-constexpr int kGraphCaptureSteps = 16;
+// Steps of a captured graph.  A replay costs 6 us between graphs, which a
+// step of its own four launches does not: 300 nodes took 25 us per step in
+// graphs of one step and take 18.7 in graphs of eight, 18.6 launched directly;
+// 131^2 41, 34 and 34.
+constexpr int kGraphSteps = 8;
 
+// Queue nsteps steps (graph replays and, for the rest, direct launches); no
+// wait.  Left to choose (2), direct launches: they are as fast on the device
+// and need no capture.
 int advance(sf_batch* b, int nsteps, int use_graph) {
-    if (use_graph == 2) use_graph = (b->graph_exec || nsteps >= kGraphCaptureSteps) ? 1 : 0;
-    if (use_graph) {
+    int s = 0;
+    if (use_graph == 1 && nsteps >= kGraphSteps) {
         if (!b->graph_exec) {
             SF_BHIP(hipStreamBeginCapture(b->stream, hipStreamCaptureModeThreadLocal));
-            enqueue_step(b);
+            for (int k = 0; k < kGraphSteps; ++k) enqueue_step(b);
             hipGraph_t g = nullptr;
             SF_BHIP(hipStreamEndCapture(b->stream, &g));
             b->graph = g;
             SF_BHIP(hipGraphInstantiate(&b->graph_exec, g, nullptr, nullptr, 0));
         }
-        for (int s = 0; s < nsteps; ++s) SF_BHIP(hipGraphLaunch(b->graph_exec, b->stream));
-    } else {
-        for (int s = 0; s < nsteps; ++s) enqueue_step(b);
+        for (; s + kGraphSteps <= nsteps; s += kGraphSteps)
+            SF_BHIP(hipGraphLaunch(b->graph_exec, b->stream));
     }
+    for (; s < nsteps; ++s) enqueue_step(b);
     launch_clock(b, 0);
     SF_BHIP(hipGetLastError());
     return 0;
@@ -951,7 +954,7 @@ int sf_batch_set_tiles(sf_batch* b, int xlen, int ylen) {
 
 // ---- autotuner ----------------------------------------------------------------
 // Times every launch shape (schedule x x-tile x y-tile x persistent grid
-// size) on the batch's own problems: each trial replays the captured step
+// size) on the batch's own problems: each trial takes the same steps
 // from the same saved state, which is restored afterwards, so tuning leaves
 // the problems exactly as it found them.
 namespace {
@@ -1003,8 +1006,8 @@ int snapshot_restore(sf_batch* b, const Snapshot& sn) {
     return 0;
 }
 
-// Mean time of one step of the current shape over `steps` graph replays
-// (after one untimed replay that captures the graph).
+// Mean time of one step of the current shape over `steps` steps (after an
+// untimed one).
 int time_shape(sf_batch* b, int steps, double* ms) {
     if (b->tables_dirty)
         if (int rc = rebuild_tables(b)) return rc;
