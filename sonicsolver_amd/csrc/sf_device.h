@@ -1,7 +1,6 @@
-// sf_device.h -- device-side pieces shared by the grid kernels
-// (sf_kernels.h) and the batched kernels (sf_batch.hip): grid descriptor,
-// stage-update arithmetic, validation flags, CFL folding and the pressure /
-// energy conversions of the boundary closure.
+// sf_device.h -- device-side pieces shared by the grid kernels and the
+// batched ones: grid descriptor, stage-update arithmetic, validation flags,
+// CFL folding and the energies of the boundary closure.
 #pragma once
 
 #include "sf_face.h"
@@ -126,23 +125,16 @@ __device__ __forceinline__ bool solved_node(const GridDev& G, int i, int j, int 
            j <= G.solved_hi[1] && k >= G.solved_lo[2] && k <= G.solved_hi[2];
 }
 
-// Whether the CFL sum takes axis d: a grid's metric is zero on an inactive
-// axis, so its term adds an exact zero and needs no test.
-template <class GT>
-__device__ __forceinline__ bool cfl_axis(const GT& G, int d) { return G.active[d]; }
-__device__ __forceinline__ bool cfl_axis(const GridDev&, int) { return true; }
-
-// Local CFL step of RusanovEOS::deltaT (SF_rusanovEOS.cpp:110-147).  GT is
-// any descriptor with gamma, active[3] and metric[3].
-template <class GT>
-__device__ __forceinline__ double local_dt(const GT& G, const double q[5], double cfl,
+// Local CFL step of RusanovEOS::deltaT (SF_rusanovEOS.cpp:110-147).  The
+// metric of an inactive axis is zero, so its term adds an exact zero.
+__device__ __forceinline__ double local_dt(const GridDev& G, const double q[5], double cfl,
                                            unsigned& flags) {
     const Closed s = close_state(q, G.gamma);
     const double c = s.c();
     double spectral = 0.0;
 #pragma unroll
     for (int d = 0; d < 3; ++d)
-        if (cfl_axis(G, d)) spectral += fma(c, G.metric[d], fabs(s.u[d] * G.metric[d]));
+        spectral += fma(c, G.metric[d], fabs(s.u[d] * G.metric[d]));
     if (!(spectral > 0.0) || !isfinite(spectral)) flags |= kFlagDt;
     return cfl / spectral;
 }
@@ -207,11 +199,7 @@ __device__ __forceinline__ bool finite_sum5(const double f[5]) {
     return isfinite(((f[0] + f[1]) + (f[2] + f[3])) + f[4]);
 }
 
-__device__ __forceinline__ void raise_flags(unsigned f, unsigned* flags) {
-    if (f) atomicOr(flags, f);
-}
-
-// raise_flags, recording the lowest tag (-1: none) before the flags are seen.
+// Raises flags f, recording the lowest tag (-1: none) before they are seen.
 __device__ __forceinline__ void raise_fault(unsigned f, unsigned* flags, long long* tag_out,
                                             long long tag) {
     if (!f) return;
@@ -274,11 +262,10 @@ __device__ __forceinline__ void check_state(const double q[5], unsigned& flags) 
 // Stage update of one node from its current value qc and (SSPRK3 after
 // the first stage, RK4) its step-start value q0v; S is the accumulated flux
 // difference and dt the step's dt (*A.dt, which no kernel of a stage
-// changes, so a sweep reads it once).  GT is any descriptor with P, jac,
-// gamma, active[3] and metric[3].  TIME fixes the time recipe (A.time) at
+// changes, so a sweep reads it once).  TIME fixes the time recipe (A.time) at
 // compile time; -1 reads it from A.
-template <int TIME = -1, class GT>
-__device__ __forceinline__ void stage_update_dt(const GT& G, const StageArgs& A, long long id,
+template <int TIME = -1>
+__device__ __forceinline__ void stage_update_dt(const GridDev& G, const StageArgs& A, long long id,
                                                 const double qc[5], const double q0v[5],
                                                 const double S[5], double dt, unsigned& flags,
                                                 double& dt_local, double qn[5]) {
@@ -308,22 +295,6 @@ __device__ __forceinline__ void stage_update_dt(const GT& G, const StageArgs& A,
     }
     check_state(qn, flags);
     if (A.reduce_dt) dt_local = local_dt(G, qn, A.cfl, flags);
-}
-
-// Block-wide minimum of a positive double into *target (one atomic; every
-// thread of the block calls it).
-__device__ __forceinline__ void block_min_atomic(double v, unsigned long long* target,
-                                                 unsigned long long* lds) {
-    unsigned long long b = wave_min_bits(
-        (v > 0.0 && isfinite(v)) ? (unsigned long long)__double_as_longlong(v)
-                                 : 0x7FF0000000000000ull);
-    const int wave = threadIdx.x >> 6, nwave = blockDim.x >> 6;
-    if ((threadIdx.x & 63) == 0) lds[wave] = b;
-    __syncthreads();
-    if (threadIdx.x == 0) {
-        for (int w = 1; w < nwave; ++w) b = lds[w] < b ? lds[w] : b;
-        if (b != 0x7FF0000000000000ull) atomicMin(target, b);
-    }
 }
 
 // Device clock: dt of the step, physical time, step count and the dt limits.

@@ -21,6 +21,7 @@
 //   y and x sweeps               k_stage_yx:    the same march along y with
 //                                               the x faces of each row taken
 //                                               from the window's rows
+//   both on small grids          k_block_z, k_block_yx: a wave per face
 //   separately, where yx_shape   k_sweep_march, then k_sweep_x (one lane per
 //   says so                      x face, the flux difference by a cross-lane
 //                                shift) or k_sweep_xl (whole lines in 64-node

@@ -529,8 +529,8 @@ void k_sweep_march(GridDev G,
 
 // ---------------------------------------------------------------------------
 // y and x faces and the stage update of the advanced nodes in one march along
-// y: a block (one wave) takes 64 columns of one z plane and up to kYxRows
-// rows.  Ghosts are read through map_node (a lane's column and a row's
+// y: a wave takes 64 columns of one z plane and up to kYxRows rows, and a
+// block one wave or kYxWaves of them, one above the other.  Ghosts are read through map_node (a lane's column and a row's
 // number are mapped once each), and next to a zeroGradient end the launch
 // writes the boundary node and first ghost of what it advances, so no ghost
 // fill is needed between stages.  At row a
@@ -545,9 +545,9 @@ void k_sweep_march(GridDev G,
 // results are theirs bit for bit.
 //
 // Against the y march and the x sweep it neither writes nor reads back the
-// y differences and reads the state once: on 512^3 21.5 GB per launch
-// instead of 16.1 + 21.7, which those two moved at the rate of a large copy
-// (3.68 + 4.77 ms); bound by FP64 issue at three waves per SIMD (two for
+// y differences and reads the state once: on 512^3 27.3 GB per launch instead
+// of 16.6 + 21.6 (7.6 ms instead of 3.7 + 4.8).  Bound by FP64 issue (87% of
+// the cycles, 86% of it FP64) at three waves per SIMD (two for
 // WENO7, whose ring is 17 KB).  yx_shape chooses the rows and columns.
 // ---------------------------------------------------------------------------
 constexpr int kYxRows = 32;
