@@ -58,27 +58,7 @@ __global__ __launch_bounds__(64) void k_step_1d(Step1dArgs W) {
     __shared__ double cur[5][64];
     const GridDev& G = W.G;
     Control* const ctl = W.ctl;
-    // a fault of an earlier step: keep the step-start state (a fault that
-    // another block raises in this step does not stop this one, so that the
-    // record holds the earliest stage's)
-    if (ctl->fault.flags && (ctl->fault.tag >> 3) < (W.tag >> 3)) return;
     const int t = threadIdx.x;
-    double dt;
-    if (W.scan) {
-        dt = __longlong_as_double((long long)wave_min_bits(W.scan[t * kDtStride]));
-        dt = fmin(dt, ctl->clock.max_dt);
-        dt = fmin(dt, ctl->clock.limit);
-        if (blockIdx.x == 0 && t == 0) {
-            ctl->clock.time += ctl->clock.dt;
-            ctl->clock.steps += 1;
-            ctl->clock.dt = dt;
-            if (W.dt_hist) W.dt_hist[W.slot] = dt;
-        }
-    } else {
-        dt = ctl->clock.dt;
-    }
-    if (blockIdx.x == 0) W.clear[t * kDtStride] = 0x7FF0000000000000ull;
-    const double lw = (FLUX == 5) ? dt / G.d[0] : 0.0;   // Lax-Wendroff dt / spacing
     const int n = G.n[0];
     const int lo = G.solved_lo[0], hi = G.solved_hi[0];
     const bool periodic = G.wrap[0] != 0;
@@ -93,15 +73,42 @@ __global__ __launch_bounds__(64) void k_step_1d(Step1dArgs W) {
         if (G.zg_lo[0]) src = max(src, lo);
         if (G.zg_hi[0]) src = min(src, hi);
     }
+    // Everything the step starts from is requested before any of it is waited
+    // for: the nodes, the accumulator holding dt, the clock, the fault record.
+    // One after the other, three round trips of a microsecond, they were a
+    // third of the launch.
     double q[5], q0[5];
-    {
-        const long long id = node_index(G, src, 0, 0);
+    const long long start = node_index(G, src, 0, 0);
 #pragma unroll
-        for (int v = 0; v < 5; ++v) {
-            q0[v] = q[v] = W.q[v * G.P + id];
-            cur[v][t] = q[v];
+    for (int v = 0; v < 5; ++v) q0[v] = W.q[v * G.P + start];
+    unsigned long long scan = 0;
+    if (W.scan) scan = W.scan[t * kDtStride];
+    const unsigned fault_flags = ctl->fault.flags;
+    const long long fault_tag = ctl->fault.tag;
+    const double clock_dt = ctl->clock.dt, max_dt = ctl->clock.max_dt, limit = ctl->clock.limit;
+#pragma unroll
+    for (int v = 0; v < 5; ++v) {
+        q[v] = q0[v];
+        cur[v][t] = q[v];
+    }
+    // a fault of an earlier step: keep the step-start state (a fault that
+    // another block raises in this step does not stop this one, so that the
+    // record holds the earliest stage's)
+    if (fault_flags && (fault_tag >> 3) < (W.tag >> 3)) return;
+    double dt = clock_dt;
+    if (W.scan) {
+        dt = __longlong_as_double((long long)wave_min_bits(scan));
+        dt = fmin(dt, max_dt);
+        dt = fmin(dt, limit);
+        if (blockIdx.x == 0 && t == 0) {
+            ctl->clock.time += clock_dt;
+            ctl->clock.steps += 1;
+            ctl->clock.dt = dt;
+            if (W.dt_hist) W.dt_hist[W.slot] = dt;
         }
     }
+    if (blockIdx.x == 0) W.clear[t * kDtStride] = 0x7FF0000000000000ull;
+    const double lw = (FLUX == 5) ? dt / G.d[0] : 0.0;   // Lax-Wendroff dt / spacing
     wave_lds_order();
     // zeroGradient ends held by this tile: lanes outside the advanced range
     // take the last advanced node's state with its rebuilt energy
