@@ -165,6 +165,7 @@ template <int SCHEME, int FLUX, int TIME, bool HAS_S>
 __global__ __launch_bounds__(kXBlock * (2 * kBlockRows + 2)) void k_block_yx(SweepArgs W,
                                                                                   YxShape sh) {
     __shared__ BlockLds<SCHEME> lds;
+    fetch_args<sizeof(SweepArgs)>();
     const unsigned chunk = gridDim.x >> 3;
     const unsigned bid = (blockIdx.x & 7u) * chunk + (blockIdx.x >> 3);
     if (bid >= sh.blocks) return;
@@ -190,6 +191,7 @@ __global__ __launch_bounds__(kXBlock * (kBlockZ + 1)) void k_block_z(
     constexpr int NS = Stencil<SCHEME>::ns;
     constexpr int H = NS / 2;
     __shared__ double fz[kBlockZ + 1][5][kXBlock];
+    fetch_args<sizeof(GridDev) + 16 + sizeof(StageArgs)>();
     const bool raised = *A.flags != 0;   // as in block_yx_tile
     const int t = threadIdx.x & (kXBlock - 1);
     const int w = __builtin_amdgcn_readfirstlane((int)threadIdx.x / kXBlock);

@@ -56,6 +56,7 @@ __global__ __launch_bounds__(64) void k_step_1d(Step1dArgs W) {
     constexpr int ST = step_stages<TIME>;
     constexpr int U = step_nodes<SCHEME, TIME>;
     __shared__ double cur[5][64];
+    fetch_args<sizeof(Step1dArgs)>();
     const GridDev& G = W.G;
     Control* const ctl = W.ctl;
     const int t = threadIdx.x;
