@@ -21,8 +21,9 @@ namespace sfamd {
 // Faces, sums and updates are those of k_stage_yx, bit for bit.  The y faces
 // at the ends of a block's rows are evaluated twice, so where the device is
 // full the march is faster (yx_shape).  A pass of 20 steps with WENO5/HLLC:
-// 40^2 0.67 -> 0.43 ms, 130^2 0.69 -> 0.45, 193 x 97 0.74 -> 0.58, 256^2 with
-// TENO5/HLLC 1.12 -> 0.75, 400^2 1.24 -> 1.11.
+// 40^2 0.67 -> 0.43 ms, 130^2 0.69 -> 0.45, 193 x 97 0.74 -> 0.58 (0.55 since
+// the clock and the arguments cost less), 256^2 with TENO5/HLLC 1.12 -> 0.75
+// (0.70), 400^2 1.24 -> 1.11.
 // ---------------------------------------------------------------------------
 constexpr int kBlockRows = 5;    // most rows of a block
 constexpr int kBlockHalo7 = 4;   // ghost layers of WENO7
