@@ -196,8 +196,10 @@ int fill_ghosts(sf_grid* g, double* q, long long tag) {
 // update adds to it.  The flux differences are therefore summed as
 // (dz + dy) + dx rather than the reference's (dx + dy) + dz, which changes
 // the last bit at most.
-// The separate x sweeps read stored ghosts: `stored` says that q has them.
-int run_sweeps(sf_grid* g, double* q, const StageArgs& A, bool stored) {
+// The separate x sweeps read stored ghosts (`stored`: q has them); the fused
+// launch reads the boundary nodes and first ghosts that a fused stage or a
+// fill wrote (`closed`: q has those).
+int run_sweeps(sf_grid* g, double* q, const StageArgs& A, bool stored, bool closed) {
     SweepCall c{g->G, q, g->S, A, g->stream, g->march_seg, g->cus, g->x_walk};
     auto sweep = [&](int axis, int mode) {
         switch (g->desc.scheme) {
@@ -218,7 +220,7 @@ int run_sweeps(sf_grid* g, double* q, const StageArgs& A, bool stored) {
     const YxShape yx = yx_shape(c);
     g->separate = yx.blocks == 0;
     g->snapped = 0;
-    if (g->separate && !stored)
+    if (g->separate ? !stored : !closed)
         if (int rc = fill_ghosts(g, q, A.tag)) return rc;
     int axes[3], na = 0;
     for (int a = 2; a >= 0; --a)
@@ -381,7 +383,8 @@ int do_stage(sf_grid* g, int s, int fold_dt) {
     const bool last = s == nstages(g->desc.time) - 1;
     A.reduce_dt = (last && fold_dt) ? 1 : 0;
     A.cfl = g->step_cfl;
-    return run_sweeps(g, g->buf[in], A, s == 0 && g->stored);
+    // a stage by the separate sweeps leaves its output's boundary as it was
+    return run_sweeps(g, g->buf[in], A, s == 0 && g->stored, s == 0 || !g->separate);
 }
 
 // Stage buffers of a step.  No stage writes the buffer that holds the
@@ -895,7 +898,7 @@ int sf_residual(sf_grid* g, double* soa_out) {
     A.dtmin = g->slots;
     A.fault_tag = &g->fault->tag;
     A.tag = next_tag(g, 0);
-    if (int rc = run_sweeps(g, g->buf[g->cur], A, g->stored != 0)) return rc;
+    if (int rc = run_sweeps(g, g->buf[g->cur], A, g->stored != 0, true)) return rc;
     const long long N = (long long)g->G.n[0] * g->G.n[1] * g->G.n[2];
     const unsigned nb = std::min<unsigned>(blocks_for(N, 256), 65535u);
     k_pack<<<nb, 256, 0, g->stream>>>(g->G, g->buf[scratch], g->stage_io, 0, 0);
