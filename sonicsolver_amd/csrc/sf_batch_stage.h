@@ -78,6 +78,14 @@ __device__ __forceinline__ void plane_tiles(const BatchStage& B, YxLds<SCHEME>& 
     }
 }
 
+// Byte offset, from column i0 of the row at `xo`, of the stored node that
+// stands for column c >= i0 of a strip that starts there.  From the row's
+// start it would pass 2^32 at column 2^29, and an arena holds longer
+// problems.
+__host__ __device__ __forceinline__ unsigned strip_offset(const GridDev& G, int i0, int c) {
+    return (unsigned)(map_node(G, 0, c) - i0 + G.xo) * 8u;
+}
+
 // The stage of 1D problems: a wave takes strips of 63 nodes, lane 0
 // evaluating the first one's lower face.  Bound like the planes' tiles: 300
 // problems of 8192 nodes take 271 us per step, 2.2 us of issue per strip and
@@ -110,10 +118,10 @@ __device__ __forceinline__ void line_tiles(const BatchStage& B, double (&row)[5]
             const SweepArgs& U = args();
             const int i = i0 + t;
             const bool node = i <= hi0 && t >= 1;
-            const unsigned off = (unsigned)(map_node(U.G, 0, min(i, last)) + U.G.xo) * 8u;
+            const unsigned off = strip_offset(U.G, i0, min(i, last));
             double pq[5], pq0[5];
 #pragma unroll
-            for (int v = 0; v < 5; ++v) pq[v] = at(U.q + v * U.G.P, off);
+            for (int v = 0; v < 5; ++v) pq[v] = at(U.q + v * U.G.P + i0, off);
             double h = 0.0;
             if (halo) h = U.q[hv * U.G.P + (map_node(U.G, 0, min(i0 + hcol, last)) + U.G.xo)];
             wave_lds_order();
@@ -134,7 +142,7 @@ __device__ __forceinline__ void line_tiles(const BatchStage& B, double (&row)[5]
                     if (side == 0) {
                         const SweepArgs& V = args();
 #pragma unroll
-                        for (int v = 0; v < 5; ++v) pq0[v] = at(V.A.q0 + v * V.G.P, off);
+                        for (int v = 0; v < 5; ++v) pq0[v] = at(V.A.q0 + v * V.G.P + i0, off);
                     }
 #pragma unroll
                     for (int v = 0; v < 5; ++v) b[v] = row[v][t + H - 1 + side];

@@ -212,7 +212,7 @@ __device__ __forceinline__ void raise_fault(unsigned f, unsigned* flags, long lo
 
 // The coordinate along axis a whose stored value stands for coordinate c, a
 // node or ghost within the halo.
-__device__ __forceinline__ int map_node(const GridDev& G, int a, int c) {
+__host__ __device__ __forceinline__ int map_node(const GridDev& G, int a, int c) {
     c = min(max(c, G.map_lo[a]), G.map_hi[a]);
     c += c < 0 ? G.wrap[a] : 0;
     return c - (c >= G.n[a] ? G.wrap[a] : 0);
