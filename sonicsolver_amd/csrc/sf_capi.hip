@@ -888,7 +888,13 @@ int sf_residual(sf_grid* g, double* soa_out) {
     if (int rc = set_device(g)) return rc;
     if (int rc = sf_step_prepare(g)) return rc;
     const int scratch = (g->cur + 1) % 3;
-    SF_HIP(hipMemsetAsync(g->buf[scratch], 0, sizeof(double) * 5 * (size_t)g->G.P, g->stream));
+    const long long N = (long long)g->G.n[0] * g->G.n[1] * g->G.n[2];
+    const unsigned nb = std::min<unsigned>(blocks_for(N, 256), 65535u);
+    // Nodes that are not advanced have no residual.  Only the nodes are
+    // cleared: the scratch buffer's ghosts beyond an end without a condition
+    // are held for the steps that use the buffer next.
+    SF_HIP(hipMemsetAsync(g->stage_io, 0, sizeof(double) * 5 * (size_t)N, g->stream));
+    k_pack<<<nb, 256, 0, g->stream>>>(g->G, g->stage_io, g->buf[scratch], 1, 0);
     StageArgs A{};
     A.q0 = g->buf[g->cur];   // a valid state, though the residual-only update reads none
     A.qout = g->buf[scratch];
@@ -899,8 +905,6 @@ int sf_residual(sf_grid* g, double* soa_out) {
     A.fault_tag = &g->fault->tag;
     A.tag = next_tag(g, 0);
     if (int rc = run_sweeps(g, g->buf[g->cur], A, g->stored != 0, true)) return rc;
-    const long long N = (long long)g->G.n[0] * g->G.n[1] * g->G.n[2];
-    const unsigned nb = std::min<unsigned>(blocks_for(N, 256), 65535u);
     k_pack<<<nb, 256, 0, g->stream>>>(g->G, g->buf[scratch], g->stage_io, 0, 0);
     SF_HIP(hipGetLastError());
     SF_HIP(hipMemcpyAsync(soa_out, g->stage_io, sizeof(double) * 5 * (size_t)N,
