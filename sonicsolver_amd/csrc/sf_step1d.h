@@ -131,11 +131,17 @@ __global__ __launch_bounds__(64) void k_step_1d(Step1dArgs W) {
         wave_lds_order();
     };
     close_ends();
-    const bool fixed_lo = !periodic && base <= -H, fixed_hi = !periodic && base + 63 >= n - 1 + H;
+    // (of the upper zeroGradient ghosts, all equal, the outermost may lie
+    // beyond lane 63, which then stands for it)
+    const bool fixed_lo = !periodic && base <= -H;
+    const bool fixed_hi = !periodic && base + 63 >= n - 1 + H - G.zg_hi[0];
     const bool inside = periodic || (c >= lo && c <= hi);   // a node the steps advance
     // the tile that owns the last advanced node owns the boundary node, too
     const int to = from_hi ? inner : t;
     const bool own = to >= ST * H && to < ST * H + U && c < n;
+    // lane t's face lies between nodes c and c + 1; those beyond an end's
+    // outer face are no faces of the grid, and what they raise is nobody's
+    const bool face = periodic || (c >= -1 && c < n);
     double dt_next = INFINITY;
     double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};   // RK4: k1 + 2 k2 + 2 k3
 #pragma clang loop unroll(disable)
@@ -179,9 +185,9 @@ __global__ __launch_bounds__(64) void k_step_1d(Step1dArgs W) {
             if (s == ST - 1) dt_next = local_dt(G, q, W.cfl, flags);
         }
         // faces and nodes outside the tile's own range count in the tile
-        // that owns them
-        const bool counts = valid && t >= ST * H - 1 && t < ST * H + U && c < n;
-        if (counts && flags) {
+        // that owns them; the owner of a boundary node owns its outer face
+        const bool raised = valid && face && flags != 0;
+        if (raised && (own || t == ST * H - 1)) {
             atomicMin((unsigned long long*)&ctl->fault.tag, (unsigned long long)(W.tag + s));
             atomicOr(&ctl->fault.stages, flags << (8 * s));
             __threadfence();
@@ -189,7 +195,7 @@ __global__ __launch_bounds__(64) void k_step_1d(Step1dArgs W) {
         }
         // a tile that holds a fault, its own or a neighbour's, stops there:
         // the stages after it would run on what the fault left
-        if (__any(valid && flags != 0)) return;
+        if (__any(raised)) return;
         wave_lds_order();
         close_ends();
     }
