@@ -139,9 +139,13 @@ __global__ __launch_bounds__(64) void k_step_1d(Step1dArgs W) {
     // the tile that owns the last advanced node owns the boundary node, too
     const int to = from_hi ? inner : t;
     const bool own = to >= ST * H && to < ST * H + U && c < n;
-    // lane t's face lies between nodes c and c + 1; those beyond an end's
-    // outer face are no faces of the grid, and what they raise is nobody's
-    const bool face = periodic || (c >= -1 && c < n);
+    // The stages in which this lane's result counts: those that leave its
+    // node's stencil whole.  None beyond an end's outer face: lane t's face
+    // lies between nodes c and c + 1, those further out are no faces of the
+    // grid, and what they raise is nobody's.
+    const int whole = min(fixed_lo ? ST : t / H, fixed_hi ? ST : (63 - t) / H);
+    const int counted = periodic || (c >= -1 && c < n) ? whole : 0;
+    const bool recorded = own || t == ST * H - 1;
     double dt_next = INFINITY;
     double acc[5] = {0.0, 0.0, 0.0, 0.0, 0.0};   // RK4: k1 + 2 k2 + 2 k3
 #pragma clang loop unroll(disable)
@@ -157,9 +161,6 @@ __global__ __launch_bounds__(64) void k_step_1d(Step1dArgs W) {
         double f5[5];
         face_flux<0, SCHEME, FLUX>(st, G.gamma, G.area[0], f5, flags, lw);
         if (!finite_sum5(f5)) flags |= kFlagFlux;
-        // the lanes whose result counts: their node's stencil is whole
-        const int margin = H * (s + 1);
-        const bool valid = (t >= margin || fixed_lo) && (t < 64 - margin || fixed_hi);
         double d5[5];
 #pragma unroll
         for (int v = 0; v < 5; ++v) d5[v] = f5[v] - lane_shift_up1(f5[v]);
@@ -186,8 +187,8 @@ __global__ __launch_bounds__(64) void k_step_1d(Step1dArgs W) {
         }
         // faces and nodes outside the tile's own range count in the tile
         // that owns them; the owner of a boundary node owns its outer face
-        const bool raised = valid && face && flags != 0;
-        if (raised && (own || t == ST * H - 1)) {
+        const bool raised = s < counted && flags != 0;
+        if (raised && recorded) {
             atomicMin((unsigned long long*)&ctl->fault.tag, (unsigned long long)(W.tag + s));
             atomicOr(&ctl->fault.stages, flags << (8 * s));
             __threadfence();
