@@ -97,6 +97,8 @@ struct Fault {
     unsigned flags;
     unsigned stages;   // k_step_1d: the flags raised by stage s at bits 8 s
     long long tag;
+    unsigned before;   // the flags as the last clock launch found them
+    unsigned unused;
 };
 enum { kPhaseFill = 6, kPhaseScan = 7 };
 

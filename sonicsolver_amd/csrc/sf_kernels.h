@@ -75,6 +75,7 @@ __global__ __launch_bounds__(kDtSlots) void k_clock(Control* c, unsigned long lo
                                                     double* dt_hist, int slot, int commit,
                                                     int next_dt, Control* snap) {
     const int t = threadIdx.x;
+    if (t == 0) c->fault.before = c->fault.flags;
     if (!c->fault.flags) {
         if (commit && t == 0) {
             c->clock.time += c->clock.dt;
@@ -232,6 +233,7 @@ __global__ void k_clear_fault(Fault* fault) {
     if (threadIdx.x == 0 && blockIdx.x == 0) {
         fault->flags = 0u;
         fault->stages = 0u;
+        fault->before = 0u;
         fault->tag = -1;
     }
 }

@@ -59,3 +59,60 @@ def test_faces_beyond_an_end_stop_nothing(case, mirror):
     assert np.array_equal(out[0][0], out[1][0])
     assert np.array_equal(out[0][1], out[1][1])
     assert out[0][2] == out[1][2]
+
+
+def _no_pressure_at(q, k):
+    q = q.copy()
+    q[4, k] = -1.0
+    return q
+
+
+@pytest.mark.parametrize("time", ["euler", "ssprk3", "rk4"])
+@pytest.mark.parametrize("node,phase", [(1, 6), (200, 7)])
+def test_a_fault_before_the_run_is_kept(node, phase, time):
+    """Raised by the ghost fill (phase 6) or the CFL scan (7) of the state a
+    run starts from, or by the residual or the scan before the run, a fault
+    stops the run's first step like every launch: flags, step and phase stay
+    as they were recorded, and nothing advances."""
+    n = 401
+    kw, q = wl.riemann_1d(n - 1, (1.0, 0.0, 1.0), (0.5, 0.0, 0.5), 0.5)
+    bad = _no_pressure_at(q, node)
+    desc = make_desc(n=(n, 1, 1), active=(1, 0, 0), d=(kw["d"][0], 1.0, 1.0), time=time)
+
+    def run(g):
+        with pytest.raises(SonicError):
+            g.run(3, 0.4)
+
+    def scan(g):
+        with pytest.raises(SonicError):
+            g.prepare()
+            g.compute_dt(0.4)
+
+    def residual(g):
+        with pytest.raises(SonicError):
+            g.residual()
+
+    for before in (None, scan, residual):
+        got = []
+        for walk in (0, -1):
+            with Grid(desc) as g:
+                g.set_x_walk(walk)
+                g.upload(q)
+                g.run(2, 0.4)
+                g.upload(bad)
+                if before:
+                    before(g)
+                first = g.fault() if before else None
+                run(g)
+                got.append((g.fault(), g.clock(), g.download()[:, 2:-2]))
+                if before:
+                    assert got[-1][0] == first
+                # a sound state runs again from the accumulators left behind
+                g.upload(q)
+                got[-1] += (g.run(4, 0.4), g.download())
+        assert got[0][0] == got[1][0]
+        if before is not residual:
+            assert got[1][0][2] == phase
+        assert got[0][1] == got[1][1]
+        for k in (2, 3, 4):
+            assert np.array_equal(got[0][k], got[1][k])
