@@ -84,8 +84,7 @@ __global__ __launch_bounds__(64) void k_step_1d(Step1dArgs W) {
     for (int v = 0; v < 5; ++v) q0[v] = W.q[v * G.P + start];
     unsigned long long scan = 0;
     if (W.scan) scan = W.scan[t * kDtStride];
-    const unsigned fault_flags = ctl->fault.flags, fault_before = ctl->fault.before;
-    const long long fault_tag = ctl->fault.tag;
+    const unsigned fault_flags = ctl->fault.flags;
     const double clock_dt = ctl->clock.dt, max_dt = ctl->clock.max_dt, limit = ctl->clock.limit;
 #pragma unroll
     for (int v = 0; v < 5; ++v) {
@@ -96,10 +95,14 @@ __global__ __launch_bounds__(64) void k_step_1d(Step1dArgs W) {
     // found (the CFL scan's and the ghost fill's carry the first step's
     // number): keep the step-start state.  A fault that another block raises
     // in this step does not stop this one, so that the record holds the
-    // earliest stage's.
-    if (__builtin_expect(fault_flags != 0, 0) &&
-        (fault_before || (fault_tag >> 3) < (W.tag >> 3)))
-        return;
+    // earliest stage's; which step's it is is read after its flags, as they
+    // are published after the tag.
+    if (__builtin_expect(fault_flags != 0, 0)) {
+        const Fault& f = ctl->fault;
+        (void)__hip_atomic_load(&f.flags, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
+        const long long tag = __hip_atomic_load(&f.tag, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+        if (f.before || (tag >> 3) < (W.tag >> 3)) return;
+    }
     double dt = clock_dt;
     if (W.scan) {
         dt = __longlong_as_double((long long)wave_min_bits(scan));
