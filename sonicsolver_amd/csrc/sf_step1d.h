@@ -122,12 +122,14 @@ __global__ __launch_bounds__(64) void k_step_1d(Step1dArgs W) {
     // take the last advanced node's state with its rebuilt energy
     const bool from_lo = G.zg_lo[0] && c < lo, from_hi = G.zg_hi[0] && c > hi;
     const int inner = from_lo ? lo - base : from_hi ? hi - base : t;
+    unsigned end_flags = 0;
     const auto close_ends = [&] {
         if (from_lo || from_hi) {
             double qi[5];
 #pragma unroll
             for (int v = 0; v < 5; ++v) qi[v] = cur[v][inner];
             const EndEnergy e = end_energy(qi, G.gamma);
+            end_flags = e.ok ? 0u : kFlagState;
             qi[4] = c == lo - 1 || c == hi + 1 ? e.node : e.ghost;
 #pragma unroll
             for (int v = 0; v < 5; ++v) {
@@ -164,7 +166,7 @@ __global__ __launch_bounds__(64) void k_step_1d(Step1dArgs W) {
 #pragma unroll
             for (int v = 0; v < 5; ++v) st[x][v] = cur[v][at];
         }
-        unsigned flags = 0;
+        unsigned flags = end_flags;   // of the end closed before this stage
         double f5[5];
         face_flux<0, SCHEME, FLUX>(st, G.gamma, G.area[0], f5, flags, lw);
         if (!finite_sum5(f5)) flags |= kFlagFlux;
@@ -206,6 +208,11 @@ __global__ __launch_bounds__(64) void k_step_1d(Step1dArgs W) {
         if (__any(raised)) return;
         wave_lds_order();
         close_ends();
+    }
+    if (end_flags && own) {   // of the end closed after the last stage
+        atomicMin((unsigned long long*)&ctl->fault.tag, (unsigned long long)(W.tag + kPhaseFill));
+        __threadfence();
+        atomicOr(&ctl->fault.flags, end_flags);
     }
     if (own) {
         const long long id = node_index(G, c, 0, 0);

@@ -571,7 +571,9 @@ constexpr int kYxWaves = 4, kYxWaveRows = 8;   // blocks of several waves
 
 // Node (i, j, k) at id was advanced to qn: next to a zeroGradient end, write
 // the boundary node and the first ghost layer (which stands for the others,
-// map_node).
+// map_node).  Returns whether the end's pressures are positive, which
+// check_state's test of qn decides alike except where the internal energy is
+// within some ulps of the kinetic energy.
 // Filling the ghosts by launches of their own took four 4-5 us launches per
 // stage in 2D and six in 3D, latency alone: a pass of 20 steps on 853^2 takes
 // 3.51 ms without them and 4.31 with, on 193 x 97 0.83 and 1.87.
@@ -839,7 +841,8 @@ __device__ __forceinline__ void stage_yx_tile(const SweepArgs& W, const Args& ar
             const long long nid = id + i + xo;
             stage_update_dt<TIME>(U.G, U.A, nid, pq, pq0, s5, dt_step, flags, dl, qn);
             const SweepArgs& V = args();
-            write_ends<CORNERS>(V.G, V.A.qout, i, a, k, nid, qn);
+            const bool ends = write_ends<CORNERS>(V.G, V.A.qout, i, a, k, nid, qn);
+            if (!ends && !flags) flags = kFlagState;   // a raised check has stopped the run
             dt_local = fmin(dt_local, dl);
         }
     }
