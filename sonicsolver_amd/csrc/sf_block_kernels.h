@@ -83,7 +83,7 @@ __device__ __forceinline__ void block_yx_tile(const SweepArgs& W, const Args& ar
             }
             unsigned fy = 0;
             face_flux<1, SCHEME, FLUX>(st, W.G.gamma, W.G.area[1], f, fy, lwy);
-            if (!finite_sum5(f)) fy |= kFlagFlux;
+            if (!finite5(f)) fy |= kFlagFlux;
             if (node) flags |= fy;
 #pragma unroll
             for (int v = 0; v < 5; ++v) lds.fy[w][v][t] = f[v];

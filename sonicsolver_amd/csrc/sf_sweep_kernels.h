@@ -779,7 +779,7 @@ __device__ __forceinline__ void stage_yx_tile(const SweepArgs& W, const Args& ar
                         for (int v = 0; v < 5; ++v) b[v] = win[side ? rb : ra][v][t + H - 1];
                     },
                     T.G.gamma, T.G.area[1], f, fy, lwy);
-                if (!finite_sum5(f)) fy |= kFlagFlux;
+                if (!finite5(f)) fy |= kFlagFlux;
             }
             if (WAVES > 1 && a < a0) {
                 if (w > 0) {
