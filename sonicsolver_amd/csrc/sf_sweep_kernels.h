@@ -825,7 +825,9 @@ __device__ __forceinline__ void stage_yx_tile(const SweepArgs& W, const Args& ar
 #pragma unroll
         for (int v = 0; v < 5; ++v) {
             const double up = lane_shift_up1(f5[v]);
-            lower[v] = t == 0 ? first[v][a - a0] : up;
+            // a helper lane's own difference goes unused, and where there is
+            // one nothing wrote the first faces
+            lower[v] = helper == 0 && t == 0 ? first[v][a - a0] : up;
         }
         if (node) {
             const SweepArgs& U = args();
