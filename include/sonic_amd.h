@@ -315,14 +315,14 @@ int sf_batch_memory(const sf_batch *batch, size_t *used_nodes, size_t *free_node
                     int *items);
 /* Tile shape of the stages: tiles of 1D problems of xlen nodes (63, 127 or
  * 255, in strips of 63), of 2D problems of 63 or 64 columns by ylen rows
- * (4..4096; more than 32 count as 32).  Until it is called, both are chosen
- * by cost for the problems that the batch holds.  Takes effect at the next
- * step; results do not depend on it. */
+ * (4..4096; more than 32 count as 32).  0, as until it is called: chosen by
+ * cost for the problems that the batch holds.  Takes effect at the next step;
+ * results do not depend on it. */
 int sf_batch_set_tiles(sf_batch *batch, int xlen, int ylen);
 /* Persistent grid size of the stages in workgroups per compute unit
- * (1..64), or 0 for as many as each stage kernel keeps resident (the
- * runtime's occupancy figure).  Until it is called, every tile has a
- * workgroup of its own.  Results do not depend on it. */
+ * (1..64), 0 for as many as each stage kernel keeps resident (the runtime's
+ * occupancy figure), or -1, as until it is called, for a workgroup per tile.
+ * Results do not depend on it. */
 int sf_batch_set_occupancy(sf_batch *batch, int blocks_per_cu);
 /* Stage schedule: fused != 0 runs one launch per stage for every
  * (scheme, flux) variant (workgroup ranges assigned per variant; one launch
@@ -336,16 +336,18 @@ int sf_batch_set_schedule(sf_batch *batch, int fused);
  * sf_batch_step returns SF_E_NUMERIC. */
 int sf_batch_faults(sf_batch *batch, uint32_t *flags);
 
-/* Launch shape chosen by sf_batch_autotune. */
+/* Launch shape chosen by sf_batch_autotune, in the values of
+ * sf_batch_set_tiles, _occupancy and _schedule. */
 typedef struct {
     int xlen, ylen, blocks_per_cu, fused;
     double ms_per_step;      /* mean step time of the chosen shape            */
-    int candidates;          /* shapes timed                                  */
+    int candidates;          /* shapes timed against the one the batch had    */
 } sf_batch_tuning;
-/* Time every launch shape (schedule, x tile, y tile, persistent grid size)
- * on the admitted problems for trial_steps steps each, from a saved state
- * that is restored after every trial, and keep the fastest.  The problems'
- * states and clocks are unchanged on return. */
+/* Time the launch shape that the batch has and others (schedule, x tile where
+ * it holds 1D problems, y tile where it holds 2D ones, persistent grid size) on
+ * the admitted problems for trial_steps steps each, from a saved state that is
+ * restored after every trial, and keep the fastest.  The problems' states and
+ * clocks are unchanged on return. */
 int sf_batch_autotune(sf_batch *batch, int trial_steps, sf_batch_tuning *out);
 
 #ifdef __cplusplus

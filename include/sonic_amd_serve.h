@@ -69,8 +69,8 @@ int sf_server_drain(sf_server *server, double timeout_s);
 int sf_server_stats(sf_server *server, sf_serve_stats *stats);
 /* Launch shape of the batch (as sf_batch_set_tiles / _occupancy /
  * _schedule); applied before the loop's next pass.  Without a call the
- * batch's defaults hold: tile lengths chosen by cost for the problems it
- * holds, a workgroup per tile, one launch for every variant. */
+ * batch's defaults hold (0, 0, -1, 1): tile lengths chosen by cost for the
+ * problems it holds, a workgroup per tile, one launch for every variant. */
 int sf_server_set_shape(sf_server *server, int xlen, int ylen, int blocks_per_cu, int fused);
 /* How each pass launches its steps, as sf_batch_step's use_graph: 0 direct
  * launches, 1 replayed hipGraphs, 2 (the default) the library's choice.

@@ -188,8 +188,9 @@ class Batch:
         return out
 
     def autotune(self, trial_steps: int = 3) -> dict:
-        """Time every launch shape on the admitted problems and keep the
-        fastest; the problems' states and clocks are left unchanged."""
+        """Time the launch shape that the batch has and others on the admitted
+        problems and keep the fastest; the problems' states and clocks are left
+        unchanged."""
         t = Tuning()
         _check(self._lib.sf_batch_autotune(self._h, int(trial_steps), ctypes.byref(t)))
         return {name: getattr(t, name) for name, _ in t._fields_}

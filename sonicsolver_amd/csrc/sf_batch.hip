@@ -941,9 +941,10 @@ int sf_batch_memory(const sf_batch* b, size_t* used_nodes, size_t* free_nodes, i
 
 int sf_batch_set_tiles(sf_batch* b, int xlen, int ylen) {
     if (!b) return bfail(SF_E_ARG, "sf_batch_set_tiles: null batch");
-    if (xlen != 63 && xlen != 127 && xlen != 255)
-        return bfail(SF_E_ARG, "sf_batch_set_tiles: x tile must be 63, 127 or 255 nodes");
-    if (ylen < 4 || ylen > 4096) return bfail(SF_E_ARG, "sf_batch_set_tiles: y tile out of range");
+    if (xlen != 0 && xlen != 63 && xlen != 127 && xlen != 255)
+        return bfail(SF_E_ARG, "sf_batch_set_tiles: x tile must be 63, 127 or 255 nodes, or 0");
+    if (ylen != 0 && (ylen < 4 || ylen > 4096))
+        return bfail(SF_E_ARG, "sf_batch_set_tiles: y tile out of range");
     b->xlen = xlen;
     b->ylen = ylen;
     b->tables_dirty = true;
@@ -953,10 +954,13 @@ int sf_batch_set_tiles(sf_batch* b, int xlen, int ylen) {
 }  // extern "C"
 
 // ---- autotuner ----------------------------------------------------------------
-// Times every launch shape (schedule x x-tile x y-tile x persistent grid
-// size) on the batch's own problems: each trial takes the same steps
-// from the same saved state, which is restored afterwards, so tuning leaves
-// the problems exactly as it found them.
+// Times launch shapes (schedule x x-tile x y-tile x persistent grid size) on
+// the batch's own problems: each trial takes the same steps from the same
+// saved state, which is restored afterwards, so tuning leaves the problems
+// exactly as it found them.  The shape that the batch has, the automatic one
+// unless it was set, is timed first and kept unless another is faster; what
+// the batch holds no problems for keeps its setting.  Trials launch directly:
+// a captured graph would be charged with its capture.
 namespace {
 
 struct Snapshot {
@@ -1011,13 +1015,13 @@ int snapshot_restore(sf_batch* b, const Snapshot& sn) {
 int time_shape(sf_batch* b, int steps, double* ms) {
     if (b->tables_dirty)
         if (int rc = rebuild_tables(b)) return rc;
-    if (int rc = advance(b, 1, 1)) return rc;
+    if (int rc = advance(b, 1, 0)) return rc;
     hipEvent_t e0 = nullptr, e1 = nullptr;
     SF_BHIP(hipEventCreate(&e0));
     SF_BHIP(hipEventCreate(&e1));
     int rc = 0;
     if (hipEventRecord(e0, b->stream) != hipSuccess) rc = bfail(SF_E_HIP, "event record failed");
-    if (!rc) rc = advance(b, steps, 1);
+    if (!rc) rc = advance(b, steps, 0);
     if (!rc && hipEventRecord(e1, b->stream) != hipSuccess)
         rc = bfail(SF_E_HIP, "event record failed");
     if (!rc && hipEventSynchronize(e1) != hipSuccess) rc = bfail(SF_E_HIP, "event wait failed");
@@ -1041,52 +1045,42 @@ extern "C" int sf_batch_autotune(sf_batch* b, int trial_steps, sf_batch_tuning* 
     if (b->nactive == 0) return bfail(SF_E_STATE, "sf_batch_autotune: the batch is empty");
     Snapshot sn;
     int rc = snapshot_save(b, sn);
-    const int keep[4] = {b->xlen, b->ylen, b->blocks_per_cu, b->fused};
-    sf_batch_tuning best{};
-    best.ms_per_step = 1e300;
+    using Shape = sf_batch_tuning;
+    const auto set = [&](const Shape& sh) {
+        b->xlen = sh.xlen;
+        b->ylen = sh.ylen;
+        b->blocks_per_cu = sh.blocks_per_cu;
+        b->fused = sh.fused;
+        b->tables_dirty = true;
+    };
+    const auto timed = [&](Shape& sh) {
+        set(sh);
+        if (int e = time_shape(b, trial_steps, &sh.ms_per_step)) return e;
+        return snapshot_restore(b, sn);
+    };
+    const Shape own{b->xlen, b->ylen, b->blocks_per_cu, b->fused, 0.0, 0};
+    Shape best = own;
+    if (!rc) rc = timed(best);
+    bool any1d = false;
+    for (int s = 0; s < b->item_capacity; ++s) any1d = any1d || (b->used[s] && b->items[s].n1 == 1);
     int tried = 0;
-    const int xlens[3] = {63, 127, 255};
-    const int occs[5] = {0, 2, 4, 8, 16};   // 0: as many as stay resident
-    std::vector<int> ysegs = b->any2d ? std::vector<int>{8, 16, 32}
-                                     : std::vector<int>{std::max(b->ylen, 4)};
+    const std::vector<int> xlens = any1d ? std::vector<int>{63, 127, 255} : std::vector<int>{own.xlen};
+    const std::vector<int> ylens = b->any2d ? std::vector<int>{8, 16, 32} : std::vector<int>{own.ylen};
     for (int fused = 0; fused < 2 && !rc; ++fused)
         for (int xl : xlens)
-            for (int ys : ysegs)
-                for (int oc : occs) {
+            for (int yl : ylens)
+                for (int oc : {0, 2, 4, 8, 16}) {   // 0: as many as stay resident
                     if (rc) break;
-                    b->fused = fused;
-                    b->xlen = xl;
-                    b->ylen = ys;
-                    b->blocks_per_cu = oc;
-                    b->tables_dirty = true;
-                    double ms = 0.0;
-                    rc = time_shape(b, trial_steps, &ms);
-                    if (!rc) rc = snapshot_restore(b, sn);
+                    Shape sh{xl, yl, oc, fused, 0.0, 0};
+                    rc = timed(sh);
                     if (rc) break;
                     ++tried;
-                    if (ms < best.ms_per_step) {
-                        best.xlen = xl;
-                        best.ylen = ys;
-                        best.blocks_per_cu = oc;
-                        best.fused = fused;
-                        best.ms_per_step = ms;
-                    }
+                    if (sh.ms_per_step < best.ms_per_step) best = sh;
                 }
     if (sn.q) (void)hipFree(sn.q);
-    if (rc) {
-        b->xlen = keep[0];
-        b->ylen = keep[1];
-        b->blocks_per_cu = keep[2];
-        b->fused = keep[3];
-        b->tables_dirty = true;
-        return rc;
-    }
+    set(rc ? own : best);
+    if (rc) return rc;
     best.candidates = tried;
-    b->xlen = best.xlen;
-    b->ylen = best.ylen;
-    b->blocks_per_cu = best.blocks_per_cu;
-    b->fused = best.fused;
-    b->tables_dirty = true;
     *out = best;
     return 0;
 }
@@ -1100,10 +1094,10 @@ extern "C" int sf_batch_set_schedule(sf_batch* b, int fused) {
 
 extern "C" int sf_batch_set_occupancy(sf_batch* b, int blocks_per_cu) {
     if (!b) return bfail(SF_E_ARG, "sf_batch_set_occupancy: null batch");
-    if (blocks_per_cu < 0 || blocks_per_cu > 64)
+    if (blocks_per_cu < -1 || blocks_per_cu > 64)
         return bfail(SF_E_ARG,
-                     "sf_batch_set_occupancy: 1..64 workgroups per compute unit, or 0 for "
-                     "as many as stay resident");
+                     "sf_batch_set_occupancy: 1..64 workgroups per compute unit, 0 for as "
+                     "many as stay resident, or -1 for one per tile");
     b->blocks_per_cu = blocks_per_cu;
     drop_graph(b);
     return 0;

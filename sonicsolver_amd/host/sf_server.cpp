@@ -98,7 +98,7 @@ struct sf_server {
     Clock::time_point first_submit, last_done;
 
     bool shape_pending = false;
-    int shape[4] = {255, 32, 16, 0};   // xlen, ylen, blocks per CU, fused
+    int shape[4] = {0, 0, -1, 1};      // xlen, ylen, blocks per CU, fused
     int launch = 2;                      // sf_batch_step's use_graph
 
     // loop thread only
@@ -535,8 +535,8 @@ int sf_server_stats(sf_server* s, sf_serve_stats* st) {
 
 int sf_server_set_shape(sf_server* s, int xlen, int ylen, int blocks_per_cu, int fused) {
     if (!s) return fail(SF_E_ARG, "sf_server_set_shape: null server");
-    if ((xlen != 63 && xlen != 127 && xlen != 255) || ylen < 4 || ylen > 4096 ||
-        blocks_per_cu < 0 || blocks_per_cu > 64)
+    if ((xlen != 0 && xlen != 63 && xlen != 127 && xlen != 255) ||
+        (ylen != 0 && (ylen < 4 || ylen > 4096)) || blocks_per_cu < -1 || blocks_per_cu > 64)
         return fail(SF_E_ARG, "sf_server_set_shape: shape out of range (see sf_batch_set_tiles)");
     std::lock_guard<std::mutex> lk(s->mu);
     s->shape[0] = xlen;
