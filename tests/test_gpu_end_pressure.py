@@ -16,7 +16,7 @@ pytestmark = pytest.mark.gpu
 def _state(rng, n):
     N = int(np.prod(n))
     rho = 1 + 0.3 * rng.random(N)
-    u, v = 3 + rng.random(N), 0.5 * rng.normal(size=N) * (len(n) > 1)
+    u, v = 3 + rng.random(N), 0.5 * rng.normal(size=N)
     p = 0.5 + 0.5 * rng.random(N)
     return np.stack([rho, rho * u, rho * v, 0 * u, p / 0.4 + 0.5 * rho * (u * u + v * v)])
 
@@ -31,7 +31,7 @@ def _fault(g, q, dt):
     return g.fault()
 
 
-@pytest.mark.parametrize("n,seeds", [((12, 10), 60), ((40,), 150), ((9, 7, 6), 60)])
+@pytest.mark.parametrize("n,seeds", [((12, 10), 150), ((40,), 150), ((9, 7, 6), 60)])
 def test_fused_launches_refuse_what_the_fill_refuses(n, seeds):
     desc = make_desc(n=n, bc=("transmissive",) * 3, d=(0.1,) * len(n) + (1.0,) * (3 - len(n)),
                      scheme="weno5", flux="hllc", time="euler")
