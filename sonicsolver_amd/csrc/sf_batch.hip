@@ -72,7 +72,7 @@ __global__ __launch_bounds__(256) void k_batch_prepare(BatchDev B, const int* __
 #pragma unroll
         for (int v = 0; v < 5; ++v) qq[v] = q[v * G.P + id];
         best = fmin(best, local_dt(G, qq, W.A.cfl, flags));
-        if (!write_ends<true>(G, q, i, j, 0, id, qq)) flags |= kFlagState;
+        write_ends<true>(G, q, i, j, 0, id, qq, flags);
     }
     if (flags) atomicOr(&B.flags[slot], flags);
     const unsigned long long b = wave_min_bits(

@@ -161,8 +161,7 @@ __device__ __forceinline__ void line_tiles(const BatchStage& B, double (&row)[5]
                 const long long id = i + V.G.xo;
                 stage_update_dt<SF_TIME_SSPRK3>(V.G, V.A, id, pq, pq0, s5, dt_step, flags, dl, qn);
                 const SweepArgs& X = args();
-                const bool ends = write_ends(X.G, X.A.qout, i, 0, 0, id, qn);
-                if (!ends && !flags) flags = kFlagState;   // a raised check has stopped the run
+                write_ends<false, false>(X.G, X.A.qout, i, 0, 0, id, qn, flags);
                 dt_local = fmin(dt_local, dl);
             }
         }

@@ -154,8 +154,7 @@ __device__ __forceinline__ void block_yx_tile(const SweepArgs& W, const Args& ar
             for (int v = 0; v < 5; ++v) pq[v] = st[H - 1][v];
             stage_update_dt<TIME>(U.G, U.A, nid, pq, pq0, s5, dt_step, flags, dl, qn);
             const SweepArgs& V = args();
-            const bool ends = write_ends<CORNERS>(V.G, V.A.qout, i, a, k, nid, qn);
-            if (!ends && !flags) flags = kFlagState;   // a raised check has stopped the run
+            write_ends<CORNERS>(V.G, V.A.qout, i, a, k, nid, qn, flags);
             dt_local = dl;
         }
     }

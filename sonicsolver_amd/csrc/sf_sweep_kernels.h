@@ -571,22 +571,26 @@ constexpr int kYxWaves = 4, kYxWaveRows = 8;   // blocks of several waves
 
 // Node (i, j, k) at id was advanced to qn: next to a zeroGradient end, write
 // the boundary node and the first ghost layer (which stands for the others,
-// map_node).  Returns whether the end's pressures are positive, which
-// check_state's test of qn decides alike except where the internal energy is
-// within some ulps of the kinetic energy.
+// map_node).  Raises kFlagState where the end's pressures are not positive,
+// which check_state's test of qn decides alike except where the internal
+// energy is within some ulps of the kinetic energy.  RUN: only where no check
+// is raised already, which stops a grid's run; a batch's problem finishes its
+// step.
 // Filling the ghosts by launches of their own took four 4-5 us launches per
 // stage in 2D and six in 3D, latency alone: a pass of 20 steps on 853^2 takes
 // 3.51 ms without them and 4.31 with, on 193 x 97 0.83 and 1.87.
-template <bool CORNERS = false>
-__device__ __forceinline__ bool write_ends(const GridDev& G, double* __restrict__ out, int i,
-                                           int j, int k, long long id, const double qn[5]) {
+template <bool CORNERS = false, bool RUN = !CORNERS>
+__device__ __forceinline__ void write_ends(const GridDev& G, double* __restrict__ out, int i,
+                                           int j, int k, long long id, const double qn[5],
+                                           unsigned& flags) {
     const int c[3] = {i, j, k};
     bool at_end = false;
 #pragma unroll
     for (int a = 0; a < 3; ++a)
         at_end |= (G.zg_lo[a] && c[a] == G.solved_lo[a]) || (G.zg_hi[a] && c[a] == G.solved_hi[a]);
-    if (!at_end) return true;
+    if (!at_end) return;
     const EndEnergy e = end_energy(qn, G.gamma);
+    if (!e.ok && !(RUN && flags)) flags |= kFlagState;
 #pragma unroll
     for (int a = 0; a < 3; ++a)
 #pragma unroll
@@ -613,7 +617,6 @@ __device__ __forceinline__ bool write_ends(const GridDev& G, double* __restrict_
             for (int v = 0; v < 5; ++v) out[v * G.P + at] = v == 4 ? e.node : qn[v];
         }
     }
-    return e.ok;
 }
 
 // Orders the LDS accesses of a wave's lanes among themselves: the hardware
@@ -843,8 +846,7 @@ __device__ __forceinline__ void stage_yx_tile(const SweepArgs& W, const Args& ar
             const long long nid = id + i + xo;
             stage_update_dt<TIME>(U.G, U.A, nid, pq, pq0, s5, dt_step, flags, dl, qn);
             const SweepArgs& V = args();
-            const bool ends = write_ends<CORNERS>(V.G, V.A.qout, i, a, k, nid, qn);
-            if (!ends && !flags) flags = kFlagState;   // a raised check has stopped the run
+            write_ends<CORNERS>(V.G, V.A.qout, i, a, k, nid, qn, flags);
             dt_local = fmin(dt_local, dl);
         }
     }
