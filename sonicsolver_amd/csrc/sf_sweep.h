@@ -102,15 +102,16 @@ int launch_sweep_fm(const SweepCall& c, int axis) {
         if constexpr (MODE != kFinal) {
             return -1;
         } else {
-            // Grids with at least 256 x lines per CU (16 lines for every
-            // wave slot at four waves per SIMD) walk whole lines
-            // (k_sweep_xl): 512^3 ran its x sweep in 5.03 ms against 5.59
-            // with the flattened tiles, 256^3 in 0.67 against 0.77 with
-            // WENO5/HLLC, 0.67 against 0.77 with WENO5/Steger-Warming, 0.82
-            // against 1.03 with TENO5/HLLC, 1.21 against 1.44 with
-            // WENO7/HLLC and 0.72 against 0.77 with WENO3/HLLC; 2D grids and
-            // smaller 3D ones, with too few lines to fill the device, keep
-            // the tiles.
+            // What comes here (yx_shape): residuals, 1D grids, 2D and 3D ones
+            // narrower than 32 nodes that fill the device, and a chosen walk.
+            // Grids of 64 columns and at least 256 x lines per CU (16 for
+            // every wave slot at four waves per SIMD) walk whole lines, which
+            // by itself only residuals of large grids do: their x sweep on
+            // 256^3 takes 0.49 ms against 0.53 with the flattened tiles with
+            // WENO5/HLLC, 0.74 against 0.81 with TENO5, 0.78 against 0.85 with
+            // WENO7, 0.47 against 0.51 with WENO3, on 384^3 2.30 against 2.43;
+            // with too few lines to fill the device, on 128^3, 0.078 against
+            // 0.074.
             // The line walk addresses a lane's stage operands by a 32-bit
             // byte offset of up to one variable (8 P bytes) past the tile.
             const SweepArgs W{G, c.q, c.S, c.A};
@@ -307,7 +308,9 @@ inline YxShape block_shape(int nx, int ny, int nz, int cus) {
 // Blocks of four waves: 853^2 2.94 -> 2.83 ms a pass of 20 steps, 600^2 1.82
 // -> 1.71, 64^3 2.49 -> 2.38, 1000^2 (10 steps) 2.03 -> 1.94, 900^2 with
 // TENO5/HLLC 2.45 -> 2.37; with the long tiles of the largest grids there is
-// little to share, and they take one (512^3 71.6 ms, 72.9 with four).
+// little to share, and they take one (512^3 71.6 ms, 72.9 with four; on
+// 2048^2 with TENO5/HLLC four waves of eight rows take 5.06 against the 5.13
+// of the long single ones, which the cost does not see).
 //
 // Small grids take k_block_yx, up to the number of waves per SIMD at which it
 // stays ahead of the march with every scheme: 8 in 2D (400^2, passes of 20

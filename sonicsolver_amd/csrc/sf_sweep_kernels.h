@@ -22,7 +22,7 @@ constexpr int kXBlock = 64;
 
 // The x sweeps' arguments, and the wave's own view of them in the kernel
 // argument segment.  A sweep has about 90 uniform values (variable pointers,
-// grid constants, ranges of ghost copies); held across the tile loop they
+// grid constants, the ranges of its ends); held across the tile loop they
 // exceed the scalar registers, and each restored one costs a v_readlane in
 // the loop that the FP64 pipe is waiting for (90 of an x line tile's 880
 // vector instructions).  sweep_args() hides where its pointer comes from, so
